@@ -1,0 +1,372 @@
+// CSR SpMM in 16-lane groups for gfx950 (wave64): C = alpha*A*B + beta*C with contiguous rows of B.
+//
+// Sixteen lanes -- one DPP row -- own one row of A and up to 256 bytes of dense columns; a wave takes four rows, so one
+// 128-bit load instruction fetches four rows of B.  The group reads sixteen entries of its row with one coalesced
+// load; every lane turns its entry's column into the byte offset of that row of B once, and the entries go round
+// the group with DPP broadcasts inside the address addition and the multiply-adds -- no LDS crossbar (whose
+// ds_bpermutes alone held the kernel this one replaced at 0.31 ms on a 27-point stencil of 2^20 rows, n = 64) and no
+// 64-bit address arithmetic in the entry loop.  GC lanes cover the dense columns of a chunk; where they are fewer than
+// sixteen the group's 16 / GC parts take every (16 / GC)-th entry and their sums meet at the end.
+//
+// What bounds it: random columns, the L2-miss path (whole 128-byte lines at about 7 TB/s); columns that neighbouring
+// rows share, the L1-to-register path (64 bytes per clock and compute unit).
+#pragma once
+
+#include <utility>
+
+#include "device_utils.hpp"
+
+namespace asamd {
+
+constexpr int kGroupThreads = 256;
+constexpr int kGroupRows = kGroupThreads / 16;  // rows of A that a workgroup has in work at one time
+constexpr int kGroupBytes = 256;                // dense columns of one chunk, in bytes
+// A row of more entries than this is taken by all sixteen groups of the workgroup together: one group would hold the
+// workgroup up (a power-law graph of 0.7 M rows, longest row 16 727, complex64, n = 11: 3.55 ms with a lane group per
+// row whatever its length).
+constexpr int kGroupLongRow = 256;
+constexpr unsigned kGroupNoRow = 0x80000000u;  // an offset that the buffer's range check turns away (B within 2 GiB)
+
+template <typename T>
+constexpr int kGroupV = 16 / (int)sizeof(T);  // elements of one 128-bit load
+
+template <typename T>
+struct GroupVec {
+  T e[kGroupV<T>];
+};
+// the same in memory, where only the element's own alignment is known (wide global accesses may be unaligned)
+template <typename T>
+struct __attribute__((packed, aligned(alignof(T) < 8 ? alignof(T) : 8))) GroupLoose {
+  unsigned w[4];
+};
+
+// value of lane J of the caller's part of GC lanes (a DPP row holds 16 / GC parts)
+template <int GC, int J>
+__device__ __forceinline__ int part_bcast(int v, bool upper) {
+  if constexpr (GC == 16) {
+    return __builtin_amdgcn_update_dpp(0, v, 0x150 + J, 0xF, 0xF, true);  // row_newbcast:J
+  } else if constexpr (GC == 8) {
+    const int lo = __builtin_amdgcn_update_dpp(0, v, 0x150 + J, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, v, 0x158 + J, 0xF, 0xF, true);
+    return upper ? hi : lo;
+  } else {
+    static_assert(GC == 4, "four, eight or sixteen column lanes");
+    return __builtin_amdgcn_update_dpp(0, v, J * 0x55, 0xF, 0xF, true);  // quad_perm:[J,J,J,J]
+  }
+}
+template <int GC, int J, typename T>
+__device__ __forceinline__ T part_bcast_t(T v, bool upper) {
+  struct Words { int w[sizeof(T) / 4]; };
+  Words a = __builtin_bit_cast(Words, v);
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(T) / 4); ++i) a.w[i] = part_bcast<GC, J>(a.w[i], upper);
+  return __builtin_bit_cast(T, a);
+}
+
+// lanes of a wave whose position in their part of GC lanes is in [lo, hi)
+template <int GC>
+constexpr uint64_t part_lanes(int lo, int hi) {
+  uint64_t m = 0;
+  for (int l = 0; l < 64; ++l)
+    if (l % GC >= lo && l % GC < hi) m |= (uint64_t)1 << l;
+  return m;
+}
+
+// f(0), f(1), ... with compile-time numbers
+template <typename F, int... U>
+__device__ __forceinline__ void for_each_const(F& f, std::integer_sequence<int, U...>) {
+  (f(std::integral_constant<int, U>{}), ...);
+}
+
+// where a lane's L pieces of a row of B lie
+template <bool NARROW, int L>
+struct GroupB {
+  BufferRsrc rsrc;         // NARROW: all of B, within 2 GiB
+  const char* p;           // otherwise: the chunk's first column of row 0
+  unsigned lane_bytes[L];  // the lane's pieces of row 0 there, in bytes
+  int64_t row_bytes;
+};
+
+// One block of sixteen entries of a row, an entry per lane: lane l of a group holds entry part + S * (place in the part),
+// so that step j of part p takes entry p + S j of the block.  Kept as loaded until the block is worked on: arithmetic on it
+// here would wait for the loads.
+template <typename T>
+struct GroupBlock {
+  T val;
+  int col;
+  bool live;
+};
+
+template <typename T, int GC>
+__device__ __forceinline__ GroupBlock<T> group_fetch(int64_t j0, int64_t end, const T* __restrict__ val,
+                                                     const int* __restrict__ col_ind) {
+  const int l16 = threadIdx.x & 15;
+  const int64_t j = j0 + l16 / GC + (16 / GC) * (l16 % GC);
+  GroupBlock<T> e;
+  e.live = j < end;
+  // Every lane loads, the ones past the end entry 0 (there is one): a load under a branch would be waited for where the
+  // branches meet.  (Not non-temporally: a block is half a cache line of column numbers, and the line's other half is the
+  // row's next block.  2^20 rows of 32 random entries, n = 64: 1.29 -> 1.24 ms.)
+  e.col = col_ind[e.live ? j : 0];
+  e.val = val[e.live ? j : 0];
+  return e;
+}
+
+// acc += a block's entries times the lane's columns of B; all lanes of the wave come here together
+template <typename T, int GC, bool NARROW, int L, bool FAR>
+__device__ __forceinline__ void group_work(const GroupBlock<T>& e, T alpha, int base, const GroupB<NARROW, L>& b,
+                                           T (&acc)[L * kGroupV<T>]) {
+  constexpr int V = kGroupV<T>;
+  const bool upper = GC == 8 && (threadIdx.x & 8);
+  const uint64_t mask = __builtin_amdgcn_ballot_w64(e.live);
+  const T weight = e.live ? alpha * e.val : T(0);
+  unsigned off = kGroupNoRow;
+  int off_hi = 0;
+  if constexpr (NARROW) {
+    if (e.live) off = (unsigned)(e.col - base) * (unsigned)b.row_bytes;
+  } else {
+    const int64_t o = e.live ? (int64_t)(e.col - base) * b.row_bytes : 0;
+    off = (unsigned)o;
+    off_hi = (int)(o >> 32);
+  }
+  auto steps = [&](auto first, auto count) {
+    constexpr int J0 = decltype(first)::value, N = decltype(count)::value;
+    GroupVec<T> bv[N][L];
+    bool has[N];
+    auto load = [&](auto u) {
+      constexpr int U = decltype(u)::value;
+      const unsigned lo = (unsigned)part_bcast<GC, J0 + U>((int)off, upper);
+      if constexpr (NARROW) {
+#pragma unroll
+        for (int q = 0; q < L; ++q) bv[U][q] = buffer_load<GroupVec<T>>(b.rsrc, (int)(lo + b.lane_bytes[q]));
+      } else {
+        has[U] = part_bcast<GC, J0 + U>((int)e.live, upper) != 0;
+        const int hi = part_bcast<GC, J0 + U>(off_hi, upper);
+        if (has[U]) {
+#pragma unroll
+          for (int q = 0; q < L; ++q)
+            bv[U][q] = __builtin_bit_cast(
+                GroupVec<T>, *reinterpret_cast<const GroupLoose<T>*>(b.p + (((int64_t)hi << 32) | lo) + b.lane_bytes[q]));
+        }
+      }
+    };
+    auto add = [&](auto u) {
+      constexpr int U = decltype(u)::value;
+      const T w = part_bcast_t<GC, J0 + U>(weight, upper);
+      // (a lane group whose row has ended adds 0 * 0: its offset was turned away)
+      if (NARROW || has[U]) {
+#pragma unroll
+        for (int q = 0; q < L; ++q) {
+#pragma unroll
+          for (int i = 0; i < V; ++i) acc[q * V + i] = fma_t(w, bv[U][q].e[i], acc[q * V + i]);
+        }
+      }
+    };
+    for_each_const(load, std::make_integer_sequence<int, N>{});
+    for_each_const(add, std::make_integer_sequence<int, N>{});
+  };
+  // Loads in flight per wave: four (eight took 20 registers more and were no faster).  FAR: one at a time where most lanes
+  // have an entry and neighbouring rows begin far apart: the L2-miss path is full either way, and fewer requests
+  // in it go faster (2^20 rows of 32 random entries, fp32, n = 64: 1.26 -> 1.21 ms; chunks
+  // of two loads a lane have as many lines in flight by themselves, 438 520 rows of 21 entries, fp64, n = 63: 0.69 -> 0.65;
+  // rows of few entries and B within
+  // the caches are latency-bound and lose up to a third).
+  if constexpr (FAR) {
+    const int c0 = __builtin_amdgcn_readlane(e.col, 0), c1 = __builtin_amdgcn_readlane(e.col, 16);
+    const int c2 = __builtin_amdgcn_readlane(e.col, 32), c3 = __builtin_amdgcn_readlane(e.col, 48);
+    if (__builtin_popcountll(mask) >= 48 && (unsigned)(c1 - c0 + 256) > 512u && (unsigned)(c3 - c2 + 256) > 512u) {
+      auto one = [&](auto j) { steps(j, std::integral_constant<int, 1>{}); };
+      for_each_const(one, std::make_integer_sequence<int, GC>{});
+      return;
+    }
+  }
+  auto four = [&](auto q) {
+    constexpr int J = 4 * decltype(q)::value;
+    if (mask & part_lanes<GC>(J, J + 4)) steps(std::integral_constant<int, J>{}, std::integral_constant<int, 4>{});
+  };
+  for_each_const(four, std::make_integer_sequence<int, GC / 4>{});
+}
+
+// acc += the entries [j0, end) of a row, every group with a range of its own; the parts' sums are not yet joined
+template <typename T, int GC, bool NARROW, int L, bool FAR>
+__device__ __forceinline__ void group_walk(int64_t j0, int64_t end, T alpha, const T* __restrict__ val,
+                                           const int* __restrict__ col_ind, int base, const GroupB<NARROW, L>& b,
+                                           T (&acc)[L * kGroupV<T>]) {
+  GroupBlock<T> cur = group_fetch<T, GC>(j0, end, val, col_ind);
+  while (__builtin_amdgcn_ballot_w64(j0 + 16 < end)) {  // the next sixteen travel while these are worked on
+    j0 += 16;
+    const GroupBlock<T> next = group_fetch<T, GC>(j0, end, val, col_ind);
+    group_work<T, GC, NARROW, L, FAR>(cur, alpha, base, b, acc);
+    cur = next;
+  }
+  group_work<T, GC, NARROW, L, FAR>(cur, alpha, base, b, acc);
+}
+
+// every part of the group receives the sum over the parts
+template <int GC, typename T, int N>
+__device__ __forceinline__ void group_join(T (&acc)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    if constexpr (GC <= 8) acc[i] += dpp_mov<0x128>(acc[i]);  // row_ror:8
+    if constexpr (GC <= 4) acc[i] += dpp_mov<0x124>(acc[i]);  // row_ror:4
+  }
+}
+
+typedef int Loose4 __attribute__((ext_vector_type(4), aligned(4)));
+
+// the V columns from c on, but not the first `first` of them; nt: C bypasses the caches
+template <typename T>
+__device__ __forceinline__ void group_store_row(T* __restrict__ c, int first, const T* acc, T beta, bool nt) {
+  constexpr int V = kGroupV<T>;
+  if (first == 0) {
+    GroupVec<T> out;
+    if (beta == T(0)) {
+#pragma unroll
+      for (int i = 0; i < V; ++i) out.e[i] = acc[i];
+    } else {
+      const Loose4* p = reinterpret_cast<const Loose4*>(c);
+      const GroupVec<T> old = __builtin_bit_cast(GroupVec<T>, nt ? __builtin_nontemporal_load(p) : *p);
+#pragma unroll
+      for (int i = 0; i < V; ++i) out.e[i] = old.e[i] * beta + acc[i];
+    }
+    if (nt) __builtin_nontemporal_store(__builtin_bit_cast(Loose4, out), reinterpret_cast<Loose4*>(c));
+    else *reinterpret_cast<Loose4*>(c) = __builtin_bit_cast(Loose4, out);
+  } else {
+#pragma unroll
+    for (int i = 1; i < V; ++i)
+      if (i >= first) c[i] = beta == T(0) ? acc[i] : c[i] * beta + acc[i];
+  }
+}
+
+// grid.x: blocks of kGroupRows rows (COLC: kWave); grid.y: chunks of `chunk` dense columns, chunk y at
+// B + y * b_chunk_bytes (b_bytes: what may be read from B on, NARROW only).  ldb in elements; C element (r, c) at
+// r * c_row + c * c_col (one of the two strides is 1: COLC when it is the rows').  b_padded: 16 bytes behind every row of
+// B may be read (a layout made here); otherwise n is at least kGroupV<T>.  L: 128-bit loads per lane and row of B, the
+// chunk's columns [q * GC * V, (q + 1) * GC * V) in load q.  c_nt: row-major C, which is touched once, bypasses the caches.
+// FAR: see group_work.
+template <typename T, int GC, bool NARROW, bool COLC, int L, bool FAR>
+__global__ __launch_bounds__(kGroupThreads) void spmm_group_kernel(
+    int m, int n, T alpha, const T* __restrict__ val, const int* __restrict__ row_ptr, const int* __restrict__ col_ind,
+    int base, const T* __restrict__ B, int64_t ldb, int64_t b_chunk_bytes, unsigned b_bytes, bool b_padded, T beta,
+    T* __restrict__ C, int64_t c_row, int64_t c_col, int chunk, bool c_nt) {
+  constexpr int V = kGroupV<T>;
+  constexpr int kCols = GC * V;
+  constexpr int kTileRows = COLC ? kWave : kGroupRows;
+  __shared__ T s_part[kGroupRows * kCols * L];          // the groups' sums of a long row
+  __shared__ T s_tile[COLC ? kCols * (kWave + 1) : 1];  // COLC: the rows' sums, column by column
+  __shared__ int s_ptr[kTileRows + 1];
+  static_assert(!COLC || L == 1, "column-major C with one load per lane");
+  const unsigned bid = xcd_contiguous_id(blockIdx.x, gridDim.x);
+  const int64_t row0 = (int64_t)bid * kTileRows;
+  const int nrows = m - row0 < kTileRows ? (int)(m - row0) : kTileRows;
+  if (threadIdx.x <= nrows) s_ptr[threadIdx.x] = row_ptr[row0 + threadIdx.x];
+  const int group = threadIdx.x / 16;
+  const int lane = threadIdx.x % kWave;
+  const int cl = threadIdx.x % GC;
+  const int cbeg = blockIdx.y * chunk;
+  const int cn = n - cbeg < chunk ? n - cbeg : chunk;
+  // the lane's columns: V from c0 on; the last lane's are moved back where the chunk ends inside them (`first`: how many
+  // of them its neighbour has as well), lanes past the end load what lane 0 loads and store nothing
+  int c0[L], first[L];
+  bool owns[L];
+  GroupB<NARROW, L> b;
+  if constexpr (NARROW) b.rsrc = make_rsrc(B, (int)b_bytes);
+  b.p = reinterpret_cast<const char*>(B) + (int64_t)blockIdx.y * b_chunk_bytes;
+  b.row_bytes = ldb * (int64_t)sizeof(T);
+#pragma unroll
+  for (int q = 0; q < L; ++q) {
+    c0[q] = q * kCols + cl * V;
+    first[q] = 0;
+    owns[q] = c0[q] < cn && threadIdx.x % 16 < GC;
+    if (c0[q] >= cn) {
+      c0[q] = 0;
+    } else if (c0[q] + V > cn && !b_padded) {
+      first[q] = c0[q] + V - cn;
+      c0[q] = cn - V;
+    }
+    // (relative to B, not to the chunk: the columns moved back may lie in the chunk before)
+    const int64_t at = (NARROW ? (int64_t)blockIdx.y * b_chunk_bytes : 0) + (int64_t)c0[q] * (int64_t)sizeof(T);
+    b.lane_bytes[q] = (unsigned)at;
+  }
+  auto put = [&](int r, const T(&acc)[L * V]) {  // the tile's row r: the lanes that own columns
+#pragma unroll
+    for (int q = 0; q < L; ++q) {
+      if (!owns[q]) continue;
+      const int have = cn - c0[q] < V ? cn - c0[q] : V;  // (fewer than V with a padded B only)
+      if constexpr (COLC) {
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+          if (i >= first[q] && i < have) s_tile[(c0[q] + i) * (kWave + 1) + r] = acc[q * V + i];
+      } else {
+        T* c = C + (row0 + r) * c_row + cbeg + c0[q];
+        if (have == V) {
+          group_store_row<T>(c, first[q], &acc[q * V], beta, c_nt);
+        } else {
+#pragma unroll
+          for (int i = 0; i < V; ++i)
+            if (i < have) c[i] = beta == T(0) ? acc[q * V + i] : c[i] * beta + acc[q * V + i];
+        }
+      }
+    }
+  };
+  __syncthreads();
+#pragma unroll 1
+  for (int pass = 0; pass < kTileRows / kGroupRows; ++pass) {
+    const int r = pass * kGroupRows + group;
+    int64_t start = 0, end = 0;
+    bool there = r < nrows;
+    if (there) {
+      start = (int64_t)s_ptr[r] - base;
+      end = (int64_t)s_ptr[r + 1] - base;
+    }
+    if (end - start > kGroupLongRow) {
+      there = false;
+      end = start;
+    }
+    T acc[L * V];
+#pragma unroll
+    for (int i = 0; i < L * V; ++i) acc[i] = T(0);
+    group_walk<T, GC, NARROW, L, FAR>(start, end, alpha, val, col_ind, base, b, acc);
+    group_join<GC>(acc);
+    if (there) put(r, acc);
+  }
+  // the workgroup's long rows, one after the other, their entries dealt to the groups
+  uint64_t long_rows = __builtin_amdgcn_ballot_w64(lane < nrows && s_ptr[lane + 1] - s_ptr[lane] > kGroupLongRow);
+  for (; long_rows; long_rows &= long_rows - 1) {  // (the same in every wave)
+    const int r = __builtin_ctzll(long_rows);
+    const int64_t start = (int64_t)s_ptr[r] - base, end = (int64_t)s_ptr[r + 1] - base;
+    const int64_t per = ((end - start + kGroupRows - 1) / kGroupRows + 15) & ~(int64_t)15;
+    const int64_t mine0 = start + per * group < end ? start + per * group : end;
+    const int64_t mine1 = mine0 + per < end ? mine0 + per : end;
+    T acc[L * V];
+#pragma unroll
+    for (int i = 0; i < L * V; ++i) acc[i] = T(0);
+    group_walk<T, GC, NARROW, L, FAR>(mine0, mine1, alpha, val, col_ind, base, b, acc);
+    group_join<GC>(acc);
+    if (threadIdx.x % 16 < GC) {
+#pragma unroll
+      for (int i = 0; i < L * V; ++i) s_part[(group * GC + cl) * L * V + i] = acc[i];
+    }
+    __syncthreads();
+    if (group == 0) {
+      for (int g = 1; g < kGroupRows; ++g) {
+#pragma unroll
+        for (int i = 0; i < L * V; ++i) acc[i] += s_part[(g * GC + cl) * L * V + i];
+      }
+      put(r, acc);
+    }
+    __syncthreads();
+  }
+  if constexpr (COLC) {
+    __syncthreads();
+    if (lane < nrows) {
+      for (int c = threadIdx.x / kWave; c < cn; c += kGroupThreads / kWave) {
+        T* out = C + row0 + lane + (int64_t)(cbeg + c) * c_col;
+        const T sum = s_tile[c * (kWave + 1) + lane];
+        nt_store(beta == T(0) ? sum : nt_load(out) * beta + sum, out);
+      }
+    }
+  }
+}
+
+}  // namespace asamd

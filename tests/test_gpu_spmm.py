@@ -328,3 +328,36 @@ def test_row_major_rows_that_share_columns(gpu, mat, n, dtype, kernel, monkeypat
                     assert np.array_equal(out.view(np.uint8), again.view(np.uint8))
         finally:
             da.free()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("lengths", [
+    # blocks of sixteen entries, the longest row of one lane group and the first that the workgroup shares, rows beyond a
+    # whole tile; the mean keeps short rows of B on four lanes each, whose long rows begin beyond 256
+    [0, 1, 15, 16, 17, 31, 255, 256, 257, 0, 1025] + [3] * 300,
+    # the same on sixteen and sixty-four lanes (long rows beyond 1024 and 4096)
+    [0, 1023, 1024, 1025, 2, 17] + [20] * 90,
+    [4095, 4096, 4097, 0, 64] + [100] * 12,
+    [20] * 130,
+], ids=["few", "some", "many", "even"])
+def test_widths_around_the_tiles(gpu, lengths, dtype):
+    """Dense widths around every form of the row kernels: whole short rows (one to four loads), 4, 8 and 16 column
+    lanes, two loads a lane, several chunks; and, column-major, the panels of 256, 128 and fewer bytes."""
+    v = 16 // np.dtype(dtype).itemsize
+    a = csr_from_lengths(lengths, 5003, dtype, base=1)
+    da = DeviceCsr(a)
+    try:
+        for n in sorted({1, v - 1, v, v + 1, 2 * v + 1, 3 * v + 1, 4 * v, 4 * v + 1, 8 * v + 1, 12 * v + 1, 16 * v - 1, 16 * v,
+                         16 * v + 1, 24 * v + 3, 32 * v + 1}):
+            if n == 0:
+                continue
+            B = wl.uniform(a.cols * n, dtype, 7)
+            C0 = wl.uniform(a.rows * n, dtype, 8)
+            announce("spmm around the tiles", len(lengths), n, np.dtype(dtype).name)
+            for beta in (0.0, 0.5):
+                out = run_csrmm(gpu, da, capi.ALPHA_SPARSE_LAYOUT_ROW_MAJOR, 0, 1.25, B, n, beta, C0, n, n, a.cols)
+                check(a, 1.25, B.reshape(-1, n), beta, C0.reshape(-1, n), out.reshape(-1, n), "row-major n=%d" % n)
+                out = run_csrmm(gpu, da, capi.ALPHA_SPARSE_LAYOUT_COLUMN_MAJOR, 0, 1.25, B, a.cols, beta, C0, a.rows, n, a.cols)
+                check(a, 1.25, B.reshape(n, -1).T, beta, C0.reshape(n, -1).T, out.reshape(n, -1).T, "column-major n=%d" % n)
+    finally:
+        da.free()
