@@ -151,6 +151,11 @@ class asamd_xlds_layout(Structure):  # include/alsparse_amd_kernels.h
                 ("dtype", c_int32), ("nnz", c_int32), ("base", c_int32)]
 
 
+class asamd_pattern_layout(Structure):  # include/alsparse_amd_kernels.h
+    _fields_ = [("pid", c_void_p), ("dist", c_void_p), ("block_off", c_void_p), ("stride", c_int32), ("group", c_int32),
+                ("device_bytes", ctypes.c_int64)]
+
+
 class asamd_dense_strides(Structure):
     _fields_ = [("b_row_stride", ctypes.c_int64), ("b_col_stride", ctypes.c_int64),
                 ("c_row_stride", ctypes.c_int64), ("c_col_stride", ctypes.c_int64)]
@@ -360,6 +365,9 @@ _COMMON = {
     "asamd_narrow_columns": [_P, _I, _I, _P, _P],
     "asamd_narrow_rel_columns": [_P, _I, _I, _I, _I, _P, _P, _P, _P],
     "asamd_spmv_stream_rel16": [_P, POINTER(asamd_spmv_args), _I, _I, _P],
+    "asamd_patterns_build": [_P, _I, _I, _I, _I, _I, _P, _P, POINTER(asamd_pattern_layout)],
+    "asamd_patterns_free": [POINTER(asamd_pattern_layout)],
+    "asamd_spmv_patterns": [_P, POINTER(asamd_spmv_args), POINTER(asamd_pattern_layout)],
     "asamd_spmv_xlds_narrow": [_P, POINTER(asamd_spmv_args), _I, _P],
     "asamd_xlds_slices": [_I, _I],
     "asamd_xlds_build": [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P],

@@ -36,6 +36,8 @@ struct asamd_csr_plan {
   uint16_t *d_col16;       /* x in LDS, one slice: the column numbers as 16-bit words (structure promised fixed) */
   int16_t *d_rel16;        /* staged row blocks: the columns as 16-bit distances from the workgroup's first row */
   int rel16_group;         /* the lanes per row they were made for */
+  asamd_pattern_layout pat; /* staged row blocks: a pattern number per row instead of the columns */
+  int pinned;              /* the family was set from outside: the staged row blocks then read columns (or distances) */
   int watched;             /* laid out for asamd_csr_plan_csrmv_watched: its fingerprints are the caller's account */
   void *d_eval;            /* ELL copy: ell_width * m values, column-major */
   int32_t *d_ecol;         /* ... and zero-based columns */
@@ -437,6 +439,7 @@ static void account(asamd_csr_plan *p) {
   if (p->d_block_row) b += ((int64_t)st->merge_blocks + 1) * 4;
   if (p->d_col16) b += ((int64_t)st->nnz + 4) * 2;
   if (p->d_rel16) b += ((int64_t)st->nnz + 4) * 2;
+  b += p->pat.device_bytes;
   b += p->tiled.device_bytes + p->hot.device_bytes + p->binned.device_bytes + p->xlds.device_bytes;
   if (st->ell_built) b += (int64_t)st->m * st->ell_width * ((int64_t)p->val_size + 4);
   for (int w = 0; w < 2; ++w)
@@ -530,6 +533,7 @@ static int run_algo(hipStream_t s, const asamd_csr_plan *p, int algo, const asam
     case ASAMD_SPMV_ROWCONST:
       return asamd_spmv_rowconst(s, a, st->const_len);
     case ASAMD_SPMV_STREAM:
+      if (p->pat.pid && !p->pinned && ((uintptr_t)a->val & 15u) == 0) return asamd_spmv_patterns(s, a, &p->pat);
       if (p->d_rel16 && p->rel16_group == stream_group(p, 0) && ((uintptr_t)a->val & 15u) == 0)
         return asamd_spmv_stream_rel16(s, a, p->rel16_group, st->max_len, p->d_rel16);
       return asamd_spmv_stream(s, a, stream_group(p, 0), st->max_len, st->first_offset);
@@ -1037,6 +1041,8 @@ static double model_ms(const asamd_csr_plan *p, int algo) {
       if (vs >= 16.0 && rate > 4.2) rate = 4.2;
       /* 16-bit distances for columns: half of the bytes they save shows (27-point stencil, 160^3 points: 0.204 ->
        * 0.181 ms with 4-byte values, 0.300 -> 0.274 with 8-byte ones) */
+      /* a pattern number per row for the columns: the values, row_ptr, the numbers, x and y are what is left */
+      if (p->pat.pid) return hypot2((bytes - 4.0 * nnz + m) / 6.2e9, 0.5 * gather);
       if (p->d_rel16) return hypot2((bytes - 1.0 * nnz) / (rate * 1e9), gather);
       break;
     case ASAMD_SPMV_VECTOR: rate = 2.4 * vector_utilisation(st, p->auto_width); break;
@@ -1330,6 +1336,23 @@ static hipError_t plan_create(hipStream_t stream, int32_t m, int32_t n, int32_t 
       }
     }
   }
+  /* Staged row blocks whose rows follow few patterns (grids): a byte per row for the column numbers.  From 2^20 entries
+   * on: below, a multiply is one launch's latency (5-point Laplacian on 300 x 333, fp64: 3.7 us with the columns, 4.4
+   * with the patterns; on 900 x 1100, fp32: 11.3 against 7.2).  Values of 16 bytes stay with the ELL copy (5-point
+   * Laplacian on 1500 x 1400: 59 us against 84). */
+  if (col_ind && st->trusted && trusted != 3 && (p->auto_algo == ASAMD_SPMV_STREAM || (trusted == 2 && stream_ok(p))) &&
+      nnz >= (trusted == 2 ? 1 : 1 << 20) && p->val_size <= 8 && st->first_offset == 0 && st->min_len >= 1 &&
+      env_int("ALSPARSE_AMD_STREAM_PATTERNS", 1) > 0) {
+    e = (hipError_t)asamd_patterns_build(stream, m, nnz, base, stream_group(p, 0), st->max_len, row_ptr, col_ind, &p->pat);
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError(); /* the caller's columns serve */
+      e = hipSuccess;
+    }
+    if (e != hipSuccess) {
+      asamd_csr_plan_destroy(p);
+      return e;
+    }
+  }
   if (col_ind && st->trusted && trusted != 3 && (p->auto_algo == ASAMD_SPMV_STREAM || (trusted == 2 && stream_ok(p))) &&
       (p->dtype == ASAMD_DTYPE_FLOAT || p->dtype == ASAMD_DTYPE_DOUBLE) && nnz >= 1 && st->first_offset == 0 &&
       (trusted == 2 || (double)nnz * (4.0 + val_size) + ((double)m + n) * val_size > 400.0e6) &&
@@ -1337,7 +1360,8 @@ static hipError_t plan_create(hipStream_t stream, int32_t m, int32_t n, int32_t 
     /* staged row blocks and a structure that stays: where every entry lies within 32 767 columns of its workgroup's
      * first row (a discretisation, a band) the kernel reads 16-bit distances instead of the column numbers.  Pays
      * on matrices well beyond the memory-side cache (256 MB): 27-point stencil on 160^3 points 0.204 -> 0.177 ms,
-     * nothing on the 5-point Laplacian on 2048^2 (336 MB). */
+     * nothing on the 5-point Laplacian on 2048^2 (336 MB).  Made beside row patterns too: a multiply whose family was
+     * set from outside runs the staged kernel with them. */
     int32_t *too_far = (int32_t *)p->d_setup;
     int32_t h_far = 1;
     p->rel16_group = stream_group(p, 0);
@@ -1424,6 +1448,7 @@ static hipError_t plan_create(hipStream_t stream, int32_t m, int32_t n, int32_t 
       return e;
     }
   }
+  if (p->pat.pid && p->auto_algo != ASAMD_SPMV_STREAM && trusted != 2) asamd_patterns_free(&p->pat);
   if (p->d_rel16 && p->auto_algo != ASAMD_SPMV_STREAM && trusted != 2) {
     (void)hipFree(p->d_rel16); /* another family was kept */
     p->d_rel16 = NULL;
@@ -1452,6 +1477,7 @@ void asamd_csr_plan_destroy(asamd_csr_plan *p) {
   if (p->d_block_row) (void)hipFree(p->d_block_row);
   if (p->d_col16) (void)hipFree(p->d_col16);
   if (p->d_rel16) (void)hipFree(p->d_rel16);
+  asamd_patterns_free(&p->pat);
   if (p->d_setup) (void)hipFree(p->d_setup);
   if (p->d_fp) (void)hipFree(p->d_fp);
   free_tiled(p);
@@ -1554,6 +1580,7 @@ int asamd_csr_plan_set_algo(asamd_csr_plan *p, int32_t algo) {
   switch (algo) {
     case ASAMD_SPMV_AUTO:
       p->st.algo = p->auto_algo;
+      p->pinned = 0;
       return hipSuccess;
     case ASAMD_SPMV_ROWCONST:
       if (!rowconst_ok(p)) return hipErrorInvalidValue;
@@ -1587,5 +1614,6 @@ int asamd_csr_plan_set_algo(asamd_csr_plan *p, int32_t algo) {
       return hipErrorInvalidValue;
   }
   p->st.algo = algo;
+  p->pinned = 1;
   return hipSuccess;
 }

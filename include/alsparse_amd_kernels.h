@@ -156,6 +156,23 @@ int asamd_spmv_stream_rel16(hipStream_t stream, const asamd_spmv_args *a, int32_
                             const int16_t *rel16);
 int asamd_spmv_stream(hipStream_t stream, const asamd_spmv_args *a, int32_t group, int32_t max_len,
                       int32_t first_offset);
+/* Rows that follow few patterns (discretisations on grids): the list of a row's distances (column - row) is one of at
+ * most 256, so a byte per row and a small table stand for the column numbers.  Made once for a structure that stays and
+ * for THIS `group`; the record is left EMPTY (pid NULL, not an error) where there are more patterns, a row is empty or
+ * rows are longer than 64.  Element types of at most 8 bytes, val 16-byte aligned,
+ * row_ptr[0] == base.  (No
+ * counterpart in the reference, whose kernel reads every column: dcu_gemv_vector.h:14-57.) */
+typedef struct {
+  unsigned char *pid;   /* m pattern numbers; NULL: no layout (owns the one allocation) */
+  int32_t *dist;        /* 256 x stride distances */
+  int32_t *block_off;   /* where the entries of every workgroup's 256 / group rows begin, and the last one's end */
+  int32_t stride, group;
+  int64_t device_bytes;
+} asamd_pattern_layout;
+int asamd_patterns_build(hipStream_t stream, int32_t m, int32_t nnz, int32_t base, int32_t group, int32_t max_len,
+                         const int32_t *row_ptr, const int32_t *col_ind, asamd_pattern_layout *out);
+void asamd_patterns_free(asamd_pattern_layout *layout);
+int asamd_spmv_patterns(hipStream_t stream, const asamd_spmv_args *a, const asamd_pattern_layout *layout);
 
 /* Merge-path: the (m + nnz) items are cut into blocks of ASAMD_MERGE_THREADS * ipt items (ipt: 4, 8, or
  * 16 for real types of at most 8 bytes; 4 only for 16-byte values).  block_row: blocks + 1 merge
