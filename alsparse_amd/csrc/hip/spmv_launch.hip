@@ -447,9 +447,11 @@ extern "C" int asamd_merge_partition(hipStream_t s, int32_t m, int32_t nnz, cons
   return hipGetLastError();
 }
 
+extern "C" int32_t asamd_merge_self_blocks(void) { return kMergeSelfBlocks; }
+
 extern "C" int asamd_spmv_merge(hipStream_t s, const asamd_spmv_args* a, int32_t ipt, const int32_t* block_row,
                                 int32_t* carry_row, void* carry_val, void* head_val) {
-  if (!a || !block_row || !carry_row || !carry_val || !head_val) return hipErrorInvalidValue;
+  if (!a || !carry_row || !carry_val || !head_val) return hipErrorInvalidValue;
   return by_dtype(a->dtype, [&](auto* tag) -> int {
     using T = std::remove_pointer_t<decltype(tag)>;
     if (!args_ok<T>(a)) return hipErrorInvalidValue;

@@ -74,7 +74,29 @@ static __global__ __launch_bounds__(256) void merge_partition_kernel(int m, int 
   block_row[b] = (int)lo;
 }
 
-// IPT items per thread, kMergeThreads * IPT items per workgroup.  WIDE: val and col_ind are 16-byte aligned
+// The same coordinate found by a whole wave: 64 probes at a time, all lanes return it.
+static __device__ __forceinline__ int merge_coordinate(int m, int nnz, const int* __restrict__ row_ptr, int base, int64_t d) {
+  const int lane = threadIdx.x % kWave;
+  int64_t lo = d > nnz ? d - nnz : 0;
+  int64_t hi = d < m ? d : m;  // the answer lies in [lo, hi]
+  while (lo < hi) {
+    const int64_t step = (hi - lo + kWave - 1) / kWave;
+    const int64_t mid = lo + (lane + 1) * step - 1;  // ascending over the lanes; rows from the first false one on are false
+    const int64_t at = mid < hi ? mid : hi - 1;
+    const bool done = mid < hi && (int64_t)row_ptr[at + 1] - base <= d - at - 1;
+    const int below = __popcll(__builtin_amdgcn_ballot_w64(done));
+    lo += below * step;
+    if (lo + step - 1 < hi) hi = lo + step - 1;
+  }
+  return (int)lo;
+}
+// Up to this many workgroups find their two coordinates themselves, two of a workgroup's waves one each.  A launch of
+// its own for them costs 4.4 us, three rounds of probes in the L2 about one; a workgroup's probes are 64 lines a round,
+// though, where neighbouring threads of the table's kernel share theirs, so large matrices keep the table.
+constexpr int kMergeSelfBlocks = 4096;
+
+// IPT items per thread, kMergeThreads * IPT items per workgroup.  block_row: the coordinates, or null (every workgroup
+// searches for its own).  WIDE: val and col_ind are 16-byte aligned
 // and the workgroup's entries are read as pieces of four from the multiple of four at or before its first
 // entry (a quarter of the memory instructions); a workgroup whose last piece would reach past the end of
 // the arrays reads entry by entry.
@@ -99,8 +121,19 @@ __global__ __launch_bounds__(kMergeThreads) void spmv_merge_kernel(
   const int64_t total = (int64_t)m + nnz;
   const int64_t d0 = (int64_t)b * kItems;
   const int64_t d1 = d0 + kItems < total ? d0 + kItems : total;
-  const int row_b = block_row[b];
-  const int row_e = block_row[b + 1];
+  int row_b, row_e;
+  if (block_row) {
+    row_b = block_row[b];
+    row_e = block_row[b + 1];
+  } else {
+    if (tid < 2 * kWave) {
+      const int r = merge_coordinate(m, nnz, row_ptr, base, tid < kWave ? d0 : d1);
+      if (tid % kWave == 0) s_wrow[tid / kWave] = r;
+    }
+    __syncthreads();
+    row_b = __builtin_amdgcn_readfirstlane(s_wrow[0]);
+    row_e = __builtin_amdgcn_readfirstlane(s_wrow[1]);
+  }
   const int64_t nnz_b = d0 - row_b;
   const int64_t nnz_e = d1 - row_e;
   int rows_cnt = row_e - row_b;

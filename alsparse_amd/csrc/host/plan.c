@@ -574,8 +574,8 @@ static int run_algo(hipStream_t s, const asamd_csr_plan *p, int algo, const asam
     case ASAMD_SPMV_MERGE: {
       const size_t nb = (size_t)st->merge_blocks;
       const int32_t *block_row = p->d_block_row;
-      if (!block_row) {
-        /* structure not promised fixed: the coordinates are computed for this call */
+      if (!block_row && st->merge_blocks > asamd_merge_self_blocks()) {
+        /* structure not promised fixed: the coordinates are computed for this call (few workgroups: by themselves) */
         int32_t *fresh = (int32_t *)ws_take(&ws, (nb + 1) * 4);
         if (!fresh) return -1;
         const int e = asamd_merge_partition(s, st->m, st->nnz, a->row_ptr, st->base, st->merge_blocks,
