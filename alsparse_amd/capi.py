@@ -384,6 +384,7 @@ _COMMON = {
     "asamd_csr2coo_workspace_bytes": [_I],
     "asamd_csr2coo": [_P, _P, _I, _I, _P, _I],
     "asamd_csr2coo_ws": [_P, _P, _I, _I, _P, _I, _P, c_size_t],
+    "asamd_csr2ell_width_ws": [_P, _I, _P, POINTER(_I), _P, c_size_t],
     "asamd_csr2ell_width": [_P, _I, _P, POINTER(_I)],
     "asamd_warmup": [_P],
     "asamd_s_csrmv_noalloc": [_P, _I, _I, _I, _I, c_float, _P, _P, _P, _P, c_float, _P],

@@ -50,22 +50,26 @@ __device__ __forceinline__ int wave_max_scan(int v) {
   return v;
 }
 
-// chunk_row[b] = largest r with row_ptr[r] - base <= b * kCooChunk, for b in [0, chunks]: one thread and
-// one binary search per chunk boundary, all of them in flight together (inside the chunk kernel the
-// same searches are a chain of dependent loads that each workgroup waits for)
+// chunk_row[b] = largest r with row_ptr[r] - base <= b * kCooChunk, for b in [0, chunks]: a wave per chunk boundary
+// probes 64 places at once, four rounds of loads for 2^24 rows where a thread's binary search waits for 24 (20 M entries
+// in 4 M rows: 11.3 -> 5.2 us).  All boundaries are in flight together; inside the chunk kernel every workgroup would wait
+// for its own.
 __global__ __launch_bounds__(256) void csr2coo_chunk_rows_kernel(const int* __restrict__ row_ptr, int nnz, int m,
                                                                  int base, int chunks, int* __restrict__ chunk_row) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  const int lane = threadIdx.x % kWave;
+  const int b = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (256 / kWave) + threadIdx.x / kWave));
   if (b > chunks) return;
   int64_t k = (int64_t)b * kCooChunk;
   if (k > nnz - 1) k = nnz - 1;  // the last boundary: the row of the last entry
-  int lo = 0, hi = m - 1;
+  int64_t lo = 0, hi = m - 1;
   while (lo < hi) {
-    const int mid = (int)(((int64_t)lo + hi + 1) >> 1);
-    if ((int64_t)row_ptr[mid] - base <= k) lo = mid;
-    else hi = mid - 1;
+    const int64_t step = (hi - lo + kWave - 1) / kWave;
+    const int64_t p = lo + (lane + 1) * step;
+    const bool not_after = p <= hi && (int64_t)row_ptr[p <= hi ? p : hi] - base <= k;
+    lo += __popcll(__builtin_amdgcn_ballot_w64(not_after)) * step;
+    hi = lo + step - 1 < hi ? lo + step - 1 : hi;
   }
-  chunk_row[b] = lo;
+  if (lane == 0) chunk_row[b] = (int)lo;
 }
 
 // chunk_row: the table above, or null (then every workgroup searches for its own rows)
@@ -176,8 +180,7 @@ extern "C" int asamd_csr2coo_ws(hipStream_t stream, const int32_t* row_ptr, int3
   int* chunk_row = nullptr;
   if (workspace && workspace_bytes >= asamd_csr2coo_workspace_bytes(nnz) && (uintptr_t)workspace % alignof(int) == 0) {
     chunk_row = (int*)workspace;
-    csr2coo_chunk_rows_kernel<<<(unsigned)((chunks + 1 + 255) / 256), 256, 0, stream>>>(row_ptr, nnz, m, base, chunks,
-                                                                                        chunk_row);
+    csr2coo_chunk_rows_kernel<<<(unsigned)((chunks + 1 + 3) / 4), 256, 0, stream>>>(row_ptr, nnz, m, base, chunks, chunk_row);
   }
   if (stores_bypass_caches((size_t)nnz * sizeof(int)))
     csr2coo_kernel<true><<<(unsigned)chunks, kCooThreads, 0, stream>>>(row_ptr, nnz, m, coo_row, base, chunk_row);
@@ -194,11 +197,12 @@ extern "C" int asamd_csr2coo(hipStream_t stream, const int32_t* row_ptr, int32_t
 // ---------------------------------------------------------------------------
 // csr2ell_width: max over rows of row_ptr[r+1] - row_ptr[r].
 // ---------------------------------------------------------------------------
+// out[workgroup] = the largest of the rows the workgroup looked at.  (One atomic maximum per workgroup on one word cost
+// more than reading row_ptr: 4 M rows 16.4 us, 5.9 this way.)
+constexpr int kWidthBlocks = 1024;
 __global__ __launch_bounds__(256) void max_row_len_kernel(int m, const int* __restrict__ row_ptr,
                                                           int* __restrict__ out) {
-  __shared__ int s_max;
-  if (threadIdx.x == 0) s_max = 0;
-  __syncthreads();
+  __shared__ int s_max[256 / kWave];
   int lmax = 0;
   // eight rows per thread and trip, all sixteen loads issued before the first is used
   constexpr int kU = 8;
@@ -215,28 +219,42 @@ __global__ __launch_bounds__(256) void max_row_len_kernel(int m, const int* __re
 #pragma unroll
     for (int u = 0; u < kU; ++u) lmax = max(lmax, hi[u] - lo[u]);
   }
-  atomicMax(&s_max, lmax);
+  lmax = __builtin_amdgcn_readlane(wave_max_scan(lmax), kWave - 1);
+  if (threadIdx.x % kWave == 0) s_max[threadIdx.x / kWave] = lmax;
   __syncthreads();
-  if (threadIdx.x == 0) atomicMax(out, s_max);
+  if (threadIdx.x == 0) {
+    for (int w = 0; w < 256 / kWave; ++w) lmax = max(lmax, s_max[w]);
+    out[blockIdx.x] = lmax;
+  }
 }
 
-__global__ void zero_int_kernel(int* p) { *p = 0; }
-
-extern "C" int asamd_csr2ell_width(hipStream_t stream, int32_t m, const int32_t* row_ptr,
-                                   int32_t* width_host) {
+extern "C" int asamd_csr2ell_width_ws(hipStream_t stream, int32_t m, const int32_t* row_ptr, int32_t* width_host,
+                                      void* workspace, size_t workspace_bytes) {
   if (!row_ptr || !width_host || m <= 0) return hipErrorInvalidValue;
   int* d = nullptr;
-  hipError_t e = hipMalloc(&d, sizeof(int));
+  hipError_t e = hipSuccess;
+  const bool given = workspace && workspace_bytes >= kWidthBlocks * sizeof(int) && (uintptr_t)workspace % alignof(int) == 0;
+  if (given) d = (int*)workspace;
+  else e = hipMalloc(&d, kWidthBlocks * sizeof(int));
   if (e != hipSuccess) return e;
-  zero_int_kernel<<<1, 1, 0, stream>>>(d);
-  // every workgroup ends with one atomic on the same word: few, long-running workgroups
   int grid = (int)(((int64_t)m + 256 * 8 - 1) / (256 * 8));
-  if (grid > 1024) grid = 1024;
+  if (grid > kWidthBlocks) grid = kWidthBlocks;
   max_row_len_kernel<<<grid, 256, 0, stream>>>(m, row_ptr, d);
-  e = hipMemcpyAsync(width_host, d, sizeof(int), hipMemcpyDeviceToHost, stream);
+  e = hipGetLastError();
+  int part[kWidthBlocks];
+  if (e == hipSuccess) e = hipMemcpyAsync(part, d, (size_t)grid * sizeof(int), hipMemcpyDeviceToHost, stream);
   if (e == hipSuccess) e = hipStreamSynchronize(stream);
-  (void)hipFree(d);
+  if (e == hipSuccess) {
+    int width = 0;
+    for (int b = 0; b < grid; ++b) width = part[b] > width ? part[b] : width;
+    *width_host = width;
+  }
+  if (!given) (void)hipFree(d);
   return e;
+}
+
+extern "C" int asamd_csr2ell_width(hipStream_t stream, int32_t m, const int32_t* row_ptr, int32_t* width_host) {
+  return asamd_csr2ell_width_ws(stream, m, row_ptr, width_host, nullptr, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -247,7 +265,18 @@ extern "C" int asamd_csr2ell_width(hipStream_t stream, int32_t m, const int32_t*
 // than the LDS window are read from global memory directly.
 // ---------------------------------------------------------------------------
 constexpr int kEllRows = 256;
-constexpr int kEllWindow = 4096;  // staged entries per workgroup pass (half of it for 16-byte values)
+// Staged entries per workgroup (at most half of it for 16-byte values): as many as 256 rows of the ELL's width hold, so
+// that short rows leave room for more workgroups on a compute unit -- always 4 096 were 50 KB for 8-byte values, three
+// workgroups (5-point Laplacian of 4 M rows, fp64: 102 -> 93 us).
+constexpr int kEllWindow = 4096;
+template <typename T>
+constexpr int ell_window(int width) {
+  const int most = sizeof(T) > 8 ? kEllWindow / 2 : kEllWindow;  // at most 32 KiB of staged values
+  return width < most / kEllRows ? width * kEllRows : most;
+}
+// staged entry p lives at p + p / 32: lanes read slot s of consecutive rows, i.e. positions a row
+// length apart, and without the skew rows of 16 or 32 entries would all fall into a few LDS banks
+__host__ __device__ constexpr int ell_at(int p) { return p + (p >> 5); }
 
 // WIDE: val and col_ind are 16-byte aligned; the staged range is then read as pieces of four entries from the
 // multiple of four at or before its start (a quarter of the load instructions); pieces that would reach past
@@ -256,14 +285,11 @@ template <typename T, bool NTS, bool WIDE>
 __global__ __launch_bounds__(kEllRows) void csr2ell_kernel(
     int m, const T* __restrict__ val, const int* __restrict__ row_ptr,
     const int* __restrict__ col_ind, int csr_base, int ell_base, int width,
-    T* __restrict__ ell_val, int* __restrict__ ell_col, const int* __restrict__ gate) {
+    T* __restrict__ ell_val, int* __restrict__ ell_col, int window, const int* __restrict__ gate) {
   if (gate && *gate == 0) return;  // a refresh behind the value guard: nothing has changed
-  constexpr int kWindow = sizeof(T) > 8 ? kEllWindow / 2 : kEllWindow;  // at most 32 KiB of staged values
-  // staged entry p lives at p + p / 32: lanes read slot s of consecutive rows, i.e. positions a row
-  // length apart, and without the skew rows of 16 or 32 entries would all fall into a few LDS banks
-  auto at = [](int p) { return p + (p >> 5); };
-  __shared__ T s_val[kWindow + kWindow / 32];
-  __shared__ int s_col[kWindow + kWindow / 32];
+  extern __shared__ __align__(16) unsigned char s_ell[];  // ell_at(window) values, then as many columns
+  T* s_val = reinterpret_cast<T*>(s_ell);
+  int* s_col = reinterpret_cast<int*>(s_ell + (size_t)ell_at(window) * sizeof(T));
   const int64_t row_first = (int64_t)blockIdx.x * kEllRows;
   const int64_t row = row_first + threadIdx.x;
   int64_t row_last = row_first + kEllRows;
@@ -275,7 +301,7 @@ __global__ __launch_bounds__(kEllRows) void csr2ell_kernel(
     my_begin = (int64_t)row_ptr[row] - csr_base;
     my_end = (int64_t)row_ptr[row + 1] - csr_base;
   }
-  const bool staged = blk_end - blk_begin <= kWindow;  // workgroup-uniform
+  const bool staged = blk_end - blk_begin <= window;  // workgroup-uniform
   if (staged && WIDE) {
     const int count = (int)(blk_end - blk_begin);
     const int64_t limit = (int64_t)row_ptr[m] - csr_base;  // entries in the arrays
@@ -314,8 +340,8 @@ __global__ __launch_bounds__(kEllRows) void csr2ell_kernel(
           for (int j = 0; j < 4; ++j) {
             const int p = k + j - head;
             if (p >= 0 && p < count) {
-              s_val[at(p)] = v[u].get(j);
-              s_col[at(p)] = cc[j];
+              s_val[ell_at(p)] = v[u].get(j);
+              s_col[ell_at(p)] = cc[j];
             }
           }
         }
@@ -341,8 +367,8 @@ __global__ __launch_bounds__(kEllRows) void csr2ell_kernel(
       for (int u = 0; u < kU; ++u) {
         const int p = p0 + u * kEllRows;
         if (p < count) {
-          s_val[at(p)] = v[u];
-          s_col[at(p)] = c[u];
+          s_val[ell_at(p)] = v[u];
+          s_col[ell_at(p)] = c[u];
         }
       }
     }
@@ -356,8 +382,8 @@ __global__ __launch_bounds__(kEllRows) void csr2ell_kernel(
     if (s < len) {
       if (staged) {
         const int p = (int)(my_begin - blk_begin) + s;
-        v = s_val[at(p)];
-        c = s_col[at(p)] - csr_base + ell_base;
+        v = s_val[ell_at(p)];
+        c = s_col[ell_at(p)] - csr_base + ell_base;
       } else {
         v = val[my_begin + s];
         c = col_ind[my_begin + s] - csr_base + ell_base;
@@ -384,8 +410,11 @@ static int csr2ell_impl(hipStream_t stream, int m, const T* val, const int* rp, 
   const unsigned grid = (unsigned)(((int64_t)m + kEllRows - 1) / kEllRows);
   const bool nts = stores_bypass_caches((size_t)m * (size_t)width * (sizeof(T) + sizeof(int)));
   const bool wide = (((uintptr_t)val | (uintptr_t)ci) & 15u) == 0;
-#define ASAMD_CSR2ELL(NTS, WIDE) \
-  csr2ell_kernel<T, NTS, WIDE><<<grid, kEllRows, 0, stream>>>(m, val, rp, ci, csr_base, ell_base, width, ell_val, ell_col, gate)
+  const int window = ell_window<T>(width);
+  const size_t lds = (size_t)ell_at(window) * (sizeof(T) + sizeof(int));
+#define ASAMD_CSR2ELL(NTS, WIDE)                                                                                      \
+  csr2ell_kernel<T, NTS, WIDE><<<grid, kEllRows, lds, stream>>>(m, val, rp, ci, csr_base, ell_base, width, ell_val,   \
+                                                                ell_col, window, gate)
   if (nts && wide) ASAMD_CSR2ELL(true, true);
   else if (nts) ASAMD_CSR2ELL(true, false);
   else if (wide) ASAMD_CSR2ELL(false, true);
