@@ -7,7 +7,7 @@
 //   the index base of the descriptor is honoured).
 //
 //   COO (entries grouped by row, as csr2coo leaves them): every wave owns one
-//   contiguous run of entries and reduces it 64 at a time with a segmented
+//   contiguous run of entries and reduces it 256 at a time (64 with 16-byte values), with a segmented
 //   scan across its lanes (DPP only); the last lane of every row segment adds the
 //   segment's sum to y, the open segment at the end of a step is carried into
 //   the next one in registers.  Replaces
@@ -24,6 +24,8 @@
 //   scaled by beta beforehand, as in the reference (:161-169).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "alsparse_amd_kernels.h"
 #include "device_utils.hpp"
@@ -42,8 +44,40 @@ __global__ __launch_bounds__(256) void scale_y_kernel(int m, T beta, T* __restri
 }
 
 constexpr int kCooThreads = 256;
-constexpr int kCooSteps = 16;                        // 64-entry steps per wave (more when the workspace is short)
+constexpr int kCooWaveEntries = 1024;                // entries per wave (more when the workspace is short)
 constexpr int kCooWaves = kCooThreads / kWave;
+
+constexpr int kCooLane = 4;                 // consecutive entries per lane and step
+constexpr int kCooStep = kCooLane * kWave;  // entries of a wave's step
+
+template <typename T>
+struct CooStep {
+  static constexpr int n = kCooLane;
+  struct Ints { int e[n]; } row, col;
+  struct Vals { T e[n]; } val;
+};
+// The step's `count` entries (at most kCooStep) from entry k0 on: wide loads through buffer resources that end with
+// the step, so nothing behind the wave's entries is read and no load waits for a condition.
+template <typename P, int AUX>
+__device__ __forceinline__ P coo_pieces(BufferRsrc r, int lane) {
+  if constexpr (sizeof(P) <= 16) {
+    return buffer_load<P, AUX>(r, (int)sizeof(P) * lane);
+  } else {
+    struct Pieces { Int4 p[sizeof(P) / 16]; } v;
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(P) / 16); ++i) v.p[i] = buffer_load<Int4, AUX>(r, (int)sizeof(P) * lane + 16 * i);
+    return __builtin_bit_cast(P, v);
+  }
+}
+template <typename T, bool NTI, bool NTV>
+__device__ __forceinline__ CooStep<T> coo_load(const T* __restrict__ val, const int* __restrict__ row,
+                                               const int* __restrict__ col, int64_t k0, int count, int lane) {
+  CooStep<T> s;
+  s.row = coo_pieces<typename CooStep<T>::Ints, NTI ? 2 : 0>(make_rsrc(row + k0, count * 4), lane);
+  s.col = coo_pieces<typename CooStep<T>::Ints, NTI ? 2 : 0>(make_rsrc(col + k0, count * 4), lane);
+  s.val = coo_pieces<typename CooStep<T>::Vals, NTV ? 2 : 0>(make_rsrc(val + k0, count * (int)sizeof(T)), lane);
+  return s;
+}
 
 // With boundary slots (b_row != nullptr): the wave's first and last row segment -- the ones that may belong
 // to rows shared with the neighbouring waves -- do not go to y but to slots 2w (head) and 2w + 1 (tail) of
@@ -51,8 +85,172 @@ constexpr int kCooWaves = kCooThreads / kWave;
 // Entries that are grouped by row therefore reach every y through a single addition of a sum formed in a
 // fixed order: the result is the same from run to run.
 // NTI / NTV: the index streams / the values are loaded non-temporally (see stream_policy.hpp)
+//
+// The next step's entries are in flight while this one's are summed.  Bound by memory and by the additions to y, whose
+// lines are fetched for them.  One entry per lane and step was bound by its instructions and by 13-row pieces of y per
+// atomic: 5-point Laplacian of 6 M rows, fp32 (30 M entries, 411 MB) 123 us with the scaling and the boundary pass,
+// 89 now; 2048^2, fp64 108 -> 87; 27-point stencil of 10^6 points, fp32 106 -> 71.
 template <typename T, bool NTI, bool NTV>
 __global__ __launch_bounds__(kCooThreads) void coomv_kernel(int64_t nnz, int m, int n, T alpha,
+                                                            const T* __restrict__ coo_val,
+                                                            const int* __restrict__ coo_row,
+                                                            const int* __restrict__ coo_col, int base,
+                                                            const T* __restrict__ x, T* __restrict__ y, int per_wave,
+                                                            int* __restrict__ b_row, T* __restrict__ b_val) {
+  __shared__ int s_row[kCooWaves][kCooStep];  // a wave's own part only: no barriers
+  __shared__ T s_sum[kCooWaves][kCooStep];
+  const int lane = threadIdx.x % kWave;
+  const int in_group = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int64_t wave = (int64_t)blockIdx.x * kCooWaves + in_group;
+  int* const out_row = s_row[in_group];
+  T* const out_sum = s_sum[in_group];
+  const int64_t begin = wave * per_wave;
+  const int64_t end = begin + per_wave < nnz ? begin + per_wave : nnz;
+  if (begin >= end) {
+    if (b_row && lane < 2) b_row[2 * wave + lane] = -1;  // a wave past the end: empty slots
+    return;
+  }
+  const bool slots = b_row != nullptr;
+  bool emitted = !slots;  // whether the wave's first segment has gone out (wave-uniform); without slots: nothing special
+  int carry_row = -1;     // open segment handed from one step to the next (same in all lanes)
+  T carry_val = T(0);
+  int head_row = -1;
+  T head_val = T(0);
+  constexpr int E = kCooLane, kStep = kCooStep;
+  auto step_count = [&](int64_t k0) { return k0 >= end ? 0 : (int)(end - k0 < kStep ? end - k0 : kStep); };
+  // A step's sums go out through LDS, in order: neighbouring lanes then add to neighbouring rows, 64 at a time, where an
+  // instruction per position in the lane would touch every line of y four times.  They go out behind the NEXT step's
+  // gathers: loads and additions return in order, and gathers issued behind them would wait for y's lines.
+  int pending = 0;
+  auto drain = [&] {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (int i = lane; i < pending; i += kWave) atomic_add(&y[out_row[i]], alpha * out_sum[i]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  };
+  CooStep<T> cur = coo_load<T, NTI, NTV>(coo_val, coo_row, coo_col, begin, step_count(begin), lane);
+  for (int64_t k0 = begin; k0 < end; k0 += kStep) {
+    const int count = step_count(k0);
+    int r[E], c[E];
+    T v[E], xv[E];
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      const int rr = cur.row.e[j] - base, cc = cur.col.e[j] - base;
+      const bool ok = E * lane + j < count && (unsigned)rr < (unsigned)m && (unsigned)cc < (unsigned)n;
+      r[j] = ok ? rr : -1;
+      c[j] = ok ? cc : 0;  // (n > 0 where there are entries: x[0] exists)
+    }
+#pragma unroll
+    for (int j = 0; j < E; ++j) xv[j] = x[c[j]];
+    const auto val = cur.val;
+    // (behind the last step: an empty range, no request)
+    cur = coo_load<T, NTI, NTV>(coo_val, coo_row, coo_col, k0 + kStep, step_count(k0 + kStep), lane);
+    drain();
+#pragma unroll
+    for (int j = 0; j < E; ++j) v[j] = r[j] >= 0 ? val.e[j] * xv[j] : T(0);
+    const int r0 = lane_bcast(r[0], 0);
+    const bool flush = carry_row != r0 && carry_row >= 0;  // the carried segment ended with the last step
+    if (flush && !emitted) {
+      head_row = carry_row;
+      head_val = carry_val;
+    }
+    if (lane == 0) {
+      if (carry_row == r0) v[0] = carry_val + v[0];
+      else if (flush && emitted) atomic_add(&y[carry_row], alpha * carry_val);
+    }
+    if (flush) emitted = true;
+    bool cut[E];  // whether a segment ends behind position j inside the lane
+    T run[E];     // the segment that position j belongs to, summed from its start in the lane
+    bool any_cut = false;
+    run[0] = v[0];
+#pragma unroll
+    for (int j = 0; j + 1 < E; ++j) {
+      cut[j] = r[j] != r[j + 1];
+      any_cut = any_cut || cut[j];
+      run[j + 1] = cut[j] ? v[j + 1] : run[j] + v[j + 1];
+    }
+    // rows of the neighbouring lanes through DPP wave shifts (lane 0 sees -2, lane 63 sees -2: never a row)
+    const int r_prev = __builtin_amdgcn_update_dpp(-2, r[E - 1], 0x138, 0xF, 0xF, false);  // wave_shr:1
+    const int r_next = __builtin_amdgcn_update_dpp(-2, r[0], 0x130, 0xF, 0xF, false);      // wave_shl:1
+    const bool joins = lane != 0 && r_prev == r[0];  // the lane's first segment began in a lane before it
+    const T open = segmented_scan(run[E - 1], any_cut || !joins);
+    // the ends of segments and their sums: behind entry j, and behind the lane's last entry (lane 63's stays open)
+    bool ends[E];
+    T sum[E];
+    const T from = dpp_mov<0x138>(open);  // wave_shr:1: what the lanes before have of the lane's first segment
+    bool in_first = joins;
+#pragma unroll
+    for (int j = 0; j + 1 < E; ++j) {
+      ends[j] = cut[j] && r[j] >= 0;
+      sum[j] = in_first ? from + run[j] : run[j];
+      in_first = in_first && !cut[j];
+    }
+    ends[E - 1] = lane < kWave - 1 && r_next != r[E - 1] && r[E - 1] >= 0;
+    sum[E - 1] = open;
+    if (!emitted) {
+      bool any_end = false;
+#pragma unroll
+      for (int j = 0; j < E; ++j) any_end = any_end || ends[j];
+      const uint64_t end_mask = __builtin_amdgcn_ballot_w64(any_end);
+      if (end_mask) {  // the wave's first segment ends inside this step: it goes to the slot
+        const int f = __builtin_ctzll(end_mask);
+        int row1 = -1;
+        T val1 = T(0);
+        bool found = false;
+#pragma unroll
+        for (int j = 0; j < E; ++j) {
+          const bool here = ends[j] && !found;
+          row1 = here ? r[j] : row1;
+          val1 = here ? sum[j] : val1;
+          found = found || ends[j];
+          if (here && lane == f) ends[j] = false;
+        }
+        head_row = lane_bcast(row1, f);
+        head_val = lane_bcast(val1, f);
+        emitted = true;
+      }
+    }
+    int at = 0;
+    pending = 0;
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      const uint64_t mask = __builtin_amdgcn_ballot_w64(ends[j]);
+      at += __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+      pending += __popcll(mask);
+    }
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      if (ends[j]) {
+        out_row[at] = r[j];
+        out_sum[at] = sum[j];
+        ++at;
+      }
+    }
+    carry_row = lane_bcast(r[E - 1], kWave - 1);
+    carry_val = lane_bcast(open, kWave - 1);
+  }
+  drain();
+  if (!slots) {
+    if (lane == 0 && carry_row >= 0) atomic_add(&y[carry_row], alpha * carry_val);
+    return;
+  }
+  if (!emitted) {  // one segment (or none) in the whole wave: it is the head, there is no tail
+    head_row = carry_row;
+    head_val = carry_val;
+    carry_row = -1;
+  }
+  if (lane == 0) {
+    b_row[2 * wave] = head_row;
+    b_val[2 * wave] = head_val;
+    b_row[2 * wave + 1] = carry_row;
+    b_val[2 * wave + 1] = carry_val;
+  }
+}
+
+// The same with one entry per lane and step, for 16-byte values: four of them would lie 64 bytes apart from lane to lane,
+// and the sums that the wide form keeps for later are 20 bytes each (27-point stencil of 216 000 points, complex128: 44 us
+// this way, 69 with four entries per lane, 57 with one in the wide form).
+template <typename T, bool NTI, bool NTV>
+__global__ __launch_bounds__(kCooThreads) void coomv_narrow_kernel(int64_t nnz, int m, int n, T alpha,
                                                             const T* __restrict__ coo_val,
                                                             const int* __restrict__ coo_row,
                                                             const int* __restrict__ coo_col, int base,
@@ -191,9 +389,9 @@ int coomv_impl(hipStream_t stream, int32_t m, int32_t n, int64_t nnz, T alpha, c
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
   }
-  if (nnz == 0) return (int)hipSuccess;
+  if (nnz == 0 || n == 0) return (int)hipSuccess;  // (no column: every entry lies outside the matrix)
   // two boundary slots (row, sum) per wave in the workspace; a short workspace means longer waves
-  int per_wave = kWave * kCooSteps;
+  int per_wave = kCooWaveEntries;
   int* b_row = nullptr;
   T* b_val = nullptr;
   const size_t slot_bytes = 2 * (sizeof(T) + sizeof(int));
@@ -201,8 +399,8 @@ int coomv_impl(hipStream_t stream, int32_t m, int32_t n, int64_t nnz, T alpha, c
     const int64_t max_waves = (int64_t)(workspace_bytes / slot_bytes) / kCooWaves * kCooWaves;
     int64_t waves = (nnz + per_wave - 1) / per_wave;
     if (waves > max_waves) {
-      const int64_t steps = (nnz + max_waves * kWave - 1) / (max_waves * kWave);
-      if (steps * kWave < INT32_MAX / 2) per_wave = (int)(steps * kWave);
+      const int64_t steps = (nnz + max_waves * kCooStep - 1) / (max_waves * kCooStep);
+      if (steps * kCooStep < INT32_MAX / 2) per_wave = (int)(steps * kCooStep);
       waves = (nnz + per_wave - 1) / per_wave;
     }
     if (waves <= max_waves) {
@@ -215,9 +413,13 @@ int coomv_impl(hipStream_t stream, int32_t m, int32_t n, int64_t nnz, T alpha, c
   if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
   // (21 M-entry Laplacian, fp64: indices non-temporal and values not 100 us, all three non-temporal 107 us)
   const int policy = stream_policy((double)nnz, sizeof(T), ((double)m + (double)n) * (double)sizeof(T), false, 8.0);
+  constexpr auto kernel_of = [](auto nti, auto ntv) {
+    if constexpr (sizeof(T) > 8) return coomv_narrow_kernel<T, decltype(nti)::value, decltype(ntv)::value>;
+    else return coomv_kernel<T, decltype(nti)::value, decltype(ntv)::value>;
+  };
 #define ASAMD_COO_LAUNCH(NTI, NTV)                                                                                    \
-  coomv_kernel<T, NTI, NTV><<<(unsigned)grid, kCooThreads, 0, stream>>>(nnz, m, n, alpha, coo_val, coo_row, coo_col, base, \
-                                                                        x, y, per_wave, b_row, b_val)
+  kernel_of(std::bool_constant<NTI>{}, std::bool_constant<NTV>{})<<<(unsigned)grid, kCooThreads, 0, stream>>>(        \
+      nnz, m, n, alpha, coo_val, coo_row, coo_col, base, x, y, per_wave, b_row, b_val)
   if (policy == 0) ASAMD_COO_LAUNCH(false, false);
   else if (policy == kStreamNtValues) ASAMD_COO_LAUNCH(false, true);
   else if (policy == kStreamNtIndices) ASAMD_COO_LAUNCH(true, false);
