@@ -258,21 +258,30 @@ extern "C" int asamd_csr2ell_width(hipStream_t stream, int32_t m, const int32_t*
 }
 
 // ---------------------------------------------------------------------------
-// csr2ell: a workgroup owns kEllRows consecutive rows.  Their entries form one
+// csr2ell: a workgroup owns up to kEllRows consecutive rows.  Their entries form one
 // contiguous range of the CSR streams, which is read coalesced into LDS in
 // windows; slot s of row j is then written to [s*m + j], consecutive lanes on
 // consecutive rows, so both sides of the transpose stay coalesced.  Rows longer
 // than the LDS window are read from global memory directly.
 // ---------------------------------------------------------------------------
 constexpr int kEllRows = 256;
-// Staged entries per workgroup (at most half of it for 16-byte values): as many as 256 rows of the ELL's width hold, so
-// that short rows leave room for more workgroups on a compute unit -- always 4 096 were 50 KB for 8-byte values, three
-// workgroups (5-point Laplacian of 4 M rows, fp64: 102 -> 93 us).
+// Staged entries per workgroup, at most (half of it for 16-byte values): 32 KiB of staged values.  A workgroup takes as
+// many of 256, 128, 64, 32 rows as fit at the ELL's width -- rows that did not fit were read from global memory, a row
+// length apart from lane to lane (27-point stencil of 753 000 points, fp64, all three conversion calls: 438 -> 144 us) --
+// and asks for LDS for those rows only: always 4 096 entries were 50 KB for 8-byte values, three workgroups on a compute
+// unit (5-point Laplacian of 4 M rows, fp64: 102 -> 93 us).  Wider than 32 rows fit: 256 rows, not staged.
 constexpr int kEllWindow = 4096;
 template <typename T>
+constexpr int kEllMost = sizeof(T) > 8 ? kEllWindow / 2 : kEllWindow;
+template <typename T>
+constexpr int ell_rows(int width) {
+  for (int rows = kEllRows; rows >= 32; rows /= 2)
+    if (width <= kEllMost<T> / rows) return rows;
+  return kEllRows;
+}
+template <typename T>
 constexpr int ell_window(int width) {
-  const int most = sizeof(T) > 8 ? kEllWindow / 2 : kEllWindow;  // at most 32 KiB of staged values
-  return width < most / kEllRows ? width * kEllRows : most;
+  return width < kEllMost<T> / ell_rows<T>(width) ? width * ell_rows<T>(width) : kEllMost<T>;
 }
 // staged entry p lives at p + p / 32: lanes read slot s of consecutive rows, i.e. positions a row
 // length apart, and without the skew rows of 16 or 32 entries would all fall into a few LDS banks
@@ -285,14 +294,16 @@ template <typename T, bool NTS, bool WIDE>
 __global__ __launch_bounds__(kEllRows) void csr2ell_kernel(
     int m, const T* __restrict__ val, const int* __restrict__ row_ptr,
     const int* __restrict__ col_ind, int csr_base, int ell_base, int width,
-    T* __restrict__ ell_val, int* __restrict__ ell_col, int window, const int* __restrict__ gate) {
+    T* __restrict__ ell_val, int* __restrict__ ell_col, int window, int rows, const int* __restrict__ gate) {
   if (gate && *gate == 0) return;  // a refresh behind the value guard: nothing has changed
   extern __shared__ __align__(16) unsigned char s_ell[];  // ell_at(window) values, then as many columns
   T* s_val = reinterpret_cast<T*>(s_ell);
   int* s_col = reinterpret_cast<int*>(s_ell + (size_t)ell_at(window) * sizeof(T));
-  const int64_t row_first = (int64_t)blockIdx.x * kEllRows;
-  const int64_t row = row_first + threadIdx.x;
-  int64_t row_last = row_first + kEllRows;
+  // a power of two of rows, kEllRows / rows threads each: those take the row's slots in turn
+  const int64_t row_first = (int64_t)blockIdx.x * rows;
+  const int64_t row = row_first + (threadIdx.x & (rows - 1));
+  const int first_slot = threadIdx.x / rows, slot_step = kEllRows / rows;
+  int64_t row_last = row_first + rows;
   if (row_last > m) row_last = m;
   const int64_t blk_begin = (int64_t)row_ptr[row_first] - csr_base;
   const int64_t blk_end = (int64_t)row_ptr[row_last] - csr_base;
@@ -376,7 +387,7 @@ __global__ __launch_bounds__(kEllRows) void csr2ell_kernel(
   }
   if (row >= m) return;
   const int len = (int)(my_end - my_begin);
-  for (int s = 0; s < width; ++s) {
+  for (int s = first_slot; s < width; s += slot_step) {
     T v = T(0);
     int c = ell_base;
     if (s < len) {
@@ -407,14 +418,15 @@ static int csr2ell_impl(hipStream_t stream, int m, const T* val, const int* rp, 
   if (!val || !rp || !ci || !ell_val || !ell_col || m <= 0 || width < 0) return hipErrorInvalidValue;
   if (((uintptr_t)val | (uintptr_t)ell_val) % alignof(T)) return hipErrorInvalidValue;
   if (width == 0) return hipSuccess;
-  const unsigned grid = (unsigned)(((int64_t)m + kEllRows - 1) / kEllRows);
+  const int rows = ell_rows<T>(width);
+  const unsigned grid = (unsigned)(((int64_t)m + rows - 1) / rows);
   const bool nts = stores_bypass_caches((size_t)m * (size_t)width * (sizeof(T) + sizeof(int)));
   const bool wide = (((uintptr_t)val | (uintptr_t)ci) & 15u) == 0;
   const int window = ell_window<T>(width);
   const size_t lds = (size_t)ell_at(window) * (sizeof(T) + sizeof(int));
 #define ASAMD_CSR2ELL(NTS, WIDE)                                                                                      \
   csr2ell_kernel<T, NTS, WIDE><<<grid, kEllRows, lds, stream>>>(m, val, rp, ci, csr_base, ell_base, width, ell_val,   \
-                                                                ell_col, window, gate)
+                                                                ell_col, window, rows, gate)
   if (nts && wide) ASAMD_CSR2ELL(true, true);
   else if (nts) ASAMD_CSR2ELL(true, false);
   else if (wide) ASAMD_CSR2ELL(false, true);
