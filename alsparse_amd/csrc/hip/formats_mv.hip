@@ -25,8 +25,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <type_traits>
-
 #include "alsparse_amd_kernels.h"
 #include "device_utils.hpp"
 #include "spmv_ell.hpp"
@@ -413,17 +411,21 @@ int coomv_impl(hipStream_t stream, int32_t m, int32_t n, int64_t nnz, T alpha, c
   if (grid > 0x7fffffff) return (int)hipErrorInvalidValue;
   // (21 M-entry Laplacian, fp64: indices non-temporal and values not 100 us, all three non-temporal 107 us)
   const int policy = stream_policy((double)nnz, sizeof(T), ((double)m + (double)n) * (double)sizeof(T), false, 8.0);
-  constexpr auto kernel_of = [](auto nti, auto ntv) {
-    if constexpr (sizeof(T) > 8) return coomv_narrow_kernel<T, decltype(nti)::value, decltype(ntv)::value>;
-    else return coomv_kernel<T, decltype(nti)::value, decltype(ntv)::value>;
-  };
-#define ASAMD_COO_LAUNCH(NTI, NTV)                                                                                    \
-  kernel_of(std::bool_constant<NTI>{}, std::bool_constant<NTV>{})<<<(unsigned)grid, kCooThreads, 0, stream>>>(        \
-      nnz, m, n, alpha, coo_val, coo_row, coo_col, base, x, y, per_wave, b_row, b_val)
-  if (policy == 0) ASAMD_COO_LAUNCH(false, false);
-  else if (policy == kStreamNtValues) ASAMD_COO_LAUNCH(false, true);
-  else if (policy == kStreamNtIndices) ASAMD_COO_LAUNCH(true, false);
-  else ASAMD_COO_LAUNCH(true, true);
+  // (the kernel is named in the launch: through a pointer that a lambda returned, clang's function sanitizer read the words
+  // in front of the kernel's handle as a callee's and left the launch out)
+#define ASAMD_COO_LAUNCH(KERNEL, NTI, NTV)                                                                            \
+  KERNEL<T, NTI, NTV><<<(unsigned)grid, kCooThreads, 0, stream>>>(nnz, m, n, alpha, coo_val, coo_row, coo_col, base,  \
+                                                                  x, y, per_wave, b_row, b_val)
+#define ASAMD_COO_BY_POLICY(KERNEL)                                                 \
+  do {                                                                              \
+    if (policy == 0) ASAMD_COO_LAUNCH(KERNEL, false, false);                        \
+    else if (policy == kStreamNtValues) ASAMD_COO_LAUNCH(KERNEL, false, true);      \
+    else if (policy == kStreamNtIndices) ASAMD_COO_LAUNCH(KERNEL, true, false);     \
+    else ASAMD_COO_LAUNCH(KERNEL, true, true);                                      \
+  } while (0)
+  if constexpr (sizeof(T) > 8) ASAMD_COO_BY_POLICY(coomv_narrow_kernel);
+  else ASAMD_COO_BY_POLICY(coomv_kernel);
+#undef ASAMD_COO_BY_POLICY
 #undef ASAMD_COO_LAUNCH
   if (b_row) {
     const int64_t slots = grid * kCooWaves * 2;
