@@ -363,10 +363,9 @@ static void spmm_rows(const SpmmCall<T>& a, int n, int k, const T* B, int64_t ld
   const bool whole_lines = (ldb * (int64_t)sizeof(T)) % 128 == 0 && (uintptr_t)B % 128 == 0;
   const bool colc = a.c_row == 1 && a.c_col != 1;
   const int full = (whole_lines || colc ? 1 : 2) * kGroupBytes / (int)sizeof(T);
-  const int chunks = (n + full - 1) / full;
-  const int chunk = ((n + chunks - 1) / chunks + V - 1) / V * V;
+  const GroupChunks g = group_chunks(n, full, V);
   const unsigned __int128 span = (unsigned __int128)(k > 0 ? k - 1 : 0) * (unsigned __int128)ldb * sizeof(T) + (uint64_t)n * sizeof(T);
-  spmm_group<T>(a, n, chunk, (n + chunk - 1) / chunk, B, ldb, chunk,
+  spmm_group<T>(a, n, g.chunk, g.count, B, ldb, g.chunk,
                 k > 0 && span < ((unsigned __int128)1 << 31) ? (uint64_t)span : 0, false, C);
 }
 

@@ -78,12 +78,48 @@ __device__ __forceinline__ void for_each_const(F& f, std::integer_sequence<int, 
   (f(std::integral_constant<int, U>{}), ...);
 }
 
+// ---- which columns a lane takes (host and device: the arithmetic is checked without a GPU) --------------------
+// `count` chunks of `chunk` columns, whole loads of v each, as even as that allows; the last ends with column n and may hold
+// fewer than v columns (n = 961, at most 64 a chunk, v = 4: fifteen of 64, then one column).
+struct GroupChunks {
+  int chunk, count;
+};
+__host__ __device__ constexpr GroupChunks group_chunks(int n, int most, int v) {
+  const int even = (int)(((int64_t)n + most - 1) / most);
+  const int chunk = (int)((((int64_t)n + even - 1) / even + v - 1) / v * v);
+  return {chunk, (int)(((int64_t)n + chunk - 1) / chunk)};
+}
+
+// The lane at column c of a chunk of cn columns loads V columns from c0 on and stores all but the first `first` of them.
+// Where the chunk ends inside a load it is moved back (what its neighbour has as well is `first`), into the chunk before
+// where this one holds fewer than V columns: c0 is negative then, and every row of B has the columns there.  Lanes past the
+// end load what is sure to be there and store nothing.  padded: 16 bytes behind a row may be read, nothing is moved.
+struct GroupColumns {
+  int c0, first;
+  bool owns;
+};
+template <int V>
+__host__ __device__ constexpr GroupColumns group_columns(int c, int cn, bool padded) {
+  const int last = padded || cn - V > c ? c : cn - V;
+  if (c < cn) return {last, c - last, true};
+  return {padded || cn >= V ? 0 : cn - V, 0, false};
+}
+
+// Where that load begins, in bytes: from B's row on (`narrow`: offsets into all of B, never negative there), otherwise from
+// the chunk's first column on, which may be negative and stays signed when it is added to a 64-bit address.
+__host__ __device__ constexpr int group_lane_bytes(bool narrow, int64_t chunk_bytes, int c0, int size) {
+  return (int)((narrow ? chunk_bytes : 0) + (int64_t)c0 * size);
+}
+__host__ __device__ constexpr int64_t group_far_bytes(int row_hi, unsigned row_lo, int lane_bytes) {
+  return (int64_t)(((uint64_t)(unsigned)row_hi << 32) | row_lo) + lane_bytes;
+}
+
 // where a lane's L pieces of a row of B lie
 template <bool NARROW, int L>
 struct GroupB {
-  BufferRsrc rsrc;         // NARROW: all of B, within 2 GiB
-  const char* p;           // otherwise: the chunk's first column of row 0
-  unsigned lane_bytes[L];  // the lane's pieces of row 0 there, in bytes
+  BufferRsrc rsrc;    // NARROW: all of B, within 2 GiB
+  const char* p;      // otherwise: the chunk's first column of row 0
+  int lane_bytes[L];  // group_lane_bytes of the lane's pieces
   int64_t row_bytes;
 };
 
@@ -138,7 +174,7 @@ __device__ __forceinline__ void group_work(const GroupBlock<T>& e, T alpha, int 
       const unsigned lo = (unsigned)part_bcast<GC, J0 + U>((int)off, upper);
       if constexpr (NARROW) {
 #pragma unroll
-        for (int q = 0; q < L; ++q) bv[U][q] = buffer_load<GroupVec<T>>(b.rsrc, (int)(lo + b.lane_bytes[q]));
+        for (int q = 0; q < L; ++q) bv[U][q] = buffer_load<GroupVec<T>>(b.rsrc, (int)(lo + (unsigned)b.lane_bytes[q]));
       } else {
         has[U] = part_bcast<GC, J0 + U>((int)e.live, upper) != 0;
         const int hi = part_bcast<GC, J0 + U>(off_hi, upper);
@@ -146,7 +182,7 @@ __device__ __forceinline__ void group_work(const GroupBlock<T>& e, T alpha, int 
 #pragma unroll
           for (int q = 0; q < L; ++q)
             bv[U][q] = __builtin_bit_cast(
-                GroupVec<T>, *reinterpret_cast<const GroupLoose<T>*>(b.p + (((int64_t)hi << 32) | lo) + b.lane_bytes[q]));
+                GroupVec<T>, *reinterpret_cast<const GroupLoose<T>*>(b.p + group_far_bytes(hi, lo, b.lane_bytes[q])));
         }
       }
     };
@@ -265,8 +301,6 @@ __global__ __launch_bounds__(kGroupThreads) void spmm_group_kernel(
   const int cl = threadIdx.x % GC;
   const int cbeg = blockIdx.y * chunk;
   const int cn = n - cbeg < chunk ? n - cbeg : chunk;
-  // the lane's columns: V from c0 on; the last lane's are moved back where the chunk ends inside them (`first`: how many
-  // of them its neighbour has as well), lanes past the end load what lane 0 loads and store nothing
   int c0[L], first[L];
   bool owns[L];
   GroupB<NARROW, L> b;
@@ -275,18 +309,11 @@ __global__ __launch_bounds__(kGroupThreads) void spmm_group_kernel(
   b.row_bytes = ldb * (int64_t)sizeof(T);
 #pragma unroll
   for (int q = 0; q < L; ++q) {
-    c0[q] = q * kCols + cl * V;
-    first[q] = 0;
-    owns[q] = c0[q] < cn && threadIdx.x % 16 < GC;
-    if (c0[q] >= cn) {
-      c0[q] = 0;
-    } else if (c0[q] + V > cn && !b_padded) {
-      first[q] = c0[q] + V - cn;
-      c0[q] = cn - V;
-    }
-    // (relative to B, not to the chunk: the columns moved back may lie in the chunk before)
-    const int64_t at = (NARROW ? (int64_t)blockIdx.y * b_chunk_bytes : 0) + (int64_t)c0[q] * (int64_t)sizeof(T);
-    b.lane_bytes[q] = (unsigned)at;
+    const GroupColumns mine = group_columns<V>(q * kCols + cl * V, cn, b_padded);
+    c0[q] = mine.c0;
+    first[q] = mine.first;
+    owns[q] = mine.owns && threadIdx.x % 16 < GC;
+    b.lane_bytes[q] = group_lane_bytes(NARROW, (int64_t)blockIdx.y * b_chunk_bytes, mine.c0, (int)sizeof(T));
   }
   auto put = [&](int r, const T(&acc)[L * V]) {  // the tile's row r: the lanes that own columns
 #pragma unroll
