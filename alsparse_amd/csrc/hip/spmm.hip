@@ -376,13 +376,16 @@ static int csrmm_impl(hipStream_t s, int m, int n, int k, int nnz, T alpha, cons
   if (!val || !rp || !ci || !B || !C || !st || m <= 0 || n <= 0) return hipErrorInvalidValue;
   if (((uintptr_t)val | (uintptr_t)B | (uintptr_t)C) % alignof(T)) return hipErrorInvalidValue;
   const SpmmCall<T> a{s, m, k, nnz, alpha, val, rp, ci, base, beta, st->c_row_stride, st->c_col_stride};
-  if (n == 1 || st->b_col_stride == 1) {
+  // The row kernels load entry 0 for a lane without one: a matrix without entries is the strided kernel's, which then reads
+  // row_ptr only.
+  const bool entries = nnz > 0;
+  if (entries && (n == 1 || st->b_col_stride == 1)) {
     // rows of op(B) are contiguous; C in either layout (a single dense column has unit stride whatever the layout says)
     if (n == 1 || st->c_col_stride == 1 || st->c_row_stride == 1) {
       spmm_rows<T>(a, n, k, B, st->b_row_stride, C);
       return hipGetLastError();
     }
-  } else if (colmajor_nn(st, n) && ws && k > 0 && (uintptr_t)ws % 16 == 0 && ws_bytes >= workspace_bytes(sizeof(T), n, k, st)) {
+  } else if (entries && colmajor_nn(st, n) && ws && k > 0 && (uintptr_t)ws % 16 == 0 && ws_bytes >= workspace_bytes(sizeof(T), n, k, st)) {
     const PanelPlan plan = plan_panels((int)sizeof(T), n, k);
     int c0 = 0;
     for (int i = 0; i < plan.kinds; ++i) {

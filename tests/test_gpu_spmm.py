@@ -361,3 +361,30 @@ def test_widths_around_the_tiles(gpu, lengths, dtype):
                 check(a, 1.25, B.reshape(n, -1).T, beta, C0.reshape(n, -1).T, out.reshape(n, -1).T, "column-major n=%d" % n)
     finally:
         da.free()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("n", [1, 5, 70])
+def test_kernel_abi_without_entries(gpu, n, dtype):
+    """asamd_?_csrmm_ws on a matrix without entries, whose arrays hold nothing: C = beta * C in both layouts.  (The public
+    calls return before that and leave C alone.)"""
+    lib = capi.load()
+    m, k = 100, 30
+    T = capi.scalar_type(dtype)
+    C0, B = wl.uniform(m * n, dtype, 4), wl.uniform(k * n, dtype, 5)
+    rp, empty = hiprt.DeviceArray.from_numpy(np.ones(m + 1, dtype=np.int32)), hiprt.DeviceArray((0,), dtype)
+    dB, ws = hiprt.DeviceArray.from_numpy(B), hiprt.DeviceArray((1 << 20,), np.uint8)
+    try:
+        for st in (capi.asamd_dense_strides(n, 1, n, 1), capi.asamd_dense_strides(1, k, 1, m), capi.asamd_dense_strides(n, 1, 1, m)):
+            for beta in (0.0, 0.5):
+                announce("csrmm_ws without entries", n, np.dtype(dtype).name, st.b_row_stride, st.c_row_stride, beta)
+                dC = hiprt.DeviceArray.from_numpy(np.full_like(C0, np.nan) if beta == 0 else C0)
+                assert getattr(lib, "asamd_%s_csrmm_ws" % capi.prefix(dtype))(
+                    None, m, n, k, 0, T(1.5), empty.c_ptr(), rp.c_ptr(), empty.c_ptr(), 1, dB.c_ptr(), T(beta), dC.c_ptr(),
+                    byref(st), ws.c_ptr(), 1 << 20) == 0
+                hiprt.synchronize()
+                assert np.array_equal(dC.to_numpy(), (C0 * dtype(beta)).astype(dtype))
+                dC.free()
+    finally:
+        for d in (rp, empty, dB, ws):
+            d.free()
