@@ -311,17 +311,18 @@ static void spmm_short(const SpmmCall<T>& a, int n, const T* B, int64_t ldb, T* 
 template <typename T, int GC, bool COLC, int L>
 static void launch_group(const SpmmCall<T>& a, int n, int chunk, int chunks, const T* B, int64_t ldb, int64_t chunk_elems,
                          uint64_t span, bool padded, T* C) {
-  constexpr int tile = COLC ? kWave : kGroupRows;
-  const dim3 grid((unsigned)(((int64_t)a.m + tile - 1) / tile), (unsigned)chunks);
+  constexpr int full = COLC ? kWave : kGroupRows;
+  const GroupTile tile = group_tile(a.m, chunks, full);
+  const dim3 grid((unsigned)(((int64_t)a.m + tile.rows - 1) / tile.rows), (unsigned)chunks);
   // Beyond the memory-side cache together: C, which is touched once, should not push B out of it, and B's rows mostly
   // come from memory (FAR, where rows of sixteen entries and more fill the groups' blocks).
   const bool big = ((double)a.k + (double)a.m) * (double)n * (double)sizeof(T) > 256.0e6;
 #define ASAMD_GROUP(NARROW, FAR)                                                                               \
   spmm_group_kernel<T, GC, NARROW, COLC, L, FAR><<<grid, kGroupThreads, 0, a.s>>>(                             \
       a.m, n, a.alpha, a.val, a.rp, a.ci, a.base, B, ldb, chunk_elems * (int64_t)sizeof(T), (unsigned)span, padded, \
-      a.beta, C, a.c_row, a.c_col, chunk, big)
+      a.beta, C, a.c_row, a.c_col, chunk, tile, big)
   if constexpr (GC == 16) {
-    if (span > 0 && (big || L == 2) && a.nnz >= 16 * (int64_t)a.m) {
+    if (span > 0 && tile.rows == full && (big || L == 2) && a.nnz >= 16 * (int64_t)a.m) {
       ASAMD_GROUP(true, true);
       return;
     }

@@ -90,6 +90,24 @@ __host__ __device__ constexpr GroupChunks group_chunks(int n, int most, int v) {
   return {chunk, (int)(((int64_t)n + chunk - 1) / chunk)};
 }
 
+// How many rows of A a workgroup takes, and from how many entries on its sixteen groups share a row.  Whole tiles (`most`
+// rows) where those make two workgroups per compute unit; fewer rows where the matrix has not so many, down to one: a
+// workgroup takes its long rows one after the other, and groups without a row are what shared rows are dealt to.
+// us, whole tiles against this: 2 000 rows of 1 500 entries, fp32, n = 64: 168 -> 49; 400 of 4 000, fp64, n = 40: 1 255 -> 83;
+// 512 of 8 000, column-major, fp32, n = 16: 1 043 -> 37.  Against four workgroups per compute unit: 4 000 rows of 64, n = 64:
+// 5.9 (7.3), 2 000 of 1 500, n = 64: 49 (60), n = 200: 300 (233).
+constexpr int kGroupFill = 512;
+constexpr int kGroupLongLeast = 64;  // entries: the join of the groups' sums is not worth less (400 rows of 40: the same)
+struct GroupTile {
+  int rows, long_row;
+};
+__host__ __device__ constexpr GroupTile group_tile(int m, int chunks, int most) {
+  int rows = most;
+  while (rows > 1 && ((int64_t)m + rows - 1) / rows * chunks < kGroupFill) rows /= 2;
+  const int share = rows < kGroupRows ? kGroupLongRow / kGroupRows * rows : kGroupLongRow;
+  return {rows, share < kGroupLongLeast ? kGroupLongLeast : share};
+}
+
 // The lane at column c of a chunk of cn columns loads V columns from c0 on and stores all but the first `first` of them.
 // Where the chunk ends inside a load it is moved back (what its neighbour has as well is `first`), into the chunk before
 // where this one holds fewer than V columns: c0 is negative then, and every row of B has the columns there.  Lanes past the
@@ -135,10 +153,10 @@ struct GroupBlock {
 };
 
 template <typename T, int GC>
-__device__ __forceinline__ GroupBlock<T> group_fetch(int64_t j0, int64_t end, const T* __restrict__ val,
+__device__ __forceinline__ GroupBlock<T> group_fetch(unsigned j0, unsigned end, const T* __restrict__ val,
                                                      const int* __restrict__ col_ind) {
   const int l16 = threadIdx.x & 15;
-  const int64_t j = j0 + l16 / GC + (16 / GC) * (l16 % GC);
+  const unsigned j = j0 + l16 / GC + (16 / GC) * (l16 % GC);
   GroupBlock<T> e;
   e.live = j < end;
   // Every lane loads, the ones past the end entry 0 (there is one): a load under a branch would be waited for where the
@@ -224,14 +242,16 @@ __device__ __forceinline__ void group_work(const GroupBlock<T>& e, T alpha, int 
   for_each_const(four, std::make_integer_sequence<int, GC / 4>{});
 }
 
-// acc += the entries [j0, end) of a row, every group with a range of its own; the parts' sums are not yet joined
+// acc += the blocks of sixteen entries of a row at j0, j0 + step, ... before `end`, every group with blocks of its own; the
+// parts' sums are not yet joined.  (Positions are below 2^31, so that an unsigned one a step past the end has not wrapped;
+// 64-bit ones took 2 to 14 registers more.)
 template <typename T, int GC, bool NARROW, int L, bool FAR>
-__device__ __forceinline__ void group_walk(int64_t j0, int64_t end, T alpha, const T* __restrict__ val,
+__device__ __forceinline__ void group_walk(unsigned j0, unsigned end, unsigned step, T alpha, const T* __restrict__ val,
                                            const int* __restrict__ col_ind, int base, const GroupB<NARROW, L>& b,
                                            T (&acc)[L * kGroupV<T>]) {
   GroupBlock<T> cur = group_fetch<T, GC>(j0, end, val, col_ind);
-  while (__builtin_amdgcn_ballot_w64(j0 + 16 < end)) {  // the next sixteen travel while these are worked on
-    j0 += 16;
+  while (__builtin_amdgcn_ballot_w64(j0 + step < end)) {  // the next sixteen travel while these are worked on
+    j0 += step;
     const GroupBlock<T> next = group_fetch<T, GC>(j0, end, val, col_ind);
     group_work<T, GC, NARROW, L, FAR>(cur, alpha, base, b, acc);
     cur = next;
@@ -275,8 +295,8 @@ __device__ __forceinline__ void group_store_row(T* __restrict__ c, int first, co
   }
 }
 
-// grid.x: blocks of kGroupRows rows (COLC: kWave); grid.y: chunks of `chunk` dense columns, chunk y at
-// B + y * b_chunk_bytes (b_bytes: what may be read from B on, NARROW only).  ldb in elements; C element (r, c) at
+// grid.x: blocks of tile.rows rows, a power of two of at most kGroupRows (COLC: kWave; FAR: exactly that many); grid.y:
+// chunks of `chunk` dense columns, chunk y at B + y * b_chunk_bytes (b_bytes: what may be read from B on, NARROW only).  ldb in elements; C element (r, c) at
 // r * c_row + c * c_col (one of the two strides is 1: COLC when it is the rows').  b_padded: 16 bytes behind every row of
 // B may be read (a layout made here); otherwise n is at least kGroupV<T>.  L: 128-bit loads per lane and row of B, the
 // chunk's columns [q * GC * V, (q + 1) * GC * V) in load q.  c_nt: row-major C, which is touched once, bypasses the caches.
@@ -285,7 +305,7 @@ template <typename T, int GC, bool NARROW, bool COLC, int L, bool FAR>
 __global__ __launch_bounds__(kGroupThreads) void spmm_group_kernel(
     int m, int n, T alpha, const T* __restrict__ val, const int* __restrict__ row_ptr, const int* __restrict__ col_ind,
     int base, const T* __restrict__ B, int64_t ldb, int64_t b_chunk_bytes, unsigned b_bytes, bool b_padded, T beta,
-    T* __restrict__ C, int64_t c_row, int64_t c_col, int chunk, bool c_nt) {
+    T* __restrict__ C, int64_t c_row, int64_t c_col, int chunk, GroupTile tile, bool c_nt) {
   constexpr int V = kGroupV<T>;
   constexpr int kCols = GC * V;
   constexpr int kTileRows = COLC ? kWave : kGroupRows;
@@ -294,9 +314,13 @@ __global__ __launch_bounds__(kGroupThreads) void spmm_group_kernel(
   __shared__ int s_ptr[kTileRows + 1];
   static_assert(!COLC || L == 1, "column-major C with one load per lane");
   const unsigned bid = xcd_contiguous_id(blockIdx.x, gridDim.x);
-  const int64_t row0 = (int64_t)bid * kTileRows;
-  const int nrows = m - row0 < kTileRows ? (int)(m - row0) : kTileRows;
-  if (threadIdx.x <= nrows) s_ptr[threadIdx.x] = row_ptr[row0 + threadIdx.x];
+  // (FAR: constants, runtime values took 30 to 50 registers more and two of six waves per SIMD there)
+  const int tile_rows = FAR ? kTileRows : tile.rows;
+  const int long_row = FAR ? kGroupLongRow : tile.long_row;
+  const int64_t row0 = (int64_t)bid * tile_rows;
+  if (row0 >= m) return;
+  const int nrows = m - row0 < tile_rows ? (int)(m - row0) : tile_rows;
+  if ((int)threadIdx.x <= nrows) s_ptr[threadIdx.x] = row_ptr[row0 + threadIdx.x];
   const int group = threadIdx.x / 16;
   const int lane = threadIdx.x % kWave;
   const int cl = threadIdx.x % GC;
@@ -340,36 +364,36 @@ __global__ __launch_bounds__(kGroupThreads) void spmm_group_kernel(
   __syncthreads();
 #pragma unroll 1
   for (int pass = 0; pass < kTileRows / kGroupRows; ++pass) {
+    if (pass > 0 && pass * kGroupRows >= nrows) break;
     const int r = pass * kGroupRows + group;
-    int64_t start = 0, end = 0;
+    int start = 0, end = 0;
     bool there = r < nrows;
     if (there) {
-      start = (int64_t)s_ptr[r] - base;
-      end = (int64_t)s_ptr[r + 1] - base;
+      start = s_ptr[r] - base;
+      end = s_ptr[r + 1] - base;
     }
-    if (end - start > kGroupLongRow) {
+    if (end - start > long_row) {
       there = false;
       end = start;
     }
     T acc[L * V];
 #pragma unroll
     for (int i = 0; i < L * V; ++i) acc[i] = T(0);
-    group_walk<T, GC, NARROW, L, FAR>(start, end, alpha, val, col_ind, base, b, acc);
+    group_walk<T, GC, NARROW, L, FAR>(start, end, 16, alpha, val, col_ind, base, b, acc);
     group_join<GC>(acc);
     if (there) put(r, acc);
   }
-  // the workgroup's long rows, one after the other, their entries dealt to the groups
-  uint64_t long_rows = __builtin_amdgcn_ballot_w64(lane < nrows && s_ptr[lane + 1] - s_ptr[lane] > kGroupLongRow);
+  // The workgroup's long rows, one after the other.  The groups take blocks of sixteen in turn, so that a workgroup sweeps the
+  // row together: rows of ascending columns then read neighbouring rows of B at one time (a sixteenth of the row each:
+  // 2 000 rows of 1 500, fp32, n = 64, 71 us against 49).
+  uint64_t long_rows = __builtin_amdgcn_ballot_w64(lane < nrows && s_ptr[lane + 1] - s_ptr[lane] > long_row);
   for (; long_rows; long_rows &= long_rows - 1) {  // (the same in every wave)
     const int r = __builtin_ctzll(long_rows);
-    const int64_t start = (int64_t)s_ptr[r] - base, end = (int64_t)s_ptr[r + 1] - base;
-    const int64_t per = ((end - start + kGroupRows - 1) / kGroupRows + 15) & ~(int64_t)15;
-    const int64_t mine0 = start + per * group < end ? start + per * group : end;
-    const int64_t mine1 = mine0 + per < end ? mine0 + per : end;
+    const int start = s_ptr[r] - base, end = s_ptr[r + 1] - base;
     T acc[L * V];
 #pragma unroll
     for (int i = 0; i < L * V; ++i) acc[i] = T(0);
-    group_walk<T, GC, NARROW, L, FAR>(mine0, mine1, alpha, val, col_ind, base, b, acc);
+    group_walk<T, GC, NARROW, L, FAR>(start + 16 * group, end, 16 * kGroupRows, alpha, val, col_ind, base, b, acc);
     group_join<GC>(acc);
     if (threadIdx.x % 16 < GC) {
 #pragma unroll

@@ -1,6 +1,6 @@
 // TEST INFRASTRUCTURE.  The column arithmetic of the sixteen-lane SpMM groups (spmm_group.hpp), enumerated on the host: for
 // every width, element size and chunk width each lane's load lies inside its row of B, in both address forms, and
-// every column is stored once.  Prints the first violation and returns 1, or returns 0.
+// every column is stored once; and the rows that a workgroup takes, for every number of rows.  Prints the first violation and returns 1, or returns 0.
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -51,8 +51,25 @@ static bool check(int chunk_bytes_most) {
   return V == 1 || narrow_chunks > 0;
 }
 
+// Every row is one workgroup's: a power of two of rows each, the last workgroup begins before row m.
+static bool check_tiles() {
+  for (int most : {kGroupRows, (int)kWave})
+    for (int chunks : {1, 2, 4, 1000})
+      for (int64_t m = 1; m < 2147483647; m = m < 70000 ? m + 1 : m * 3 + 1) {
+        const GroupTile t = group_tile((int)m, chunks, most);
+        const int64_t grid = (m + t.rows - 1) / t.rows;
+        const bool whole = (m + most - 1) / most * chunks >= kGroupFill;
+        if (t.rows < 1 || t.rows > most || (t.rows & (t.rows - 1)) || (grid - 1) * t.rows >= m || grid * t.rows < m ||
+            t.long_row < kGroupLongLeast || t.long_row > kGroupLongRow || (whole && (t.rows != most || t.long_row != kGroupLongRow))) {
+          printf("m = %lld, %d chunks, tiles of at most %d: %d rows, long from %d\n", (long long)m, chunks, most, t.rows, t.long_row);
+          return false;
+        }
+      }
+  return true;
+}
+
 int main() {
-  bool ok = true;
+  bool ok = check_tiles();
   for (int bytes : {kGroupBytes, 2 * kGroupBytes}) ok = check<4>(bytes) && check<8>(bytes) && check<16>(bytes) && ok;
   return ok ? 0 : 1;
 }

@@ -388,3 +388,32 @@ def test_kernel_abi_without_entries(gpu, n, dtype):
     finally:
         for d in (rp, empty, dB, ws):
             d.free()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.complex128], ids=["f32", "f64", "c128"])
+@pytest.mark.parametrize("m,chunks", [(1, 1), (5, 3), (511, 1), (513, 1), (2049, 1), (8191, 1), (8193, 1), (130, 5)])
+def test_few_rows_of_many_entries(gpu, m, chunks, dtype):
+    """Matrices of so few rows that a workgroup takes one, two, ... sixteen of them (sixty-four with column-major C), and rows
+    around the lengths from which its groups share a row (64 to 256, by the rows it takes)."""
+    from helpers_shapes import complex_vector
+    vector = complex_vector if np.dtype(dtype).kind == "c" else wl.uniform
+    rng = np.random.default_rng(m)
+    lengths = rng.choice([0, 1, 17, 63, 64, 65, 128, 129, 256, 257], size=m, p=[0.1] * 10 if m < 1000 else [0.3, 0.3, 0.3] + [0.1 / 7] * 7)
+    lengths[0] = 1025
+    row_ptr = np.concatenate([[0], np.cumsum(lengths)])
+    col = rng.integers(0, 900, size=int(row_ptr[-1]))
+    a = wl.Csr(m, 900, row_ptr.astype(np.int32), col.astype(np.int32), vector(col.size, dtype, 7), 0, "few rows")
+    n = 16 * (16 // np.dtype(dtype).itemsize) * chunks + (chunks > 1)
+    B, C0 = vector(900 * n, dtype, 5), vector(m * n, dtype, 4)
+    da = DeviceCsr(a)
+    try:
+        for layout, row, b, c in ((capi.ALPHA_SPARSE_LAYOUT_ROW_MAJOR, True, n, n), (capi.ALPHA_SPARSE_LAYOUT_COLUMN_MAJOR, False, 900, m)):
+            announce("spmm few rows", m, n, np.dtype(dtype).name, layout)
+            out = run_csrmm(gpu, da, layout, 0, 1.25, B, b, 0.5, C0, c, n, 900)
+            B2, C02, C2 = (np.ascontiguousarray(v.reshape(-1, n) if row else v.reshape(n, -1).T) for v in (B, C0, out))
+            ref = orc.csrmm_plain(a, 1.25, B2, 0.5, C02)
+            err = orc.csrmm_err(a, 1.25, B2, 0.5, C02, C2, ref)
+            tol = 1e-4 if np.dtype(dtype) == np.float32 else 1e-12
+            assert err.zero_den_mismatch == 0 and err.full <= tol, (m, n, err)
+    finally:
+        da.free()

@@ -1,5 +1,5 @@
 """Which columns of B and C the lanes of the sixteen-lane SpMM groups take, for every width up to 36 chunks and both address
-forms (tests/host_checks/group_columns.hip, compiled for the host and run: no GPU)."""
+forms, and which rows of A their workgroups (tests/host_checks/group_columns.hip, compiled for the host and run: no GPU)."""
 import os
 import subprocess
 
