@@ -357,14 +357,15 @@ static void spmm_rows(const SpmmCall<T>& a, int n, int k, const T* B, int64_t ld
     spmm_short<T>(a, n, B, ldb, C);
     return;
   }
-  // Chunks of equal widths (whole 128-bit loads): 79 columns of fp32 are 40 and 39, not 64 and 15.  256 bytes wide where
-  // the chunks are whole cache lines: one slice of B is live at a time.  Where they are not, every chunk of a row begins
-  // and ends inside a line, and wider chunks fetch fewer lines twice: 512 bytes (438 520 rows of 21 random entries, fp64,
-  // n = 63: 0.80 -> 0.68 ms).
+  // Where rows of B are whole cache lines the chunks are, too, of up to 256 bytes: one slice of B is live at a time and no
+  // line is fetched for two chunks (300 000 rows of 20 random entries, us, chunks as even as whole loads allow / of whole
+  // lines: fp32, n = 96 425 / 324, n = 224 1045 / 724; fp64, n = 48 432 / 330; complex128, n = 40 772 / 559).  Where they
+  // are not, every chunk begins and ends inside a line: equal widths (79 columns of fp32 are 40 and 39, not 64 and 15), and
+  // 512 bytes, which fetch fewer lines twice (438 520 rows of 21 random entries, fp64, n = 63: 0.80 -> 0.68 ms).
   const bool whole_lines = (ldb * (int64_t)sizeof(T)) % 128 == 0 && (uintptr_t)B % 128 == 0;
   const bool colc = a.c_row == 1 && a.c_col != 1;
   const int full = (whole_lines || colc ? 1 : 2) * kGroupBytes / (int)sizeof(T);
-  const GroupChunks g = group_chunks(n, full, V);
+  const GroupChunks g = group_chunks(n, full, whole_lines ? 128 / (int)sizeof(T) : V);
   const unsigned __int128 span = (unsigned __int128)(k > 0 ? k - 1 : 0) * (unsigned __int128)ldb * sizeof(T) + (uint64_t)n * sizeof(T);
   spmm_group<T>(a, n, g.chunk, g.count, B, ldb, g.chunk,
                 k > 0 && span < ((unsigned __int128)1 << 31) ? (uint64_t)span : 0, false, C);

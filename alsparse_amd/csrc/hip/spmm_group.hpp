@@ -79,8 +79,8 @@ __device__ __forceinline__ void for_each_const(F& f, std::integer_sequence<int, 
 }
 
 // ---- which columns a lane takes (host and device: the arithmetic is checked without a GPU) --------------------
-// `count` chunks of `chunk` columns, whole loads of v each, as even as that allows; the last ends with column n and may hold
-// fewer than v columns (n = 961, at most 64 a chunk, v = 4: fifteen of 64, then one column).
+// `count` chunks of `chunk` columns, whole units of v each (a load, or a line), as even as that allows; the last ends with
+// column n and may hold fewer columns than a load (n = 961, at most 64 a chunk: fifteen of 64, then one column).
 struct GroupChunks {
   int chunk, count;
 };

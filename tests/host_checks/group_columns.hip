@@ -11,14 +11,14 @@
 using namespace asamd;
 
 template <int SIZE>
-static bool check(int chunk_bytes_most) {
+static bool check(int chunk_bytes_most, bool lines) {
   constexpr int V = 16 / SIZE;
-  const int most = chunk_bytes_most / SIZE;
+  const int most = chunk_bytes_most / SIZE, unit = lines ? 128 / SIZE : V;
   int64_t narrow_chunks = 0;
   for (int n = 2 * V + 1; n <= 36 * most; ++n) {
-    const GroupChunks g = group_chunks(n, most, V);
+    const GroupChunks g = group_chunks(n, most, unit);
     std::vector<int> stored(n, 0);
-    bool ok = g.chunk >= 1 && g.chunk <= most && g.chunk % V == 0 && (int64_t)g.chunk * (g.count - 1) < n &&
+    bool ok = g.chunk >= 1 && g.chunk <= most && g.chunk % unit == 0 && (int64_t)g.chunk * (g.count - 1) < n &&
               (int64_t)g.chunk * g.count >= n;
     for (int y = 0; ok && y < g.count; ++y) {
       const int cbeg = y * g.chunk, cn = n - cbeg < g.chunk ? n - cbeg : g.chunk;
@@ -70,6 +70,7 @@ static bool check_tiles() {
 
 int main() {
   bool ok = check_tiles();
-  for (int bytes : {kGroupBytes, 2 * kGroupBytes}) ok = check<4>(bytes) && check<8>(bytes) && check<16>(bytes) && ok;
+  for (int bytes : {kGroupBytes, 2 * kGroupBytes})
+    for (bool lines : {false, true}) ok = check<4>(bytes, lines) && check<8>(bytes, lines) && check<16>(bytes, lines) && ok;
   return ok ? 0 : 1;
 }
