@@ -24,7 +24,6 @@
 namespace asamd {
 
 constexpr int kPatternSlots = 256;   // a pattern's number is one byte
-constexpr int kPatternProbes = 32;   // slots looked at before a matrix is taken to have too many patterns
 constexpr int kPatternMaxLen = 64;   // entries per row; 64 KiB of distances at most, of which a matrix touches a few lines
 
 // What the builder leaves in one allocation besides the rows' pattern numbers.
@@ -38,7 +37,8 @@ struct PatternScratch {
 
 // One thread per row: the row's distances from LDS (the block's entries are one contiguous range, read with unit stride),
 // hashed, and the hash looked up in an open-addressed table of 256 slots, entered where it is new.  Which slot a pattern
-// gets depends on the order of arrival; nothing that a multiply computes does.
+// gets depends on the order of arrival; nothing that a multiply computes does.  All slots are probed before the matrix is
+// taken to have too many patterns: which of them a shorter search still reaches depends on the order of arrival as well.
 static __global__ __launch_bounds__(kStreamRows) void pattern_rows_kernel(int m, int base, int rows_per_group,
                                                                           int max_len, const int* __restrict__ row_ptr,
                                                                           const int* __restrict__ col_ind,
@@ -78,7 +78,8 @@ static __global__ __launch_bounds__(kStreamRows) void pattern_rows_kernel(int m,
   }
   const unsigned long long key = h | 1;  // never 0
   int slot = (int)(h >> 56);
-  for (int p = 0; p < kPatternProbes; ++p, slot = (slot + 1) % kPatternSlots) {
+  for (int p = 0; p < kPatternSlots; ++p, slot = (slot + 1) % kPatternSlots) {
+    if (p % 32 == 31 && __atomic_load_n(&tab->fail, __ATOMIC_RELAXED)) return;  // (a table that others found full)
     unsigned long long seen = __atomic_load_n(&tab->key[slot], __ATOMIC_RELAXED);
     if (seen == 0) {
       seen = atomicCAS(&tab->key[slot], 0ull, key);

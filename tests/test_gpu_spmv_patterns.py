@@ -130,6 +130,34 @@ def test_matrices_without_the_layout(gpu, what):
         da.free()
 
 
+@pytest.mark.parametrize("count", [250, 255, 256, 257])
+def test_every_slot_of_the_table_is_used(gpu, count):
+    """As many patterns as a byte can number have the layout whatever order they arrive in, one more never has: rows of
+    two entries, the second `d` columns behind the first, every `d` from 1 to `count` (a row's first distance is 0)."""
+    rng = np.random.default_rng(count)
+    m = 20000
+    d = np.concatenate([np.arange(1, count + 1), rng.integers(1, count + 1, size=m - count)])
+    rng.shuffle(d)
+    col = np.stack([np.arange(m), np.arange(m) + d], axis=1).astype(np.int32).reshape(-1)
+    a = wl.Csr(m, m + count, (2 * np.arange(m + 1)).astype(np.int32), col, wl.uniform(2 * m, np.float64, 7), 0, "pairs")
+    x, y0 = wl.uniform(a.cols, a.dtype, 3), wl.uniform(a.rows, a.dtype, 4)
+    da = DeviceCsr(a)
+    try:
+        for attempt in range(8):
+            announce("patterns:", count, "patterns, attempt", attempt)
+            layout = _build(da)
+            try:
+                assert bool(layout.pid) == (count <= 256)
+                if layout.pid:
+                    st, y = _multiply(da, layout, 1.5, x, 0.5, y0)
+                    assert st == 0
+                    check_spmv(a, 1.5, x, 0.5, y0, y, "%d patterns" % count)
+            finally:
+                capi.load().asamd_patterns_free(byref(layout))
+    finally:
+        da.free()
+
+
 def test_an_analysed_stencil_keeps_patterns_and_reads_the_callers_values(gpu):
     """27-point stencil of 45 x 44 x 43 points (2.1 M entries) through the public API: patterns instead of a copy, the
     values read in place (new ones need nothing), and a value array that is not 16-byte aligned still multiplies."""
