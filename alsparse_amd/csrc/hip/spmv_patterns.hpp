@@ -11,8 +11,8 @@
 // Bound by memory.  us per multiply over four matrices in turn, before (32-bit columns, 16-bit distances or the ELL copy,
 // whichever the analysis kept) and now: 5-point Laplacian 2048^2 fp64 67.4 -> 50.4 (256 MB moved, 5.1 TB/s), fp32
 // 49.6 -> 31.9; 27-point stencil of 101 x 100 x 97 points complex64 72.5 -> 50.8, fp64 69.9 -> 50.8; of 160^3 points fp32
-// 179 -> 105; of 60 x 50 x 47 points fp32 10.7 -> 6.1.  Under a million entries the launch is all there is and the
-// staged kernel has the shorter chain of loads (300 x 333, fp64: 3.7 against 4.4).  16-byte values: the ELL copy stays
+// 179 -> 105; of 60 x 50 x 47 points fp32 10.7 -> 6.1.  Rows far shorter than the longest, and small matrices, stay with
+// the columns (patterns_pay in plan.c).  16-byte values: the ELL copy stays
 // ahead (5-point Laplacian of 2.1 M rows 58.7 against 84.4).
 //
 // The reference has no counterpart (src/kernel/dcu/level2/mv/csrmv/dcu_gemv_vector.h:14-57 reads every column).

@@ -122,6 +122,30 @@ static int stream_group(const asamd_csr_plan *p, int regular_only) {
 }
 static int stream_ok(const asamd_csr_plan *p) { return stream_group(p, 0) > 0; }
 
+/* Whether the staged row blocks gain from row patterns.  The pattern kernel gathers for every lane of a row as many
+ * elements of x as the longest row needs, so what decides is those gathers over the entries.  Time with patterns over time
+ * with columns, rows of L entries every fourth, shorter ones between, 12 M and 60 M entries, the worst of one matrix
+ * again and again and four in turn:
+ *   4-byte values, one or four lanes per row: 1.23 0.96-1.00, 1.33 0.82, 1.45 1.07, 1.6 1.12, 2.0 1.35
+ *                  two lanes per row:         1.23 1.13, 1.5 1.30-1.41 (1.06, the 27-point stencil: 0.58)
+ *   fp64,          one or two lanes:          1.23 0.95-1.02, 1.47 0.98-1.06, 1.6 1.06, 1.75 1.14-1.15, 2.0 1.2
+ *                  more:                      1.5 0.90, 1.75 0.95, 2.0 0.97-1.04, 2.5 1.17
+ *   complex64,     one or two lanes:          1.5 0.92, 1.75 1.0, 1.9 0.97, 2.0 1.05-1.09
+ *                  more:                      2.0 0.90, 2.5 0.95-0.98, 3.0 1.03
+ * From 2^20 entries on: below, a multiply is one launch's latency, and the staged kernel has the shorter chain of loads
+ * (5-point Laplacian on 300 x 333, fp64: 3.7 us with the columns, 4.4 with the patterns; on 900 x 1100, fp32: 11.3
+ * against 7.2).
+ * Values of 16 bytes stay with the ELL copy (5-point Laplacian on 1500 x 1400: 59 us against 84). */
+static int patterns_pay(const asamd_csr_plan *p) {
+  const asamd_csr_stats *st = &p->st;
+  const int g = stream_group(p, 0);
+  if (g < 1 || p->val_size > 8 || st->nnz < 1 << 20) return 0;
+  int per_lane = (st->max_len + g - 1) / g;
+  if (per_lane > 8) per_lane += per_lane & 1;
+  const double most = p->val_size == 4 ? (g == 2 ? 1.15 : 1.4) : is_complex(p) ? (g <= 2 ? 1.9 : 2.5) : (g <= 2 ? 1.5 : 2.0);
+  return (double)st->m * per_lane * g <= most * (double)st->nnz;
+}
+
 /* x in LDS: for an x that crowds the L1 (32 KB) and fits the LDS, on matrices large enough for 256 persistent
  * workgroups.  4 M x 16 entries, fp32: rowconst 0.105 / 0.125 / 0.20 / 0.25 / 0.29 ms with 4 / 16 / 32 / 64 / 128 KB of x,
  * this kernel 0.127 ms whatever x; fp64 with 128 KB of x 0.37 against 0.18 ms.  ALSPARSE_AMD_XLDS=0 leaves it out. */
@@ -1336,12 +1360,10 @@ static hipError_t plan_create(hipStream_t stream, int32_t m, int32_t n, int32_t 
       }
     }
   }
-  /* Staged row blocks whose rows follow few patterns (grids): a byte per row for the column numbers.  From 2^20 entries
-   * on: below, a multiply is one launch's latency (5-point Laplacian on 300 x 333, fp64: 3.7 us with the columns, 4.4
-   * with the patterns; on 900 x 1100, fp32: 11.3 against 7.2).  Values of 16 bytes stay with the ELL copy (5-point
-   * Laplacian on 1500 x 1400: 59 us against 84). */
-  if (col_ind && st->trusted && trusted != 3 && (p->auto_algo == ASAMD_SPMV_STREAM || (trusted == 2 && stream_ok(p))) &&
-      nnz >= (trusted == 2 ? 1 : 1 << 20) && p->val_size <= 8 && st->first_offset == 0 && st->min_len >= 1 &&
+  /* Staged row blocks whose rows follow few patterns (grids): a byte per row for the column numbers. */
+  if (col_ind && st->trusted && trusted != 3 &&
+      (trusted == 2 ? stream_ok(p) && nnz >= 1 && p->val_size <= 8 : p->auto_algo == ASAMD_SPMV_STREAM && patterns_pay(p)) &&
+      st->first_offset == 0 && st->min_len >= 1 &&
       env_int("ALSPARSE_AMD_STREAM_PATTERNS", 1) > 0) {
     e = (hipError_t)asamd_patterns_build(stream, m, nnz, base, stream_group(p, 0), st->max_len, row_ptr, col_ind, &p->pat);
     if (e == hipErrorOutOfMemory) {

@@ -158,6 +158,43 @@ def test_every_slot_of_the_table_is_used(gpu, count):
         da.free()
 
 
+@pytest.mark.parametrize("name,entries,short,long,every,want", [
+    ("f32", 2000000, 5, 5, 1, True),
+    ("f32", 1000000, 5, 5, 1, False),   # a launch's latency
+    ("f32", 2000000, 2, 12, 10, False),  # 12 gathers for every row of 3 entries on average
+    ("f32", 2000000, 3, 4, 4, True),
+    ("f32", 2000000, 18, 24, 4, False),  # two lanes a row
+    ("f64", 2000000, 1, 8, 9, False),
+    ("f64", 2000000, 14, 24, 4, True),
+    ("c64", 2000000, 3, 6, 4, True),
+])
+def test_uneven_rows_stay_with_the_columns(gpu, name, entries, short, long, every, want):
+    """The analysis keeps patterns where the gathers of rows padded to the longest are worth it: rows of `short` entries,
+    every `every`-th of `long`, all of two patterns."""
+    lib, dtype = capi.load(), DTYPES[name]
+    rows = int(entries * every / ((every - 1) * short + long)) if every > 1 else entries // long
+    lengths = np.where(np.arange(rows) % every == 0, long, short)
+    row_ptr = np.concatenate([[0], np.cumsum(lengths)])
+    row = np.repeat(np.arange(rows), lengths)
+    col = (row + 7 * (np.arange(row.size) - row_ptr[row])).astype(np.int32)
+    a = wl.Csr(rows, rows + 7 * long, row_ptr.astype(np.int32), col, _vector(row.size, dtype, 9), 0, "uneven")
+    x, y0 = _vector(a.cols, dtype, 3), _vector(a.rows, dtype, 4)
+    da = DeviceCsr(a)
+    descr, info = capi.make_descr(), capi.alphasparse_dcu_mat_info_t()
+    assert lib.alphasparse_dcu_create_mat_info(byref(info)) == 0
+    try:
+        assert getattr(lib, "alphasparse_dcu_%s_csrmv_analysis" % capi.prefix(dtype))(
+            gpu.h, 0, a.rows, a.cols, a.nnz, byref(descr), da.val.c_ptr(), da.row_ptr.c_ptr(), da.col.c_ptr(), info) == 0
+        st = lib.asamd_analysis_stats(info).contents
+        assert st.algo == capi.ASAMD_SPMV_STREAM
+        announce("patterns: uneven rows", name, entries, short, long, every)
+        assert (st.device_bytes >= a.rows) == want, "a byte per row with patterns, a constant without"
+        _check(a, 1.5, x, 0.5, y0, run_csrmv(gpu, da, 1.5, x, 0.5, y0, info=info), "uneven rows")
+    finally:
+        lib.alphasparse_dcu_destroy_mat_info(info)
+        da.free()
+
+
 def test_an_analysed_stencil_keeps_patterns_and_reads_the_callers_values(gpu):
     """27-point stencil of 45 x 44 x 43 points (2.1 M entries) through the public API: patterns instead of a copy, the
     values read in place (new ones need nothing), and a value array that is not 16-byte aligned still multiplies."""
