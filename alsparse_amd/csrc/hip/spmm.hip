@@ -15,8 +15,13 @@
 //
 // Arithmetic follows the row-major plain kernel
 // (src/plain/kernel/level3/mm/gemm/gemm_x_csr_row_plain.c:11-19): alpha is
-// folded into each value, products are accumulated with fma in entry order,
-// then C = beta*C + acc.  beta == 0 never reads C.
+// folded into each value, products are accumulated with fma, then
+// C = beta*C + acc.  beta == 0 never reads C.  The strided kernel adds a row's
+// products in entry order.  The others deal them out by position -- the short
+// kernel to W lanes or, long rows, to the workgroup; the group kernel to 16 / GC
+// parts of a lane group (one for chunks of more than 128 bytes) or, long rows, to
+// sixteen groups -- and join the partial sums in a fixed order, so the same call
+// returns the same bits.
 
 #include <hip/hip_runtime.h>
 

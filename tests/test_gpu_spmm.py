@@ -116,9 +116,8 @@ def test_random_structures_widths_and_layouts(gpu, seed, dtype):
 @pytest.mark.parametrize("maker", [lambda: wl.stencil3d(64, 60, 56, np.float32), lambda: wl.uniform_rows(215040, 215040, 12, np.float32)],
                          ids=["stencil", "random_columns"])
 def test_row_major_operand_of_the_middle_sizes(gpu, maker):
-    """A dense operand of 48 to 384 MiB: which row-major kernel runs is decided by a look at the matrix (do
-    neighbouring rows share columns?) on the first multiply.  Both answers, twice each (the second multiply
-    reuses the first one's answer), against the oracle."""
+    """A dense operand of 48 to 384 MiB, beyond an XCD's L2 and around the size of the memory-side cache: matrices whose
+    neighbouring rows share columns and matrices whose rows do not, twice each, against the oracle."""
     a = maker()
     n = 64
     assert 48 << 20 < a.cols * n * 4 <= 384 << 20
@@ -270,14 +269,13 @@ def _band(rows, cols, width, dtype, base=0, seed=11):
 
 
 SHARED = {
-    # 27-point stencil: nine runs of three consecutive columns per row; 32 rows share their rows of B
+    # 27-point stencil: nine runs of three consecutive columns per row
     "stencil27": lambda dt, base: wl.stencil3d(20, 18, 16, dt, base=base),
     "laplace": lambda dt, base: wl.laplace2d(90, 70, dt, base=base),
-    # 32 rows x 100 entries exceed the staged entries: the run is halved, then fits
     "band100": lambda dt, base: _band(3000, 2600, 100, dt, base),
-    # rows whose own columns exceed the tile: halved down to one row, which one wave multiplies from global memory
+    # rows that the sixteen lane groups of a workgroup share
     "band300": lambda dt, base: _band(700, 900, 300, dt, base),
-    # a matrix with fewer rows than one workgroup takes, and one that ends inside a run
+    # a matrix of hardly more rows than one workgroup takes, and one that ends inside a workgroup
     "band_short": lambda dt, base: _band(19, 40, 7, dt, base),
     "band_tail": lambda dt, base: _band(32 * 5 + 3, 400, 9, dt, base),
 }
@@ -288,13 +286,12 @@ SHARED = {
 @pytest.mark.parametrize("n", [33, 64, 100, 128])
 @pytest.mark.parametrize("kernel", ["chosen", "lds"])
 def test_row_major_rows_that_share_columns(gpu, mat, n, dtype, kernel, monkeypatch):
-    """Matrices whose neighbouring rows share columns.  "chosen": the kernel the library picks by itself (a
-    device-side look at the structure where the size of B does not decide); "lds": the opt-in kernel that stages
-    the distinct rows of B of a run of rows of A in LDS.  Aligned and padded leading dimensions (128-bit and
-    element-wise loads), both bases, beta zero and not."""
+    """Matrices whose neighbouring rows share columns.  Aligned and padded leading dimensions (rows of B that are whole cache
+    lines and rows that are not), both bases, beta zero and not.  "lds": with ALSPARSE_AMD_SPMM_LDS in the environment, which
+    once chose a kernel and must change nothing."""
     from helpers_shapes import complex_vector, complexify, real_dtype
     if kernel == "lds":
-        monkeypatch.setenv("ALSPARSE_AMD_SPMM_LDS", "1")  # read by the library at every call
+        monkeypatch.setenv("ALSPARSE_AMD_SPMM_LDS", "1")
     else:
         monkeypatch.delenv("ALSPARSE_AMD_SPMM_LDS", raising=False)
     cx = np.iscomplexobj(np.zeros(1, dtype))
@@ -323,7 +320,7 @@ def test_row_major_rows_that_share_columns(gpu, mat, n, dtype, kernel, monkeypat
                     if beta == 0:
                         assert err.strict <= tol, "%s n=%d: %r" % (mat, n, err)
                     assert np.array_equal(out[:, n:], Cfull[:, n:]), "padding columns of C were touched"
-                    # the same bits on a second run: sums are formed in CSR order whatever slot a column got
+                    # the same bits on a second run: a row's parts and their order depend on its entries alone
                     again = run_csrmm(gpu, da, capi.ALPHA_SPARSE_LAYOUT_ROW_MAJOR, 0, alpha, Bfull, ldb, beta, Cfull, ldc, n, a.cols)
                     assert np.array_equal(out.view(np.uint8), again.view(np.uint8))
         finally:
@@ -415,5 +412,63 @@ def test_few_rows_of_many_entries(gpu, m, chunks, dtype):
             err = orc.csrmm_err(a, 1.25, B2, 0.5, C02, C2, ref)
             tol = 1e-4 if np.dtype(dtype) == np.float32 else 1e-12
             assert err.zero_den_mismatch == 0 and err.full <= tol, (m, n, err)
+    finally:
+        da.free()
+
+
+def _far_matrix(m, cols, per_row, dtype, base):
+    """Rows of random columns of at least sixteen entries on average, some without entries and some that a workgroup shares."""
+    rng = np.random.default_rng(m + per_row)
+    lengths = np.full(m, per_row)
+    lengths[::97], lengths[5::1001], lengths[7::1501] = 0, 300, 257
+    row_ptr = np.concatenate([[0], np.cumsum(lengths)])
+    return wl.Csr(m, cols, (row_ptr + base).astype(np.int32), (rng.integers(0, cols, size=int(row_ptr[-1])) + base).astype(np.int32),
+                  None, base, "far rows")
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.complex64, np.complex128], ids=["f32", "f64", "c64", "c128"])
+@pytest.mark.parametrize("m", [8192, 8207])
+def test_two_loads_a_lane_one_row_of_b_in_flight(gpu, m, dtype):
+    """Chunks of more than 256 bytes over whole tiles of rows of sixteen entries and more: one and several chunks, the last load
+    moved back by every number of columns; both matrices end inside and at the end of a workgroup's tile."""
+    from helpers_shapes import complex_vector
+    vector = complex_vector if np.dtype(dtype).kind == "c" else wl.uniform
+    v = 16 // np.dtype(dtype).itemsize
+    a = _far_matrix(m, 3001, 20, dtype, 1)
+    a.values = vector(a.col_ind.size, dtype, 7)
+    da = DeviceCsr(a)
+    try:
+        for n in (16 * v + 1, 24 * v + v - 1, 32 * v - 1, 64 * v + 1 if m == 8192 else 17 * v):
+            ldb = n + (1 if n % (8 * v) == 0 else 0)  # (rows of B that are whole cache lines take one load a lane)
+            assert a.nnz >= 16 * m and (ldb * np.dtype(dtype).itemsize) % 128
+            B, C0 = vector(a.cols * ldb, dtype, 5).reshape(a.cols, ldb), vector(m * n, dtype, 4)
+            announce("spmm two loads a lane", m, n, np.dtype(dtype).name)
+            out = run_csrmm(gpu, da, capi.ALPHA_SPARSE_LAYOUT_ROW_MAJOR, 0, 1.25, B, ldb, 0.5, C0, n, n, a.cols)
+            B2, C02, C2 = np.ascontiguousarray(B[:, :n]), C0.reshape(m, n), out.reshape(m, n)
+            err = orc.csrmm_err(a, 1.25, B2, 0.5, C02, C2, orc.csrmm_plain(a, 1.25, B2, 0.5, C02))
+            tol = 1e-4 if np.dtype(dtype).name in ("float32", "complex64") else 1e-12
+            assert err.zero_den_mismatch == 0 and err.full <= tol, (m, n, err)
+    finally:
+        da.free()
+
+
+@pytest.mark.parametrize("n", [64, 65])
+def test_operands_beyond_the_memory_side_cache(gpu, n):
+    """B and C of more than 256 MB together under rows of sixteen entries and more: one row of B in flight with one load a lane,
+    row-major C past the caches, and column-major C with B laid out in panels (whole tiles of 64 rows) and with B^T."""
+    m, k = 32768 + 9, 1050001
+    a = _far_matrix(m, k, 18, np.float32, 0)
+    a.values = wl.uniform(a.col_ind.size, np.float32, 7)
+    assert a.nnz >= 16 * m and (m + k) * n * 4 > 256e6
+    B, C0 = wl.uniform(k * n, np.float32, 5), wl.uniform(m * n, np.float32, 4)
+    da = DeviceCsr(a)
+    ROW, COL = capi.ALPHA_SPARSE_LAYOUT_ROW_MAJOR, capi.ALPHA_SPARSE_LAYOUT_COLUMN_MAJOR
+    try:
+        for layout, trans, ldb, ldc in ((ROW, 0, n, n), (COL, 0, k, m), (COL, 1, n, m)):
+            announce("spmm beyond the memory-side cache", n, layout, trans)
+            out = run_csrmm(gpu, da, layout, trans, 1.25, B, ldb, 0.5, C0, ldc, n, k)
+            B2 = B.reshape(n, k).T if (layout, trans) == (COL, 0) else B.reshape(k, n)
+            C02, C2 = (x.reshape(m, n) if layout == ROW else x.reshape(n, m).T for x in (C0, out))
+            check(a, 1.25, B2, 0.5, C02, C2, "layout %d trans %d n=%d" % (layout, trans, n))
     finally:
         da.free()
