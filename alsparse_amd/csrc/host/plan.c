@@ -1475,6 +1475,7 @@ static hipError_t plan_create(hipStream_t stream, int32_t m, int32_t n, int32_t 
     (void)hipFree(p->d_rel16); /* another family was kept */
     p->d_rel16 = NULL;
   }
+  st->row_patterns = p->pat.pid != NULL;
   account(p);
   *out = p;
   return hipSuccess;
@@ -1603,6 +1604,7 @@ int asamd_csr_plan_set_algo(asamd_csr_plan *p, int32_t algo) {
     case ASAMD_SPMV_AUTO:
       p->st.algo = p->auto_algo;
       p->pinned = 0;
+      p->st.row_patterns = p->pat.pid != NULL;
       return hipSuccess;
     case ASAMD_SPMV_ROWCONST:
       if (!rowconst_ok(p)) return hipErrorInvalidValue;
@@ -1637,5 +1639,6 @@ int asamd_csr_plan_set_algo(asamd_csr_plan *p, int32_t algo) {
   }
   p->st.algo = algo;
   p->pinned = 1;
+  p->st.row_patterns = 0;
   return hipSuccess;
 }

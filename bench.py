@@ -37,14 +37,23 @@ MEASURED_TRAFFIC_BYTES = {
     (4, "merge-path"): (3.19e9, "profiles/spmv_merge_C4.txt"),
     (4, "merge-path, hot columns in LDS"): (2.85e9, "profiles/spmv_merge_hot_C4.txt"),
     (2, "ell copy"): (356.6e6, "profiles/spmv_ell_copy_C2.txt"),
+    (2, "row-block stream, row patterns"): (256.2e6, "profiles/spmv_patterns_laplace_stencil.txt"),
     (2, "row-block stream"): (338.8e6, "profiles/spmv_stream_C2.txt"),
-    (5, "spmm row-major"): (9.27e9, "profiles/spmm_rowmajor_C5.txt"),
+    (5, "spmm row-major"): (9.18e9, "profiles/spmm_rowmajor_C5.txt"),
 }
 
 
 def measured_traffic(cfg, kernel):
     """(bytes, source file) of the counter measurement recorded for this configuration and kernel, or (None, None)."""
     return MEASURED_TRAFFIC_BYTES.get((cfg, kernel), (None, None))
+
+
+def algo_name(stats):
+    """The kernel family that an analysis chose."""
+    from alsparse_amd import capi
+    if stats.algo == capi.ASAMD_SPMV_STREAM and stats.row_patterns:
+        return "row-block stream, row patterns"
+    return capi.ALGO_NAMES.get(stats.algo, "?")
 
 
 WORKLOAD_NAMES = {
@@ -240,7 +249,7 @@ def run_spmv(cfg, steps, warmup, cpu_baseline, check, transpose=False, vendor=Fa
     if transpose and analysed:
         assert stats.transpose_built != 0, "no room for the transposed copy"
         stats = lib.asamd_analysis_transpose_stats(info).contents
-    algo = capi.ALGO_NAMES.get(stats.algo, "?")
+    algo = algo_name(stats)
     if stats.algo == capi.ASAMD_SPMV_VECTOR:
         algo += "(W=%d)" % stats.vector_width
     if transpose and not analysed:
@@ -301,7 +310,7 @@ def run_spmv(cfg, steps, warmup, cpu_baseline, check, transpose=False, vendor=Fa
                 raise RuntimeError("csrmv status %d" % s)
         cold = time_steps(cold_step, steps, warmup, hiprt)
         cold["copies"] = cold_copies
-        cold["kernel"] = capi.ALGO_NAMES.get(lib.asamd_analysis_stats(copies[0][1]).contents.algo, "?")
+        cold["kernel"] = algo_name(lib.asamd_analysis_stats(copies[0][1]).contents)
         for arrs, inf in copies:
             lib.alphasparse_dcu_destroy_mat_info(inf)
             for d in arrs:
@@ -718,7 +727,8 @@ def run_ceilings(steps, warmup, short=False):
 
 def against_ceiling(cfg, r, ceilings):
     """The measured ceiling that bounds the configuration's kernel, named, and how close the kernel runs to it.
-    C2 streams its algorithmic bytes once: the non-temporal read rate.  C3's tiled pair moves its streams twice
+    C2 streams its algorithmic bytes once (with row patterns: values, row offsets and a byte per row): the non-temporal
+    read rate.  C3's tiled pair moves its streams twice
     (products out and in again): its real traffic (counter measurement, `traffic`) against the copy rate.
     C4 and the row kernels on C3 gather single elements of x that miss the L1: entries per second against the
     4-byte gather rates from an L2-resident array and from one of x's size.  C5 fetches one 256-byte row of B per
@@ -737,6 +747,15 @@ def against_ceiling(cfg, r, ceilings):
         got = r["traffic"] / ms / 1e9
         return {"ceiling": "plain copy of 2 GiB (probe kernel); achieved = measured HBM traffic of the kernel pair / time",
                 "ceiling_value": c["tb_per_s"], "achieved": got, "unit": "TB/s of real traffic",
+                "frac_of_ceiling": got / c["tb_per_s"]}
+    if cfg == 2 and kernel.endswith("row patterns"):
+        if not r.get("traffic"):
+            return None
+        c = ceilings["read_2GiB_nontemporal"]
+        ms = r["cold"]["ms"] if r.get("cold") else ms  # (the counters were read with several sets of arrays in turn, too)
+        got = r["traffic"] / ms / 1e9
+        return {"ceiling": "non-temporal read of 2 GiB (probe kernel); achieved = measured HBM traffic / time of the cold "
+                           "multiply", "ceiling_value": c["tb_per_s"], "achieved": got, "unit": "TB/s of real traffic",
                 "frac_of_ceiling": got / c["tb_per_s"]}
     if cfg == 2 and (kernel.startswith("row-block stream") or kernel.startswith("ell")):
         c = ceilings["read_2GiB_nontemporal"]

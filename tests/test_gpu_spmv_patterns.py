@@ -189,6 +189,12 @@ def test_uneven_rows_stay_with_the_columns(gpu, name, entries, short, long, ever
         assert st.algo == capi.ASAMD_SPMV_STREAM
         announce("patterns: uneven rows", name, entries, short, long, every)
         assert (st.device_bytes >= a.rows) == want, "a byte per row with patterns, a constant without"
+        assert st.row_patterns == want
+        if want:  # (a family set from outside reads columns)
+            for algo, patterns in ((capi.ASAMD_SPMV_STREAM, 0), (capi.ASAMD_SPMV_AUTO, 1)):
+                assert lib.asamd_analysis_set_algo(info, algo) == 0
+                assert lib.asamd_analysis_stats(info).contents.row_patterns == patterns
+                _check(a, 1.5, x, 0.5, y0, run_csrmv(gpu, da, 1.5, x, 0.5, y0, info=info), "uneven rows")
         _check(a, 1.5, x, 0.5, y0, run_csrmv(gpu, da, 1.5, x, 0.5, y0, info=info), "uneven rows")
     finally:
         lib.alphasparse_dcu_destroy_mat_info(info)
