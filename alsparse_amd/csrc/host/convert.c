@@ -44,7 +44,8 @@ alphasparse_status_t alphasparse_dcu_csr2ell_width(alphasparse_dcu_handle_t hand
     return ALPHA_SPARSE_STATUS_SUCCESS;
   }
   if (csr_row_ptr == NULL) return ALPHA_SPARSE_STATUS_INVALID_POINTER;
-  ASAMD_HIP_STATUS(asamd_csr2ell_width_ws(handle->stream, m, csr_row_ptr, ell_width, handle->buffer, handle->buffer_size));
+  /* (not in the handle's scratch, which a multiply on another stream of the handle may still be using) */
+  ASAMD_HIP_STATUS(asamd_csr2ell_width(handle->stream, m, csr_row_ptr, ell_width));
   return ALPHA_SPARSE_STATUS_SUCCESS;
 }
 

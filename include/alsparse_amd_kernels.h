@@ -444,7 +444,7 @@ int asamd_csr2coo_ws(hipStream_t stream, const int32_t *row_ptr, int32_t nnz, in
  * src/core/format/convert_ell_x_coo.c:46-52. */
 int asamd_csr2ell_width(hipStream_t stream, int32_t m, const int32_t *row_ptr,
                         int32_t *width_host);
-/* The same with a device workspace: 4 KiB of it save an allocation. */
+/* The same with a device workspace (4 KiB of it are used). */
 int asamd_csr2ell_width_ws(hipStream_t stream, int32_t m, const int32_t *row_ptr, int32_t *width_host, void *workspace,
                            size_t workspace_bytes);
 
