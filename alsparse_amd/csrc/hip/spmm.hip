@@ -217,7 +217,9 @@ static bool colmajor_nn(const asamd_dense_strides* st, int n) {
 // panel's rows start on line boundaries: as many panels of 256 bytes as fit, and of what is left a panel of 128 bytes and
 // a small one of the next power of two, up to 64 -- 17 columns of fp64 are one line and 8 bytes that stay in the L2s,
 // where rows of 136 bytes end to end take 2.06 lines each (262 147^2 x 16, n = 17: 0.30 -> 0.13 ms with all of this
-// file's column-major path) -- or one of 256 where more than 192 are left.
+// file's column-major path) -- or one of 256 where more than 192 are left.  tight: what is left in panels of its powers of
+// two instead, as many elements as B has (17 columns of fp32 are 16 and 1, not rows of 32): for a workspace that has no room
+// for more, at one more pass over A per panel.
 struct Panel {
   int cols, stride;   // columns, elements from row to row
   int64_t at;         // element offset of the first such panel in the workspace
@@ -225,11 +227,11 @@ struct Panel {
   int64_t elems;      // elements from panel to panel
 };
 struct PanelPlan {
-  Panel p[3];
+  Panel p[1 + 6];
   int kinds;
   int64_t total;  // elements
 };
-static PanelPlan plan_panels(int val_size, int n, int64_t k) {
+static PanelPlan plan_panels(int val_size, int n, int64_t k, bool tight) {
   PanelPlan plan{};
   const int full = kGroupBytes / val_size, line = full / 2;
   auto add = [&](int cols, int stride, int count) {
@@ -244,6 +246,10 @@ static PanelPlan plan_panels(int val_size, int n, int64_t k) {
   };
   if (n / full > 0) add(full, full, n / full);
   int rest = n % full;
+  for (int cols = line; tight && cols > 0; cols /= 2) {
+    if (rest & cols) add(cols, cols, 1);
+  }
+  if (tight) return plan;
   if (rest > line && (rest - line) * val_size <= 64) {
     add(line, line, 1);
     rest -= line;
@@ -256,9 +262,9 @@ static PanelPlan plan_panels(int val_size, int n, int64_t k) {
   return plan;
 }
 
-static size_t workspace_bytes(size_t val_size, int n, int k, const asamd_dense_strides* st) {
+static size_t workspace_bytes(size_t val_size, int n, int k, const asamd_dense_strides* st, bool tight) {
   if (!st || n <= 0 || k <= 0 || !colmajor_nn(st, n)) return 0;
-  return (size_t)plan_panels((int)val_size, n, k).total * val_size;
+  return (size_t)plan_panels((int)val_size, n, k, tight).total * val_size;
 }
 
 // ---- launching -------------------------------------------------------------------------------------
@@ -392,8 +398,9 @@ static int csrmm_impl(hipStream_t s, int m, int n, int k, int nnz, T alpha, cons
       spmm_rows<T>(a, n, k, B, st->b_row_stride, C);
       return hipGetLastError();
     }
-  } else if (entries && colmajor_nn(st, n) && ws && k > 0 && (uintptr_t)ws % 16 == 0 && ws_bytes >= workspace_bytes(sizeof(T), n, k, st)) {
-    const PanelPlan plan = plan_panels((int)sizeof(T), n, k);
+  } else if (entries && colmajor_nn(st, n) && ws && k > 0 && (uintptr_t)ws % 16 == 0 &&
+             (ws_bytes >= workspace_bytes(sizeof(T), n, k, st, false) || ws_bytes >= workspace_bytes(sizeof(T), n, k, st, true))) {
+    const PanelPlan plan = plan_panels((int)sizeof(T), n, k, ws_bytes < workspace_bytes(sizeof(T), n, k, st, false));
     int c0 = 0;
     for (int i = 0; i < plan.kinds; ++i) {
       const Panel& p = plan.p[i];
@@ -440,7 +447,11 @@ extern "C" int asamd_s_csrmm(hipStream_t stream, int32_t m, int32_t n, int32_t k
 extern "C" size_t asamd_csrmm_workspace_bytes(int32_t val_size, int32_t m, int32_t n, int32_t k,
                                               const asamd_dense_strides* strides) {
   (void)m;
-  return (val_size == 4 || val_size == 8 || val_size == 16) ? workspace_bytes((size_t)val_size, n, k, strides) : 0;
+  return (val_size == 4 || val_size == 8 || val_size == 16) ? workspace_bytes((size_t)val_size, n, k, strides, false) : 0;
+}
+
+extern "C" size_t asamd_csrmm_least_workspace_bytes(int32_t val_size, int32_t n, int32_t k, const asamd_dense_strides* strides) {
+  return (val_size == 4 || val_size == 8 || val_size == 16) ? workspace_bytes((size_t)val_size, n, k, strides, true) : 0;
 }
 
 extern "C" int asamd_s_csrmm_ws(hipStream_t stream, int32_t m, int32_t n, int32_t k, int32_t nnz, float alpha,

@@ -406,10 +406,13 @@ int asamd_z_csrmm_plain(hipStream_t stream, int32_t m, int32_t n, asamd_complex1
  * (k*n elements) in a caller-provided device workspace; without one, or with too
  * small a one, the multiply falls back to gathering B element by element, which
  * is tens of times slower.  asamd_csrmm_workspace_bytes returns what those strides
- * need (0 for every other layout).  The workspace only has to live until the
- * call's kernels have run on `stream`. */
+ * need (0 for every other layout), asamd_csrmm_least_workspace_bytes how little serves
+ * (about k*n elements, where the other rounds rows of the copy up to cache lines; slower).
+ * The workspace only has to live until the call's kernels have run on `stream`. */
 size_t asamd_csrmm_workspace_bytes(int32_t val_size, int32_t m, int32_t n, int32_t k,
                                    const asamd_dense_strides *strides);
+size_t asamd_csrmm_least_workspace_bytes(int32_t val_size, int32_t n, int32_t k,
+                                         const asamd_dense_strides *strides);
 int asamd_s_csrmm_ws(hipStream_t stream, int32_t m, int32_t n, int32_t k, int32_t nnz, float alpha,
                      const float *val, const int32_t *row_ptr, const int32_t *col_ind, int32_t base,
                      const float *B, float beta, float *C, const asamd_dense_strides *strides,

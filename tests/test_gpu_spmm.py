@@ -472,3 +472,44 @@ def test_operands_beyond_the_memory_side_cache(gpu, n):
             check(a, 1.25, B2, 0.5, C02, C2, "layout %d trans %d n=%d" % (layout, trans, n))
     finally:
         da.free()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.complex64, np.complex128], ids=["f32", "f64", "c64", "c128"])
+@pytest.mark.parametrize("per_row", [3, 20])
+def test_column_major_with_room_for_b_alone(gpu, per_row, dtype):
+    """A workspace of as many elements as B has: its copy in panels of powers of two, every width up to a full panel and one
+    more; a byte less takes the kernel that gathers B in place."""
+    from helpers_shapes import complex_vector
+    vector = complex_vector if np.dtype(dtype).kind == "c" else wl.uniform
+    lib, size, letter = capi.load(), np.dtype(dtype).itemsize, capi.prefix(dtype)
+    scalar = capi.scalar_type(dtype)
+    m, k = 530, 401
+    a = _far_matrix(m, k, per_row, dtype, 1)
+    a.values = vector(a.col_ind.size, dtype, 7)
+    da = DeviceCsr(a)
+    try:
+        for n in sorted({2, 3, 7, 64 // size + 1, 128 // size - 1, 128 // size, 128 // size + 1, 256 // size - 1, 256 // size, 256 // size + 3}):
+            st = capi.asamd_dense_strides(1, k, 1, m)
+            least = lib.asamd_csrmm_least_workspace_bytes(size, n, k, byref(st))
+            most = lib.asamd_csrmm_workspace_bytes(size, m, n, k, byref(st))
+            assert k * n * size <= least <= k * n * size + 7 * 512
+            B, C0 = vector(k * n, dtype, 5), vector(m * n, dtype, 4)
+            dB, ws = hiprt.DeviceArray.from_numpy(B), hiprt.DeviceArray((most + least,), np.uint8)
+            B2, C02 = np.ascontiguousarray(B.reshape(n, k).T), np.ascontiguousarray(C0.reshape(n, m).T)
+            ref = orc.csrmm_plain(a, 1.25, B2, 0.5, C02)
+            for room in (min(least, most) - 1, least, most):
+                announce("spmm column-major, workspace", n, np.dtype(dtype).name, per_row, room)
+                dC = hiprt.DeviceArray.from_numpy(C0)
+                assert getattr(lib, "asamd_%s_csrmm_ws" % letter)(
+                    None, m, n, k, a.nnz, scalar(1.25), da.val.c_ptr(), da.row_ptr.c_ptr(), da.col.c_ptr(), 1, dB.c_ptr(),
+                    scalar(0.5), dC.c_ptr(), byref(st), ws.c_ptr(), room) == 0
+                hiprt.synchronize()
+                C2 = np.ascontiguousarray(dC.to_numpy().reshape(n, m).T)
+                err = orc.csrmm_err(a, 1.25, B2, 0.5, C02, C2, ref)
+                tol = 1e-4 if np.dtype(dtype).name in ("float32", "complex64") else 1e-12
+                assert err.zero_den_mismatch == 0 and err.full <= tol, (n, room, err)
+                dC.free()
+            dB.free()
+            ws.free()
+    finally:
+        da.free()
