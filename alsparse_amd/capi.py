@@ -136,7 +136,7 @@ class asamd_csr_stats(Structure):
                 ("tile_long_blocks", c_int32), ("value_check", c_int32), ("tune_mode", c_int32),
                 ("device_bytes", c_int64), ("workspace_bytes", c_int64),
                 ("lines_per_entry_wave", c_float), ("lines_per_entry_segment", c_float),
-                ("xlds_slices", c_int32), ("row_patterns", c_int32)]
+                ("xlds_slices", c_int32), ("row_patterns", c_int32), ("row_sums", c_int32)]
 
 
 class asamd_spmv_args(Structure):  # include/alsparse_amd_kernels.h
@@ -347,6 +347,10 @@ _COMMON = {
     "asamd_tiled_free": [_P],
     "asamd_tiled_gather_values": [_P, _P, _P, _P],
     "asamd_spmv_tiled": [_P, POINTER(asamd_spmv_args), _P, _P, _P, _P],
+    "asamd_sums_build": [_P, _I, _I, _I, _I, _I, _P, _P, _P, c_int64, _P],
+    "asamd_sums_free": [_P],
+    "asamd_sums_refresh_values": [_P, _P, _P, _P],
+    "asamd_spmv_sums": [_P, POINTER(asamd_spmv_args), _P, _P],
     "asamd_hot_build": [_P, _I, _I, _I, _I, _I, _P, _P, _I, _I, _I, _P],
     "asamd_hot_free": [_P],
     "asamd_spmv_hot": [_P, POINTER(asamd_spmv_args), _P, _P, _P, _P, _P],

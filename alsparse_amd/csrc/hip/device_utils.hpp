@@ -312,6 +312,13 @@ __device__ __forceinline__ T group_sum(T v) {
   return v;
 }
 
+// Orders this wave's LDS traffic: the LDS works through a wave's instructions in order, so all that is
+// needed is that the compiler keeps them in program order.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // ---- buffer loads with the hardware's range check ------------------------------
 // A raw buffer resource over [p, p + bytes): loads at byte offsets >= bytes return zero and touch
 // no memory.  0x00020000 is the 32-bit data format word of gfx9 resources.

@@ -19,13 +19,6 @@
 
 using namespace asamd;
 
-// dst[i] = src[i * stride]
-__global__ __launch_bounds__(256) void strided_gather_kernel(int count, const int* __restrict__ src, int64_t stride,
-                                                             int* __restrict__ dst) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < count) dst[i] = src[(int64_t)i * stride];
-}
-
 // Cuts groups [0, groups) with cumulative entry counts off[0..groups] into
 // consecutive blocks of at most max_groups groups holding about `target`
 // entries each.  group_block[g] = block of group g; returns the block starts
@@ -44,16 +37,6 @@ static std::vector<int> cut_blocks(const int* off, int groups, int max_groups, i
   }
   start.push_back(groups);
   return start;
-}
-
-template <typename T>
-static void launch_gather_tiles(hipStream_t s, const asamd_tiled_layout* L, const void* val, const int32_t* gate) {
-  // eight tiles to a wave at a time, eight workgroups abreast (one per XCD), as many as the chip holds at once
-  const int64_t per_xcd = ((int64_t)(L->row_blocks + 7) / 8) * ((L->col_blocks + 7) / 8);
-  int64_t grid = (per_xcd + 3) / 4 * 8;
-  if (grid > 8 * 512) grid = 8 * 512;
-  gather_values_tiles_kernel<T, false><<<(unsigned)grid, 256, 0, s>>>(L->tperm, (const T*)val, (T*)L->tval, L->tile_ptr,
-                                                                     L->col_blocks, L->row_blocks, gate);
 }
 
 // Equal-entry column / row blocks, stable sort of the entries by (column block,
@@ -255,7 +238,7 @@ static hipError_t build_tiled(hipStream_t stream, asamd_tiled_layout* L, const i
                                                                                 d_tile_ptr);
     if constexpr (kPayloadSort) {
       L->tile_ptr = d_tile_ptr;  // stays with the layout: the values are gathered tile by tile, now and later
-      launch_gather_tiles<T>(stream, L, val, nullptr);
+      launch_gather_tiles<T>(stream, L->tperm, L->tile_ptr, L->col_blocks, L->row_blocks, val, L->tval, nullptr);
     }
     // Entries in tiles of 65..128 entries: if they are few, phase 2 runs in its one-entry-per-lane form
     // (twice the tiles in flight) and leaves those tiles to phase 3.
@@ -373,11 +356,11 @@ static hipError_t build_tiled(hipStream_t stream, asamd_tiled_layout* L, const i
     e = hipFuncSetAttribute((const void*)tiled_products_kernel<T, true>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, kSliceBytes);
   if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void*)tiled_reduce_kernel<T, 1>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, TileDims<T>::red_lds_bytes);
+    e = hipFuncSetAttribute((const void*)tiled_reduce_kernel<T, 1, false>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kLdsPerCu);
   if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void*)tiled_reduce_kernel<T, 2>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, TileDims<T>::red_lds_bytes);
+    e = hipFuncSetAttribute((const void*)tiled_reduce_kernel<T, 2, false>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kLdsPerCu);
   if (h_cnt) (void)hipHostFree(h_cnt);
   if (L->tile_ptr == d_tile_ptr) d_tile_ptr = nullptr;
   if (kPayloadSort) d_perm = nullptr;  // part of the arena
@@ -464,13 +447,13 @@ extern "C" int asamd_spmv_tiled(hipStream_t s, const asamd_spmv_args* a, const a
     }
     const unsigned red_grid = (unsigned)((L->row_blocks + TileDims<T>::red_waves - 1) / TileDims<T>::red_waves);
     if (L->entries_per_lane == 1)
-      tiled_reduce_kernel<T, 1><<<red_grid, TileDims<T>::red_threads, TileDims<T>::red_lds_bytes, s>>>(
-          L->m, L->row_blocks, L->col_blocks, L->row_block_start, (const TileRange*)L->ranges, L->trow, prod, alpha,
-          beta, y, skip);
+      tiled_reduce_kernel<T, 1, false><<<red_grid, TileDims<T>::red_threads, TileDims<T>::red_lds_bytes, s>>>(
+          L->row_blocks, L->col_blocks, TileDims<T>::rows, L->row_block_start, nullptr, (const TileRange*)L->ranges,
+          L->trow, prod, alpha, beta, y, skip);
     else
-      tiled_reduce_kernel<T, 2><<<red_grid, TileDims<T>::red_threads, TileDims<T>::red_lds_bytes, s>>>(
-          L->m, L->row_blocks, L->col_blocks, L->row_block_start, (const TileRange*)L->ranges, L->trow, prod, alpha,
-          beta, y, skip);
+      tiled_reduce_kernel<T, 2, false><<<red_grid, TileDims<T>::red_threads, TileDims<T>::red_lds_bytes, s>>>(
+          L->row_blocks, L->col_blocks, TileDims<T>::rows, L->row_block_start, nullptr, (const TileRange*)L->ranges,
+          L->trow, prod, alpha, beta, y, skip);
     if (L->n_long_chunks > 0) {
       const int waves = kLongThreads / kWave, narrow = L->n_long_narrow, wide = L->n_long_chunks - narrow;
       const LongBlock* list = (const LongBlock*)L->long_list;
@@ -497,7 +480,7 @@ extern "C" int asamd_tiled_gather_values(hipStream_t s, const asamd_tiled_layout
   return by_dtype(L->dtype, [&](auto* tag) -> int {
     using T = std::remove_pointer_t<decltype(tag)>;
     if ((uintptr_t)val % alignof(T)) return hipErrorInvalidValue;
-    launch_gather_tiles<T>(s, L, val, gate);
+    launch_gather_tiles<T>(s, L->tperm, L->tile_ptr, L->col_blocks, L->row_blocks, val, L->tval, gate);
     return hipGetLastError();
   });
 }

@@ -44,13 +44,6 @@ struct HotDims {
   static constexpr int lds_cols = table_bytes / (int)sizeof(T);
 };
 
-// Orders this wave's LDS traffic: the LDS works through a wave's instructions in order, so all that is
-// needed is that the compiler keeps them in program order.
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 template <typename T>
 __global__ __launch_bounds__(256) void hot_prepare_kernel(int hc, const int* __restrict__ hot_cols,
                                                           const T* __restrict__ x, T* __restrict__ x_front) {

@@ -113,6 +113,13 @@ struct LongFinish {  // a row block whose long tiles were dealt to several workg
 };
 
 // ---- analysis ----------------------------------------------------------------
+// dst[i] = src[i * stride]
+static __global__ __launch_bounds__(256) void strided_gather_kernel(int count, const int* __restrict__ src, int64_t stride,
+                                                             int* __restrict__ dst) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < count) dst[i] = src[(int64_t)i * stride];
+}
+
 // Entries per group of 256 columns (for cutting equal-entry column blocks), counted on a sample:
 // every stride-th run of kCountRun consecutive entries.  The counts only steer where the blocks are
 // cut, so a few million samples are as good as all entries, and the atomics (which collide on hot
@@ -267,6 +274,17 @@ __global__ __launch_bounds__(256) void gather_values_tiles_kernel(const unsigned
         if (mine < len[u]) nt_store(CONJ ? conj_t(v[u]) : v[u], out + lo[u] + mine);
     }
   }
+}
+
+template <typename T>
+void launch_gather_tiles(hipStream_t s, const unsigned* perm, const int* tile_ptr, int col_blocks, int row_blocks,
+                         const void* val, void* out, const int* gate) {
+  // eight tiles to a wave at a time, eight workgroups abreast (one per XCD), as many as the chip holds at once
+  const int64_t per_xcd = ((int64_t)(row_blocks + 7) / 8) * ((col_blocks + 7) / 8);
+  int64_t grid = (per_xcd + 3) / 4 * 8;
+  if (grid > 8 * 512) grid = 8 * 512;
+  gather_values_tiles_kernel<T, false><<<(unsigned)grid, 256, 0, s>>>(perm, (const T*)val, (T*)out, tile_ptr, col_blocks,
+                                                                      row_blocks, gate);
 }
 
 // Entries in sorted order: values, columns and rows local to their blocks.
@@ -514,15 +532,16 @@ __device__ __forceinline__ void add_rows(T* acc, int r, T v, bool valid_arg) {
 // 1 takes tiles of up to kWave entries with twice as many in flight (for the same number of outstanding
 // loads: where tiles are short -- wide values make narrow column blocks -- the loads of the second half
 // would all come back empty, and the bytes in flight, which bound the speed, would halve).
-template <typename T, int H>
+// DISTINCT: no tile holds a row twice (row-sum tiles, spmv_sums.hpp), so nothing has to be combined first.
+template <typename T, int H, bool DISTINCT>
 __global__ __launch_bounds__(TileDims<T>::red_threads) void tiled_reduce_kernel(
-    int m, int row_blocks, int col_blocks, const int* __restrict__ row_block_start,
-    const TileRange* __restrict__ ranges, const unsigned short* __restrict__ t_row,
+    int row_blocks, int col_blocks, int rows_cap, const int* __restrict__ row_block_start,
+    const int* __restrict__ run_ptr, const TileRange* __restrict__ ranges, const unsigned short* __restrict__ t_row,
     const T* __restrict__ prod, T alpha, T beta, T* __restrict__ y, const int* __restrict__ skip) {
   if (skip && *skip) return;  // the caller's guard found that the layout no longer describes the matrix
   extern __shared__ __align__(16) unsigned char smem[];
   T* s_acc = reinterpret_cast<T*>(smem);
-  constexpr int kTileRows = TileDims<T>::rows;
+  const int kTileRows = rows_cap;  // no row block of the layout has more
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int rb = blockIdx.x * TileDims<T>::red_waves + wave;
@@ -530,6 +549,9 @@ __global__ __launch_bounds__(TileDims<T>::red_threads) void tiled_reduce_kernel(
   T* acc = s_acc + wave * (kTileRows + kWave);
   for (int i = lane; i < kTileRows + kWave; i += kWave) acc[i] = T(0);
 
+  // The row block's tiles: one per column block, or (run_ptr) a list of its own.
+  const TileRange* my = ranges + (run_ptr ? (int64_t)run_ptr[rb] : (int64_t)rb * col_blocks);
+  const int tiles = run_ptr ? run_ptr[rb + 1] - run_ptr[rb] : col_blocks;
   // Wave-private accumulators.  Every tile listed in `ranges` has at most H * 64 entries: H per lane.
   // The wave keeps kSlots tiles in flight in a ring of registers: step s adds the tile in slot s
   // and at once loads the tile kSlots further on into it, so the loads of the next kSlots - 1 tiles are
@@ -545,12 +567,11 @@ __global__ __launch_bounds__(TileDims<T>::red_threads) void tiled_reduce_kernel(
   T sv[kSlots][H];
   int sr[kSlots][H];
   int slen[kSlots];
-  const TileRange* my = ranges + (int64_t)rb * col_blocks;
   auto load_ranges = [&](int group) {  // 64 tile ranges, one coalesced load
-    // no select on the loaded value (it would wait for the load at once): tiles past col_blocks are
+    // no select on the loaded value (it would wait for the load at once): tiles past the last are
     // cut off in issue()
     const int cb = group * kWave + lane;
-    return my[cb < col_blocks ? cb : 0];
+    return my[cb < tiles ? cb : 0];
   };
   const int r_none = kTileRows + lane;  // "no entry": the lane's dummy row behind the accumulators
   // the tile ranges of a group are loaded while the group before it is worked on
@@ -565,7 +586,7 @@ __global__ __launch_bounds__(TileDims<T>::red_threads) void tiled_reduce_kernel(
     const int src = ti & (kWave - 1);
     const int b0 = __builtin_amdgcn_readlane(tr.begin, src);
     const int e0 = __builtin_amdgcn_readlane(tr.end, src);
-    const int len = ti < col_blocks ? e0 - b0 : 0;
+    const int len = ti < tiles ? e0 - b0 : 0;
     slen[s] = len;
     const BufferRsrc rv = make_rsrc(prod + b0, len * (int)sizeof(T));
     const BufferRsrc rr = make_rsrc(t_row + b0, len * 2);
@@ -579,6 +600,11 @@ __global__ __launch_bounds__(TileDims<T>::red_threads) void tiled_reduce_kernel(
   auto consume = [&](int s) {
     const int len = slen[s];
     // a lane without an entry holds value zero already; its row becomes the lane's dummy row
+    if constexpr (DISTINCT) {
+      static_assert(H == 1, "one run, one instruction");
+      acc[lane < len ? sr[s][0] : r_none] += sv[s][0];
+      return;
+    }
     add_rows<true>(acc, lane < len ? sr[s][0] : r_none, sv[s][0], true);
     if constexpr (H == 2) {
       if (len > kWave)  // wave-uniform
@@ -592,7 +618,7 @@ __global__ __launch_bounds__(TileDims<T>::red_threads) void tiled_reduce_kernel(
     // outstanding at that wait is the smaller of what the two ways into the loop guarantee
     __builtin_amdgcn_sched_barrier(0);
   }
-  for (int t0 = 0; t0 < col_blocks; t0 += kSlots) {
+  for (int t0 = 0; t0 < tiles; t0 += kSlots) {
 #pragma unroll
     for (int s = 0; s < kSlots; ++s) {
       consume(s);

@@ -29,6 +29,7 @@ struct asamd_csr_plan {
   int merge_ipt;           /* items per thread of the merge-path kernel (4, 8 or 16) */
   int32_t *d_block_row;    /* merge-path coordinates of a structure promised fixed, merge_blocks + 1 ints */
   asamd_tiled_layout tiled;
+  asamd_sums_layout sums;  /* row-sum tiles: what AUTO runs, whatever the family, where they are laid out (build_sums) */
   asamd_hot_layout hot;
   asamd_binned_layout binned;
   asamd_xlds_layout xlds;  /* column slices for the kernel that holds x in LDS (an x of several LDS fills) */
@@ -41,14 +42,16 @@ struct asamd_csr_plan {
   int watched;             /* laid out for asamd_csr_plan_csrmv_watched: its fingerprints are the caller's account */
   void *d_eval;            /* ELL copy: ell_width * m values, column-major */
   int32_t *d_ecol;         /* ... and zero-based columns */
-  const void *copy_val_src; /* the value array that the tiled / ELL copy was taken from */
+  const void *copy_val_src; /* the value array that the tiled / ELL / row-sum copy was taken from */
   asamd_trans_copy tr[2];  /* CSR copies of the transpose [0] and of the conjugate transpose [1] */
   int lazy_transpose;      /* build a copy on the first transposed multiply */
-  uint64_t *d_fp;          /* 3 device words: fingerprints of the values that the copies were taken from
-                              (tiled / ELL, A^T, A^H) */
+  uint64_t *d_fp;          /* 4 device words: fingerprints of the values that the copies were taken from
+                              (tiled / ELL / slices, A^T, A^H, row-sum tiles) */
   void *d_setup;           /* device scratch of the plan's own set-up work (statistics, first fingerprints) */
 };
 
+#define FP_WORDS 4
+#define FP_SUMS 3
 #define SETUP_BYTES (ASAMD_GUARD_WS_BYTES + 1024)
 
 static const int kValSize[4] = {4, 8, 8, 16};
@@ -314,6 +317,11 @@ static void free_ell(asamd_csr_plan *p) {
   p->st.ell_built = 0;
 }
 
+static void free_sums(asamd_csr_plan *p) {
+  asamd_sums_free(&p->sums);
+  p->st.row_sums = 0;
+}
+
 static void free_hot(asamd_csr_plan *p) {
   asamd_hot_free(&p->hot);
   p->st.hot_built = 0;
@@ -422,7 +430,10 @@ static size_t algo_scratch(const asamd_csr_plan *p, int algo) {
 }
 
 static int has_value_copy(const asamd_csr_plan *p) {
-  return p->st.tiled_built || p->st.ell_built || p->xlds.val != NULL;
+  return p->st.tiled_built || p->st.ell_built || p->xlds.val != NULL || p->sums.tval != NULL;
+}
+static size_t sums_scratch(const asamd_csr_plan *p) {
+  return p->sums.tval ? align256((size_t)p->sums.sums * (size_t)p->val_size) : 0;
 }
 /* the families whose kernels read values that the plan keeps */
 static int holds_values(const asamd_csr_plan *p, int algo) {
@@ -444,6 +455,7 @@ size_t asamd_csr_plan_workspace_bytes(const asamd_csr_plan *p) {
     const size_t s = algo_scratch(p, a);
     if (s > need) need = s;
   }
+  if (sums_scratch(p) > need) need = sums_scratch(p);
   if (has_value_copy(p)) need += align256(ASAMD_GUARD_WS_BYTES);
   {
     const size_t s = align256(ASAMD_GUARD_WS_BYTES) + align256(trans_ylds_scratch(p));
@@ -459,12 +471,13 @@ size_t asamd_csr_plan_workspace_bytes(const asamd_csr_plan *p) {
 
 static void account(asamd_csr_plan *p) {
   asamd_csr_stats *st = &p->st;
-  int64_t b = SETUP_BYTES + 3 * 8;
+  int64_t b = SETUP_BYTES + FP_WORDS * 8;
   if (p->d_block_row) b += ((int64_t)st->merge_blocks + 1) * 4;
   if (p->d_col16) b += ((int64_t)st->nnz + 4) * 2;
   if (p->d_rel16) b += ((int64_t)st->nnz + 4) * 2;
   b += p->pat.device_bytes;
-  b += p->tiled.device_bytes + p->hot.device_bytes + p->binned.device_bytes + p->xlds.device_bytes;
+  b += p->tiled.device_bytes + p->hot.device_bytes + p->binned.device_bytes + p->xlds.device_bytes +
+       p->sums.device_bytes;
   if (st->ell_built) b += (int64_t)st->m * st->ell_width * ((int64_t)p->val_size + 4);
   for (int w = 0; w < 2; ++w)
     if (p->tr[w].plan) b += p->tr[w].t.device_bytes + p->tr[w].plan->st.device_bytes;
@@ -638,11 +651,31 @@ static hipError_t refresh_trans(hipStream_t s, asamd_csr_plan *p, int which, con
   asamd_trans_copy *t = &p->tr[which];
   hipError_t e = (hipError_t)asamd_gather_values(s, p->dtype, which == 1, p->st.nnz, t->t.perm, val, t->t.val, gate);
   if (e == hipSuccess) e = refresh_main(s, t->plan, t->t.row_ptr, t->t.col_ind, t->t.val, gate);
+  if (e == hipSuccess && t->plan->sums.tval) e = (hipError_t)asamd_sums_refresh_values(s, &t->plan->sums, t->t.val, gate);
   return e;
+}
+
+/* The row-sum tiles' multiply, or -1 where they do not serve this call: none laid out, a family set from outside, other
+ * values than those they hold, no room for their scratch or for the check of their values. */
+static int csrmv_sums(hipStream_t s, asamd_csr_plan *p, const asamd_spmv_args *a, ws_cursor ws, int guard) {
+  const asamd_csr_stats *st = &p->st;
+  if (!p->sums.tval || p->pinned || a->val != p->copy_val_src) return -1;
+  void *g = guard && st->value_check ? ws_take(&ws, ASAMD_GUARD_WS_BYTES) : NULL;
+  void *sums = ws_take(&ws, sums_scratch(p));
+  if (!sums || (guard && st->value_check && !g)) return -1;
+  if (g) {
+    int e = asamd_value_guard(s, a->val, (size_t)st->nnz * (size_t)p->val_size, st->value_check == 2, p->d_fp + FP_SUMS, g);
+    if (e == hipSuccess) e = asamd_sums_refresh_values(s, &p->sums, a->val, ASAMD_GUARD_FLAG(g));
+    if (e == hipSuccess) e = asamd_value_guard_commit(s, g, p->d_fp + FP_SUMS);
+    if (e != hipSuccess) return e;
+  }
+  return asamd_spmv_sums(s, a, &p->sums, sums);
 }
 
 static int csrmv_inner(hipStream_t s, asamd_csr_plan *p, const asamd_spmv_args *a, ws_cursor ws, int guard) {
   const asamd_csr_stats *st = &p->st;
+  const int summed = csrmv_sums(s, p, a, ws, guard);
+  if (summed != -1) return summed;
   int algo = st->algo;
   /* The tiled, ELL and slice-by-slice copies hold the values of the array they were built from.  A multiply that
    * brings another value array (same structure, new numbers) must not see the old ones: it runs the kernel that
@@ -1253,6 +1286,68 @@ static hipError_t model_copies(hipStream_t stream, asamd_csr_plan *p, const int3
   return e;
 }
 
+/* ---- row-sum tiles -----------------------------------------------------------------------------------
+ * What AUTO runs in the place of the family that was chosen, where their estimate is under 0.9 of that family's.
+ * They move vs + 2 bytes per entry and 2 vs + 2 per sum (a row's entries in one column block of 128 KB of x); measured
+ * with power-law rows and columns (1.1 .. 8.4 M rows, P = sums per entry = 0.31 .. 0.46), power-law rows over uniform
+ * columns, two and geometric row lengths, uniform rows of 3 .. 128 entries over 2 .. 64 MB of x, all types: 0.03 ms
+ * (the value guard's launches, two phases' ramps) and 4.2 TB/s, 4.9 from 4 GB on, within a fifth.  Before -> with them, us:
+ *   power law, 8.4 M rows: fp32 524 -> 250, fp64 779 -> 465; 2.1 M rows 136 -> 78, 164 -> 117; 1.1 M rows 62 -> 57, 83 -> 79;
+ *     0.6 M rows 37 -> 52, 40 -> 65 (estimate 43, 59: not laid out)
+ *   uniform rows, fp32: 1 M x 1 M x 16 103 -> 78, x 32 208 -> 120, x 64 324 -> 170, 2 M x 2 M x 16 173 -> 142, 4 M x 4 M x 16
+ *     285 -> 253, 16 M x 16 M x 16 853 -> 910 (next to no row meets a column block twice, and the tiled pair's are wider:
+ *     estimate 926 against 906, not laid out); fp64: 1 M x 1 M x 16 165 -> 120, 2 M x 2 M x 64 1215 -> 649
+ * A matrix that they serve keeps the copy of its family, for a family set from outside and for other value arrays. */
+static double sums_bytes(const asamd_csr_plan *p, double sums) {
+  const asamd_csr_stats *st = &p->st;
+  const double vs = (double)p->val_size;
+  return (double)st->nnz * (vs + 2.0) + sums * (2.0 * vs + 2.0) + ((double)st->n + (double)st->m) * vs;
+}
+static double sums_ms(const asamd_csr_plan *p, double sums) {
+  const double bytes = sums_bytes(p, sums);
+  double rate = 4.2 + 0.7 * (bytes - 1.0e9) / 3.0e9;
+  if (rate < 4.2) rate = 4.2;
+  if (rate > 4.9) rate = 4.9;
+  return 0.03 + bytes / (rate * 1e9);
+}
+
+static hipError_t build_sums(hipStream_t stream, asamd_csr_plan *p, const int32_t *row_ptr, const int32_t *col_ind,
+                             const void *val, int force) {
+  asamd_csr_stats *st = &p->st;
+  if (!st->trusted || st->first_offset != 0 || env_int("ALSPARSE_AMD_ROW_SUMS", 1) <= 0) return hipSuccess;
+  if (!asamd_tiled_fits(p->dtype, st->m, st->n, st->nnz)) return hipSuccess;
+  double most = (double)st->nnz;
+  if (force) {
+    if (p->auto_algo != ASAMD_SPMV_MERGE) return hipSuccess;
+  } else {
+    if (st->nnz < (1 << 22) || st->lines_per_entry_wave <= 0.f) return hipSuccess;
+    const int algo = p->auto_algo;
+    double kept = model_ms(p, algo == ASAMD_SPMV_MERGE_HOT || algo == ASAMD_SPMV_BINNED ? ASAMD_SPMV_MERGE : algo);
+    if (algo == ASAMD_SPMV_BINNED || algo == ASAMD_SPMV_MERGE_HOT) kept *= 0.95; /* they were kept for being faster */
+    if (holds_values(p, algo) && algo != ASAMD_SPMV_XLDS && st->value_check) kept += 0.022;
+    /* (the tiled pair's estimate runs high for 16-byte values: the transpose of 2.5 M x 2.5 M x 18, complex128, 0.63 against
+     * 0.493 ms; with them 0.506) */
+    if (algo == ASAMD_SPMV_TILED && p->val_size == 16) kept *= 0.8;
+    /* the most sums that pay: by bisection, the estimate grows with them */
+    double lo = (double)(st->m - st->hist[0]), hi = most;
+    if (!(sums_ms(p, lo) < 0.9 * kept)) return hipSuccess; /* a row leaves one sum at least */
+    for (int i = 0; i < 40; ++i) {
+      const double mid = 0.5 * (lo + hi);
+      if (sums_ms(p, mid) < 0.9 * kept) lo = mid;
+      else hi = mid;
+    }
+    most = lo;
+  }
+  hipError_t e = (hipError_t)asamd_sums_build(stream, p->dtype, st->m, st->n, st->nnz, st->base, row_ptr, col_ind, val,
+                                              (int64_t)most, &p->sums);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError(); /* optional, like every copy */
+    e = hipSuccess;
+  }
+  st->row_sums = p->sums.tval != NULL;
+  return e;
+}
+
 /* the fingerprint of the values a copy set was taken from (set-up work: plan-owned scratch, not concurrent) */
 static hipError_t first_fingerprint(hipStream_t stream, asamd_csr_plan *p, const void *val, int slot) {
   if (!p->st.value_check) return hipSuccess;
@@ -1284,7 +1379,7 @@ static hipError_t plan_create(hipStream_t stream, int32_t m, int32_t n, int32_t 
   p->watched = trusted == 3;
 
   hipError_t e = hipMalloc(&p->d_setup, SETUP_BYTES);
-  if (e == hipSuccess) e = hipMalloc((void **)&p->d_fp, 3 * sizeof(uint64_t));
+  if (e == hipSuccess) e = hipMalloc((void **)&p->d_fp, FP_WORDS * sizeof(uint64_t));
   int32_t h[ASAMD_ROW_STATS_WORDS];
   if (e == hipSuccess) e = (hipError_t)asamd_csr_row_stats(stream, m, row_ptr, (int32_t *)p->d_setup, h);
   if (e != hipSuccess) {
@@ -1441,9 +1536,11 @@ static hipError_t plan_create(hipStream_t stream, int32_t m, int32_t n, int32_t 
       st->xlds_slices = 0;
       if (p->struct_algo == ASAMD_SPMV_XLDS) p->struct_algo = p->plain_algo;
     }
+    if (e == hipSuccess && !only_tiled) e = build_sums(stream, p, row_ptr, col_ind, val, force);
     if (e == hipSuccess && has_value_copy(p)) {
       p->copy_val_src = val;
       e = first_fingerprint(stream, p, val, 0);
+      if (e == hipSuccess && p->sums.tval) e = first_fingerprint(stream, p, val, FP_SUMS);
       if (e == hipSuccess) e = hipStreamSynchronize(stream);
     }
     if (e != hipSuccess) {
@@ -1505,6 +1602,7 @@ void asamd_csr_plan_destroy(asamd_csr_plan *p) {
   if (p->d_fp) (void)hipFree(p->d_fp);
   free_tiled(p);
   free_ell(p);
+  free_sums(p);
   free_hot(p);
   free_binned(p);
   asamd_xlds_free(&p->xlds);
@@ -1583,9 +1681,11 @@ int asamd_csr_plan_refresh_values(hipStream_t stream, asamd_csr_plan *p, const i
   if (!p || !row_ptr || !col_ind || !val || !p->st.trusted) return hipErrorInvalidValue;
   if ((uintptr_t)val % (size_t)p->val_size) return hipErrorInvalidValue;
   hipError_t e = refresh_main(stream, p, row_ptr, col_ind, val, NULL);
+  if (e == hipSuccess && p->sums.tval) e = (hipError_t)asamd_sums_refresh_values(stream, &p->sums, val, NULL);
   if (e == hipSuccess && has_value_copy(p)) {
     p->copy_val_src = val;
     e = first_fingerprint(stream, p, val, 0);
+    if (e == hipSuccess && p->sums.tval) e = first_fingerprint(stream, p, val, FP_SUMS);
   }
   for (int which = 0; which < 2 && e == hipSuccess; ++which) {
     if (!p->tr[which].plan) continue;

@@ -243,6 +243,34 @@ int asamd_tiled_gather_values(hipStream_t stream, const asamd_tiled_layout *layo
 int asamd_spmv_tiled(hipStream_t stream, const asamd_spmv_args *a, const asamd_tiled_layout *layout,
                      void *products, void *long_scratch, const int32_t *skip);
 
+/* The tiled pair for rows that meet a column block more than once (long rows, power-law graphs): phase 1 adds up what a
+ * row has in a column block and writes one value for it.  Holds the values (tval) and the CSR position of every slot
+ * (tperm).  Per-call scratch: `sums` elements. */
+typedef struct {
+  void *tval;                /* slots values, span by span; NULL: no layout                    */
+  uint32_t *tperm;           /* slots: CSR position of the entry, or ~0                        */
+  uint16_t *tcol;            /* slots: local column; bit 15: last entry of its sum             */
+  uint16_t *srow;            /* sums: local row                                                */
+  int32_t *row_block_start;  /* row_blocks + 1                                                 */
+  int32_t *run_ptr;          /* row_blocks + 1: first of a row block's runs of sums            */
+  int32_t *span_sum;         /* spans + 1: first sum of every span                             */
+  int32_t *order;            /* spans: the order in which their values are gathered            */
+  void *runs, *chunks;
+  int32_t dtype, m, n, nnz;
+  int32_t col_blocks, row_blocks, rows_cap; /* rows_cap: rows of the tallest row block         */
+  int32_t sums, spans, n_runs, n_chunks;
+  int64_t device_bytes;
+} asamd_sums_layout;
+/* an empty record where the matrix would leave more than most_sums sums */
+int asamd_sums_build(hipStream_t stream, int32_t dtype, int32_t m, int32_t n, int32_t nnz, int32_t base,
+                     const int32_t *row_ptr, const int32_t *col_ind, const void *val, int64_t most_sums,
+                     asamd_sums_layout *out);
+void asamd_sums_free(asamd_sums_layout *layout);
+/* the values taken afresh from val; gate as for asamd_gather_values */
+int asamd_sums_refresh_values(hipStream_t stream, const asamd_sums_layout *layout, const void *val, const int32_t *gate);
+/* y = alpha*A*x + beta*y from the layout (a->val, a->row_ptr, a->col_ind are not read) */
+int asamd_spmv_sums(hipStream_t stream, const asamd_spmv_args *a, const asamd_sums_layout *layout, void *sums);
+
 /* Hot-column merge-path for power-law columns: the column stream rewritten as ranks of the popular
  * columns (pcol), whose x sits in LDS (the cols_lds most popular) or in a compact front (cols_front).
  * Structure only: values come from the caller's array.  Per-call scratch: front (cols_front elements),
