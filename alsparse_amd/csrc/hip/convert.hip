@@ -41,17 +41,6 @@ constexpr int kCooRound = kCooThreads * 4;  // entries per scan round
 constexpr int kCooRounds = 8;
 constexpr int kCooChunk = kCooRound * kCooRounds;  // 8192 entries
 
-// inclusive running maximum of non-negative values over the 64 lanes of a wave (DPP only)
-__device__ __forceinline__ int wave_max_scan(int v) {
-  v = max(v, dpp_mov_rows<0x111, 0xF>(v));  // row_shr:1
-  v = max(v, dpp_mov_rows<0x112, 0xF>(v));  // row_shr:2
-  v = max(v, dpp_mov_rows<0x114, 0xF>(v));  // row_shr:4
-  v = max(v, dpp_mov_rows<0x118, 0xF>(v));  // row_shr:8
-  v = max(v, dpp_mov_rows<0x142, 0xA>(v));  // row_bcast:15 into rows 1 and 3
-  v = max(v, dpp_mov_rows<0x143, 0xC>(v));  // row_bcast:31 into rows 2 and 3
-  return v;
-}
-
 // chunk_row[b] = largest r with row_ptr[r] - base <= b * kCooChunk, for b in [0, chunks]: a wave per chunk boundary
 // probes 64 places at once, four rounds of loads for 2^24 rows where a thread's binary search waits for 24 (20 M entries
 // in 4 M rows: 11.3 -> 5.2 us).  All boundaries are in flight together; inside the chunk kernel every workgroup would wait

@@ -236,6 +236,17 @@ __device__ __forceinline__ Cx<R> dpp_mov_rows(Cx<R> v) {
   return Cx<R>(dpp_mov_rows<Ctrl, RowMask>(v.re), dpp_mov_rows<Ctrl, RowMask>(v.im));
 }
 
+// inclusive running maximum of non-negative values over the 64 lanes of a wave (DPP only)
+__device__ __forceinline__ int wave_max_scan(int v) {
+  v = max(v, dpp_mov_rows<0x111, 0xF>(v));  // row_shr:1
+  v = max(v, dpp_mov_rows<0x112, 0xF>(v));  // row_shr:2
+  v = max(v, dpp_mov_rows<0x114, 0xF>(v));  // row_shr:4
+  v = max(v, dpp_mov_rows<0x118, 0xF>(v));  // row_shr:8
+  v = max(v, dpp_mov_rows<0x142, 0xA>(v));  // row_bcast:15 into rows 1 and 3
+  v = max(v, dpp_mov_rows<0x143, 0xC>(v));  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
 // value of the given lane, the same in every lane (v_readlane: no LDS crossbar)
 __device__ __forceinline__ int lane_bcast(int v, int src) { return __builtin_amdgcn_readlane(v, src); }
 __device__ __forceinline__ float lane_bcast(float v, int src) {

@@ -519,7 +519,7 @@ static int launch_trans_ylds(hipStream_t s, const asamd_spmv_args* a, void* part
   const int64_t grid = trans_ylds_groups(a->m);
   spmv_trans_ylds_kernel<T, W, CONJ><<<(unsigned)grid, kXldsThreads, lds, s>>>(
       a->m, a->n, scalar_of<T>(a->alpha), (const T*)a->val, a->row_ptr, a->col_ind, (const T*)a->x, (T*)partials, a->base);
-  trans_partials_sum_kernel<T><<<(unsigned)(((int64_t)a->n + 255) / 256), 256, 0, s>>>(
+  trans_partials_sum_kernel<T><<<(unsigned)(((int64_t)a->n + kPartialCols - 1) / kPartialCols), 256, 0, s>>>(
       a->n, (int)grid, (const T*)partials, scalar_of<T>(a->beta), (T*)a->y);
   return hipGetLastError();
 }
@@ -550,14 +550,116 @@ extern "C" int asamd_spmv_trans_ylds(hipStream_t s, const asamd_spmv_args* a, in
   });
 }
 
+// ---- transposed product with the columns in slices, their sums in LDS -----------------------------------
+namespace {
+struct SliceShape {
+  int parts, slices, slice_cols;
+};
+}  // namespace
+
+static int64_t trans_slices_least(int32_t dtype, int32_t n) {
+  const int sum_size = dtype == ASAMD_DTYPE_FLOAT_COMPLEX || dtype == ASAMD_DTYPE_DOUBLE_COMPLEX ? 16 : 8;
+  const int64_t max_cols = (ASAMD_XLDS_MAX_BYTES - kSliceLdsFixed) / sum_size;
+  return ((int64_t)n + max_cols - 1) / max_cols;
+}
+// parts * slices workgroups, as many as compute units: parts of about 4 096 entries (powers of two from 4 096 to 32 768 on
+// power laws of 9 000 rows 17 / 17 / 20 / 27 us, 200 000 x 500 points 12 / 15 / 21 / 24) but no more than leave one slice
+// per LDS, and one part where a chunk holds all entries, which saves the second launch.
+static SliceShape trans_slices_shape(int32_t dtype, int32_t n, int32_t nnz) {
+  const int64_t least = trans_slices_least(dtype, n);
+  const int64_t cus = xlds_compute_units();
+  int64_t parts = nnz <= kSliceChunk ? 1 : ((int64_t)nnz + 4095) / 4096;
+  if (parts > cus / least) parts = cus / least;
+  if (parts > 8) parts = parts / 8 * 8;  // a part's slices then share an XCD
+  if (parts < 1) parts = 1;
+  int64_t slices = cus / parts;
+  if (slices > ((int64_t)n + 63) / 64) slices = ((int64_t)n + 63) / 64;
+  if (slices < least) slices = least;
+  const int64_t cols = ((int64_t)n + slices - 1) / slices;
+  return {(int)parts, (int)(((int64_t)n + cols - 1) / cols), (int)cols};
+}
+
+// Where the slices beat the scatter (us, scatter / slices):
+//   * a few thousand entries and rows, one launch instead of two: a pair of products with 5 000 points of 1 000 x 1 000
+//     9.7 / 8.6, with 12 000 points (two chunks) 9.7 / 10.7
+//   * rows much longer than the mean, one lane group each in the scatter, and the popular columns that such graphs have:
+//     power law of 102 000 rows fp32 415 / 40, 400 000 rows 900 / 188 (25 slices); where the estimates say so
+//   * few columns for the entries, the atomics meet on few lines: 200 000 points x 500 columns 22 / 12, 24 M x 16 000
+//     fp64 880 / 96 (y in LDS: 182); as one slice only.
+// Everything else scatters: entries are read once per slice (uniform 7.2 M x 300 000 columns 349 / 393, its fp64 form of
+// 1 M columns 690 / 2 230), and neighbouring rows with the same columns meet in the scatter's own table (27-point stencil
+// on 60^3 points 28 / 209).
+constexpr int64_t kSlicesMost = 64;
+extern "C" int asamd_spmv_trans_slices_fit(int32_t dtype, int32_t m, int32_t n, int32_t nnz, int32_t max_len) {
+  if (m < 1 || n < 1 || nnz < 1 || dtype_size(dtype) == 0) return 0;
+  if (nnz <= kSliceChunk && m <= kSliceChunk) return trans_slices_least(dtype, n) <= 8;
+  const double ratio = (double)max_len * (double)m / (double)nnz;  // longest row over the mean
+  const int64_t least = trans_slices_least(dtype, n);
+  // picoseconds: 2.9 per entry and slice; an atomic 50, and a trip of the longest row's lane group 0.7 us
+  if (max_len >= 128 && ratio >= 16.0)
+    return least <= kSlicesMost && 2.9 * (double)nnz * (double)least <= 50.0 * (double)nnz + 0.7e6 * ratio;
+  return least == 1 && (int64_t)nnz >= (int64_t)64 * n;
+}
+extern "C" size_t asamd_spmv_trans_slices_bytes(int32_t dtype, int32_t n, int32_t nnz) {
+  if (n < 1 || nnz < 1) return 0;
+  const SliceShape shape = trans_slices_shape(dtype, n, nnz);
+  return shape.parts > 1 ? (size_t)shape.parts * (size_t)n * (size_t)dtype_size(dtype) : 0;
+}
+
+template <typename T, bool CONJ>
+static int launch_trans_slices(hipStream_t s, const asamd_spmv_args* a, void* partials) {
+  const SliceShape shape = trans_slices_shape(a->dtype, a->n, a->nnz);
+  if (shape.parts > 1 && !partials) return hipErrorInvalidValue;
+  T* out = shape.parts > 1 ? (T*)partials : nullptr;
+  static std::atomic<uint64_t> allowed{0};
+  if (const hipError_t e = allow_full_lds((const void*)csrmv_trans_slices_kernel<T, CONJ>, allowed); e != hipSuccess) return e;
+  const size_t lds = kSliceLdsFixed + (size_t)shape.slice_cols * sizeof(LdsSum<T>);
+  const T beta = scalar_of<T>(a->beta);
+  csrmv_trans_slices_kernel<T, CONJ><<<(unsigned)(shape.parts * shape.slices), kSliceThreads, lds, s>>>(
+      a->m, a->n, shape.parts, shape.slice_cols, scalar_of<T>(a->alpha), (const T*)a->val, a->row_ptr, a->col_ind,
+      (const T*)a->x, beta, (T*)a->y, out, a->base);
+  if (out)
+    trans_partials_sum_kernel<T><<<(unsigned)(((int64_t)a->n + kPartialCols - 1) / kPartialCols), 256, 0, s>>>(
+        a->n, shape.parts, out, beta, (T*)a->y);
+  return hipGetLastError();
+}
+// partials: asamd_spmv_trans_slices_bytes(dtype, n, nnz) bytes of per-call scratch
+extern "C" int asamd_spmv_trans_slices(hipStream_t s, const asamd_spmv_args* a, int32_t conj, void* partials) {
+  if (!a || a->n < 1 || a->nnz < 1 || trans_slices_least(a->dtype, a->n) > kSlicesMost) return hipErrorInvalidValue;
+  return by_dtype(a->dtype, [&](auto* tag) -> int {
+    using T = std::remove_pointer_t<decltype(tag)>;
+    if (!args_ok<T>(a) || (conj && kIsReal<T>) || (uintptr_t)partials % alignof(T)) return hipErrorInvalidValue;
+    if constexpr (!kIsReal<T>) {
+      if (conj) return launch_trans_slices<T, true>(s, a, partials);
+    }
+    return launch_trans_slices<T, false>(s, a, partials);
+  });
+}
+
 // ---- transposed product as an atomic scatter ------------------------------------------------------
 template <typename T, int W, bool CONJ>
 static void launch_trans_scatter(hipStream_t s, const asamd_spmv_args* a) {
-  constexpr int rows_per_block = kTransThreads / W;
-  const unsigned grid = (unsigned)(((int64_t)a->m + rows_per_block - 1) / rows_per_block);
-  csrmv_trans_scatter_kernel<T, W, CONJ><<<grid, kTransThreads, 0, s>>>(a->m, a->n, scalar_of<T>(a->alpha),
-                                                                         (const T*)a->val, a->row_ptr, a->col_ind,
-                                                                         (const T*)a->x, (T*)a->y, a->base);
+  constexpr int groups = kTransThreads / W;
+  const int64_t blocks = ((int64_t)a->m + groups - 1) / groups;
+  const T alpha = scalar_of<T>(a->alpha);
+  const T* val = (const T*)a->val;
+  const T* x = (const T*)a->x;
+#define ASAMD_SCATTER(K, TABLE, GRID)                                                                          \
+  csrmv_trans_scatter_kernel<T, W, K, CONJ, TABLE><<<(unsigned)(GRID), kTransThreads, 0, s>>>(                 \
+      a->m, a->n, alpha, val, a->row_ptr, a->col_ind, x, (T*)a->y, a->base)
+  if constexpr (W <= 4) {
+    // short rows: a workgroup's entries are few.  Small matrices are one launch's latency, to which the table adds half a
+    // microsecond; four rows per lane group cost scattered columns 4 % (uniform 400 000 x 5 fp32: 102 and 106 us; the
+    // 5-point Laplacian on 1000^2, fp64: 39 and 36, without the table 53).
+    if (a->nnz < (1 << 17)) ASAMD_SCATTER(1, false, blocks);
+    else ASAMD_SCATTER(1, true, blocks);
+  } else {
+    // four rows per lane group where that leaves two workgroups per compute unit (27-point stencil on 60^3 points, fp64:
+    // one 34 us, four 28, without the table 119; 200 000 points in 20 000 rows, W = 8: 22 and 13)
+    if (blocks >= 2048) ASAMD_SCATTER(4, true, (blocks + 3) / 4);
+    else ASAMD_SCATTER(1, true, blocks);
+  }
+#undef ASAMD_SCATTER
 }
 
 template <typename T, bool CONJ>

@@ -360,8 +360,9 @@ __global__ __launch_bounds__(kXldsThreads) void spmv_xlds4_kernel(int m, int n_t
 // above (W lanes per row, eight rows per lane group and trip in flight), every entry adds a * x[row] to its column's
 // sum in the workgroup's LDS (LDS atomics: the order of the additions inside a workgroup is not fixed), and the
 // workgroup writes its n sums to partials + blockIdx.x * n; trans_partials_sum_kernel adds the workgroups' sums in
-// order.  The scatter with global atomics (spmv_trans.hpp) takes 3.1 ms on 4 194 304 x 32 768 x 16, fp32: every one
-// of its 67 M atomics travels to memory.
+// order.  The scatter with global atomics (spmv_trans.hpp) takes 3.1 ms on 4 194 304 x 32 768 x 16, fp32, this 0.40: every
+// one of the scatter's 67 M atomics travels to memory.  The sums keep the element type here, so that a y of a whole LDS
+// is one slice: with sums in double precision the same matrix is three slices, 0.55 ms (csrmv_trans_slices_kernel).
 template <typename T, int W, bool CONJ>
 __global__ __launch_bounds__(kXldsThreads) void spmv_trans_ylds_kernel(int m, int n, T alpha, const T* __restrict__ val,
                                                                        const int* __restrict__ row_ptr,
@@ -427,16 +428,6 @@ __global__ __launch_bounds__(kXldsThreads) void spmv_trans_ylds_kernel(int m, in
   __syncthreads();
   T* __restrict__ out = partials + (int64_t)blockIdx.x * n;
   for (int i = threadIdx.x; i < n; i += kXldsThreads) out[i] = ys[i];
-}
-// y = beta * y + (the workgroups' sums, added in the order of the workgroups)
-template <typename T>
-__global__ __launch_bounds__(256) void trans_partials_sum_kernel(int n, int groups, const T* __restrict__ partials, T beta,
-                                                                 T* __restrict__ y) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  T sum = partials[i];
-  for (int g = 1; g < groups; ++g) sum += partials[(int64_t)g * n + i];
-  y[i] = beta == T(0) ? sum : y[i] * beta + sum;
 }
 
 // ---- column slices: the table of offsets, and the sum of the slices' results ------------------------------------

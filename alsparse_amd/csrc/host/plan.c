@@ -440,11 +440,19 @@ static int holds_values(const asamd_csr_plan *p, int algo) {
   return algo == ASAMD_SPMV_TILED || algo == ASAMD_SPMV_ELL || (algo == ASAMD_SPMV_XLDS && p->xlds.val != NULL);
 }
 
-/* per-call scratch of the transposed multiply that keeps y in LDS, or 0 where the atomic scatter runs */
+/* The transposed multiply without a copy: sums in LDS, the columns in slices or all of y (else the atomic scatter runs), and
+ * its per-call scratch. */
+static int trans_slices_ok(const asamd_csr_plan *p) {
+  const asamd_csr_stats *st = &p->st;
+  return asamd_spmv_trans_slices_fit(p->dtype, st->m, st->n, st->nnz, st->max_len) && env_int("ALSPARSE_AMD_XLDS", 1) > 0;
+}
 static size_t trans_ylds_scratch(const asamd_csr_plan *p) {
   const asamd_csr_stats *st = &p->st;
   if (st->nnz < (1 << 20) || st->first_offset != 0 || env_int("ALSPARSE_AMD_XLDS", 1) <= 0) return 0;
   return asamd_spmv_trans_ylds_bytes(p->dtype, st->m, st->n);
+}
+static size_t trans_scratch(const asamd_csr_plan *p) {
+  return align256(trans_slices_ok(p) ? asamd_spmv_trans_slices_bytes(p->dtype, p->st.n, p->st.nnz) : trans_ylds_scratch(p));
 }
 
 size_t asamd_csr_plan_workspace_bytes(const asamd_csr_plan *p) {
@@ -458,8 +466,8 @@ size_t asamd_csr_plan_workspace_bytes(const asamd_csr_plan *p) {
   if (sums_scratch(p) > need) need = sums_scratch(p);
   if (has_value_copy(p)) need += align256(ASAMD_GUARD_WS_BYTES);
   {
-    const size_t s = align256(ASAMD_GUARD_WS_BYTES) + align256(trans_ylds_scratch(p));
-    if (trans_ylds_scratch(p) && s > need) need = s;
+    const size_t s = align256(ASAMD_GUARD_WS_BYTES) + trans_scratch(p);
+    if (trans_scratch(p) && s > need) need = s;
   }
   for (int w = 0; w < 2; ++w)
     if (p->tr[w].plan) {
@@ -779,11 +787,13 @@ int asamd_csr_plan_csrmv(hipStream_t s, asamd_csr_plan *p, int32_t op, const voi
       return csrmv_inner(s, t->plan, &at, ws, 0);
     }
   }
-  /* y in LDS where it fits and the matrix is large enough for a workgroup per compute unit to pay */
-  const size_t ylds = trans_ylds_scratch(p);
-  if (ylds) {
-    void *partials = ws_take(&ws, ylds);
-    if (partials) return asamd_spmv_trans_ylds(s, &a, p->auto_width, which == 1, partials);
+  const size_t scratch = trans_scratch(p);
+  void *partials = scratch ? ws_take(&ws, scratch) : NULL;
+  if (trans_slices_ok(p)) {
+    if (partials || !scratch) return asamd_spmv_trans_slices(s, &a, which == 1, partials);
+  } else if (partials) {
+    /* y in LDS where it fits and the matrix is large enough for a workgroup per compute unit to pay */
+    return asamd_spmv_trans_ylds(s, &a, p->auto_width, which == 1, partials);
   }
   return asamd_spmv_trans_scatter(s, &a, p->auto_width, which == 1);
 }

@@ -190,8 +190,8 @@ int asamd_spmv_merge(hipStream_t stream, const asamd_spmv_args *a, int32_t ipt, 
                      int32_t *carry_row, void *carry_val, void *head_val);
 
 /* Transposed / conjugate-transposed product without a copy: y (n elements) is scaled by beta, then
- * `width` lanes per row scatter alpha*op(a)*x[row] with hardware float atomics, the traversal of
- * src/kernel/dcu/level2/mv/csrmv/dcu_gemv_x_csr_trans.cpp:11-68 and dcu_gemv_c_csr_conj.cpp:22-75.
+ * `width` lanes per row scatter alpha*op(a)*x[row], a workgroup's share of a column in one hardware float atomic where
+ * its table in LDS has room for the column: the traversal of src/kernel/dcu/level2/mv/csrmv/dcu_gemv_x_csr_trans.cpp:11-68 and dcu_gemv_c_csr_conj.cpp:22-75.
  * x has m elements.  conj != 0: complex types only. */
 int asamd_spmv_trans_scatter(hipStream_t stream, const asamd_spmv_args *a, int32_t width, int32_t conj);
 /* The same for a matrix of so few columns that y (n elements) fits a compute unit's LDS (asamd_spmv_xlds_fits):
@@ -199,6 +199,13 @@ int asamd_spmv_trans_scatter(hipStream_t stream, const asamd_spmv_args *a, int32
  * asamd_spmv_trans_ylds_bytes(dtype, m, n) bytes of per-call scratch (0: the matrix does not suit). */
 size_t asamd_spmv_trans_ylds_bytes(int32_t dtype, int32_t m, int32_t n);
 int asamd_spmv_trans_ylds(hipStream_t stream, const asamd_spmv_args *a, int32_t width, int32_t conj, void *partials);
+/* The same without global atomics, for a matrix whose columns make few enough slices of a compute unit's LDS
+ * (up to 64): equal pieces of the entries, a slice's sums in LDS.  asamd_spmv_trans_slices_fit: whether that is the better
+ * kernel for a matrix whose longest row has max_len entries.  partials: asamd_spmv_trans_slices_bytes(dtype, n, nnz) bytes
+ * of per-call scratch (0: none is needed). */
+int asamd_spmv_trans_slices_fit(int32_t dtype, int32_t m, int32_t n, int32_t nnz, int32_t max_len);
+size_t asamd_spmv_trans_slices_bytes(int32_t dtype, int32_t n, int32_t nnz);
+int asamd_spmv_trans_slices(hipStream_t stream, const asamd_spmv_args *a, int32_t conj, void *partials);
 
 /* ---- re-ordered copies of a CSR matrix ("layouts") and the kernels that multiply with them ------
  * A layout is a plain record of device pointers and counts, filled by its *_build call (which
