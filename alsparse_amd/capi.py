@@ -339,6 +339,8 @@ _COMMON = {
     "asamd_merge_partition": [_P, _I, _I, _P, _I, _I, _I, _P],
     "asamd_merge_self_blocks": [],
     "asamd_spmv_merge": [_P, POINTER(asamd_spmv_args), _I, _P, _P, _P, _P],
+    "asamd_spmv_permuted": [_P, POINTER(asamd_spmv_args), _I, _I, _P],
+    "asamd_spmv_merge_permuted": [_P, POINTER(asamd_spmv_args), _I, _P, _P, _P, _P, _P, _I],
     "asamd_spmv_trans_scatter": [_P, POINTER(asamd_spmv_args), _I, _I],
     "asamd_spmv_trans_ylds_bytes": [_I, _I, _I],
     "asamd_spmv_trans_ylds": [_P, POINTER(asamd_spmv_args), _I, _I, _P],

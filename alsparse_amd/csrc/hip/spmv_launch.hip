@@ -63,6 +63,38 @@ extern "C" int asamd_spmv_vector(hipStream_t s, const asamd_spmv_args* a, int32_
   return asamd_spmv_vector_if(s, a, width, nullptr);
 }
 
+template <typename T, int W, bool CONJ>
+static void launch_permuted(hipStream_t s, const asamd_spmv_args* a, const uint32_t* perm) {
+  constexpr int rows = kRowsBlock / W;
+  spmv_permuted_kernel<T, W, CONJ><<<(unsigned)(((int64_t)a->m + rows - 1) / rows), kRowsBlock, 0, s>>>(
+      a->m, scalar_of<T>(a->alpha), (const T*)a->val, perm, a->row_ptr, a->col_ind, (const T*)a->x, scalar_of<T>(a->beta),
+      (T*)a->y, a->base);
+}
+template <typename T, bool CONJ>
+static int permuted(hipStream_t s, const asamd_spmv_args* a, int width, const uint32_t* perm) {
+  switch (width) {
+    case 2: launch_permuted<T, 2, CONJ>(s, a, perm); break;
+    case 4: launch_permuted<T, 4, CONJ>(s, a, perm); break;
+    case 8: launch_permuted<T, 8, CONJ>(s, a, perm); break;
+    case 16: launch_permuted<T, 16, CONJ>(s, a, perm); break;
+    case 32: launch_permuted<T, 32, CONJ>(s, a, perm); break;
+    case 64: launch_permuted<T, 64, CONJ>(s, a, perm); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+extern "C" int asamd_spmv_permuted(hipStream_t s, const asamd_spmv_args* a, int32_t width, int32_t conj, const uint32_t* perm) {
+  if (!a || !perm) return hipErrorInvalidValue;
+  return by_dtype(a->dtype, [&](auto* tag) -> int {
+    using T = std::remove_pointer_t<decltype(tag)>;
+    if (!args_ok<T>(a) || (conj && kIsReal<T>)) return hipErrorInvalidValue;
+    if constexpr (!kIsReal<T>) {
+      if (conj) return permuted<T, true>(s, a, width, perm);
+    }
+    return permuted<T, false>(s, a, width, perm);
+  });
+}
+
 // ---- x in LDS ---------------------------------------------------------------------------------------
 static int xlds_compute_units() {
   static const int cus = [] {
@@ -449,8 +481,8 @@ extern "C" int asamd_merge_partition(hipStream_t s, int32_t m, int32_t nnz, cons
 
 extern "C" int32_t asamd_merge_self_blocks(void) { return kMergeSelfBlocks; }
 
-extern "C" int asamd_spmv_merge(hipStream_t s, const asamd_spmv_args* a, int32_t ipt, const int32_t* block_row,
-                                int32_t* carry_row, void* carry_val, void* head_val) {
+static int merge_launch(hipStream_t s, const asamd_spmv_args* a, int32_t ipt, const int32_t* block_row, int32_t* carry_row,
+                        void* carry_val, void* head_val, const uint32_t* perm, int32_t conj) {
   if (!a || !carry_row || !carry_val || !head_val) return hipErrorInvalidValue;
   return by_dtype(a->dtype, [&](auto* tag) -> int {
     using T = std::remove_pointer_t<decltype(tag)>;
@@ -467,9 +499,17 @@ extern "C" int asamd_spmv_merge(hipStream_t s, const asamd_spmv_args* a, int32_t
     // 128-bit loads of the streams need them 16-byte aligned
     const bool wide = (((uintptr_t)a->val | (uintptr_t)a->col_ind) & 15u) == 0;
     const int policy = csr_stream_policy(a, sizeof(T), true);
+#define ASAMD_LAUNCH_MERGE_PERM(IPT, HOW)                                                                            \
+  spmv_merge_kernel<T, IPT, false, HOW><<<nb, kMergeThreads, 0, s>>>(a->m, a->nnz, alpha, val, a->row_ptr,           \
+                                                                     a->col_ind, x, beta, y, a->base, block_row,     \
+                                                                     carry_row, (T*)carry_val, (T*)head_val, 0, perm)
 #define ASAMD_LAUNCH_MERGE(IPT)                                                                                      \
   do {                                                                                                               \
-    if (wide)                                                                                                        \
+    if (perm && conj)                                                                                                \
+      ASAMD_LAUNCH_MERGE_PERM(IPT, kPermConj);                                                                       \
+    else if (perm)                                                                                                   \
+      ASAMD_LAUNCH_MERGE_PERM(IPT, kPermPlain);                                                                      \
+    else if (wide)                                                                                                        \
       spmv_merge_kernel<T, IPT, true><<<nb, kMergeThreads, 0, s>>>(a->m, a->nnz, alpha, val, a->row_ptr, a->col_ind, \
                                                                    x, beta, y, a->base, block_row, carry_row,        \
                                                                    (T*)carry_val, (T*)head_val, policy);             \
@@ -491,11 +531,24 @@ extern "C" int asamd_spmv_merge(hipStream_t s, const asamd_spmv_args* a, int32_t
       ASAMD_LAUNCH_MERGE(4);
     }
 #undef ASAMD_LAUNCH_MERGE
+#undef ASAMD_LAUNCH_MERGE_PERM
     if (nb > 1)
       merge_fixup_kernel<T><<<(nb + 255) / 256, 256, 0, s>>>(nb, a->m, alpha, beta, carry_row, (const T*)carry_val,
                                                              (const T*)head_val, y);
     return hipGetLastError();
   });
+}
+
+extern "C" int asamd_spmv_merge(hipStream_t s, const asamd_spmv_args* a, int32_t ipt, const int32_t* block_row,
+                                int32_t* carry_row, void* carry_val, void* head_val) {
+  return merge_launch(s, a, ipt, block_row, carry_row, carry_val, head_val, nullptr, 0);
+}
+extern "C" int asamd_spmv_merge_permuted(hipStream_t s, const asamd_spmv_args* a, int32_t ipt, const int32_t* block_row,
+                                         int32_t* carry_row, void* carry_val, void* head_val, const uint32_t* perm,
+                                         int32_t conj) {
+  if (!a || !perm || (conj && a->dtype != ASAMD_DTYPE_FLOAT_COMPLEX && a->dtype != ASAMD_DTYPE_DOUBLE_COMPLEX))
+    return hipErrorInvalidValue;
+  return merge_launch(s, a, ipt, block_row, carry_row, carry_val, head_val, perm, conj);
 }
 
 // ---- transposed product with y in LDS --------------------------------------------------------------

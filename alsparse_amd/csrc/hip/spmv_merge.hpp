@@ -99,13 +99,16 @@ constexpr int kMergeSelfBlocks = 4096;
 // searches for its own).  WIDE: val and col_ind are 16-byte aligned
 // and the workgroup's entries are read as pieces of four from the multiple of four at or before its first
 // entry (a quarter of the memory instructions); a workgroup whose last piece would reach past the end of
-// the arrays reads entry by entry.
-template <typename T, int IPT, bool WIDE = false>
+// the arrays reads entry by entry.  PERM (entry by entry only): entry k's value is val[perm[k]], with kPermConj its
+// conjugate (see spmv_permuted_kernel).
+enum MergePerm { kPermNone, kPermPlain, kPermConj };
+template <typename T, int IPT, bool WIDE = false, MergePerm PERM = kPermNone>
 __global__ __launch_bounds__(kMergeThreads) void spmv_merge_kernel(
     int m, int nnz, T alpha, const T* __restrict__ val, const int* __restrict__ row_ptr,
     const int* __restrict__ col_ind, const T* __restrict__ x, T beta, T* __restrict__ y, int base,
     const int* __restrict__ block_row, int* __restrict__ carry_row, T* __restrict__ carry_val,
-    T* __restrict__ head_val, int policy = kStreamNtValues | kStreamNtIndices) {
+    T* __restrict__ head_val, int policy = kStreamNtValues | kStreamNtIndices, const unsigned* __restrict__ perm = nullptr) {
+  static_assert(!WIDE || PERM == kPermNone, "the values of a piece of four lie apart");
   constexpr int kItems = kMergeThreads * IPT;
   __shared__ int s_rend[kItems + 1];  // row ends, local to this workgroup's entry range
   __shared__ T s_prod[kItems + kItems / 32 + 1];
@@ -200,13 +203,19 @@ __global__ __launch_bounds__(kMergeThreads) void spmv_merge_kernel(
     const int64_t safe = nnz_cnt > 0 ? nnz_b : 0;
     T v[IPT];
     int c[IPT];
+    [[maybe_unused]] unsigned p[IPT];
 #pragma unroll
     for (int s = 0; s < IPT; ++s) {
       const int k = tid + s * kMergeThreads;
       const int64_t kk = k < nnz_cnt ? nnz_b + k : safe;
       // the streams are touched once: non-temporal, so that they do not push x out of the caches
-      v[s] = nt_load(val + kk);
+      if constexpr (PERM == kPermNone) v[s] = nt_load(val + kk);
+      else p[s] = nt_load(perm + kk);
       c[s] = nt_load(col_ind + kk);
+    }
+    if constexpr (PERM != kPermNone) {
+#pragma unroll
+      for (int s = 0; s < IPT; ++s) v[s] = PERM == kPermConj ? conj_t(val[p[s]]) : val[p[s]];
     }
     T xv[IPT];
 #pragma unroll

@@ -79,6 +79,45 @@ __global__ __launch_bounds__(kRowsBlock) void spmv_vector_kernel(
   spmv_vector_block<T, W>(xcd_contiguous_id(blockIdx.x, gridDim.x), m, alpha, val, row_ptr, col_ind, x, beta, y, base);
 }
 
+// The same with the values where they lie in another array: entry j of a row is val[perm[j]] (CONJ: its conjugate).  The
+// small transposed product: the copy of A^T keeps its structure only, so nothing has to check that its values are still
+// the caller's (the check is four launches; they are most of a small multiply).
+template <typename T, int W, bool CONJ>
+__global__ __launch_bounds__(kRowsBlock) void spmv_permuted_kernel(
+    int m, T alpha, const T* __restrict__ val, const unsigned* __restrict__ perm, const int* __restrict__ row_ptr,
+    const int* __restrict__ col_ind, const T* __restrict__ x, T beta, T* __restrict__ y, int base) {
+  constexpr int kU = 4;
+  const int lane = threadIdx.x % W;
+  const int64_t row = (int64_t)xcd_contiguous_id(blockIdx.x, gridDim.x) * (kRowsBlock / W) + threadIdx.x / W;
+  if (row >= m) return;  // whole lane groups leave together
+  const int64_t start = (int64_t)row_ptr[row] - base;
+  const int64_t end = (int64_t)row_ptr[row + 1] - base;
+  const T* __restrict__ xb = x - base;
+  T sum = T(0);
+  // four entries per lane and trip, every load unconditional (past the end: the trip's first entry again)
+  for (int64_t j = start + lane; j < end; j += kU * W) {
+    unsigned p[kU];
+    int c[kU];
+    T v[kU], xv[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int64_t k = j + u * W < end ? j + u * W : j;
+      p[u] = perm[k];
+      c[u] = col_ind[k];
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      v[u] = val[p[u]];
+      xv[u] = xb[c[u]];
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+      if (j + u * W < end) sum = fma_t(CONJ ? conj_t(v[u]) : v[u], xv[u], sum);
+  }
+  sum = group_sum<W>(sum);
+  if (lane == 0) store_axpby(y, row, alpha, sum, beta);
+}
+
 // The stand-in for a kernel that a device-side guard may turn away: launched every time, with a small grid
 // whose workgroups walk the row blocks in turn, so that the usual case -- *run_if == 0, nothing to do -- costs
 // a few hundred empty workgroups instead of one per row block.

@@ -562,6 +562,28 @@ static int settle_algo(const asamd_csr_plan *p, int algo, const void *val, const
   return algo;
 }
 
+/* merge path; perm: NULL, or where the values of the plan's entries lie in a->val */
+static int run_merge(hipStream_t s, asamd_csr_plan *p, const asamd_spmv_args *a, ws_cursor ws, const uint32_t *perm, int conj) {
+  const asamd_csr_stats *st = &p->st;
+  const size_t nb = (size_t)st->merge_blocks, vs = (size_t)p->val_size;
+  const int32_t *block_row = p->d_block_row;
+  if (!block_row && st->merge_blocks > asamd_merge_self_blocks()) {
+    /* structure not promised fixed: the coordinates are computed for this call (few workgroups: by themselves) */
+    int32_t *fresh = (int32_t *)ws_take(&ws, (nb + 1) * 4);
+    if (!fresh) return -1;
+    const int e = asamd_merge_partition(s, st->m, st->nnz, a->row_ptr, st->base, st->merge_blocks,
+                                        ASAMD_MERGE_THREADS * p->merge_ipt, fresh);
+    if (e != hipSuccess) return e;
+    block_row = fresh;
+  }
+  int32_t *carry_row = (int32_t *)ws_take(&ws, nb * 4);
+  void *carry_val = ws_take(&ws, nb * vs);
+  void *head_val = ws_take(&ws, nb * vs);
+  if (!head_val) return -1;
+  if (perm) return asamd_spmv_merge_permuted(s, a, p->merge_ipt, block_row, carry_row, carry_val, head_val, perm, conj);
+  return asamd_spmv_merge(s, a, p->merge_ipt, block_row, carry_row, carry_val, head_val);
+}
+
 static int run_algo(hipStream_t s, const asamd_csr_plan *p, int algo, const asamd_spmv_args *a, ws_cursor ws) {
   const asamd_csr_stats *st = &p->st;
   const size_t vs = (size_t)p->val_size;
@@ -616,24 +638,8 @@ static int run_algo(hipStream_t s, const asamd_csr_plan *p, int algo, const asam
       if (!head_val) return -1;
       return asamd_spmv_hot(s, a, &p->hot, front, carry_row, carry_val, head_val);
     }
-    case ASAMD_SPMV_MERGE: {
-      const size_t nb = (size_t)st->merge_blocks;
-      const int32_t *block_row = p->d_block_row;
-      if (!block_row && st->merge_blocks > asamd_merge_self_blocks()) {
-        /* structure not promised fixed: the coordinates are computed for this call (few workgroups: by themselves) */
-        int32_t *fresh = (int32_t *)ws_take(&ws, (nb + 1) * 4);
-        if (!fresh) return -1;
-        const int e = asamd_merge_partition(s, st->m, st->nnz, a->row_ptr, st->base, st->merge_blocks,
-                                            ASAMD_MERGE_THREADS * p->merge_ipt, fresh);
-        if (e != hipSuccess) return e;
-        block_row = fresh;
-      }
-      int32_t *carry_row = (int32_t *)ws_take(&ws, nb * 4);
-      void *carry_val = ws_take(&ws, nb * vs);
-      void *head_val = ws_take(&ws, nb * vs);
-      if (!head_val) return -1;
-      return asamd_spmv_merge(s, a, p->merge_ipt, block_row, carry_row, carry_val, head_val);
-    }
+    case ASAMD_SPMV_MERGE:
+      return run_merge(s, p, a, ws, NULL, 0);
     case ASAMD_SPMV_VECTOR:
     default:
       return asamd_spmv_vector(s, a, p->auto_width);
@@ -730,6 +736,26 @@ static void fill_args(asamd_spmv_args *a, const asamd_csr_plan *p, const void *a
   a->y = y;
 }
 
+/* Small transposed products read the caller's values through the copy's permutation: one launch (two where a few rows of
+ * A^T are long) where the check of the copy's values is four of their own, and nothing to check.  us per call, this / the
+ * checked copy: 30 000 to 120 000 entries 4.6 / 18, 500 000 scattered ones 14-16 / 18-19, 1 000 000 27-30 / 19-25 (every
+ * value then moves a cache line of its own), a power law of 60 000 rows 15 / 28. */
+#define PERMUTED_MOST (1 << 19)
+
+/* Any value array with the structure of the plan; -1: no room for the scratch. */
+static int csrmv_permuted(hipStream_t s, asamd_trans_copy *t, const void *alpha, const void *val, const void *x,
+                          const void *beta, void *y, ws_cursor ws, int conj) {
+  asamd_csr_plan *p = t->plan;
+  asamd_spmv_args a;
+  fill_args(&a, p, alpha, val, t->t.row_ptr, t->t.col_ind, x, beta, y);
+  /* a lane group takes four entries per lane and trip: more lanes where the longest row has many trips, and the merge
+   * path where a wave would still have more than eight */
+  int width = p->auto_width;
+  while (width < 64 && p->st.max_len > 16 * width) width *= 2;
+  if (p->st.max_len <= 32 * width) return asamd_spmv_permuted(s, &a, width, conj, t->t.perm);
+  return run_merge(s, p, &a, ws, t->t.perm, conj);
+}
+
 static hipError_t build_transpose(hipStream_t stream, asamd_csr_plan *p, const int32_t *rp, const int32_t *ci,
                                   const void *val, int which);
 
@@ -765,6 +791,10 @@ int asamd_csr_plan_csrmv(hipStream_t s, asamd_csr_plan *p, int32_t op, const voi
         return e;
       }
     }
+  }
+  if (t->plan && st->nnz <= PERMUTED_MOST) {
+    const int e = csrmv_permuted(s, t, alpha, val, x, beta, y, ws, which == 1);
+    if (e != -1) return e;
   }
   /* the copy holds the values it was gathered from: another value array takes the scatter route below */
   if (t->plan && val == t->val_src) {

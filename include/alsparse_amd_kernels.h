@@ -189,6 +189,13 @@ int32_t asamd_merge_self_blocks(void);
 int asamd_spmv_merge(hipStream_t stream, const asamd_spmv_args *a, int32_t ipt, const int32_t *block_row,
                      int32_t *carry_row, void *carry_val, void *head_val);
 
+/* `width` lanes per row (2 .. 64), entry j of the matrix at val[perm[j]] (conj != 0, complex types only: its conjugate):
+ * the structure of a copy with the caller's own values. */
+int asamd_spmv_permuted(hipStream_t stream, const asamd_spmv_args *a, int32_t width, int32_t conj, const uint32_t *perm);
+/* ... by the merge path (asamd_spmv_merge) */
+int asamd_spmv_merge_permuted(hipStream_t stream, const asamd_spmv_args *a, int32_t ipt, const int32_t *block_row,
+                              int32_t *carry_row, void *carry_val, void *head_val, const uint32_t *perm, int32_t conj);
+
 /* Transposed / conjugate-transposed product without a copy: y (n elements) is scaled by beta, then
  * `width` lanes per row scatter alpha*op(a)*x[row], a workgroup's share of a column in one hardware float atomic where
  * its table in LDS has room for the column: the traversal of src/kernel/dcu/level2/mv/csrmv/dcu_gemv_x_csr_trans.cpp:11-68 and dcu_gemv_c_csr_conj.cpp:22-75.
