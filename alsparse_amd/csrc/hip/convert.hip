@@ -219,9 +219,11 @@ __global__ __launch_bounds__(256) void max_row_len_kernel(int m, const int* __re
   }
 }
 
-// The workgroups' maxima of a call without a workspace.  One call at a time has it; one that comes meanwhile, from another
-// thread, allocates.  (All three conversions of a 4 M-row Laplacian, fp64: 147.6 us with these words as with a workspace.)
-static __device__ int width_parts[kWidthBlocks];
+// The workgroups' maxima of a call without a workspace: 4 KB of pinned host memory, made by the first call and kept, which
+// the kernel writes itself.  A copy from the device into pageable memory behind the kernel goes to the copy engine: all
+// three conversions of a Laplacian of 0.3 M rows, fp32, 40.5 -> 31.5 us.  One call at a time has it; one that
+// comes meanwhile, from another thread, allocates.
+static int* width_parts = nullptr;
 static std::atomic_flag width_parts_taken = ATOMIC_FLAG_INIT;
 
 extern "C" int asamd_csr2ell_width_ws(hipStream_t stream, int32_t m, const int32_t* row_ptr, int32_t* width_host,
@@ -230,22 +232,28 @@ extern "C" int asamd_csr2ell_width_ws(hipStream_t stream, int32_t m, const int32
   int* d = nullptr;
   hipError_t e = hipSuccess;
   const bool given = workspace && workspace_bytes >= kWidthBlocks * sizeof(int) && (uintptr_t)workspace % alignof(int) == 0;
-  const bool parts = !given && !width_parts_taken.test_and_set(std::memory_order_acquire);
-  if (given) d = (int*)workspace;
-  else if (parts) e = hipGetSymbolAddress((void**)&d, HIP_SYMBOL(width_parts));
-  else e = hipMalloc(&d, kWidthBlocks * sizeof(int));
-  if (e != hipSuccess) {
-    if (parts) width_parts_taken.clear(std::memory_order_release);
-    return e;
+  bool parts = !given && !width_parts_taken.test_and_set(std::memory_order_acquire);
+  if (parts && !width_parts &&
+      hipHostMalloc((void**)&width_parts, kWidthBlocks * sizeof(int), hipHostMallocPortable) != hipSuccess) {
+    (void)hipGetLastError();
+    width_parts = nullptr;
+    width_parts_taken.clear(std::memory_order_release);
+    parts = false;
   }
+  if (given) d = (int*)workspace;
+  else if (parts) d = width_parts;
+  else e = hipMalloc(&d, kWidthBlocks * sizeof(int));
+  if (e != hipSuccess) return e;
   int grid = (int)(((int64_t)m + 256 * 8 - 1) / (256 * 8));
   if (grid > kWidthBlocks) grid = kWidthBlocks;
   max_row_len_kernel<<<grid, 256, 0, stream>>>(m, row_ptr, d);
   e = hipGetLastError();
-  int part[kWidthBlocks];
-  if (e == hipSuccess) e = hipMemcpyAsync(part, d, (size_t)grid * sizeof(int), hipMemcpyDeviceToHost, stream);
+  int copied[kWidthBlocks];
+  if (e == hipSuccess && !parts)
+    e = hipMemcpyAsync(copied, d, (size_t)grid * sizeof(int), hipMemcpyDeviceToHost, stream);
   if (e == hipSuccess) e = hipStreamSynchronize(stream);
   if (e == hipSuccess) {
+    const int* part = parts ? d : copied;
     int width = 0;
     for (int b = 0; b < grid; ++b) width = part[b] > width ? part[b] : width;
     *width_host = width;
