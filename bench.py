@@ -34,6 +34,7 @@ NO_ANALYSIS = False  # --no-analysis
 MEASURED_TRAFFIC_BYTES = {
     (3, "tiled two-phase"): (5.17e9, "profiles/spmv_tiled_C3.txt"),
     (3, "rowconst"): (34.6e9, "profiles/spmv_tiled_C3.txt"),
+    (4, "row-sum tiles"): (1.13e9, "profiles/spmv_sums_C4.txt"),
     (4, "merge-path"): (3.19e9, "profiles/spmv_merge_C4.txt"),
     (4, "merge-path, hot columns in LDS"): (2.85e9, "profiles/spmv_merge_hot_C4.txt"),
     (2, "ell copy"): (356.6e6, "profiles/spmv_ell_copy_C2.txt"),
@@ -53,6 +54,8 @@ def algo_name(stats):
     from alsparse_amd import capi
     if stats.algo == capi.ASAMD_SPMV_STREAM and stats.row_patterns:
         return "row-block stream, row patterns"
+    if stats.row_sums:
+        return "row-sum tiles"
     return capi.ALGO_NAMES.get(stats.algo, "?")
 
 
@@ -742,7 +745,7 @@ def against_ceiling(cfg, r, ceilings):
         got = r["nnz"] / ms * 1e3
         return {"ceiling": "random 256-byte rows gathered from 256 MiB (probe kernel)", "ceiling_value": c["rows_per_s"],
                 "achieved": got, "unit": "rows of B per second", "frac_of_ceiling": got / c["rows_per_s"]}
-    if kernel.startswith("tiled") and r.get("traffic"):
+    if kernel.startswith(("tiled", "row-sum")) and r.get("traffic"):
         c = ceilings["copy_2GiB"]
         got = r["traffic"] / ms / 1e9
         return {"ceiling": "plain copy of 2 GiB (probe kernel); achieved = measured HBM traffic of the kernel pair / time",
