@@ -345,6 +345,7 @@ _COMMON = {
     "asamd_spmv_trans_ylds_bytes": [_I, _I, _I],
     "asamd_spmv_trans_ylds": [_P, POINTER(asamd_spmv_args), _I, _I, _P],
     "asamd_spmv_trans_slices_fit": [_I, _I, _I, _I, _I],
+    "asamd_spmv_trans_slices_pay": [_I, _I, _I, c_float],
     "asamd_spmv_trans_slices_bytes": [_I, _I, _I],
     "asamd_spmv_trans_slices": [_P, POINTER(asamd_spmv_args), _I, _P],
     "asamd_tiled_fits": [_I, _I, _I, _I],
@@ -365,6 +366,7 @@ _COMMON = {
     "asamd_transpose_build": [_P, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P],
     "asamd_transpose_free": [_P],
     "asamd_csr_row_stats": [_P, _I, _P, _P, _P],
+    "asamd_csr_row_stats_lines": [_P, _I, _P, _I, _I, _I, _P, _P, _P, _P],
     "asamd_csr_locality_probe": [_P, _I, _I, _I, _P, _I, _P, POINTER(c_float)],
     "asamd_value_guard_run": [c_size_t],
     "asamd_value_guard": [_P, _P, c_size_t, _I, _P, _P],

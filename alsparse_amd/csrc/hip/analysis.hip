@@ -50,23 +50,70 @@ __global__ __launch_bounds__(256) void row_stats_kernel(int m, const int* __rest
   }
 }
 
-__global__ void stats_init_kernel(int* out) {
+__global__ void stats_init_kernel(int* out, int words) {
   const int t = threadIdx.x;
-  if (t < kStatWords) out[t] = t == 0 ? 0x7fffffff : 0;
+  if (t < words) out[t] = t == 0 ? 0x7fffffff : 0;
+}
+
+// out[kStatWords] += distinct 128-byte lines of y that a run of 1 024 entries meets, over 64 runs at even distances: a
+// bitmap in LDS that the line numbers fold onto (two of 1 024 lines rarely share one of 2^15 bits).  It rides on the
+// statistics' round trip, which a call without an analysis makes once per matrix (three short launches then, not two).
+// Nothing beyond the entries that row_ptr names is read, whatever nnz is.
+constexpr int kRunEntries = 1024;
+constexpr int kRuns = 64;
+constexpr int kRunBits = 1 << 15;
+__global__ __launch_bounds__(256) void run_lines_kernel(int m, int nnz, int base, int elem_shift,
+                                                        const int* __restrict__ row_ptr, const int* __restrict__ col_ind,
+                                                        int* __restrict__ out) {
+  __shared__ unsigned s_bits[kRunBits / 32];
+  for (int i = threadIdx.x; i < kRunBits / 32; i += 256) s_bits[i] = 0;
+  const int64_t named = (int64_t)row_ptr[m] - base;
+  const int64_t room = (named < nnz ? named : nnz) - kRunEntries;
+  if (room < 0) return;  // the whole grid
+  const int64_t begin = room * blockIdx.x / (kRuns - 1);
+  unsigned line[kRunEntries / 256];
+#pragma unroll
+  for (int q = 0; q < kRunEntries / 256; ++q)
+    line[q] = (unsigned)(((int64_t)(col_ind[begin + threadIdx.x + q * 256] - base) << elem_shift) >> 7);
+  __syncthreads();
+  int lines = 0;
+#pragma unroll
+  for (int q = 0; q < kRunEntries / 256; ++q) {
+    const unsigned bit = (line[q] ^ (line[q] >> 15) * 0x9E3779B1u) & (kRunBits - 1);
+    const unsigned old = atomicOr(&s_bits[bit >> 5], 1u << (bit & 31));
+    lines += (old >> (bit & 31)) & 1u ? 0 : 1;
+  }
+  for (int d = kWave / 2; d > 0; d >>= 1) lines += __shfl_down(lines, d, kWave);
+  if (threadIdx.x % kWave == 0) atomicAdd(out, lines);
 }
 
 extern "C" int asamd_csr_row_stats(hipStream_t stream, int32_t m, const int32_t* row_ptr, int32_t* d_scratch,
                                    int32_t* stats_host) {
+  return asamd_csr_row_stats_lines(stream, m, row_ptr, 0, 0, 4, nullptr, d_scratch, stats_host, nullptr);
+}
+
+extern "C" int asamd_csr_row_stats_lines(hipStream_t stream, int32_t m, const int32_t* row_ptr, int32_t nnz, int32_t base,
+                                         int32_t elem_bytes, const int32_t* col_ind, int32_t* d_scratch,
+                                         int32_t* stats_host, float* lines_host) {
   if (!row_ptr || !d_scratch || !stats_host || m <= 0) return hipErrorInvalidValue;
-  stats_init_kernel<<<1, 64, 0, stream>>>(d_scratch);
+  int shift = 0;
+  while ((1 << shift) < elem_bytes) ++shift;
+  if ((1 << shift) != elem_bytes || elem_bytes > 16) return hipErrorInvalidValue;
+  const bool probe = lines_host && col_ind && nnz >= kRuns * kRunEntries;
+  int words[kStatWords + 1];
+  stats_init_kernel<<<1, 64, 0, stream>>>(d_scratch, probe ? kStatWords + 1 : kStatWords);
   int64_t grid = ((int64_t)m + 255) / 256;
   if (grid > 256 * 16) grid = 256 * 16;
   row_stats_kernel<<<(unsigned)grid, 256, 0, stream>>>(m, row_ptr, d_scratch);
+  if (probe) run_lines_kernel<<<kRuns, 256, 0, stream>>>(m, nnz, base, shift, row_ptr, col_ind, d_scratch + kStatWords);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess)
-    e = hipMemcpyAsync(stats_host, d_scratch, kStatWords * sizeof(int), hipMemcpyDeviceToHost, stream);
+    e = hipMemcpyAsync(words, d_scratch, (kStatWords + (probe ? 1 : 0)) * sizeof(int), hipMemcpyDeviceToHost, stream);
   if (e == hipSuccess) e = hipStreamSynchronize(stream);
-  return e;
+  if (e != hipSuccess) return e;
+  for (int i = 0; i < kStatWords; ++i) stats_host[i] = words[i];
+  if (lines_host) *lines_host = probe ? (float)words[kStatWords] / (float)(kRuns * kRunEntries) : 0.f;
+  return hipSuccess;
 }
 
 // ---------------------------------------------------------------------------

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <cmath>
 
 #include "alsparse_amd_kernels.h"
 #include "launch_utils.hpp"
@@ -639,9 +640,9 @@ static SliceShape trans_slices_shape(int32_t dtype, int32_t n, int32_t nnz) {
 //     power law of 102 000 rows fp32 415 / 40, 400 000 rows 900 / 188 (25 slices); where the estimates say so
 //   * few columns for the entries, the atomics meet on few lines: 200 000 points x 500 columns 22 / 12, 24 M x 16 000
 //     fp64 880 / 96 (y in LDS: 182); as one slice only.
-// Everything else scatters: entries are read once per slice (uniform 7.2 M x 300 000 columns 349 / 393, its fp64 form of
-// 1 M columns 690 / 2 230), and neighbouring rows with the same columns meet in the scatter's own table (27-point stencil
-// on 60^3 points 28 / 209).
+// What is left goes by its columns (asamd_spmv_trans_slices_pay): entries are read once per slice (uniform 7.2 M x 300 000
+// columns 349 / 393, its fp64 form of 1 M columns 690 / 2 230), and neighbouring rows with the same columns meet in the
+// scatter's own table (27-point stencil on 60^3 points 28 / 209).
 constexpr int64_t kSlicesMost = 64;
 extern "C" int asamd_spmv_trans_slices_fit(int32_t dtype, int32_t m, int32_t n, int32_t nnz, int32_t max_len) {
   if (m < 1 || n < 1 || nnz < 1 || dtype_size(dtype) == 0) return 0;
@@ -652,6 +653,26 @@ extern "C" int asamd_spmv_trans_slices_fit(int32_t dtype, int32_t m, int32_t n, 
   if (max_len >= 128 && ratio >= 16.0)
     return least <= kSlicesMost && 2.9 * (double)nnz * (double)least <= 50.0 * (double)nnz + 0.7e6 * ratio;
   return least == 1 && (int64_t)nnz >= (int64_t)64 * n;
+}
+// Scattered columns, whose atomics leave the scatter's workgroups one by one.  A run of entries meets at least half the lines
+// of y that columns at random would (the 5-point Laplacian and the 27-point stencil: under 0.2 of them), and the estimates
+// in us, scatter 6 + 45 ps an entry and real component, slices 12 + 2.9 ps an entry and slice + 0.3 per MB of partial
+// sums, say so by a tenth.  Scatter / slices, us: random points, 24 a row, 10 000 columns fp32 19 / 10, 60 000 fp32 77 / 25,
+// fp64 68 / 28, complex64 149 / 37, 150 000 fp32 181 / 79; 8 a row, 60 000 fp32 28 / 18; 48 a row, 100 000 fp32 247 / 69.
+// 3 a row of 150 000 fp64 (23 / 33) and 8 a row of 400 000 fp32 (160 / 174) scatter.
+extern "C" int asamd_spmv_trans_slices_pay(int32_t dtype, int32_t n, int32_t nnz, float lines) {
+  const double size = (double)dtype_size(dtype);
+  if (n < 1 || nnz < 1 || size == 0.0) return 0;
+  const int64_t least = trans_slices_least(dtype, n);
+  if (least > kSlicesMost) return 0;
+  const double run = 1024.0, all = (double)n * size / 128.0;  // lines of y
+  const double share = (double)lines * run / (all * (1.0 - std::exp(-run / all)));
+  if (!(share >= 0.5)) return 0;
+  const bool real = dtype == ASAMD_DTYPE_FLOAT || dtype == ASAMD_DTYPE_DOUBLE;
+  const double partials = (double)asamd_spmv_trans_slices_bytes(dtype, n, nnz);
+  const double scatter = 6.0 + (real ? 45e-6 : 90e-6) * (double)nnz * (share < 1.0 ? share : 1.0);
+  const double slices = 12.0 + 2.9e-6 * (double)nnz * (double)least + 0.3e-6 * partials;
+  return slices <= 0.9 * scatter;
 }
 extern "C" size_t asamd_spmv_trans_slices_bytes(int32_t dtype, int32_t n, int32_t nnz) {
   if (n < 1 || nnz < 1) return 0;

@@ -44,6 +44,7 @@ struct asamd_csr_plan {
   int32_t *d_ecol;         /* ... and zero-based columns */
   const void *copy_val_src; /* the value array that the tiled / ELL / row-sum copy was taken from */
   asamd_trans_copy tr[2];  /* CSR copies of the transpose [0] and of the conjugate transpose [1] */
+  float trans_lines;       /* distinct lines of y per entry of a run (0: not sampled); steers the transposed scatter only */
   int lazy_transpose;      /* build a copy on the first transposed multiply */
   uint64_t *d_fp;          /* 4 device words: fingerprints of the values that the copies were taken from
                               (tiled / ELL / slices, A^T, A^H, row-sum tiles) */
@@ -440,16 +441,19 @@ static int holds_values(const asamd_csr_plan *p, int algo) {
   return algo == ASAMD_SPMV_TILED || algo == ASAMD_SPMV_ELL || (algo == ASAMD_SPMV_XLDS && p->xlds.val != NULL);
 }
 
-/* The transposed multiply without a copy: sums in LDS, the columns in slices or all of y (else the atomic scatter runs), and
- * its per-call scratch. */
-static int trans_slices_ok(const asamd_csr_plan *p) {
-  const asamd_csr_stats *st = &p->st;
-  return asamd_spmv_trans_slices_fit(p->dtype, st->m, st->n, st->nnz, st->max_len) && env_int("ALSPARSE_AMD_XLDS", 1) > 0;
-}
+/* per-call scratch of the transposed multiply that keeps y in LDS, or 0 where it does not serve */
 static size_t trans_ylds_scratch(const asamd_csr_plan *p) {
   const asamd_csr_stats *st = &p->st;
   if (st->nnz < (1 << 20) || st->first_offset != 0 || env_int("ALSPARSE_AMD_XLDS", 1) <= 0) return 0;
   return asamd_spmv_trans_ylds_bytes(p->dtype, st->m, st->n);
+}
+/* The transposed multiply without a copy: sums in LDS, the columns in slices or all of y (else the atomic scatter runs), and
+ * its per-call scratch. */
+static int trans_slices_ok(const asamd_csr_plan *p) {
+  const asamd_csr_stats *st = &p->st;
+  if (env_int("ALSPARSE_AMD_XLDS", 1) <= 0) return 0;
+  return asamd_spmv_trans_slices_fit(p->dtype, st->m, st->n, st->nnz, st->max_len) ||
+         (trans_ylds_scratch(p) == 0 && asamd_spmv_trans_slices_pay(p->dtype, st->n, st->nnz, p->trans_lines));
 }
 static size_t trans_scratch(const asamd_csr_plan *p) {
   return align256(trans_slices_ok(p) ? asamd_spmv_trans_slices_bytes(p->dtype, p->st.n, p->st.nnz) : trans_ylds_scratch(p));
@@ -1421,11 +1425,14 @@ static hipError_t plan_create(hipStream_t stream, int32_t m, int32_t n, int32_t 
   hipError_t e = hipMalloc(&p->d_setup, SETUP_BYTES);
   if (e == hipSuccess) e = hipMalloc((void **)&p->d_fp, FP_WORDS * sizeof(uint64_t));
   int32_t h[ASAMD_ROW_STATS_WORDS];
-  if (e == hipSuccess) e = (hipError_t)asamd_csr_row_stats(stream, m, row_ptr, (int32_t *)p->d_setup, h);
+  if (e == hipSuccess)
+    e = (hipError_t)asamd_csr_row_stats_lines(stream, m, row_ptr, nnz, base, val_size, col_ind, (int32_t *)p->d_setup, h,
+                                              &p->trans_lines);
   if (e != hipSuccess) {
     asamd_csr_plan_destroy(p);
     return e;
   }
+  if (!trusted) col_ind = NULL; /* nothing below may be laid out from columns that can change */
   st->min_len = h[0];
   st->max_len = h[1];
   st->first_offset = h[2] - base;

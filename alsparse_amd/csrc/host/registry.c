@@ -169,7 +169,7 @@ alphasparse_status_t asamd_plan_for_call(alphasparse_dcu_handle_t handle, const 
   if (!found) {
     asamd_csr_plan *p = NULL;
     ASAMD_HIP_STATUS(asamd_csr_plan_create_dtype(handle->stream, m, n, nnz, (const int32_t *)row_ptr,
-                                                 NULL, NULL, base, dtype, /*trusted=*/0, &p));
+                                                 (const int32_t *)col_ind, NULL, base, dtype, /*trusted=*/0, &p));
     asamd_record *r = (asamd_record *)calloc(1, sizeof(*r));
     if (!r) {
       asamd_csr_plan_destroy(p);

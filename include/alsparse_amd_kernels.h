@@ -211,6 +211,8 @@ int asamd_spmv_trans_ylds(hipStream_t stream, const asamd_spmv_args *a, int32_t 
  * kernel for a matrix whose longest row has max_len entries.  partials: asamd_spmv_trans_slices_bytes(dtype, n, nnz) bytes
  * of per-call scratch (0: none is needed). */
 int asamd_spmv_trans_slices_fit(int32_t dtype, int32_t m, int32_t n, int32_t nnz, int32_t max_len);
+/* Whether it is the better kernel for scattered columns: lines per entry as asamd_csr_row_stats_lines gives them. */
+int asamd_spmv_trans_slices_pay(int32_t dtype, int32_t n, int32_t nnz, float lines);
 size_t asamd_spmv_trans_slices_bytes(int32_t dtype, int32_t n, int32_t nnz);
 int asamd_spmv_trans_slices(hipStream_t stream, const asamd_spmv_args *a, int32_t conj, void *partials);
 
@@ -347,6 +349,11 @@ void asamd_transpose_free(asamd_transpose_layout *layout);
 #define ASAMD_ROW_STATS_WORDS (3 + ASAMD_HIST_BINS)
 int asamd_csr_row_stats(hipStream_t stream, int32_t m, const int32_t *row_ptr, int32_t *d_scratch,
                         int32_t *stats_host);
+/* The same, and *lines_host = distinct 128-byte lines of y (elements of elem_bytes) per entry that runs of 1 024 entries
+ * meet, sampled; 0 where col_ind is NULL or nnz is under 65 536.  d_scratch: one device int more. */
+int asamd_csr_row_stats_lines(hipStream_t stream, int32_t m, const int32_t *row_ptr, int32_t nnz, int32_t base,
+                              int32_t elem_bytes, const int32_t *col_ind, int32_t *d_scratch, int32_t *stats_host,
+                              float *lines_host);
 /* 64-bit fingerprint of the structure arrays (m + 1 offsets, nnz columns): equal arrays give equal
  * values.  d_scratch: 8 device bytes, 8-byte aligned.  Synchronises `stream`; *hash_host is a host word. */
 int asamd_csr_structure_hash(hipStream_t stream, int32_t m, int32_t nnz, const int32_t *row_ptr,
