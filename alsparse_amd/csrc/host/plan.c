@@ -39,6 +39,7 @@ struct asamd_csr_plan {
   int rel16_group;         /* the lanes per row they were made for */
   asamd_pattern_layout pat; /* staged row blocks: a pattern number per row instead of the columns */
   int pinned;              /* the family was set from outside: the staged row blocks then read columns (or distances) */
+  int of_transpose;        /* the analysis of a copy of A^T or A^H: A's plan checks the values, the caller sets no family */
   int watched;             /* laid out for asamd_csr_plan_csrmv_watched: its fingerprints are the caller's account */
   void *d_eval;            /* ELL copy: ell_width * m values, column-major */
   int32_t *d_ecol;         /* ... and zero-based columns */
@@ -673,6 +674,11 @@ static hipError_t refresh_trans(hipStream_t s, asamd_csr_plan *p, int which, con
   return e;
 }
 
+/* How the row-sum tiles' values are checked against the caller's.  Where they stand in for a family that reads csr_val on
+ * every multiply, a change of any single value has to show in the next product: every byte is fingerprinted.  Where that
+ * family holds a copy itself they are checked as that copy is. */
+static int sums_check_all(const asamd_csr_plan *p) { return p->st.value_check == 2 || !holds_values(p, p->auto_algo); }
+
 /* The row-sum tiles' multiply, or -1 where they do not serve this call: none laid out, a family set from outside, other
  * values than those they hold, no room for their scratch or for the check of their values. */
 static int csrmv_sums(hipStream_t s, asamd_csr_plan *p, const asamd_spmv_args *a, ws_cursor ws, int guard) {
@@ -682,7 +688,7 @@ static int csrmv_sums(hipStream_t s, asamd_csr_plan *p, const asamd_spmv_args *a
   void *sums = ws_take(&ws, sums_scratch(p));
   if (!sums || (guard && st->value_check && !g)) return -1;
   if (g) {
-    int e = asamd_value_guard(s, a->val, (size_t)st->nnz * (size_t)p->val_size, st->value_check == 2, p->d_fp + FP_SUMS, g);
+    int e = asamd_value_guard(s, a->val, (size_t)st->nnz * (size_t)p->val_size, sums_check_all(p), p->d_fp + FP_SUMS, g);
     if (e == hipSuccess) e = asamd_sums_refresh_values(s, &p->sums, a->val, ASAMD_GUARD_FLAG(g));
     if (e == hipSuccess) e = asamd_value_guard_commit(s, g, p->d_fp + FP_SUMS);
     if (e != hipSuccess) return e;
@@ -1331,16 +1337,17 @@ static hipError_t model_copies(hipStream_t stream, asamd_csr_plan *p, const int3
 }
 
 /* ---- row-sum tiles -----------------------------------------------------------------------------------
- * What AUTO runs in the place of the family that was chosen, where their estimate is under 0.9 of that family's.
+ * What AUTO runs in the place of the family that was chosen, where their estimate is under 0.83 of that family's and, with
+ * the fingerprint of every byte that they need in the place of a family that reads csr_val, under 0.95.
  * They move vs + 2 bytes per entry and 2 vs + 2 per sum (a row's entries in one column block of 128 KB of x); measured
  * with power-law rows and columns (1.1 .. 8.4 M rows, P = sums per entry = 0.31 .. 0.46), power-law rows over uniform
  * columns, two and geometric row lengths, uniform rows of 3 .. 128 entries over 2 .. 64 MB of x, all types: 0.03 ms
- * (the value guard's launches, two phases' ramps) and 4.2 TB/s, 4.9 from 4 GB on, within a fifth.  Before -> with them, us:
- *   power law, 8.4 M rows: fp32 524 -> 250, fp64 779 -> 465; 2.1 M rows 136 -> 78, 164 -> 117; 1.1 M rows 62 -> 57, 83 -> 79;
- *     0.6 M rows 37 -> 52, 40 -> 65 (estimate 43, 59: not laid out)
- *   uniform rows, fp32: 1 M x 1 M x 16 103 -> 78, x 32 208 -> 120, x 64 324 -> 170, 2 M x 2 M x 16 173 -> 142, 4 M x 4 M x 16
- *     285 -> 253, 16 M x 16 M x 16 853 -> 910 (next to no row meets a column block twice, and the tiled pair's are wider:
- *     estimate 926 against 906, not laid out); fp64: 1 M x 1 M x 16 165 -> 120, 2 M x 2 M x 64 1215 -> 649
+ * (the value guard's launches, two phases' ramps) and 4.65 TB/s, 4.9 from 4 GB on; the estimate is within a tenth of 40 of 46
+ * timings and within 17 % of all, the families' are within a quarter.  Before -> with them, the check included, us:
+ *   power law, 8.4 M rows: fp32 527 -> 323, 2.1 M rows 124 -> 87; 1.1 M rows 62 -> 60 (not laid out)
+ *   uniform rows, fp32: 1 M x 1 M x 16 93 -> 79, x 32 189 -> 137, x 64 324 -> 170, 2 M x 2 M x 16 173 -> 142;
+ *     4 M x 4 M x 16 285 -> 253 (not laid out), 16 M x 16 M x 16 853 -> 910 (next to no row meets a column block twice, and
+ *     the tiled pair's are wider: not laid out); fp64: 1 M x 1 M x 16 161 -> 115, 2 M x 2 M x 64 1215 -> 649
  * A matrix that they serve keeps the copy of its family, for a family set from outside and for other value arrays. */
 static double sums_bytes(const asamd_csr_plan *p, double sums) {
   const asamd_csr_stats *st = &p->st;
@@ -1349,8 +1356,8 @@ static double sums_bytes(const asamd_csr_plan *p, double sums) {
 }
 static double sums_ms(const asamd_csr_plan *p, double sums) {
   const double bytes = sums_bytes(p, sums);
-  double rate = 4.2 + 0.7 * (bytes - 1.0e9) / 3.0e9;
-  if (rate < 4.2) rate = 4.2;
+  double rate = 4.65 + 0.25 * (bytes - 1.0e9) / 3.0e9;
+  if (rate < 4.65) rate = 4.65;
   if (rate > 4.9) rate = 4.9;
   return 0.03 + bytes / (rate * 1e9);
 }
@@ -1367,17 +1374,28 @@ static hipError_t build_sums(hipStream_t stream, asamd_csr_plan *p, const int32_
     if (st->nnz < (1 << 22) || st->lines_per_entry_wave <= 0.f) return hipSuccess;
     const int algo = p->auto_algo;
     double kept = model_ms(p, algo == ASAMD_SPMV_MERGE_HOT || algo == ASAMD_SPMV_BINNED ? ASAMD_SPMV_MERGE : algo);
-    if (algo == ASAMD_SPMV_BINNED || algo == ASAMD_SPMV_MERGE_HOT) kept *= 0.95; /* they were kept for being faster */
+    if (algo == ASAMD_SPMV_BINNED || algo == ASAMD_SPMV_MERGE_HOT) {
+      /* they were kept for being faster; with 8-byte values merge-path's estimate runs low (power law of 2.1 / 4.2 / 8.4 M
+       * rows, hot columns: 0.179 / 0.363 / 0.790 ms, estimated at 0.158 / 0.328 / 0.672) */
+      kept *= p->val_size < 8 ? 0.95 : 1.1;
+    }
     if (holds_values(p, algo) && algo != ASAMD_SPMV_XLDS && st->value_check) kept += 0.022;
     /* (the tiled pair's estimate runs high for 16-byte values: the transpose of 2.5 M x 2.5 M x 18, complex128, 0.63 against
      * 0.493 ms; with them 0.506) */
     if (algo == ASAMD_SPMV_TILED && p->val_size == 16) kept *= 0.8;
+    double most_ms = 0.83 * kept;
+    /* every byte fingerprinted (sums_check_all): 0.21 ms for 1 GiB, arrays of up to 32 MiB are read whole anyway; the copy of
+     * A^T stands behind the check of A's values */
+    const double beyond = (double)st->nnz * (double)p->val_size - (double)ASAMD_GUARD_FULL_BYTES;
+    if (st->value_check && !p->of_transpose && !holds_values(p, algo) && beyond > 0.0 &&
+        0.95 * kept - beyond / 5.1e9 < most_ms)
+      most_ms = 0.95 * kept - beyond / 5.1e9;
     /* the most sums that pay: by bisection, the estimate grows with them */
     double lo = (double)(st->m - st->hist[0]), hi = most;
-    if (!(sums_ms(p, lo) < 0.9 * kept)) return hipSuccess; /* a row leaves one sum at least */
+    if (!(sums_ms(p, lo) < most_ms)) return hipSuccess; /* a row leaves one sum at least */
     for (int i = 0; i < 40; ++i) {
       const double mid = 0.5 * (lo + hi);
-      if (sums_ms(p, mid) < 0.9 * kept) lo = mid;
+      if (sums_ms(p, mid) < most_ms) lo = mid;
       else hi = mid;
     }
     most = lo;
@@ -1395,15 +1413,15 @@ static hipError_t build_sums(hipStream_t stream, asamd_csr_plan *p, const int32_
 /* the fingerprint of the values a copy set was taken from (set-up work: plan-owned scratch, not concurrent) */
 static hipError_t first_fingerprint(hipStream_t stream, asamd_csr_plan *p, const void *val, int slot) {
   if (!p->st.value_check) return hipSuccess;
-  hipError_t e = (hipError_t)asamd_value_guard(stream, val, (size_t)p->st.nnz * (size_t)p->val_size,
-                                               p->st.value_check == 2, NULL, p->d_setup);
+  const int full = slot == FP_SUMS ? sums_check_all(p) : p->st.value_check == 2;
+  hipError_t e = (hipError_t)asamd_value_guard(stream, val, (size_t)p->st.nnz * (size_t)p->val_size, full, NULL, p->d_setup);
   if (e == hipSuccess) e = (hipError_t)asamd_value_guard_commit(stream, p->d_setup, p->d_fp + slot);
   return e;
 }
 
 static hipError_t plan_create(hipStream_t stream, int32_t m, int32_t n, int32_t nnz, const int32_t *row_ptr,
                               const int32_t *col_ind, const void *val, int32_t base, int32_t dtype, int32_t trusted,
-                              asamd_csr_plan **out) {
+                              int of_transpose, asamd_csr_plan **out) {
   if (!out || !row_ptr || m <= 0 || nnz < 0 || dtype < ASAMD_DTYPE_FLOAT || dtype > ASAMD_DTYPE_DOUBLE_COMPLEX)
     return hipErrorInvalidValue;
   const int val_size = kValSize[dtype];
@@ -1421,6 +1439,7 @@ static hipError_t plan_create(hipStream_t stream, int32_t m, int32_t n, int32_t 
   p->dtype = dtype;
   p->val_size = val_size;
   p->watched = trusted == 3;
+  p->of_transpose = of_transpose;
 
   hipError_t e = hipMalloc(&p->d_setup, SETUP_BYTES);
   if (e == hipSuccess) e = hipMalloc((void **)&p->d_fp, FP_WORDS * sizeof(uint64_t));
@@ -1630,13 +1649,13 @@ int asamd_csr_plan_create(hipStream_t stream, int32_t m, int32_t n, int32_t nnz,
                           asamd_csr_plan **out) {
   if (val_size != 4 && val_size != 8) return hipErrorInvalidValue;
   return plan_create(stream, m, n, nnz, row_ptr, col_ind, val, base,
-                     val_size == 4 ? ASAMD_DTYPE_FLOAT : ASAMD_DTYPE_DOUBLE, trusted, out);
+                     val_size == 4 ? ASAMD_DTYPE_FLOAT : ASAMD_DTYPE_DOUBLE, trusted, 0, out);
 }
 
 int asamd_csr_plan_create_dtype(hipStream_t stream, int32_t m, int32_t n, int32_t nnz, const int32_t *row_ptr,
                                 const int32_t *col_ind, const void *val, int32_t base, int32_t dtype, int32_t trusted,
                                 asamd_csr_plan **out) {
-  return plan_create(stream, m, n, nnz, row_ptr, col_ind, val, base, dtype, trusted, out);
+  return plan_create(stream, m, n, nnz, row_ptr, col_ind, val, base, dtype, trusted, 0, out);
 }
 
 void asamd_csr_plan_destroy(asamd_csr_plan *p) {
@@ -1667,7 +1686,7 @@ static hipError_t build_transpose(hipStream_t stream, asamd_csr_plan *p, const i
                                                    val, &t->t);
   if (e == hipSuccess)
     e = plan_create(stream, st->n, st->m, st->nnz, t->t.row_ptr, t->t.col_ind, t->t.val, 0, p->dtype, /*trusted=*/1,
-                    &t->plan);
+                    /*of_transpose=*/1, &t->plan);
   if (e == hipSuccess) e = first_fingerprint(stream, p, val, 1 + which);
   if (e == hipSuccess) e = hipStreamSynchronize(stream);
   if (e != hipSuccess) {

@@ -114,15 +114,17 @@ size_t asamd_csr_plan_workspace_bytes(const asamd_csr_plan *plan);
  * multiply still gives the right result through kernels that need no scratch (a lane group per row;
  * the atomic scatter for op != 0), slowly.
  *
- * Values changed in place: a plan's copies (tiled, ELL, A^T, A^H) hold the values that `val` held when
- * they were laid out.  Before such a copy is used, a guard kernel fingerprints val and compares with
+ * Values changed in place: a plan's copies (tiled, ELL, slice by slice, row-sum tiles, A^T, A^H) hold the values that `val`
+ * held when they were laid out.  Before such a copy is used, a guard kernel fingerprints val and compares with
  * the fingerprint of the values the copy was taken from; if they differ, the copy is gathered again
  * through the permutation the plan kept -- all on the device, in stream order, no host round trip.
  * By default the fingerprint covers every byte of arrays up to 32 MiB and, of larger ones, 256 bytes
  * at a varying position of every run of asamd_value_guard_run(bytes) bytes (8 KiB for a gigabyte): a
  * caller who rewrites the array, or any contiguous stretch of at least two runs, is always noticed; one who
  * pokes single entries of a large array is noticed with probability 256 / run and should call
- * asamd_csr_plan_refresh_values (or analyse again).  ALSPARSE_AMD_VALUE_CHECK=full fingerprints every
+ * asamd_csr_plan_refresh_values (or analyse again).  Row-sum tiles that stand in for a family that keeps no
+ * values (merge-path, the hot columns, the row kernels) are the exception: every byte is fingerprinted for them, and a
+ * single changed entry counts as it does with that family.  ALSPARSE_AMD_VALUE_CHECK=full fingerprints every
  * byte (one more pass over val per multiply), =off none (the caller then refreshes by hand).  A
  * multiply that passes ANOTHER value array than the copies were taken from runs on the caller's arrays. */
 int asamd_csr_plan_csrmv(hipStream_t stream, asamd_csr_plan *plan, int32_t op, const void *alpha, const void *val,

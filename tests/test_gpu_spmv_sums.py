@@ -171,6 +171,33 @@ def test_values_follow_the_caller(gpu):
         p.close()
 
 
+def test_single_values_poked_into_a_graph_count(gpu):
+    """Merge-path and the hot-column kernel read csr_val on every multiply; the tiles that stand in for them hold a copy of
+    it, 92 MB here, of which the usual check reads a quarter: one changed value anywhere has to show in the next product
+    all the same."""
+    a = wl.powerlaw_rmat(21, 50000, np.float32)
+    lib = capi.load()
+    assert int(lib.asamd_value_guard_run(a.nnz * 4)) >= 1024, "an array of which the usual check reads a part"
+    rng = np.random.default_rng(17)
+    x = wl.uniform(a.cols, a.dtype, 3)
+    x[np.abs(x) < 0.1] = 0.5
+    y0 = np.zeros(a.rows, np.float32)
+    p = Plan(a, 1)
+    try:
+        announce("row sums, single values poked")
+        assert p.stats.row_sums == 1 and p.stats.value_check == 1
+        assert p.stats.algo in (capi.ASAMD_SPMV_MERGE, capi.ASAMD_SPMV_MERGE_HOT)
+        vals = a.values.copy()
+        p.multiply(1.0, x, 0.0, y0)
+        for k in list(rng.integers(0, a.nnz, 8)) + [a.nnz - 1, 0]:
+            vals[k] = np.float32(1000.0)
+            p.da.val.copy_from(vals)
+            b = wl.Csr(a.rows, a.cols, a.row_ptr, a.col_ind, vals, a.base, "poked")
+            _check(b, 1.0, x, 0.0, y0, p.multiply(1.0, x, 0.0, y0), "value %d poked" % k)
+    finally:
+        p.close()
+
+
 @pytest.mark.parametrize("name,make,want", [
     # rows of 16, and uneven rows of 30 on average, over 4 MB of x; matrices whose x the LDS or the caches hold stay as they are
     ("uniform", lambda: wl.uniform_rows(1 << 20, 1 << 20, 16, np.float32), 1),
