@@ -1771,6 +1771,7 @@ int asamd_csr_plan_set_algo(asamd_csr_plan *p, int32_t algo) {
       p->st.algo = p->auto_algo;
       p->pinned = 0;
       p->st.row_patterns = p->pat.pid != NULL;
+      p->st.row_sums = p->sums.tval != NULL;
       return hipSuccess;
     case ASAMD_SPMV_ROWCONST:
       if (!rowconst_ok(p)) return hipErrorInvalidValue;
@@ -1806,5 +1807,6 @@ int asamd_csr_plan_set_algo(asamd_csr_plan *p, int32_t algo) {
   p->st.algo = algo;
   p->pinned = 1;
   p->st.row_patterns = 0;
+  p->st.row_sums = 0;
   return hipSuccess;
 }

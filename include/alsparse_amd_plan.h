@@ -68,7 +68,8 @@ typedef struct {
   float lines_per_entry_segment; /* ... and within runs of 32 768 consecutive entries                     */
   int32_t xlds_slices;   /* column slices of the kernel that holds x in LDS (a table of offsets exists), or 0   */
   int32_t row_patterns;  /* 1: STREAM reads a pattern number per row instead of columns (not where a family was set) */
-  int32_t row_sums;      /* 1: MERGE and MERGE_HOT run on row-sum tiles (not where a family was set)            */
+  int32_t row_sums;      /* 1: the multiply runs on row-sum tiles in the place of `algo`, whichever it is (0 where a family
+                            was set from outside)                                                                */
 } asamd_csr_stats;
 
 typedef struct asamd_csr_plan asamd_csr_plan;

@@ -163,8 +163,10 @@ def test_values_follow_the_caller(gpu):
         small.bytes = 4096
         _check(a, 1.0, x, 0.5, y0, p.multiply(1.0, x, 0.5, y0, ws=small), "no room")
         assert p.lib.asamd_csr_plan_set_algo(p.plan, ALGOS["merge"]) == 0
+        assert p.stats.row_sums == 0, "a family set from outside runs, not the tiles"
         _check(a, 1.0, x, 0.5, y0, p.multiply(1.0, x, 0.5, y0), "merge-path set from outside")
         assert p.lib.asamd_csr_plan_set_algo(p.plan, capi.ASAMD_SPMV_AUTO) == 0
+        assert p.stats.row_sums == 1
         assert np.array_equal(p.multiply(1.0, x, 0.5, y0), first)
         d_other.free()
     finally:
