@@ -901,6 +901,17 @@ int asamd_csr_plan_csrmv_watched(hipStream_t s, asamd_csr_plan *p, const void *a
 /* ---- analysis: timing the candidates ----------------------------------------------------------------- */
 enum { CAND_BASE = 0, CAND_TILED, CAND_ELL, CAND_HOT, CAND_BINNED, CAND_COUNT };
 
+/* ALSPARSE_AMD_TUNE_PICK = base | tiled | ell | hot | binned overrides the verdict among the candidates that the matrix is
+ * eligible for (for profiling a kernel that lost); -1: not set.  Row-sum tiles, which take the place of any family, are not
+ * laid out then. */
+static int env_tune_pick(void) {
+  static const char *names[CAND_COUNT] = {"base", "tiled", "ell", "hot", "binned"};
+  const char *e = getenv("ALSPARSE_AMD_TUNE_PICK");
+  for (int c = 0; e && c < CAND_COUNT; ++c)
+    if (!strcmp(e, names[c])) return c;
+  return -1;
+}
+
 typedef struct {
   hipStream_t stream;
   asamd_csr_plan *p;
@@ -1063,14 +1074,8 @@ static hipError_t tune_copies(hipStream_t stream, asamd_csr_plan *p, const int32
   int pick = 0;
   for (int c = 1; c < CAND_COUNT; ++c)
     if (cost[c] > 0.f && cost[c] < margin[c] * cost[CAND_BASE] && (pick == 0 || cost[c] < cost[pick])) pick = c;
-  /* ALSPARSE_AMD_TUNE_PICK = base | tiled | ell | hot | binned overrides the timing's verdict among the
-   * candidates that were built (for profiling a kernel that lost) */
-  const char *ev = getenv("ALSPARSE_AMD_TUNE_PICK");
-  if (ev) {
-    static const char *names[CAND_COUNT] = {"base", "tiled", "ell", "hot", "binned"};
-    for (int c = 0; c < CAND_COUNT; ++c)
-      if (!strcmp(ev, names[c]) && (c == 0 || t.best[c] > 0.f)) pick = c;
-  }
+  const int forced = env_tune_pick();
+  if (forced == CAND_BASE || (forced > 0 && t.best[forced] > 0.f)) pick = forced;
   if (pick != CAND_TILED) free_tiled(p);
   if (pick != CAND_ELL) free_ell(p);
   if (pick != CAND_HOT) free_hot(p);
@@ -1277,13 +1282,7 @@ static hipError_t model_copies(hipStream_t stream, asamd_csr_plan *p, const int3
      * 2 M x 16 384: 0.39 -> 0.25. */
     if (xlds_sized_x(p) && st->nnz >= (1 << 22) && !xlds_rows_regular(st)) want_hot = 1;
   }
-  const char *ev = getenv("ALSPARSE_AMD_TUNE_PICK");
-  int forced = -1;
-  if (ev) {
-    static const char *names[CAND_COUNT] = {"base", "tiled", "ell", "hot", "binned"};
-    for (int c = 0; c < CAND_COUNT; ++c)
-      if (!strcmp(ev, names[c])) forced = c;
-  }
+  const int forced = env_tune_pick();
   int order[4] = {CAND_BASE, CAND_BASE, CAND_BASE, CAND_BASE};
   const int tiled_wins = tiled_ok && est_tiled < 0.9 * base, ell_wins = ell_ok && est_ell < 0.95 * base;
   int k = 0;
@@ -1371,7 +1370,7 @@ static hipError_t build_sums(hipStream_t stream, asamd_csr_plan *p, const int32_
   if (force) {
     if (p->auto_algo != ASAMD_SPMV_MERGE) return hipSuccess;
   } else {
-    if (st->nnz < (1 << 22) || st->lines_per_entry_wave <= 0.f) return hipSuccess;
+    if (st->nnz < (1 << 22) || st->lines_per_entry_wave <= 0.f || env_tune_pick() >= 0) return hipSuccess;
     const int algo = p->auto_algo;
     double kept = model_ms(p, algo == ASAMD_SPMV_MERGE_HOT || algo == ASAMD_SPMV_BINNED ? ASAMD_SPMV_MERGE : algo);
     if (algo == ASAMD_SPMV_BINNED || algo == ASAMD_SPMV_MERGE_HOT) {

@@ -223,3 +223,20 @@ def test_the_analysis_lays_them_out_where_they_pay(gpu, name, make, want, monkey
     finally:
         p.close()
         q.close()
+
+
+@pytest.mark.parametrize("pick,algo", [("tiled", capi.ASAMD_SPMV_TILED), ("ell", capi.ASAMD_SPMV_ELL), ("base", None)])
+@pytest.mark.parametrize("tune", ["model", "timed"])
+def test_a_family_picked_for_the_analysis_is_the_one_that_runs(gpu, pick, algo, tune, monkeypatch):
+    """ALSPARSE_AMD_TUNE_PICK overrides the analysis' verdict: the tiles do not take the picked family's place."""
+    a = wl.uniform_rows(1 << 21, 1 << 21, 16, np.float32)
+    monkeypatch.setenv("ALSPARSE_AMD_TUNE", tune)
+    monkeypatch.setenv("ALSPARSE_AMD_TUNE_PICK", pick)
+    p = Plan(a, 1)
+    try:
+        announce("row sums, picked", pick, tune)
+        assert p.stats.row_sums == 0
+        if tune == "model":  # (a timing run picks among the copies that it found worth laying out)
+            assert p.stats.algo == algo if algo is not None else p.stats.tiled_built + p.stats.ell_built == 0
+    finally:
+        p.close()
