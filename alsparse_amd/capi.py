@@ -136,7 +136,8 @@ class asamd_csr_stats(Structure):
                 ("tile_long_blocks", c_int32), ("value_check", c_int32), ("tune_mode", c_int32),
                 ("device_bytes", c_int64), ("workspace_bytes", c_int64),
                 ("lines_per_entry_wave", c_float), ("lines_per_entry_segment", c_float),
-                ("xlds_slices", c_int32), ("row_patterns", c_int32), ("row_sums", c_int32)]
+                ("xlds_slices", c_int32), ("row_patterns", c_int32), ("row_sums", c_int32),
+                ("tune_ms_sums", c_float)]
 
 
 class asamd_spmv_args(Structure):  # include/alsparse_amd_kernels.h

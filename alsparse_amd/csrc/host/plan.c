@@ -899,7 +899,7 @@ int asamd_csr_plan_csrmv_watched(hipStream_t s, asamd_csr_plan *p, const void *a
 }
 
 /* ---- analysis: timing the candidates ----------------------------------------------------------------- */
-enum { CAND_BASE = 0, CAND_TILED, CAND_ELL, CAND_HOT, CAND_BINNED, CAND_COUNT };
+enum { CAND_BASE = 0, CAND_TILED, CAND_ELL, CAND_HOT, CAND_BINNED, CAND_COUNT, CAND_SUMS = CAND_COUNT, CAND_ALL };
 
 /* ALSPARSE_AMD_TUNE_PICK = base | tiled | ell | hot | binned overrides the verdict among the candidates that the matrix is
  * eligible for (for profiling a kernel that lost); -1: not set.  Row-sum tiles, which take the place of any family, are not
@@ -920,7 +920,7 @@ typedef struct {
   void *x, *y, *ws;
   size_t ws_bytes;
   hipEvent_t e0, e1;
-  float best[CAND_COUNT];
+  float best[CAND_ALL];
   int algos[CAND_COUNT];
   hipError_t err;
 } tune_ctx;
@@ -935,10 +935,35 @@ static void tune_reserve(tune_ctx *t, size_t bytes) {
   if (t->err == hipSuccess) t->ws_bytes = bytes;
 }
 
+static void tune_open(tune_ctx *t, hipStream_t stream, asamd_csr_plan *p, const int32_t *row_ptr, const int32_t *col_ind,
+                      const void *val) {
+  const size_t vs = (size_t)p->val_size;
+  memset(t, 0, sizeof *t);
+  t->stream = stream;
+  t->p = p;
+  t->row_ptr = row_ptr;
+  t->col_ind = col_ind;
+  t->val = val;
+  t->err = hipMalloc(&t->x, (size_t)p->st.n * vs);
+  if (t->err == hipSuccess) t->err = hipMalloc(&t->y, (size_t)p->st.m * vs);
+  if (t->err == hipSuccess) t->err = hipMemsetAsync(t->x, 0, (size_t)p->st.n * vs, stream);
+  if (t->err == hipSuccess) t->err = hipEventCreate(&t->e0);
+  if (t->err == hipSuccess) t->err = hipEventCreate(&t->e1);
+}
+
+static void tune_close(tune_ctx *t) {
+  if (t->e0) (void)hipEventDestroy(t->e0);
+  if (t->e1) (void)hipEventDestroy(t->e1);
+  if (t->x) (void)hipFree(t->x);
+  if (t->y) (void)hipFree(t->y);
+  if (t->ws) (void)hipFree(t->ws);
+}
+
+/* CAND_SUMS: the row-sum tiles where they are laid out (csrmv_inner prefers them to any family) */
 static void time_algo(tune_ctx *t, int cand) {
   asamd_csr_plan *p = t->p;
-  p->st.algo = t->algos[cand];
-  tune_reserve(t, algo_scratch(p, t->algos[cand]) + 512);
+  if (cand != CAND_SUMS) p->st.algo = t->algos[cand];
+  tune_reserve(t, (cand == CAND_SUMS ? sums_scratch(p) : algo_scratch(p, t->algos[cand])) + 512);
   static const double one[2] = {1.0, 0.0}, zero[2] = {0.0, 0.0};
   static const float onef[2] = {1.0f, 0.0f}, zerof[2] = {0.0f, 0.0f};
   const int wide = p->dtype == ASAMD_DTYPE_DOUBLE || p->dtype == ASAMD_DTYPE_DOUBLE_COMPLEX;
@@ -970,17 +995,7 @@ static hipError_t tune_copies(hipStream_t stream, asamd_csr_plan *p, const int32
   asamd_csr_stats *st = &p->st;
   const size_t vs = (size_t)p->val_size;
   tune_ctx t;
-  memset(&t, 0, sizeof t);
-  t.stream = stream;
-  t.p = p;
-  t.row_ptr = row_ptr;
-  t.col_ind = col_ind;
-  t.val = val;
-  t.err = hipMalloc(&t.x, (size_t)st->n * vs);
-  if (t.err == hipSuccess) t.err = hipMalloc(&t.y, (size_t)st->m * vs);
-  if (t.err == hipSuccess) t.err = hipMemsetAsync(t.x, 0, (size_t)st->n * vs, stream);
-  if (t.err == hipSuccess) t.err = hipEventCreate(&t.e0);
-  if (t.err == hipSuccess) t.err = hipEventCreate(&t.e1);
+  tune_open(&t, stream, p, row_ptr, col_ind, val);
   t.algos[CAND_BASE] = p->auto_algo;
   t.algos[CAND_TILED] = ASAMD_SPMV_TILED;
   t.algos[CAND_ELL] = ASAMD_SPMV_ELL;
@@ -1052,11 +1067,7 @@ static hipError_t tune_copies(hipStream_t stream, asamd_csr_plan *p, const int32
     t.err = build_binned(stream, p, row_ptr);
     if (t.err == hipSuccess && st->binned_built) time_algo(&t, CAND_BINNED);
   }
-  if (t.e0) (void)hipEventDestroy(t.e0);
-  if (t.e1) (void)hipEventDestroy(t.e1);
-  if (t.x) (void)hipFree(t.x);
-  if (t.y) (void)hipFree(t.y);
-  if (t.ws) (void)hipFree(t.ws);
+  tune_close(&t);
   st->algo = p->auto_algo;
   if (t.err != hipSuccess) return t.err;
   st->tune_ms_binned = t.best[CAND_BINNED];
@@ -1361,37 +1372,67 @@ static double sums_ms(const asamd_csr_plan *p, double sums) {
   return 0.03 + bytes / (rate * 1e9);
 }
 
+/* Every byte fingerprinted (sums_check_all): 0.21 ms for 1 GiB, arrays of up to 32 MiB are read whole anyway; the copy of A^T
+ * stands behind the check of A's values. */
+static double sums_check_ms(const asamd_csr_plan *p) {
+  const asamd_csr_stats *st = &p->st;
+  const double beyond = (double)st->nnz * (double)p->val_size - (double)ASAMD_GUARD_FULL_BYTES;
+  return st->value_check && !p->of_transpose && !holds_values(p, p->auto_algo) && beyond > 0.0 ? beyond / 5.1e9 : 0.0;
+}
+
+/* the family's own figure that the tiles are laid out against */
+static double sums_rival_ms(const asamd_csr_plan *p) {
+  const int algo = p->auto_algo;
+  double kept = model_ms(p, algo == ASAMD_SPMV_MERGE_HOT || algo == ASAMD_SPMV_BINNED ? ASAMD_SPMV_MERGE : algo);
+  if (algo == ASAMD_SPMV_BINNED || algo == ASAMD_SPMV_MERGE_HOT) {
+    /* they were kept for being faster; with 8-byte values merge-path's estimate runs low (power law of 2.1 / 4.2 / 8.4 M
+     * rows, hot columns: 0.179 / 0.363 / 0.790 ms, estimated at 0.158 / 0.328 / 0.672) */
+    kept *= p->val_size < 8 ? 0.95 : 1.1;
+  }
+  if (holds_values(p, algo) && algo != ASAMD_SPMV_XLDS && p->st.value_check) kept += 0.022;
+  /* (the tiled pair's estimate runs high for 16-byte values: the transpose of 2.5 M x 2.5 M x 18, complex128, 0.63 against
+   * 0.493 ms; with them 0.506) */
+  if (algo == ASAMD_SPMV_TILED && p->val_size == 16) kept *= 0.8;
+  return kept;
+}
+
 static hipError_t build_sums(hipStream_t stream, asamd_csr_plan *p, const int32_t *row_ptr, const int32_t *col_ind,
                              const void *val, int force) {
   asamd_csr_stats *st = &p->st;
   if (!st->trusted || st->first_offset != 0 || env_int("ALSPARSE_AMD_ROW_SUMS", 1) <= 0) return hipSuccess;
   if (!asamd_tiled_fits(p->dtype, st->m, st->n, st->nnz)) return hipSuccess;
+  const int timed = !force && !st->tune_mode;
   double most = (double)st->nnz;
+  tune_ctx t;
+  memset(&t, 0, sizeof t);
+  hipError_t e = hipSuccess;
   if (force) {
     if (p->auto_algo != ASAMD_SPMV_MERGE) return hipSuccess;
   } else {
     if (st->nnz < (1 << 22) || st->lines_per_entry_wave <= 0.f || env_tune_pick() >= 0) return hipSuccess;
-    const int algo = p->auto_algo;
-    double kept = model_ms(p, algo == ASAMD_SPMV_MERGE_HOT || algo == ASAMD_SPMV_BINNED ? ASAMD_SPMV_MERGE : algo);
-    if (algo == ASAMD_SPMV_BINNED || algo == ASAMD_SPMV_MERGE_HOT) {
-      /* they were kept for being faster; with 8-byte values merge-path's estimate runs low (power law of 2.1 / 4.2 / 8.4 M
-       * rows, hot columns: 0.179 / 0.363 / 0.790 ms, estimated at 0.158 / 0.328 / 0.672) */
-      kept *= p->val_size < 8 ? 0.95 : 1.1;
+    double most_ms = 0.0;
+    if (timed) {
+      /* ALSPARSE_AMD_TUNE=timed: the clock decides; the estimate only spares a layout that has no chance */
+      tune_open(&t, stream, p, row_ptr, col_ind, val);
+      t.algos[CAND_BASE] = p->auto_algo;
+      p->copy_val_src = val;
+      if (t.err == hipSuccess) time_algo(&t, CAND_BASE);
+      e = t.err;
+      if (e == hipSuccess && holds_values(p, p->auto_algo) && st->value_check) t.best[CAND_BASE] += 0.022f;
+      most_ms = 1.2 * (double)t.best[CAND_BASE];
+    } else {
+      const double kept = sums_rival_ms(p), check = sums_check_ms(p);
+      most_ms = 0.83 * kept;
+      if (check > 0.0 && 0.95 * kept - check < most_ms) most_ms = 0.95 * kept - check;
     }
-    if (holds_values(p, algo) && algo != ASAMD_SPMV_XLDS && st->value_check) kept += 0.022;
-    /* (the tiled pair's estimate runs high for 16-byte values: the transpose of 2.5 M x 2.5 M x 18, complex128, 0.63 against
-     * 0.493 ms; with them 0.506) */
-    if (algo == ASAMD_SPMV_TILED && p->val_size == 16) kept *= 0.8;
-    double most_ms = 0.83 * kept;
-    /* every byte fingerprinted (sums_check_all): 0.21 ms for 1 GiB, arrays of up to 32 MiB are read whole anyway; the copy of
-     * A^T stands behind the check of A's values */
-    const double beyond = (double)st->nnz * (double)p->val_size - (double)ASAMD_GUARD_FULL_BYTES;
-    if (st->value_check && !p->of_transpose && !holds_values(p, algo) && beyond > 0.0 &&
-        0.95 * kept - beyond / 5.1e9 < most_ms)
-      most_ms = 0.95 * kept - beyond / 5.1e9;
     /* the most sums that pay: by bisection, the estimate grows with them */
     double lo = (double)(st->m - st->hist[0]), hi = most;
-    if (!(sums_ms(p, lo) < most_ms)) return hipSuccess; /* a row leaves one sum at least */
+    if (e != hipSuccess || !(sums_ms(p, lo) < most_ms)) { /* a row leaves one sum at least */
+      tune_close(&t);
+      if (e != hipErrorOutOfMemory) return e;
+      (void)hipGetLastError();
+      return hipSuccess;
+    }
     for (int i = 0; i < 40; ++i) {
       const double mid = 0.5 * (lo + hi);
       if (sums_ms(p, mid) < most_ms) lo = mid;
@@ -1399,13 +1440,22 @@ static hipError_t build_sums(hipStream_t stream, asamd_csr_plan *p, const int32_
     }
     most = lo;
   }
-  hipError_t e = (hipError_t)asamd_sums_build(stream, p->dtype, st->m, st->n, st->nnz, st->base, row_ptr, col_ind, val,
-                                              (int64_t)most, &p->sums);
+  e = (hipError_t)asamd_sums_build(stream, p->dtype, st->m, st->n, st->nnz, st->base, row_ptr, col_ind, val, (int64_t)most,
+                                   &p->sums);
+  if (timed && e == hipSuccess && p->sums.tval) {
+    time_algo(&t, CAND_SUMS);
+    e = t.err;
+    st->tune_ms_sums = t.best[CAND_SUMS];
+    const double check = st->value_check ? 0.022 + sums_check_ms(p) : 0.0;
+    if (e != hipSuccess || !((double)st->tune_ms_sums + check < 0.9 * (double)t.best[CAND_BASE])) free_sums(p);
+  }
+  tune_close(&t);
   if (e == hipErrorOutOfMemory) {
     (void)hipGetLastError(); /* optional, like every copy */
     e = hipSuccess;
   }
   st->row_sums = p->sums.tval != NULL;
+  if (st->row_sums && st->tune_mode) st->tune_ms_sums = (float)sums_ms(p, (double)p->sums.sums);
   return e;
 }
 

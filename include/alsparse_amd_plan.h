@@ -70,6 +70,7 @@ typedef struct {
   int32_t row_patterns;  /* 1: STREAM reads a pattern number per row instead of columns (not where a family was set) */
   int32_t row_sums;      /* 1: the multiply runs on row-sum tiles in the place of `algo`, whichever it is (0 where a family
                             was set from outside)                                                                */
+  float tune_ms_sums;    /* timing (ALSPARSE_AMD_TUNE=timed) or estimate of the row-sum tiles, or 0              */
 } asamd_csr_stats;
 
 typedef struct asamd_csr_plan asamd_csr_plan;

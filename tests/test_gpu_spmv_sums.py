@@ -240,3 +240,26 @@ def test_a_family_picked_for_the_analysis_is_the_one_that_runs(gpu, pick, algo, 
             assert p.stats.algo == algo if algo is not None else p.stats.tiled_built + p.stats.ell_built == 0
     finally:
         p.close()
+
+
+@pytest.mark.parametrize("make", [lambda: wl.uniform_rows(1 << 21, 1 << 21, 16, np.float32),
+                                  lambda: wl.powerlaw_rmat(21, 50000, np.float32)], ids=["uniform", "powerlaw"])
+def test_a_timed_analysis_times_them(gpu, make, monkeypatch):
+    """ALSPARSE_AMD_TUNE=timed: no estimate puts a kernel that was not timed in the place of the family that won."""
+    a = make()
+    rng = np.random.default_rng(18)
+    x, y0 = _numbers(rng, a.cols, a.dtype), _numbers(rng, a.rows, a.dtype)
+    q = Plan(a, 1)
+    monkeypatch.setenv("ALSPARSE_AMD_TUNE", "timed")
+    p = Plan(a, 1)
+    try:
+        announce("row sums, timed analysis")
+        assert q.stats.row_sums == 1 and q.stats.tune_ms_sums > 0
+        assert p.stats.tune_mode == 0 and p.stats.tune_ms_sums > 0 and p.stats.tune_ms_sums != q.stats.tune_ms_sums
+        assert 0.5 * p.stats.tune_ms_sums < q.stats.tune_ms_sums < 2 * p.stats.tune_ms_sums
+        _check(a, 1.5, x, 0.5, y0, p.multiply(1.5, x, 0.5, y0), "timed")
+        y = p.multiply(1.5, x, 0.5, y0)
+        assert np.array_equal(y, q.multiply(1.5, x, 0.5, y0)) == (p.stats.row_sums == 1)
+    finally:
+        p.close()
+        q.close()
