@@ -39,6 +39,7 @@ struct asamd_csr_plan {
   int rel16_group;         /* the lanes per row they were made for */
   asamd_pattern_layout pat; /* staged row blocks: a pattern number per row instead of the columns */
   int pinned;              /* the family was set from outside: the staged row blocks then read columns (or distances) */
+  int sums_against;        /* the family that the row-sum tiles were weighed against already, or 0 (AUTO) */
   int of_transpose;        /* the analysis of a copy of A^T or A^H: A's plan checks the values, the caller sets no family */
   int watched;             /* laid out for asamd_csr_plan_csrmv_watched: its fingerprints are the caller's account */
   void *d_eval;            /* ELL copy: ell_width * m values, column-major */
@@ -1234,6 +1235,9 @@ static double model_ms(const asamd_csr_plan *p, int algo) {
   return hypot2(bytes / (rate * 1e9), gather);
 }
 
+static hipError_t build_sums(hipStream_t stream, asamd_csr_plan *p, const int32_t *row_ptr, const int32_t *col_ind,
+                             const void *val, int force);
+
 static hipError_t model_copies(hipStream_t stream, asamd_csr_plan *p, const int32_t *row_ptr, const int32_t *col_ind,
                                const void *val, int tiled_ok, int ell_ok, int hot_ok, int binned_ok) {
   asamd_csr_stats *st = &p->st;
@@ -1312,6 +1316,18 @@ static hipError_t model_copies(hipStream_t stream, asamd_csr_plan *p, const int3
     }
   }
   hipError_t e = hipSuccess;
+  if (p->of_transpose && k > 0) {
+    /* Nothing but AUTO's choice ever runs for A^T: where the tiles beat the family whose copy would be laid out first, that
+     * copy is not laid out at all (2 M x 2 M x 16, fp32: 10.5 -> 7.3 ms for A^T and 0.41 GB less; 1.5 M x 1.5 M x 24, fp64: 12.8
+   * -> 8.7 ms, 0.58 GB). */
+    static const int family[CAND_COUNT] = {0, ASAMD_SPMV_TILED, ASAMD_SPMV_ELL, ASAMD_SPMV_MERGE_HOT, ASAMD_SPMV_BINNED};
+    const int kept = p->auto_algo;
+    p->auto_algo = family[order[0]];
+    e = build_sums(stream, p, row_ptr, col_ind, val, 0);
+    p->sums_against = p->auto_algo;
+    p->auto_algo = kept;
+    if (p->sums.tval) return e;
+  }
   for (int i = 0; i < k && e == hipSuccess; ++i) {
     int built = 0, algo = p->auto_algo;
     switch (order[i]) {
@@ -1358,7 +1374,8 @@ static hipError_t model_copies(hipStream_t stream, asamd_csr_plan *p, const int3
  *   uniform rows, fp32: 1 M x 1 M x 16 93 -> 79, x 32 189 -> 137, x 64 324 -> 170, 2 M x 2 M x 16 173 -> 142;
  *     4 M x 4 M x 16 285 -> 253 (not laid out), 16 M x 16 M x 16 853 -> 910 (next to no row meets a column block twice, and
  *     the tiled pair's are wider: not laid out); fp64: 1 M x 1 M x 16 161 -> 115, 2 M x 2 M x 64 1215 -> 649
- * A matrix that they serve keeps the copy of its family, for a family set from outside and for other value arrays. */
+ * A matrix that they serve keeps the copy of its family, for a family set from outside and for other value arrays; the
+ * copy of A^T, which has neither, does not (drop_family). */
 static double sums_bytes(const asamd_csr_plan *p, double sums) {
   const asamd_csr_stats *st = &p->st;
   const double vs = (double)p->val_size;
@@ -1457,6 +1474,21 @@ static hipError_t build_sums(hipStream_t stream, asamd_csr_plan *p, const int32_
   st->row_sums = p->sums.tval != NULL;
   if (st->row_sums && st->tune_mode) st->tune_ms_sums = (float)sums_ms(p, (double)p->sums.sums);
   return e;
+}
+
+/* In the analysis of A^T the row-sum tiles replace the family for good: no family is set there, no other value array comes.
+ * What is left is the kernel on the copy's own arrays, for a workspace without room. */
+static void drop_family(asamd_csr_plan *p) {
+  free_tiled(p);
+  free_ell(p);
+  free_hot(p);
+  free_binned(p);
+  if (p->xlds.seg) {
+    asamd_xlds_free(&p->xlds);
+    p->st.xlds_slices = 0;
+    if (p->struct_algo == ASAMD_SPMV_XLDS) p->struct_algo = p->plain_algo;
+  }
+  p->auto_algo = p->st.algo = p->struct_algo;
 }
 
 /* the fingerprint of the values a copy set was taken from (set-up work: plan-owned scratch, not concurrent) */
@@ -1651,9 +1683,11 @@ static hipError_t plan_create(hipStream_t stream, int32_t m, int32_t n, int32_t 
       st->xlds_slices = 0;
       if (p->struct_algo == ASAMD_SPMV_XLDS) p->struct_algo = p->plain_algo;
     }
-    if (e == hipSuccess && !only_tiled) e = build_sums(stream, p, row_ptr, col_ind, val, force);
-    if (e == hipSuccess && has_value_copy(p)) {
-      p->copy_val_src = val;
+    if (e == hipSuccess && !only_tiled && !p->sums.tval && (p->sums_against == 0 || p->sums_against != p->auto_algo))
+      e = build_sums(stream, p, row_ptr, col_ind, val, force);
+    if (e == hipSuccess && p->of_transpose && p->sums.tval) drop_family(p);
+    if (e == hipSuccess && has_value_copy(p)) p->copy_val_src = val;
+    if (e == hipSuccess && has_value_copy(p) && !p->of_transpose) {
       e = first_fingerprint(stream, p, val, 0);
       if (e == hipSuccess && p->sums.tval) e = first_fingerprint(stream, p, val, FP_SUMS);
       if (e == hipSuccess) e = hipStreamSynchronize(stream);

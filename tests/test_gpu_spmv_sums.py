@@ -60,10 +60,10 @@ class Plan:
         self.stats = self.lib.asamd_csr_plan_stats(self.plan).contents
         self.ws = capi.Workspace(self.lib, self.plan)
 
-    def multiply(self, alpha, x, beta, y0, val=None, ws=None):
+    def multiply(self, alpha, x, beta, y0, val=None, ws=None, op=0):
         T = capi.scalar_type(self.da.a.dtype)
         dx, dy = hiprt.DeviceArray.from_numpy(x), hiprt.DeviceArray.from_numpy(y0)
-        assert capi.plan_csrmv(self.lib, None, self.plan, 0, T(alpha), (val or self.da.val).c_ptr(), self.da.row_ptr.c_ptr(),
+        assert capi.plan_csrmv(self.lib, None, self.plan, op, T(alpha), (val or self.da.val).c_ptr(), self.da.row_ptr.c_ptr(),
                                self.da.col.c_ptr(), dx.c_ptr(), T(beta), dy.c_ptr(), ws or self.ws) == 0
         hiprt.synchronize()
         y = dy.to_numpy()
@@ -263,3 +263,49 @@ def test_a_timed_analysis_times_them(gpu, make, monkeypatch):
     finally:
         p.close()
         q.close()
+
+
+def _transposed(a, op):
+    t = sp.csr_matrix((a.values if op == 1 else a.values.conj(), a.col_ind, a.row_ptr), shape=(a.rows, a.cols)).T.tocsr()
+    return wl.Csr(a.cols, a.rows, t.indptr.astype(np.int32), t.indices.astype(np.int32), t.data, 0, "op %d" % op)
+
+
+@pytest.mark.parametrize("dtype,op,m,n", [(np.float32, 1, 1 << 21, 1 << 21), (np.float64, 1, 1000003, 786433),
+                                          (np.complex64, 2, 1000003, 786433)], ids=["f32_T", "f64_T", "c64_H"])
+def test_the_copy_of_the_transpose_runs_on_them(gpu, dtype, op, m, n):
+    """The copy of A^T (A^H) with row-sum tiles: its family's own copy is not laid out beside them, values rewritten in place
+    are picked up, and a refresh takes another array."""
+    a = wl.uniform_rows(m, n, 16, np.float64)
+    rng = np.random.default_rng(19)
+    a = wl.Csr(a.rows, a.cols, a.row_ptr, a.col_ind, _numbers(rng, a.nnz, dtype), 0, a.name)
+    x, y0 = _numbers(rng, a.rows, dtype), _numbers(rng, a.cols, dtype)
+    p = Plan(a, 1)
+    try:
+        announce("row sums of the transpose", np.dtype(dtype).name, op)
+        build = p.lib.asamd_csr_plan_build_transpose if op == 1 else p.lib.asamd_csr_plan_build_conj_transpose
+        assert build(None, p.plan, p.da.row_ptr.c_ptr(), p.da.col.c_ptr(), p.da.val.c_ptr()) == 0
+        p.ws = capi.Workspace(p.lib, p.plan)
+        st = p.lib.asamd_csr_plan_transpose_stats(p.plan).contents
+        assert st.row_sums == 1 and p.stats.value_check == 1
+        assert st.tiled_built + st.ell_built + st.hot_built + st.binned_built + st.xlds_slices == 0
+        first = p.multiply(1.5, x, 0.5, y0, op=op)
+        _check(_transposed(a, op), 1.5, x, 0.5, y0, first, "values of the analysis")
+        assert np.array_equal(first, p.multiply(1.5, x, 0.5, y0, op=op))
+        b = wl.Csr(a.rows, a.cols, a.row_ptr, a.col_ind, _numbers(rng, a.nnz, dtype), 0, "other values")
+        p.da.val.copy_from(b.values)
+        t = _transposed(b, op)
+        second = p.multiply(1.5, x, 0.5, y0, op=op)
+        _check(t, 1.5, x, 0.5, y0, second, "in place")
+        small = capi.Workspace(p.lib, p.plan)
+        small.bytes = 1 << 20  # the check of the values and no room for the sums
+        _check(t, 1.5, x, 0.5, y0, p.multiply(1.5, x, 0.5, y0, op=op, ws=small), "no room")
+        d_other = hiprt.DeviceArray.from_numpy(a.values)
+        p.da.val.copy_from(np.zeros_like(a.values))
+        assert p.lib.asamd_csr_plan_refresh_values(None, p.plan, p.da.row_ptr.c_ptr(), p.da.col.c_ptr(), d_other.c_ptr()) == 0
+        assert np.array_equal(first, p.multiply(1.5, x, 0.5, y0, op=op, val=d_other)), "refreshed from another array"
+        _check(a, 1.5, y0, 0.5, x, p.multiply(1.5, y0, 0.5, x, val=d_other), "the product with A, refreshed")
+        d_other.copy_from(b.values)
+        assert np.array_equal(second, p.multiply(1.5, x, 0.5, y0, op=op, val=d_other)), "in place in the array of the refresh"
+        d_other.free()
+    finally:
+        p.close()
