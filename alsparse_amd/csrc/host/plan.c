@@ -47,6 +47,8 @@ struct asamd_csr_plan {
   const void *copy_val_src; /* the value array that the tiled / ELL / row-sum copy was taken from */
   asamd_trans_copy tr[2];  /* CSR copies of the transpose [0] and of the conjugate transpose [1] */
   float trans_lines;       /* distinct lines of y per entry of a run (0: not sampled); steers the transposed scatter only */
+  int trans_route;         /* the transposed multiply without a copy, settled when the plan is made: TRANS_* ... */
+  size_t trans_bytes;      /* ... and its per-call scratch */
   int lazy_transpose;      /* build a copy on the first transposed multiply */
   uint64_t *d_fp;          /* 4 device words: fingerprints of the values that the copies were taken from
                               (tiled / ELL / slices, A^T, A^H, row-sum tiles) */
@@ -64,7 +66,7 @@ static const int kValSize[4] = {4, 8, 8, 16};
 
 static int is_complex(const asamd_csr_plan *p) { return p->dtype >= ASAMD_DTYPE_FLOAT_COMPLEX; }
 
-/* ---- environment switches (read once) ------------------------------------------------------------ */
+/* ---- environment switches (read when a plan is made; ALSPARSE_AMD_XLDS=0 also counts later) ------------------------------------------------------------ */
 static int env_int(const char *name, int fallback) {
   const char *e = getenv(name);
   return e && *e ? atoi(e) : fallback;
@@ -443,22 +445,26 @@ static int holds_values(const asamd_csr_plan *p, int algo) {
   return algo == ASAMD_SPMV_TILED || algo == ASAMD_SPMV_ELL || (algo == ASAMD_SPMV_XLDS && p->xlds.val != NULL);
 }
 
-/* per-call scratch of the transposed multiply that keeps y in LDS, or 0 where it does not serve */
-static size_t trans_ylds_scratch(const asamd_csr_plan *p) {
+/* The transposed multiply without a copy, and its per-call scratch: sums in LDS, with the columns in slices or with all of y
+ * (where it fits and the matrix is large enough for a workgroup per compute unit to pay), or the atomic scatter.  Settled
+ * once: the estimates and the switches behind them cost half a microsecond, which a multiply of a few thousand entries
+ * shows (a pair of products, 3 000 x 9 000 x 10: 12.4 us with them on every call, 11.6 without). */
+enum { TRANS_SCATTER = 0, TRANS_SLICES, TRANS_YLDS };
+
+static void choose_trans_route(asamd_csr_plan *p) {
   const asamd_csr_stats *st = &p->st;
-  if (st->nnz < (1 << 20) || st->first_offset != 0 || env_int("ALSPARSE_AMD_XLDS", 1) <= 0) return 0;
-  return asamd_spmv_trans_ylds_bytes(p->dtype, st->m, st->n);
-}
-/* The transposed multiply without a copy: sums in LDS, the columns in slices or all of y (else the atomic scatter runs), and
- * its per-call scratch. */
-static int trans_slices_ok(const asamd_csr_plan *p) {
-  const asamd_csr_stats *st = &p->st;
-  if (env_int("ALSPARSE_AMD_XLDS", 1) <= 0) return 0;
-  return asamd_spmv_trans_slices_fit(p->dtype, st->m, st->n, st->nnz, st->max_len) ||
-         (trans_ylds_scratch(p) == 0 && asamd_spmv_trans_slices_pay(p->dtype, st->n, st->nnz, p->trans_lines));
-}
-static size_t trans_scratch(const asamd_csr_plan *p) {
-  return align256(trans_slices_ok(p) ? asamd_spmv_trans_slices_bytes(p->dtype, p->st.n, p->st.nnz) : trans_ylds_scratch(p));
+  p->trans_route = TRANS_SCATTER;
+  p->trans_bytes = 0;
+  if (env_int("ALSPARSE_AMD_XLDS", 1) <= 0) return;
+  const size_t ylds = st->nnz >= (1 << 20) && st->first_offset == 0 ? asamd_spmv_trans_ylds_bytes(p->dtype, st->m, st->n) : 0;
+  if (asamd_spmv_trans_slices_fit(p->dtype, st->m, st->n, st->nnz, st->max_len) ||
+      (ylds == 0 && asamd_spmv_trans_slices_pay(p->dtype, st->n, st->nnz, p->trans_lines))) {
+    p->trans_route = TRANS_SLICES;
+    p->trans_bytes = align256(asamd_spmv_trans_slices_bytes(p->dtype, st->n, st->nnz));
+  } else if (ylds) {
+    p->trans_route = TRANS_YLDS;
+    p->trans_bytes = align256(ylds);
+  }
 }
 
 size_t asamd_csr_plan_workspace_bytes(const asamd_csr_plan *p) {
@@ -471,10 +477,8 @@ size_t asamd_csr_plan_workspace_bytes(const asamd_csr_plan *p) {
   }
   if (sums_scratch(p) > need) need = sums_scratch(p);
   if (has_value_copy(p)) need += align256(ASAMD_GUARD_WS_BYTES);
-  {
-    const size_t s = align256(ASAMD_GUARD_WS_BYTES) + trans_scratch(p);
-    if (trans_scratch(p) && s > need) need = s;
-  }
+  if (p->trans_bytes && align256(ASAMD_GUARD_WS_BYTES) + p->trans_bytes > need)
+    need = align256(ASAMD_GUARD_WS_BYTES) + p->trans_bytes;
   for (int w = 0; w < 2; ++w)
     if (p->tr[w].plan) {
       const size_t s = align256(ASAMD_GUARD_WS_BYTES) + asamd_csr_plan_workspace_bytes(p->tr[w].plan);
@@ -828,13 +832,12 @@ int asamd_csr_plan_csrmv(hipStream_t s, asamd_csr_plan *p, int32_t op, const voi
       return csrmv_inner(s, t->plan, &at, ws, 0);
     }
   }
-  const size_t scratch = trans_scratch(p);
-  void *partials = scratch ? ws_take(&ws, scratch) : NULL;
-  if (trans_slices_ok(p)) {
-    if (partials || !scratch) return asamd_spmv_trans_slices(s, &a, which == 1, partials);
-  } else if (partials) {
-    /* y in LDS where it fits and the matrix is large enough for a workgroup per compute unit to pay */
-    return asamd_spmv_trans_ylds(s, &a, p->auto_width, which == 1, partials);
+  if (p->trans_route != TRANS_SCATTER && env_int("ALSPARSE_AMD_XLDS", 1) > 0) {
+    void *partials = p->trans_bytes ? ws_take(&ws, p->trans_bytes) : NULL;
+    if (p->trans_route == TRANS_SLICES && (partials || !p->trans_bytes))
+      return asamd_spmv_trans_slices(s, &a, which == 1, partials);
+    if (p->trans_route == TRANS_YLDS && partials)
+      return asamd_spmv_trans_ylds(s, &a, p->auto_width, which == 1, partials);
   }
   return asamd_spmv_trans_scatter(s, &a, p->auto_width, which == 1);
 }
@@ -1319,7 +1322,7 @@ static hipError_t model_copies(hipStream_t stream, asamd_csr_plan *p, const int3
   if (p->of_transpose && k > 0) {
     /* Nothing but AUTO's choice ever runs for A^T: where the tiles beat the family whose copy would be laid out first, that
      * copy is not laid out at all (2 M x 2 M x 16, fp32: 10.5 -> 7.3 ms for A^T and 0.41 GB less; 1.5 M x 1.5 M x 24, fp64: 12.8
-   * -> 8.7 ms, 0.58 GB). */
+     * -> 8.7 ms, 0.58 GB). */
     static const int family[CAND_COUNT] = {0, ASAMD_SPMV_TILED, ASAMD_SPMV_ELL, ASAMD_SPMV_MERGE_HOT, ASAMD_SPMV_BINNED};
     const int kept = p->auto_algo;
     p->auto_algo = family[order[0]];
@@ -1549,6 +1552,7 @@ static hipError_t plan_create(hipStream_t stream, int32_t m, int32_t n, int32_t 
   const int64_t nb = (total + merge_items - 1) / merge_items;
   st->merge_blocks = (int)nb;
   choose_algo(p);
+  choose_trans_route(p);
 
   if (st->trusted && st->first_offset == 0) {
     /* the structure is promised fixed: the merge-path coordinates are computed once */

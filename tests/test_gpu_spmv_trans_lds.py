@@ -3,6 +3,8 @@ longer than the mean; few columns) at the edges of a chunk of 8 192 entries, of 
 scatter's table in LDS (its slots meet, one or four rows per lane group, more entries than a table).  Against the oracle's
 restatement of the reference's plain transposed kernel; sums are held in double precision, so the tolerance is the one of
 every transposed product here."""
+from ctypes import byref, c_void_p
+
 import numpy as np
 import pytest
 
@@ -74,4 +76,22 @@ def test_transposed_sums_in_lds_complex(gpu, shape, dtype, op):
             metric, ref = oracle_mv(a, op, alpha, x, beta, y0)
             check(metric, alpha, x, beta, y0, y, ref, shape)
     finally:
+        da.free()
+
+
+def test_the_route_is_settled_with_the_plan(gpu, monkeypatch):
+    """A transposed multiply works nothing out anew: the scratch that a plan asks for stays what it was, whatever the
+    switches say later."""
+    a = SHAPES["skewed"][0](np.float32)
+    lib, da, plan = capi.load(), DeviceCsr(a), c_void_p()
+    try:
+        announce("route of the transposed product")
+        assert lib.asamd_csr_plan_create_dtype(None, a.rows, a.cols, a.nnz, da.row_ptr.c_ptr(), da.col.c_ptr(), None, a.base,
+                                               capi.dtype_tag(a.dtype), 0, byref(plan)) == 0
+        needed = lib.asamd_csr_plan_workspace_bytes(plan)
+        assert needed > lib.asamd_spmv_trans_slices_bytes(0, a.cols, a.nnz) > 0
+        monkeypatch.setenv("ALSPARSE_AMD_XLDS", "0")
+        assert lib.asamd_csr_plan_workspace_bytes(plan) == needed
+    finally:
+        lib.asamd_csr_plan_destroy(plan)
         da.free()
