@@ -720,7 +720,7 @@ static void launch_trans_scatter(hipStream_t s, const asamd_spmv_args* a) {
   const T* x = (const T*)a->x;
 #define ASAMD_SCATTER(K, TABLE, GRID)                                                                          \
   csrmv_trans_scatter_kernel<T, W, K, CONJ, TABLE><<<(unsigned)(GRID), kTransThreads, 0, s>>>(                 \
-      a->m, a->n, alpha, val, a->row_ptr, a->col_ind, x, (T*)a->y, a->base)
+      a->m, a->n, alpha, val, a->row_ptr, a->col_ind, x, (T*)a->y, a->base, (unsigned)(GRID))
   if constexpr (W <= 4) {
     // short rows: a workgroup's entries are few.  Small matrices are one launch's latency, to which the table adds half a
     // microsecond; four rows per lane group cost scattered columns 4 % (uniform 400 000 x 5 fp32: 102 and 106 us; the

@@ -6,9 +6,12 @@ through a function pointer has its handle there, a data object, and the optimise
 import glob
 import os
 import re
+import struct
 import subprocess
 
 import pytest
+
+from alsparse_amd import build
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HIP = os.path.join(ROOT, "alsparse_amd", "csrc", "hip")
@@ -30,3 +33,38 @@ def test_sanitized_host_code_launches_the_same_kernels(name):
     sanitized = _launched(os.path.join(HIP, name), "-Xarch_host", "-fsanitize=undefined")
     assert release, "no launch found in %s" % name
     assert sanitized == release, "launches that differ: %s" % sorted(sanitized ^ release)[:4]
+
+
+READELF = os.path.join(os.environ.get("ROCM", "/opt/rocm"), "llvm", "bin", "llvm-readelf")
+
+
+def _kernels(tmp_path):
+    """{symbol: its metadata} of every gfx950 kernel in the built library, one code object per HIP file."""
+    data = open(build.LIB_PATH, "rb").read()
+    magic, found = b"__CLANG_OFFLOAD_BUNDLE__", {}
+    for at in (m.start() for m in re.finditer(magic, data)):
+        count, = struct.unpack_from("<Q", data, at + len(magic))
+        p = at + len(magic) + 8
+        for _ in range(count):
+            offset, size, length = struct.unpack_from("<QQQ", data, p)
+            triple = data[p + 24:p + 24 + length]
+            p += 24 + length
+            if b"gfx950" not in triple or size == 0:
+                continue
+            obj = tmp_path / "object"
+            obj.write_bytes(data[at + offset:at + offset + size])
+            notes = subprocess.run([READELF, "--notes", str(obj)], stdout=subprocess.PIPE, text=True, timeout=120).stdout
+            for block in re.split(r"\n  - (?=\.)", notes[notes.index("amdhsa.kernels:"):])[1:]:
+                found[re.search(r"\.symbol:\s+'?(\S+?)\.kd", block).group(1)] = block
+    return found
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
+def test_the_transposed_products_of_small_matrices_take_no_hidden_arguments(tmp_path):
+    """A kernel that asks for its grid brings 256 bytes of hidden arguments, which the host writes on every launch; a pair of
+    products of a few thousand entries is its launches."""
+    kernels = {n: b for n, b in _kernels(tmp_path).items()
+               if re.search(r"csrmv_trans_(scatter|slices)_kernel|trans_partials_sum_kernel|scale_vec_kernel", n)}
+    assert sum("trans_scatter" in n for n in kernels) >= 40 and sum("trans_slices" in n for n in kernels) == 6
+    asking = [n for n, block in kernels.items() if "hidden_" in block]
+    assert not asking, asking[:4]
