@@ -754,8 +754,13 @@ static void fill_args(asamd_spmv_args *a, const asamd_csr_plan *p, const void *a
 /* Small transposed products read the caller's values through the copy's permutation: one launch (two where a few rows of
  * A^T are long) where the check of the copy's values is four of their own, and nothing to check.  us per call, this / the
  * checked copy: 30 000 to 120 000 entries 4.6 / 18, 500 000 scattered ones 14-16 / 18-19, 1 000 000 27-30 / 19-25 (every
- * value then moves a cache line of its own), a power law of 60 000 rows 15 / 28. */
+ * value then moves a cache line of its own), a power law of 60 000 rows 15 / 28.  With ALSPARSE_AMD_VALUE_CHECK=off the copy
+ * costs its multiply alone and is the faster one from 200 000 entries on (uniform 20 000 x 20 000 x 10 5.4 / 4.5, 40 000 x
+ * 40 000 x 12 11.7 / 4.6, power law 12.6 / 9.4; level below): only another value array, which it does not hold, comes here. */
 #define PERMUTED_MOST (1 << 19)
+static int permuted_serves(const asamd_csr_plan *p, const void *val, const void *copy_of) {
+  return p->st.nnz <= PERMUTED_MOST && (p->st.value_check || val != copy_of);
+}
 
 /* Any value array with the structure of the plan; -1: no room for the scratch. */
 static int csrmv_permuted(hipStream_t s, asamd_trans_copy *t, const void *alpha, const void *val, const void *x,
@@ -807,7 +812,7 @@ int asamd_csr_plan_csrmv(hipStream_t s, asamd_csr_plan *p, int32_t op, const voi
       }
     }
   }
-  if (t->plan && st->nnz <= PERMUTED_MOST) {
+  if (t->plan && permuted_serves(p, val, t->val_src)) {
     const int e = csrmv_permuted(s, t, alpha, val, x, beta, y, ws, which == 1);
     if (e != -1) return e;
   }
@@ -1771,9 +1776,11 @@ static hipError_t build_transpose(hipStream_t stream, asamd_csr_plan *p, const i
   asamd_trans_copy *t = &p->tr[which];
   hipError_t e = (hipError_t)asamd_transpose_build(stream, p->dtype, which == 1, st->m, st->n, st->nnz, st->base, rp, ci,
                                                    val, &t->t);
+  /* (where every product goes through the permutation nothing beside t.val, which a workspace without room falls back to, is
+   * laid out from the values) */
   if (e == hipSuccess)
-    e = plan_create(stream, st->n, st->m, st->nnz, t->t.row_ptr, t->t.col_ind, t->t.val, 0, p->dtype, /*trusted=*/1,
-                    /*of_transpose=*/1, &t->plan);
+    e = plan_create(stream, st->n, st->m, st->nnz, t->t.row_ptr, t->t.col_ind, permuted_serves(p, val, val) ? NULL : t->t.val,
+                    0, p->dtype, /*trusted=*/1, /*of_transpose=*/1, &t->plan);
   if (e == hipSuccess) e = first_fingerprint(stream, p, val, 1 + which);
   if (e == hipSuccess) e = hipStreamSynchronize(stream);
   if (e != hipSuccess) {

@@ -1,7 +1,7 @@
 """Small analysed transposed products read the caller's values through the copy's permutation: by lane groups (one to eight
 trips of four entries per lane, wider groups for longer rows) or, where a row of A^T would keep a wave longer, by the merge
 path.  Any values with the analysed structure give their own product, without a second analysis; results are reproducible."""
-from ctypes import byref
+from ctypes import byref, c_void_p
 
 import numpy as np
 import pytest
@@ -84,4 +84,51 @@ def test_small_analysed_transposed_products(gpu, shape, dtype, op):
         product(b, 2.0, 3.0, "in place")
     finally:
         lib.alphasparse_dcu_destroy_mat_info(info)
+        da.free()
+
+
+@pytest.mark.parametrize("make", [lambda: wl.uniform_rows(20000, 20000, 10, np.float32), lambda: wl.uniform_rows(20000, 20000, 17, np.float64)],
+                         ids=["f32", "f64"])
+def test_without_a_check_the_copy_multiplies(gpu, make, monkeypatch):
+    """ALSPARSE_AMD_VALUE_CHECK=off: nothing stands in front of the copy of A^T, whose multiply alone is the faster one.  The
+    product has the bits of a multiply with the copy's own arrays; another value array still gives its own product."""
+    monkeypatch.setenv("ALSPARSE_AMD_VALUE_CHECK", "off")
+    a = make()
+    x, y0 = wl.uniform(a.rows, a.dtype, 3), wl.uniform(a.cols, a.dtype, 4)
+    lib, da, T = capi.load(), DeviceCsr(a), capi.scalar_type(a.dtype)
+    plan, direct = c_void_p(), c_void_p()
+    code = capi.dtype_tag(a.dtype)
+
+    def product(p, op, arrays):
+        ws = capi.Workspace(lib, p)
+        dx, dy = hiprt.DeviceArray.from_numpy(x), hiprt.DeviceArray.from_numpy(y0)
+        assert capi.plan_csrmv(lib, None, p, op, T(1.5), *arrays, dx.c_ptr(), T(0.5), dy.c_ptr(), ws) == 0
+        hiprt.synchronize()
+        y = dy.to_numpy()
+        dx.free()
+        dy.free()
+        return y
+
+    try:
+        announce("transposed, values not checked", a.name)
+        own = (da.val.c_ptr(), da.row_ptr.c_ptr(), da.col.c_ptr())
+        assert lib.asamd_csr_plan_create_dtype(None, a.rows, a.cols, a.nnz, own[1], own[2], own[0], 0, code, 1, byref(plan)) == 0
+        assert lib.asamd_csr_plan_build_transpose(None, plan, own[1], own[2], own[0]) == 0
+        row, col, val = c_void_p(), c_void_p(), c_void_p()
+        assert lib.asamd_csr_plan_transpose_arrays(plan, 0, byref(row), byref(col), byref(val)) == 0
+        assert lib.asamd_csr_plan_create_dtype(None, a.cols, a.rows, a.nnz, row, col, val, 0, code, 1, byref(direct)) == 0
+        y = product(plan, 1, own)
+        check_trans(a, 1.5, x, 0.5, y0, y, "not checked")
+        assert np.array_equal(y, product(direct, 0, (val, row, col)))
+        b = wl.Csr(a.rows, a.cols, a.row_ptr, a.col_ind, (a.values * a.dtype.type(-2.0)).astype(a.dtype), 0, "other")
+        other = hiprt.DeviceArray.from_numpy(b.values)
+        check_trans(b, 1.5, x, 0.5, y0, product(plan, 1, (other.c_ptr(),) + own[1:]), "another array")
+        da.val.copy_from(b.values)
+        assert lib.asamd_csr_plan_refresh_values(None, plan, own[1], own[2], own[0]) == 0
+        check_trans(b, 1.5, x, 0.5, y0, product(plan, 1, own), "refreshed")
+        other.free()
+    finally:
+        if direct:
+            lib.asamd_csr_plan_destroy(direct)
+        lib.asamd_csr_plan_destroy(plan)
         da.free()
