@@ -349,6 +349,7 @@ _COMMON = {
     "asamd_spmv_trans_slices_pay": [_I, _I, _I, c_float],
     "asamd_spmv_trans_slices_bytes": [_I, _I, _I],
     "asamd_spmv_trans_slices": [_P, POINTER(asamd_spmv_args), _I, _P],
+    "asamd_spmv_trans_slices_gaps": [_P, POINTER(asamd_spmv_args), _I, _P],
     "asamd_tiled_fits": [_I, _I, _I, _I],
     "asamd_tiled_build": [_P, _I, _I, _I, _I, _I, _P, _P, _P, _I, _I, _P],
     "asamd_tiled_free": [_P],

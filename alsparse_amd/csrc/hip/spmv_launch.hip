@@ -680,16 +680,16 @@ extern "C" size_t asamd_spmv_trans_slices_bytes(int32_t dtype, int32_t n, int32_
   return shape.parts > 1 ? (size_t)shape.parts * (size_t)n * (size_t)dtype_size(dtype) : 0;
 }
 
-template <typename T, bool CONJ>
+template <typename T, bool CONJ, bool GAPS>
 static int launch_trans_slices(hipStream_t s, const asamd_spmv_args* a, void* partials) {
   const SliceShape shape = trans_slices_shape(a->dtype, a->n, a->nnz);
   if (shape.parts > 1 && !partials) return hipErrorInvalidValue;
   T* out = shape.parts > 1 ? (T*)partials : nullptr;
   static std::atomic<uint64_t> allowed{0};
-  if (const hipError_t e = allow_full_lds((const void*)csrmv_trans_slices_kernel<T, CONJ>, allowed); e != hipSuccess) return e;
+  if (const hipError_t e = allow_full_lds((const void*)csrmv_trans_slices_kernel<T, CONJ, GAPS>, allowed); e != hipSuccess) return e;
   const size_t lds = kSliceLdsFixed + (size_t)shape.slice_cols * sizeof(LdsSum<T>);
   const T beta = scalar_of<T>(a->beta);
-  csrmv_trans_slices_kernel<T, CONJ><<<(unsigned)(shape.parts * shape.slices), kSliceThreads, lds, s>>>(
+  csrmv_trans_slices_kernel<T, CONJ, GAPS><<<(unsigned)(shape.parts * shape.slices), kSliceThreads, lds, s>>>(
       a->m, a->n, shape.parts, shape.slice_cols, scalar_of<T>(a->alpha), (const T*)a->val, a->row_ptr, a->col_ind,
       (const T*)a->x, beta, (T*)a->y, out, a->base);
   if (out)
@@ -698,16 +698,23 @@ static int launch_trans_slices(hipStream_t s, const asamd_spmv_args* a, void* pa
   return hipGetLastError();
 }
 // partials: asamd_spmv_trans_slices_bytes(dtype, n, nnz) bytes of per-call scratch
-extern "C" int asamd_spmv_trans_slices(hipStream_t s, const asamd_spmv_args* a, int32_t conj, void* partials) {
+template <bool GAPS>
+static int trans_slices(hipStream_t s, const asamd_spmv_args* a, int32_t conj, void* partials) {
   if (!a || a->n < 1 || a->nnz < 1 || trans_slices_least(a->dtype, a->n) > kSlicesMost) return hipErrorInvalidValue;
   return by_dtype(a->dtype, [&](auto* tag) -> int {
     using T = std::remove_pointer_t<decltype(tag)>;
     if (!args_ok<T>(a) || (conj && kIsReal<T>) || (uintptr_t)partials % alignof(T)) return hipErrorInvalidValue;
     if constexpr (!kIsReal<T>) {
-      if (conj) return launch_trans_slices<T, true>(s, a, partials);
+      if (conj) return launch_trans_slices<T, true, GAPS>(s, a, partials);
     }
-    return launch_trans_slices<T, false>(s, a, partials);
+    return launch_trans_slices<T, false, GAPS>(s, a, partials);
   });
+}
+extern "C" int asamd_spmv_trans_slices(hipStream_t s, const asamd_spmv_args* a, int32_t conj, void* partials) {
+  return trans_slices<false>(s, a, conj, partials);
+}
+extern "C" int asamd_spmv_trans_slices_gaps(hipStream_t s, const asamd_spmv_args* a, int32_t conj, void* partials) {
+  return trans_slices<true>(s, a, conj, partials);
 }
 
 // ---- transposed product as an atomic scatter ------------------------------------------------------

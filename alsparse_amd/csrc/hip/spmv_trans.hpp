@@ -144,11 +144,16 @@ __global__ __launch_bounds__(kTransThreads) void csrmv_trans_scatter_kernel(
 // parts in order.  Entries are read once per slice: a part's slices run on one XCD (parts a multiple of eight) and meet
 // in its L2.
 //
-// Rows that start in a chunk mark their place, a running maximum names every entry's row.
+// Rows that start in a chunk mark their place, a running maximum names every entry's row.  That walk takes 0.86 us for
+// 1 024 rows, and all rows of a run of empty ones fall to one part.  With GAPS a chunk over which more than kSliceWalk rows
+// start is not walked to its end: its entries look their rows up, a thread its first one's among all, the others' between
+// that and the next thread's.  us, scatter / without / with: 4 M rows, all 400 000 entries in the last 100 000 of them
+// 77 / 3 310 / 27; 1 M rows, the second half of two entries each 79 / 431 / 34; no such runs: 19 / 18.7 / 19.1.
 constexpr int kSliceThreads = 1024;
 constexpr int kSlicePer = 8;  // entries per thread and chunk
 constexpr int kSliceChunk = kSliceThreads * kSlicePer;
 constexpr int kSliceWaves = kSliceThreads / kWave;
+constexpr int kSliceWalk = 8 * kSliceThreads;
 constexpr int kSliceLdsFixed = (kSliceChunk + 2 * kSliceWaves) * (int)sizeof(int);
 // largest r in [0, m) with row_ptr[r] - base <= k (0 if there is none): a whole wave, 64 probes at a time
 static __device__ __forceinline__ int row_of_entry(int m, const int* __restrict__ row_ptr, int base, int64_t k) {
@@ -164,7 +169,7 @@ static __device__ __forceinline__ int row_of_entry(int m, const int* __restrict_
   return (int)lo;
 }
 
-template <typename T, bool CONJ>
+template <typename T, bool CONJ, bool GAPS>
 __global__ __launch_bounds__(kSliceThreads) void csrmv_trans_slices_kernel(
     int m, int n, int parts, int slice_cols, T alpha, const T* __restrict__ val, const int* __restrict__ row_ptr,
     const int* __restrict__ col_ind, const T* __restrict__ x, T beta, T* __restrict__ y, T* __restrict__ partials, int base) {
@@ -172,6 +177,7 @@ __global__ __launch_bounds__(kSliceThreads) void csrmv_trans_slices_kernel(
   int* __restrict__ s_row = reinterpret_cast<int*>(slice_bytes);
   int* __restrict__ s_part = s_row + kSliceChunk;  // a wave's largest mark
   int* __restrict__ s_first = s_part + kSliceWaves;
+  int* __restrict__ s_more = s_first + 1;  // more rows start over the chunk than were walked
   using S = LdsSum<T>;
   S* __restrict__ s_sum = reinterpret_cast<S*>(slice_bytes + kSliceLdsFixed);
 
@@ -201,35 +207,69 @@ __global__ __launch_bounds__(kSliceThreads) void csrmv_trans_slices_kernel(
 #pragma unroll
     for (int q = 0; q < kSlicePer / 4; ++q) mine[q] = Int4{0, 0, 0, 0};
     __syncthreads();
-    for (int64_t i = 1 + tid; r0 + i < m; i += kSliceThreads) {  // ascending offsets: past the chunk, all later ones are too
+    int64_t i = 1 + tid;
+    for (; (!GAPS || i <= kSliceWalk) && r0 + i < m; i += kSliceThreads) {  // ascending offsets: past the chunk, all later ones are too
       const int64_t pos = (int64_t)row_ptr[r0 + i] - base - k0;
       if (pos >= len) break;
       atomicMax(&s_row[pos > 0 ? pos : 0], (int)i);
     }
-    __syncthreads();
-    int mk[kSlicePer];
-#pragma unroll
-    for (int q = 0; q < kSlicePer / 4; ++q) {
-      const Int4 w = mine[q];
-      mk[4 * q] = w.x, mk[4 * q + 1] = w.y, mk[4 * q + 2] = w.z, mk[4 * q + 3] = w.w;
-    }
-#pragma unroll
-    for (int q = 1; q < kSlicePer; ++q) mk[q] = max(mk[q], mk[q - 1]);
-    const int incl = wave_max_scan(mk[kSlicePer - 1]);
-    int lead = __builtin_amdgcn_update_dpp(0, incl, 0x138, 0xF, 0xF, true);  // wave_shr:1, lane 0 gets 0
-    if (tid % kWave == kWave - 1) s_part[wave] = incl;
+    if (GAPS && tid == kSliceThreads - 1) *s_more = i > kSliceWalk;  // the thread that walks row r0 + kSliceWalk
     __syncthreads();
     int last = 0;
+    if (GAPS && *s_more) {
+      // (the row of the chunk's last entry; at least row r0 + kSliceWalk, where row_ptr ascends)
+      const int64_t to = row_of_entry(m, row_ptr, base, k0 + len - 1) - r0;
+      const int most = to > 1 ? (int)to : 1;
+      auto starts_by = [&](int r, int k) __attribute__((always_inline)) {  // row r0 + r starts at or before entry k0 + k
+        return (int64_t)row_ptr[r0 + r] - base - k0 <= k;
+      };
+      const int k1 = tid * kSlicePer;
+      int lo = 0;  // the row of the thread's first entry
+      for (int step = 1 << (31 - __builtin_clz(most)); step > 0; step >>= 1) {
+        const int r = most - lo >= step ? lo + step : 0;
+        if (r > 0 && starts_by(r, k1 < len ? k1 : len - 1)) lo = r;
+      }
+      s_row[k1] = lo;
+      __syncthreads();
+      const int hi = tid + 1 < kSliceThreads ? s_row[k1 + kSlicePer] : most;  // the others' lie up to the next thread's
+      int at[kSlicePer];
 #pragma unroll
-    for (int w = 0; w < kSliceWaves; ++w) {
-      const int pw = s_part[w];
-      if (w < wave) lead = max(lead, pw);
-      last = max(last, pw);
+      for (int q = 0; q < kSlicePer; ++q) at[q] = lo;
+      for (int step = hi > lo ? 1 << (31 - __builtin_clz(hi - lo)) : 0; step > 0; step >>= 1) {
+#pragma unroll
+        for (int q = 1; q < kSlicePer; ++q) {
+          const int r = hi - at[q] >= step ? at[q] + step : lo;
+          if (r > at[q] && starts_by(r, k1 + q < len ? k1 + q : len - 1)) at[q] = r;
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < kSlicePer / 4; ++q) mine[q] = Int4{at[4 * q], at[4 * q + 1], at[4 * q + 2], at[4 * q + 3]};
+      __syncthreads();
+      last = s_row[len - 1];
+    } else {
+      int mk[kSlicePer];
+#pragma unroll
+      for (int q = 0; q < kSlicePer / 4; ++q) {
+        const Int4 w = mine[q];
+        mk[4 * q] = w.x, mk[4 * q + 1] = w.y, mk[4 * q + 2] = w.z, mk[4 * q + 3] = w.w;
+      }
+#pragma unroll
+      for (int q = 1; q < kSlicePer; ++q) mk[q] = max(mk[q], mk[q - 1]);
+      const int incl = wave_max_scan(mk[kSlicePer - 1]);
+      int lead = __builtin_amdgcn_update_dpp(0, incl, 0x138, 0xF, 0xF, true);  // wave_shr:1, lane 0 gets 0
+      if (tid % kWave == kWave - 1) s_part[wave] = incl;
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < kSliceWaves; ++w) {
+        const int pw = s_part[w];
+        if (w < wave) lead = max(lead, pw);
+        last = max(last, pw);
+      }
+#pragma unroll
+      for (int q = 0; q < kSlicePer / 4; ++q)
+        mine[q] = Int4{max(lead, mk[4 * q]), max(lead, mk[4 * q + 1]), max(lead, mk[4 * q + 2]), max(lead, mk[4 * q + 3])};
+      __syncthreads();
     }
-#pragma unroll
-    for (int q = 0; q < kSlicePer / 4; ++q)
-      mine[q] = Int4{max(lead, mk[4 * q]), max(lead, mk[4 * q + 1]), max(lead, mk[4 * q + 2]), max(lead, mk[4 * q + 3])};
-    __syncthreads();
     T v[kSlicePer], t[kSlicePer];
     bool in[kSlicePer];
 #pragma unroll

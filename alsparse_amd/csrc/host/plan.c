@@ -449,7 +449,7 @@ static int holds_values(const asamd_csr_plan *p, int algo) {
  * (where it fits and the matrix is large enough for a workgroup per compute unit to pay), or the atomic scatter.  Settled
  * once: the estimates and the switches behind them cost half a microsecond, which a multiply of a few thousand entries
  * shows (a pair of products, 3 000 x 9 000 x 10: 12.4 us with them on every call, 11.6 without). */
-enum { TRANS_SCATTER = 0, TRANS_SLICES, TRANS_YLDS };
+enum { TRANS_SCATTER = 0, TRANS_SLICES, TRANS_SLICES_GAPS, TRANS_YLDS };
 
 static void choose_trans_route(asamd_csr_plan *p) {
   const asamd_csr_stats *st = &p->st;
@@ -459,7 +459,8 @@ static void choose_trans_route(asamd_csr_plan *p) {
   const size_t ylds = st->nnz >= (1 << 20) && st->first_offset == 0 ? asamd_spmv_trans_ylds_bytes(p->dtype, st->m, st->n) : 0;
   if (asamd_spmv_trans_slices_fit(p->dtype, st->m, st->n, st->nnz, st->max_len) ||
       (ylds == 0 && asamd_spmv_trans_slices_pay(p->dtype, st->n, st->nnz, p->trans_lines))) {
-    p->trans_route = TRANS_SLICES;
+    /* (as many empty rows, if they lie side by side, as take one part's workgroups 7 us to pass) */
+    p->trans_route = st->hist[0] >= 8192 ? TRANS_SLICES_GAPS : TRANS_SLICES;
     p->trans_bytes = align256(asamd_spmv_trans_slices_bytes(p->dtype, st->n, st->nnz));
   } else if (ylds) {
     p->trans_route = TRANS_YLDS;
@@ -841,6 +842,8 @@ int asamd_csr_plan_csrmv(hipStream_t s, asamd_csr_plan *p, int32_t op, const voi
     void *partials = p->trans_bytes ? ws_take(&ws, p->trans_bytes) : NULL;
     if (p->trans_route == TRANS_SLICES && (partials || !p->trans_bytes))
       return asamd_spmv_trans_slices(s, &a, which == 1, partials);
+    if (p->trans_route == TRANS_SLICES_GAPS && (partials || !p->trans_bytes))
+      return asamd_spmv_trans_slices_gaps(s, &a, which == 1, partials);
     if (p->trans_route == TRANS_YLDS && partials)
       return asamd_spmv_trans_ylds(s, &a, p->auto_width, which == 1, partials);
   }

@@ -215,6 +215,8 @@ int asamd_spmv_trans_slices_fit(int32_t dtype, int32_t m, int32_t n, int32_t nnz
 int asamd_spmv_trans_slices_pay(int32_t dtype, int32_t n, int32_t nnz, float lines);
 size_t asamd_spmv_trans_slices_bytes(int32_t dtype, int32_t n, int32_t nnz);
 int asamd_spmv_trans_slices(hipStream_t stream, const asamd_spmv_args *a, int32_t conj, void *partials);
+/* ... for a matrix that may have long runs of empty rows */
+int asamd_spmv_trans_slices_gaps(hipStream_t stream, const asamd_spmv_args *a, int32_t conj, void *partials);
 
 /* ---- re-ordered copies of a CSR matrix ("layouts") and the kernels that multiply with them ------
  * A layout is a plain record of device pointers and counts, filled by its *_build call (which

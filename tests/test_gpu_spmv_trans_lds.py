@@ -3,12 +3,14 @@ longer than the mean; few columns) at the edges of a chunk of 8 192 entries, of 
 scatter's table in LDS (its slots meet, one or four rows per lane group, more entries than a table).  Against the oracle's
 restatement of the reference's plain transposed kernel; sums are held in double precision, so the tolerance is the one of
 every transposed product here."""
+import ctypes
+import time
 from ctypes import byref, c_void_p
 
 import numpy as np
 import pytest
 
-from alsparse_amd import capi, workloads as wl
+from alsparse_amd import capi, hiprt, workloads as wl
 from helpers import DeviceCsr, announce
 from helpers_shapes import csr_from_lengths
 from test_gpu_complex import H_, T_, check, complexify, oracle_mv, real_dtype, run_csrmv
@@ -95,3 +97,81 @@ def test_the_route_is_settled_with_the_plan(gpu, monkeypatch):
     finally:
         lib.asamd_csr_plan_destroy(plan)
         da.free()
+
+
+def rows_between_empty_ones(m, rows, lengths, cols, dt, base=0):
+    """A matrix of m rows, all empty but the given ones."""
+    per_row = np.zeros(m, np.int64)
+    per_row[np.asarray(rows)] = lengths
+    return csr_from_lengths(per_row.tolist(), cols, dt, base=base)
+
+
+#: the rows that start over a chunk end at the walk's last row, one past it, far past it
+EMPTY_ROWS = {
+    "walked_to_the_end": lambda dt: rows_between_empty_ones(8193, [0, 8192], [200, 300], 400, dt),
+    "one_more": lambda dt: rows_between_empty_ones(8194, [0, 8193], [200, 300], 400, dt),
+    "last_walked_row_ends_the_chunk": lambda dt: rows_between_empty_ones(40000, [0, 8192, 8193, 39999], [8191, 1, 9000, 3], 9001, dt),
+    "empty_in_front": lambda dt: rows_between_empty_ones(300000, np.arange(290000, 300000), 4, 130, dt, base=1),
+    "empty_behind": lambda dt: rows_between_empty_ones(300000, np.arange(10000), 4, 130, dt),
+    "every_fortieth": lambda dt: rows_between_empty_ones(400000, np.arange(0, 400000, 40), 3, 300, dt),
+    "runs": lambda dt: rows_between_empty_ones(200001, np.arange(200001)[(np.arange(200001) // 20000) % 2 == 1], 2, 3000, dt),
+}
+
+
+@pytest.mark.parametrize("entry", ["asamd_spmv_trans_slices", "asamd_spmv_trans_slices_gaps"], ids=["walked", "gaps"])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("shape", sorted(EMPTY_ROWS))
+def test_slices_over_long_runs_of_empty_rows(gpu, shape, dtype, entry):
+    """Chunks over which more rows start than are walked look their entries' rows up."""
+    a = EMPTY_ROWS[shape](dtype)
+    code = capi.dtype_tag(a.dtype)
+    x, y0 = wl.uniform(a.rows, dtype, 3), wl.uniform(a.cols, dtype, 4)
+    da, lib, T = DeviceCsr(a), capi.load(), capi.scalar_type(dtype)
+    dx, args = hiprt.DeviceArray.from_numpy(x), capi.asamd_spmv_args()
+    part = hiprt.DeviceArray((max(1, lib.asamd_spmv_trans_slices_bytes(code, a.cols, a.nnz)),), np.uint8)
+    try:
+        for alpha, beta in ((1.0, 0.0), (2.0, 3.0)):
+            announce("csrmv trans, empty rows", shape, np.dtype(dtype).name, alpha, beta)
+            dy, al, be = hiprt.DeviceArray.from_numpy(y0), T(alpha), T(beta)
+            args.dtype, args.m, args.n, args.nnz, args.base = code, a.rows, a.cols, a.nnz, a.base
+            args.alpha, args.beta = ctypes.addressof(al), ctypes.addressof(be)
+            args.val, args.row_ptr, args.col_ind, args.x, args.y = (v.ptr for v in (da.val, da.row_ptr, da.col, dx, dy))
+            assert getattr(lib, entry)(None, byref(args), 0, part.c_ptr()) == 0
+            hiprt.synchronize()
+            check_trans(a, alpha, x, beta, y0, dy.to_numpy(), shape)
+            dy.free()
+    finally:
+        part.free()
+        dx.free()
+        da.free()
+
+
+def test_empty_rows_side_by_side_cost_no_more_than_the_scatter(gpu, monkeypatch):
+    """4 M rows, all 400 000 entries in the last 100 000 of them and one long row, whose length makes the slices the choice:
+    one part's workgroups met all the empty rows, and walked over them (40 times the scatter's time)."""
+    a = rows_between_empty_ones(4000001, np.arange(3900001, 4000001), [4] * 99999 + [300], 15000, np.float32)
+    assert capi.load().asamd_spmv_trans_slices_fit(0, a.rows, a.cols, a.nnz, 300) == 1
+    x, y0 = wl.uniform(a.rows, a.dtype, 3), wl.uniform(a.cols, a.dtype, 4)
+    best = []
+    for switch in ("1", "0"):
+        monkeypatch.setenv("ALSPARSE_AMD_XLDS", switch)  # 0: the scatter
+        da = DeviceCsr(a)
+        dx, dy = hiprt.DeviceArray.from_numpy(x), hiprt.DeviceArray.from_numpy(y0)
+        al, be, descr = ctypes.c_float(1.0), ctypes.c_float(0.0), capi.make_descr()
+        announce("empty rows side by side", switch)
+        took = []
+        for _ in range(6):
+            hiprt.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(10):
+                assert capi.load().alphasparse_dcu_s_csrmv(gpu.h, T_, a.rows, a.cols, a.nnz, byref(al), byref(descr), da.val.c_ptr(),
+                                                           da.row_ptr.c_ptr(), da.col.c_ptr(), None, dx.c_ptr(), byref(be),
+                                                           dy.c_ptr()) == 0
+            hiprt.synchronize()
+            took.append(time.perf_counter() - t0)
+        check_trans(a, 1.0, x, 0.0, y0, dy.to_numpy(), "switch " + switch)
+        best.append(min(took[1:]))
+        for d in (dx, dy):
+            d.free()
+        da.free()
+    assert best[0] <= 2.0 * best[1], best
