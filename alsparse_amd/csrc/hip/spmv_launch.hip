@@ -644,14 +644,24 @@ static SliceShape trans_slices_shape(int32_t dtype, int32_t n, int32_t nnz) {
 // columns 349 / 393, its fp64 form of 1 M columns 690 / 2 230), and neighbouring rows with the same columns meet in the
 // scatter's own table (27-point stencil on 60^3 points 28 / 209).
 constexpr int64_t kSlicesMost = 64;
+// What a part's workgroups take to pass the rows beyond one for two entries (those are in the figures above): 0.86 us for
+// 1 024 of them.  1 M entries in 20 M rows, scatter / slices, us: 15 000 columns 147 / 91, 750 000 (six parts) 149 / 2 900.
+extern "C" double asamd_spmv_trans_slices_rows_us(int32_t dtype, int32_t m, int32_t n, int32_t nnz) {
+  if (n < 1 || nnz < 1 || dtype_size(dtype) == 0) return 0.0;
+  const double beyond = (double)m - 0.5 * (double)nnz;
+  return beyond > 0.0 ? 0.86 / 1024.0 * beyond / trans_slices_shape(dtype, n, nnz).parts : 0.0;
+}
 extern "C" int asamd_spmv_trans_slices_fit(int32_t dtype, int32_t m, int32_t n, int32_t nnz, int32_t max_len) {
   if (m < 1 || n < 1 || nnz < 1 || dtype_size(dtype) == 0) return 0;
   if (nnz <= kSliceChunk && m <= kSliceChunk) return trans_slices_least(dtype, n) <= 8;
-  const double ratio = (double)max_len * (double)m / (double)nnz;  // longest row over the mean
+  // trips of the longest row's lane group in the scatter: as many lanes as the mean row has entries, two at least
+  const double mean = (double)nnz / (double)m;
+  const double trips = (double)max_len / (mean > 2.0 ? mean : 2.0);
   const int64_t least = trans_slices_least(dtype, n);
-  // picoseconds: 2.9 per entry and slice; an atomic 50, and a trip of the longest row's lane group 0.7 us
-  if (max_len >= 128 && ratio >= 16.0)
-    return least <= kSlicesMost && 2.9 * (double)nnz * (double)least <= 50.0 * (double)nnz + 0.7e6 * ratio;
+  // picoseconds: 2.9 per entry and slice; an atomic 50, and a trip 0.7 us
+  if (max_len >= 128 && trips >= 16.0)
+    return least <= kSlicesMost && 2.9 * (double)nnz * (double)least + 1e6 * asamd_spmv_trans_slices_rows_us(dtype, m, n, nnz) <=
+                                       50.0 * (double)nnz + 0.7e6 * trips;
   return least == 1 && (int64_t)nnz >= (int64_t)64 * n;
 }
 // Scattered columns, whose atomics leave the scatter's workgroups one by one.  A run of entries meets at least half the lines

@@ -145,15 +145,17 @@ __global__ __launch_bounds__(kTransThreads) void csrmv_trans_scatter_kernel(
 // in its L2.
 //
 // Rows that start in a chunk mark their place, a running maximum names every entry's row.  That walk takes 0.86 us for
-// 1 024 rows, and all rows of a run of empty ones fall to one part.  With GAPS a chunk over which more than kSliceWalk rows
-// start is not walked to its end: its entries look their rows up, a thread its first one's among all, the others' between
-// that and the next thread's.  us, scatter / without / with: 4 M rows, all 400 000 entries in the last 100 000 of them
-// 77 / 3 310 / 27; 1 M rows, the second half of two entries each 79 / 431 / 34; no such runs: 19 / 18.7 / 19.1.
+// 1 024 rows, and all rows of a run of empty ones fall to one part.  With GAPS the rows of a chunk are counted after
+// kSliceWalk of them; more than kSliceLook are not walked (the walk to there takes what follows): the chunk's entries look
+// their rows up, a thread its first one's among all, the others' between that and the next thread's.  us, scatter / without /
+// with: 4 M rows, all 400 000 entries in the last 100 000 of them 78 / 3 300 / 37; 1 M rows, the second half of two entries
+// each, 79 / 431 / 44; 20 M rows, every fortieth of two, 147 / 84 / 103; 200 000 rows, every second of eight, 62 / 18.5 / 19.3.
 constexpr int kSliceThreads = 1024;
 constexpr int kSlicePer = 8;  // entries per thread and chunk
 constexpr int kSliceChunk = kSliceThreads * kSlicePer;
 constexpr int kSliceWaves = kSliceThreads / kWave;
-constexpr int kSliceWalk = 8 * kSliceThreads;
+constexpr int kSliceWalk = 24 * kSliceThreads;
+constexpr int kSliceLook = 40 * kSliceThreads;
 constexpr int kSliceLdsFixed = (kSliceChunk + 2 * kSliceWaves) * (int)sizeof(int);
 // largest r in [0, m) with row_ptr[r] - base <= k (0 if there is none): a whole wave, 64 probes at a time
 static __device__ __forceinline__ int row_of_entry(int m, const int* __restrict__ row_ptr, int base, int64_t k) {
@@ -208,18 +210,27 @@ __global__ __launch_bounds__(kSliceThreads) void csrmv_trans_slices_kernel(
     for (int q = 0; q < kSlicePer / 4; ++q) mine[q] = Int4{0, 0, 0, 0};
     __syncthreads();
     int64_t i = 1 + tid;
-    for (; (!GAPS || i <= kSliceWalk) && r0 + i < m; i += kSliceThreads) {  // ascending offsets: past the chunk, all later ones are too
-      const int64_t pos = (int64_t)row_ptr[r0 + i] - base - k0;
-      if (pos >= len) break;
-      atomicMax(&s_row[pos > 0 ? pos : 0], (int)i);
-    }
+    const auto walk = [&](int64_t most) __attribute__((always_inline)) {
+      for (; i <= most && r0 + i < m; i += kSliceThreads) {  // ascending offsets: past the chunk, all later ones are too
+        const int64_t pos = (int64_t)row_ptr[r0 + i] - base - k0;
+        if (pos >= len) break;
+        atomicMax(&s_row[pos > 0 ? pos : 0], (int)i);
+      }
+    };
+    walk(GAPS ? kSliceWalk : m);
     if (GAPS && tid == kSliceThreads - 1) *s_more = i > kSliceWalk;  // the thread that walks row r0 + kSliceWalk
     __syncthreads();
-    int last = 0;
+    int last = 0, most = 0;
     if (GAPS && *s_more) {
-      // (the row of the chunk's last entry; at least row r0 + kSliceWalk, where row_ptr ascends)
+      // the row of the chunk's last entry (at least row r0 + kSliceWalk, where row_ptr ascends)
       const int64_t to = row_of_entry(m, row_ptr, base, k0 + len - 1) - r0;
-      const int most = to > 1 ? (int)to : 1;
+      most = to > 1 ? (int)to : 1;
+      if (most <= kSliceLook) {
+        walk(m);
+        __syncthreads();
+      }
+    }
+    if (GAPS && most > kSliceLook) {
       auto starts_by = [&](int r, int k) __attribute__((always_inline)) {  // row r0 + r starts at or before entry k0 + k
         return (int64_t)row_ptr[r0 + r] - base - k0 <= k;
       };

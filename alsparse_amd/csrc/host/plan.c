@@ -458,7 +458,9 @@ static void choose_trans_route(asamd_csr_plan *p) {
   if (env_int("ALSPARSE_AMD_XLDS", 1) <= 0) return;
   const size_t ylds = st->nnz >= (1 << 20) && st->first_offset == 0 ? asamd_spmv_trans_ylds_bytes(p->dtype, st->m, st->n) : 0;
   if (asamd_spmv_trans_slices_fit(p->dtype, st->m, st->n, st->nnz, st->max_len) ||
-      (ylds == 0 && asamd_spmv_trans_slices_pay(p->dtype, st->n, st->nnz, p->trans_lines))) {
+      (ylds == 0 && asamd_spmv_trans_slices_pay(p->dtype, st->n, st->nnz, p->trans_lines) &&
+       /* (not a matrix of far more rows than entries: an atomic of the scatter is 45 ps) */
+       asamd_spmv_trans_slices_rows_us(p->dtype, st->m, st->n, st->nnz) <= 45e-6 * (double)st->nnz)) {
     /* (as many empty rows, if they lie side by side, as take one part's workgroups 7 us to pass) */
     p->trans_route = st->hist[0] >= 8192 ? TRANS_SLICES_GAPS : TRANS_SLICES;
     p->trans_bytes = align256(asamd_spmv_trans_slices_bytes(p->dtype, st->n, st->nnz));

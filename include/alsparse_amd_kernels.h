@@ -213,6 +213,8 @@ int asamd_spmv_trans_ylds(hipStream_t stream, const asamd_spmv_args *a, int32_t 
 int asamd_spmv_trans_slices_fit(int32_t dtype, int32_t m, int32_t n, int32_t nnz, int32_t max_len);
 /* Whether it is the better kernel for scattered columns: lines per entry as asamd_csr_row_stats_lines gives them. */
 int asamd_spmv_trans_slices_pay(int32_t dtype, int32_t n, int32_t nnz, float lines);
+/* What the slices' workgroups take to pass the rows of a matrix that has far more of them than entries, in us. */
+double asamd_spmv_trans_slices_rows_us(int32_t dtype, int32_t m, int32_t n, int32_t nnz);
 size_t asamd_spmv_trans_slices_bytes(int32_t dtype, int32_t n, int32_t nnz);
 int asamd_spmv_trans_slices(hipStream_t stream, const asamd_spmv_args *a, int32_t conj, void *partials);
 /* ... for a matrix that may have long runs of empty rows */

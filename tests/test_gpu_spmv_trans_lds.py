@@ -108,9 +108,11 @@ def rows_between_empty_ones(m, rows, lengths, cols, dt, base=0):
 
 #: the rows that start over a chunk end at the walk's last row, one past it, far past it
 EMPTY_ROWS = {
-    "walked_to_the_end": lambda dt: rows_between_empty_ones(8193, [0, 8192], [200, 300], 400, dt),
-    "one_more": lambda dt: rows_between_empty_ones(8194, [0, 8193], [200, 300], 400, dt),
-    "last_walked_row_ends_the_chunk": lambda dt: rows_between_empty_ones(40000, [0, 8192, 8193, 39999], [8191, 1, 9000, 3], 9001, dt),
+    "walked_to_the_end": lambda dt: rows_between_empty_ones(24577, [0, 24576], [200, 300], 400, dt),
+    "one_more": lambda dt: rows_between_empty_ones(24578, [0, 24577], [200, 300], 400, dt),
+    "last_walked_row_ends_the_chunk": lambda dt: rows_between_empty_ones(40000, [0, 24576, 24577, 39999], [8191, 1, 9000, 3], 9001, dt),
+    "counted_and_walked": lambda dt: rows_between_empty_ones(42000, [0, 40959, 40960], [200, 300, 7], 400, dt),
+    "one_more_than_walked": lambda dt: rows_between_empty_ones(42000, [0, 40960, 40961], [200, 300, 7], 400, dt),
     "empty_in_front": lambda dt: rows_between_empty_ones(300000, np.arange(290000, 300000), 4, 130, dt, base=1),
     "empty_behind": lambda dt: rows_between_empty_ones(300000, np.arange(10000), 4, 130, dt),
     "every_fortieth": lambda dt: rows_between_empty_ones(400000, np.arange(0, 400000, 40), 3, 300, dt),

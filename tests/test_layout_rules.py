@@ -40,3 +40,18 @@ def test_slice_counts_hold_x_and_prefer_even_shares_of_the_compute_units():
     assert lib.asamd_xlds_slices(0, 131072) == 4
     assert lib.asamd_xlds_slices(1, 100000) == 5      # nothing within a quarter divides 256
     assert lib.asamd_xlds_slices(0, 0) == 0 and lib.asamd_xlds_slices(9, 100) == 0
+
+
+def test_the_longest_row_is_counted_in_trips_of_the_scatters_lanes():
+    """The scatter gives a row as many lanes as the mean row has entries, two at least: empty rows do not make its longest
+    row any longer."""
+    lib = capi.load()
+    fit = lib.asamd_spmv_trans_slices_fit
+    # 64 trips of two lanes, whatever the empty rows: 1 M entries in 40 slices (116 us) scatter (50 + 45)
+    assert [fit(0, m, 750000, 1000000, 128) for m in (500000, 2000000, 100000000)] == [0, 0, 0]
+    # 14 slices, 41 us, and 18 parts, which pass 100 M rows in 4.7 ms
+    assert [fit(0, m, 250000, 1000000, 128) for m in (500000, 1000000, 100000000)] == [1, 1, 0]
+    assert lib.asamd_spmv_trans_slices_rows_us(0, 500000, 250000, 1000000) == 0.0
+    assert 4000 < lib.asamd_spmv_trans_slices_rows_us(0, 100000000, 250000, 1000000) < 6000
+    # means above two are the mean, as they were: power law of 102 000 rows, 10 a row, one of 2 500
+    assert fit(0, 102000, 102000, 1000000, 2500) == 1 and fit(0, 102000, 102000, 1000000, 127) == 0
