@@ -39,6 +39,16 @@ static std::vector<int> cut_blocks(const int* off, int groups, int max_groups, i
   return start;
 }
 
+template <typename T>
+static void launch_gather_tiles(hipStream_t s, const asamd_tiled_layout* L, const void* val, const int32_t* gate) {
+  // eight tiles to a wave at a time, eight workgroups abreast (one per XCD), as many as the chip holds at once
+  const int64_t per_xcd = ((int64_t)(L->row_blocks + 7) / 8) * ((L->col_blocks + 7) / 8);
+  int64_t grid = (per_xcd + 3) / 4 * 8;
+  if (grid > 8 * 512) grid = 8 * 512;
+  gather_values_tiles_kernel<T, false><<<(unsigned)grid, 256, 0, s>>>(L->tperm, (const T*)val, (T*)L->tval, L->tile_ptr,
+                                                                     L->col_blocks, L->row_blocks, gate);
+}
+
 // Equal-entry column / row blocks, stable sort of the entries by (column block,
 // row block), then the arrays of both phases in that order and the tile tables.
 template <typename T>
@@ -238,7 +248,7 @@ static hipError_t build_tiled(hipStream_t stream, asamd_tiled_layout* L, const i
                                                                                 d_tile_ptr);
     if constexpr (kPayloadSort) {
       L->tile_ptr = d_tile_ptr;  // stays with the layout: the values are gathered tile by tile, now and later
-      launch_gather_tiles<T>(stream, L->tperm, L->tile_ptr, L->col_blocks, L->row_blocks, val, L->tval, nullptr);
+      launch_gather_tiles<T>(stream, L, val, nullptr);
     }
     // Entries in tiles of 65..128 entries: if they are few, phase 2 runs in its one-entry-per-lane form
     // (twice the tiles in flight) and leaves those tiles to phase 3.
@@ -480,7 +490,7 @@ extern "C" int asamd_tiled_gather_values(hipStream_t s, const asamd_tiled_layout
   return by_dtype(L->dtype, [&](auto* tag) -> int {
     using T = std::remove_pointer_t<decltype(tag)>;
     if ((uintptr_t)val % alignof(T)) return hipErrorInvalidValue;
-    launch_gather_tiles<T>(s, L->tperm, L->tile_ptr, L->col_blocks, L->row_blocks, val, L->tval, gate);
+    launch_gather_tiles<T>(s, L, val, gate);
     return hipGetLastError();
   });
 }

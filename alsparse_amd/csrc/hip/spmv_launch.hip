@@ -510,7 +510,7 @@ static int merge_launch(hipStream_t s, const asamd_spmv_args* a, int32_t ipt, co
       ASAMD_LAUNCH_MERGE_PERM(IPT, kPermConj);                                                                       \
     else if (perm)                                                                                                   \
       ASAMD_LAUNCH_MERGE_PERM(IPT, kPermPlain);                                                                      \
-    else if (wide)                                                                                                        \
+    else if (wide)                                                                                                   \
       spmv_merge_kernel<T, IPT, true><<<nb, kMergeThreads, 0, s>>>(a->m, a->nnz, alpha, val, a->row_ptr, a->col_ind, \
                                                                    x, beta, y, a->base, block_row, carry_row,        \
                                                                    (T*)carry_val, (T*)head_val, policy);             \

@@ -276,17 +276,6 @@ __global__ __launch_bounds__(256) void gather_values_tiles_kernel(const unsigned
   }
 }
 
-template <typename T>
-void launch_gather_tiles(hipStream_t s, const unsigned* perm, const int* tile_ptr, int col_blocks, int row_blocks,
-                         const void* val, void* out, const int* gate) {
-  // eight tiles to a wave at a time, eight workgroups abreast (one per XCD), as many as the chip holds at once
-  const int64_t per_xcd = ((int64_t)(row_blocks + 7) / 8) * ((col_blocks + 7) / 8);
-  int64_t grid = (per_xcd + 3) / 4 * 8;
-  if (grid > 8 * 512) grid = 8 * 512;
-  gather_values_tiles_kernel<T, false><<<(unsigned)grid, 256, 0, s>>>(perm, (const T*)val, (T*)out, tile_ptr, col_blocks,
-                                                                      row_blocks, gate);
-}
-
 // Entries in sorted order: values, columns and rows local to their blocks.
 template <typename T>
 __global__ __launch_bounds__(256) void tile_gather_kernel(

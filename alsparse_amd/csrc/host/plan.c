@@ -576,7 +576,8 @@ static int settle_algo(const asamd_csr_plan *p, int algo, const void *val, const
 }
 
 /* merge path; perm: NULL, or where the values of the plan's entries lie in a->val */
-static int run_merge(hipStream_t s, asamd_csr_plan *p, const asamd_spmv_args *a, ws_cursor ws, const uint32_t *perm, int conj) {
+static int run_merge(hipStream_t s, const asamd_csr_plan *p, const asamd_spmv_args *a, ws_cursor ws, const uint32_t *perm,
+                     int conj) {
   const asamd_csr_stats *st = &p->st;
   const size_t nb = (size_t)st->merge_blocks, vs = (size_t)p->val_size;
   const int32_t *block_row = p->d_block_row;
