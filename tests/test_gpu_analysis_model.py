@@ -87,9 +87,12 @@ def test_model_and_timing_choose_the_same_family(gpu, shape):
         da.free()
 
 
-def test_default_analysis_through_the_public_api_multiplies_correctly(gpu):
-    """The public analysis call under default settings (model), followed by multiplies, on the tiled shape."""
+@pytest.mark.parametrize("sums", [0, 1], ids=["family", "row_sums"])
+def test_default_analysis_through_the_public_api_multiplies_correctly(gpu, sums, monkeypatch):
+    """The public analysis call under default settings (model), followed by multiplies, on the tiled shape: with the
+    row-sum tiles that take its place by default, and without them."""
     lib = capi.load()
+    monkeypatch.setenv("ALSPARSE_AMD_ROW_SUMS", str(sums))
     a = wl.uniform_rows(1 << 21, 1 << 21, 16, np.float32)
     x, y0 = wl.uniform(a.cols, a.dtype, 3), wl.uniform(a.rows, a.dtype, 4)
     da = DeviceCsr(a)
@@ -101,9 +104,9 @@ def test_default_analysis_through_the_public_api_multiplies_correctly(gpu):
         assert lib.alphasparse_dcu_s_csrmv_analysis(gpu.h, 0, a.rows, a.cols, a.nnz, byref(descr), da.val.c_ptr(),
                                                     da.row_ptr.c_ptr(), da.col.c_ptr(), info) == 0
         st = lib.asamd_analysis_stats(info).contents
-        assert st.tune_mode == 1 and st.algo == capi.ASAMD_SPMV_TILED
+        assert st.tune_mode == 1 and st.algo == capi.ASAMD_SPMV_TILED and st.row_sums == sums
         assert st.ell_built == 0 and st.binned_built == 0, "the model lays out only the copy it keeps"
-        check_spmv(a, 1.5, x, 0.5, y0, run_csrmv(gpu, da, 1.5, x, 0.5, y0, info), "model-chosen tiled copy")
+        check_spmv(a, 1.5, x, 0.5, y0, run_csrmv(gpu, da, 1.5, x, 0.5, y0, info), "model-chosen tiled copy, row sums %d" % sums)
     finally:
         lib.alphasparse_dcu_destroy_mat_info(info)
         da.free()

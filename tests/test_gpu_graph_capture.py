@@ -14,8 +14,8 @@ from oracle import oracle as orc
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("shape", ["powerlaw_merge", "laplace_ell", "uniform_tiled", "transposed"])
-def test_analysed_csrmv_replays_from_a_hip_graph(gpu, shape):
+@pytest.mark.parametrize("shape", ["powerlaw_merge", "laplace_ell", "uniform_tiled", "uniform_row_sums", "transposed"])
+def test_analysed_csrmv_replays_from_a_hip_graph(gpu, shape, monkeypatch):
     lib, hip = capi.load(), hiprt.lib()
     dtype = np.float64 if shape == "laplace_ell" else np.float32
     if shape == "powerlaw_merge":
@@ -23,7 +23,11 @@ def test_analysed_csrmv_replays_from_a_hip_graph(gpu, shape):
     elif shape == "laplace_ell":
         a = wl.laplace2d(700, 600, dtype)
     else:
-        a = wl.uniform_rows(1 << 19, 1 << 22, 12, dtype)   # x = 16 MiB: the tiled copy is built and timed
+        a = wl.uniform_rows(1 << 19, 1 << 22, 12, dtype)   # x = 16 MiB: the tiled copy is built
+        if shape == "uniform_row_sums":
+            a = wl.uniform_rows(1 << 20, 1 << 20, 16, dtype)  # the tiles that add up, in a family's place
+        else:
+            monkeypatch.setenv("ALSPARSE_AMD_ROW_SUMS", "0")
     trans = capi.ALPHA_SPARSE_OPERATION_TRANSPOSE if shape == "transposed" else 0
     xlen, ylen = (a.rows, a.cols) if trans else (a.cols, a.rows)
     x, y0 = wl.uniform(xlen, dtype, 3), wl.uniform(ylen, dtype, 4)
@@ -49,6 +53,7 @@ def test_analysed_csrmv_replays_from_a_hip_graph(gpu, shape):
             h.h, trans, a.rows, a.cols, a.nnz, byref(descr), da.val.c_ptr(), da.row_ptr.c_ptr(), da.col.c_ptr(), info) == 0
         stats = lib.asamd_analysis_stats(info).contents
         announce("graph capture: analysis chose", capi.ALGO_NAMES[stats.algo])
+        assert stats.row_sums == (shape == "uniform_row_sums") and stats.tiled_built >= (shape == "uniform_tiled")
         assert multiply() == 0                                   # eager, on the stream
         hiprt.check(hip.hipStreamSynchronize(stream), "sync")
         eager = dy.to_numpy()
@@ -76,7 +81,7 @@ def test_analysed_csrmv_replays_from_a_hip_graph(gpu, shape):
             hiprt.check(hip.hipGraphLaunch(gexec, stream), "hipGraphLaunch")
             hiprt.check(hip.hipStreamSynchronize(stream), "sync")
             got = dy.to_numpy()
-            if running.tiled_built:  # checked against the oracle like the eager result
+            if running.tiled_built and not running.row_sums:  # checked against the oracle like the eager result
                 verify(got, "replay %d" % replay)
             else:
                 assert np.array_equal(got, eager), "replay %d differs from the eager result" % replay
@@ -99,6 +104,7 @@ CAPTURE_CASES += [("xlds", "narrow")]  # x fits the LDS: 20 000 columns, read as
 CAPTURE_CASES += [("xlds", "uniform")]  # 50 000 columns: two slices over a copy of the entries, behind the value guard
 # heavy-tailed rows: the tiled copy's third phase, the bins' chunked long rows, merge blocks inside one row
 CAPTURE_CASES += [(algo, "powerlaw") for algo in ("merge", "tiled", "hot", "binned")]
+CAPTURE_CASES += [("auto", "powerlaw")]  # row-sum tiles, behind the value guard
 
 
 @pytest.mark.parametrize("algo,shape", CAPTURE_CASES, ids=["%s-%s" % c for c in CAPTURE_CASES])
@@ -117,6 +123,7 @@ def test_every_kernel_family_replays_from_a_hip_graph(gpu, algo, shape):
         assert lib.asamd_csr_plan_create(stream, a.rows, a.cols, a.nnz, da.row_ptr.c_ptr(), da.col.c_ptr(),
                                          da.val.c_ptr(), a.base, a.dtype.itemsize, 2, byref(plan)) == 0
         assert lib.asamd_csr_plan_set_algo(plan, ALGOS[algo]) == 0, "this matrix can run every family"
+        assert lib.asamd_csr_plan_stats(plan).contents.row_sums == (algo == "auto")
 
         ws = capi.Workspace(lib, plan)
 

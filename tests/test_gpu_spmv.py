@@ -548,13 +548,16 @@ def test_tiled_second_phase_in_both_forms(gpu, dtype, per_row, monkeypatch):
 
 
 @pytest.mark.parametrize("m,n,per_row", [(1 << 21, 1 << 21, 16), (1 << 19, 1 << 21, 128)], ids=["16_per_row", "128_per_row"])
-def test_tiled_row_blocks_follow_the_tile_population(gpu, m, n, per_row):
+@pytest.mark.parametrize("sums", [0, 1], ids=["family", "row_sums"])
+def test_tiled_row_blocks_follow_the_tile_population(gpu, m, n, per_row, sums, monkeypatch):
     """2 M x 2 M with 16 entries per row: 52 column blocks (40 960 columns each), so a 2 048-row block would put
     630 entries into every tile and leave them all to the long-tile kernel.  The analysis cuts the blocks to
     about 200 rows (about 60 entries per tile), and the tiled pair then wins its timing run against the row
     kernels.  With 128 entries per row even the shortest row block (64 rows) would overfill its tiles: the
-    column blocks are made narrower as well (about 128 of them instead of 52)."""
+    column blocks are made narrower as well (about 128 of them instead of 52).  The product runs on the tiled pair, or on
+    the row-sum tiles that stand in for it by default."""
     lib = capi.load()
+    monkeypatch.setenv("ALSPARSE_AMD_ROW_SUMS", str(sums))
     a = wl.uniform_rows(m, n, per_row, np.float32)
     x, y0 = _vectors(a)
     da = DeviceCsr(a)
@@ -567,6 +570,7 @@ def test_tiled_row_blocks_follow_the_tile_population(gpu, m, n, per_row):
                                                     da.row_ptr.c_ptr(), da.col.c_ptr(), info) == 0
         st = lib.asamd_analysis_stats(info).contents
         assert st.tiled_built == 1 and st.algo == capi.ASAMD_SPMV_TILED, capi.ALGO_NAMES[st.algo]
+        assert st.row_sums == sums
         assert 6000 <= st.tile_row_blocks <= 12000, st.tile_row_blocks
         mean_tile = a.nnz / (st.tile_row_blocks * st.tile_col_blocks)
         assert 40 <= mean_tile <= 80, mean_tile

@@ -77,10 +77,13 @@ def test_plan_refresh_values_brings_every_copy_up_to_date(gpu, algo, dtype):
         da.free()
 
 
-def test_reanalysis_after_values_changed_in_place(gpu):
+@pytest.mark.parametrize("sums", [0, 1], ids=["family", "row_sums"])
+def test_reanalysis_after_values_changed_in_place(gpu, sums, monkeypatch):
     """Large enough for the analysis to pick the tiled copy (2 M x 2 M, 16 per row): analyse, multiply, rewrite
-    csr_val in place, analyse again (values only: several times faster than the first analysis), multiply."""
+    csr_val in place, analyse again (values only: several times faster than the first analysis), multiply -- on the tiled
+    pair and on the row-sum tiles that stand in for it by default."""
     lib = capi.load()
+    monkeypatch.setenv("ALSPARSE_AMD_ROW_SUMS", str(sums))
     a = wl.uniform_rows(1 << 21, 1 << 21, 16, np.float32)
     x, y0 = wl.uniform(a.cols, a.dtype, 3), wl.uniform(a.rows, a.dtype, 4)
     da = DeviceCsr(a)
@@ -100,13 +103,13 @@ def test_reanalysis_after_values_changed_in_place(gpu):
         announce("re-analysis", a.name)
         first_ms = analyse()
         st = lib.asamd_analysis_stats(info).contents
-        assert st.tiled_built == 1 and st.algo == capi.ASAMD_SPMV_TILED
+        assert st.tiled_built == 1 and st.algo == capi.ASAMD_SPMV_TILED and st.row_sums == sums
         check_spmv(a, 1.5, x, 0.5, y0, run_csrmv(gpu, da, 1.5, x, 0.5, y0, info), "first analysis")
         b = _with_values(a, _new_values(a, 7))
         da.val.copy_from(b.values)
         again_ms = analyse()
         st = lib.asamd_analysis_stats(info).contents
-        assert st.tiled_built == 1 and st.algo == capi.ASAMD_SPMV_TILED
+        assert st.tiled_built == 1 and st.algo == capi.ASAMD_SPMV_TILED and st.row_sums == sums
         check_spmv(b, 1.5, x, 0.5, y0, run_csrmv(gpu, da, 1.5, x, 0.5, y0, info), "after re-analysis")
         print("analysis %.2f ms, repeated on changed values %.2f ms" % (first_ms, again_ms))
         assert again_ms < 0.5 * first_ms, (first_ms, again_ms)

@@ -71,7 +71,8 @@ def test_plan_multiplies_with_the_values_of_the_moment(gpu, copy, dtype):
     if copy == "conj_transposed" and not np.iscomplexobj(np.zeros(1, dtype)):
         pytest.skip("a real matrix has no conjugate transpose in the reference's tables")
     lib = capi.load()
-    a = _matrix(lambda rd: wl.uniform_rows(7000, 9000, 12, rd), dtype)
+    # (transposed: more entries than the product that reads the caller's values through the permutation takes)
+    a = _matrix(lambda rd: wl.uniform_rows(*((7000, 9000, 12) if copy in ("tiled", "ell") else (70001, 60000, 8)), rd), dtype)
     op = {"tiled": 0, "ell": 0, "transposed": 1, "conj_transposed": 2}[copy]
     x = _vector(a.rows if op else a.cols, dtype, 3)
     y0 = _vector(a.cols if op else a.rows, dtype, 4)
@@ -119,10 +120,13 @@ def test_plan_multiplies_with_the_values_of_the_moment(gpu, copy, dtype):
         da.free()
 
 
+@pytest.mark.parametrize("sums", [0, 1], ids=["family", "row_sums"])
 @pytest.mark.parametrize("dtype", DT, ids=IDS)
-def test_analysis_then_new_values_then_csrmv_through_the_public_api(gpu, dtype):
+def test_analysis_then_new_values_then_csrmv_through_the_public_api(gpu, dtype, sums, monkeypatch):
     """alphasparse_dcu_?_csrmv_analysis -> overwrite csr_val -> alphasparse_dcu_?_csrmv(info), on a matrix large
-    enough for the analysis to keep the tiled copy by itself (x beyond an XCD's L2, scattered columns)."""
+    enough for the analysis to keep the tiled copy by itself (x beyond an XCD's L2, scattered columns), and in single
+    precision to lay out row-sum tiles in its place: with them and without."""
+    monkeypatch.setenv("ALSPARSE_AMD_ROW_SUMS", str(sums))
     lib = capi.load()
     rows = 1 << 21
     a = _matrix(lambda rd: wl.uniform_rows(rows, rows, 16, rd), dtype)
@@ -152,6 +156,7 @@ def test_analysis_then_new_values_then_csrmv_through_the_public_api(gpu, dtype):
                                                                      da.col.c_ptr(), info) == 0
         st = lib.asamd_analysis_stats(info).contents
         assert st.tiled_built == 1 and st.algo == capi.ASAMD_SPMV_TILED, "this shape is the tiled copy's"
+        assert st.row_sums == (sums and np.dtype(dtype) == np.float32)
         _check(a, 0, 1.5, x, 0.5, y0, multiply(1.5, 0.5), "after the analysis")
         b = _with_values(a, _new_values(a, 7))
         da.val.copy_from(b.values)
@@ -170,7 +175,8 @@ def test_analysis_then_new_values_then_csrmv_through_the_public_api(gpu, dtype):
         dx.free()
 
 
-def test_full_value_check_notices_a_single_entry(gpu):
+@pytest.mark.parametrize("sums", [0, 1], ids=["family", "row_sums"])
+def test_full_value_check_notices_a_single_entry(gpu, sums, monkeypatch):
     """ALSPARSE_AMD_VALUE_CHECK=full fingerprints every byte: one changed entry anywhere is seen.  (Read when an
     analysis is made.)"""
     lib = capi.load()
@@ -179,13 +185,14 @@ def test_full_value_check_notices_a_single_entry(gpu):
     x, y0 = wl.uniform(a.cols, a.dtype, 3), wl.uniform(a.rows, a.dtype, 4)
     da = DeviceCsr(a)
     plan = c_void_p()
+    monkeypatch.setenv("ALSPARSE_AMD_ROW_SUMS", str(sums))
     os.environ["ALSPARSE_AMD_VALUE_CHECK"] = "full"
     try:
         announce("full value check")
         assert lib.asamd_csr_plan_create(None, a.rows, a.cols, a.nnz, da.row_ptr.c_ptr(), da.col.c_ptr(), da.val.c_ptr(),
                                          a.base, 4, 1, byref(plan)) == 0
         st = lib.asamd_csr_plan_stats(plan).contents
-        assert st.value_check == 2 and st.algo == capi.ASAMD_SPMV_TILED
+        assert st.value_check == 2 and st.algo == capi.ASAMD_SPMV_TILED and st.row_sums == sums
         ws = capi.Workspace(lib, plan)
         dx = hiprt.DeviceArray.from_numpy(x)
         for k in (12345677, a.nnz - 1, 0):
@@ -239,8 +246,8 @@ def test_small_workspace_still_multiplies_correctly(gpu):
         da.free()
 
 
-@pytest.mark.parametrize("shape", ["powerlaw", "tiled", "slices"])
-def test_one_analysis_from_two_handles_at_once(gpu, shape):
+@pytest.mark.parametrize("shape", ["powerlaw", "tiled", "slices", "row_sums"])
+def test_one_analysis_from_two_handles_at_once(gpu, shape, monkeypatch):
     """Two handles, each with a stream of its own, multiply with ONE info concurrently: every scratch word of a
     multiply lives in its handle's buffer, so each result equals the serial one bit for bit."""
     lib, hip = capi.load(), hiprt.lib()
@@ -249,7 +256,8 @@ def test_one_analysis_from_two_handles_at_once(gpu, shape):
     elif shape == "slices":
         a = wl.uniform_rows(1 << 18, 1 << 17, 64, np.float32)  # x in LDS slice by slice: the slices' sums per call
     else:
-        a = wl.uniform_rows(1 << 21, 1 << 21, 16, np.float32)  # tiled: the product array per call
+        a = wl.uniform_rows(1 << 21, 1 << 21, 16, np.float32)  # tiled: the product array per call; row sums: the sums
+        monkeypatch.setenv("ALSPARSE_AMD_ROW_SUMS", "1" if shape == "row_sums" else "0")
     da = DeviceCsr(a)
     info = capi.alphasparse_dcu_mat_info_t()
     assert lib.alphasparse_dcu_create_mat_info(byref(info)) == 0
@@ -269,7 +277,8 @@ def test_one_analysis_from_two_handles_at_once(gpu, shape):
         assert lib.alphasparse_dcu_s_csrmv_analysis(handles[0].h, 0, a.rows, a.cols, a.nnz, byref(descr), da.val.c_ptr(),
                                                     da.row_ptr.c_ptr(), da.col.c_ptr(), info) == 0
         st = lib.asamd_analysis_stats(info).contents
-        want = {"powerlaw": capi.ASAMD_SPMV_MERGE, "slices": capi.ASAMD_SPMV_XLDS, "tiled": capi.ASAMD_SPMV_TILED}[shape]
+        want = {"powerlaw": capi.ASAMD_SPMV_MERGE, "slices": capi.ASAMD_SPMV_XLDS}.get(shape, capi.ASAMD_SPMV_TILED)
+        assert st.row_sums == (shape == "row_sums")
         assert st.algo == want and (shape != "slices" or st.xlds_slices >= 2), (st.algo, st.xlds_slices)
 
         def multiply(i, reps):
