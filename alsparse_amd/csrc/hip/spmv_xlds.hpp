@@ -360,8 +360,8 @@ __global__ __launch_bounds__(kXldsThreads) void spmv_xlds4_kernel(int m, int n_t
 // above (W lanes per row, eight rows per lane group and trip in flight), every entry adds a * x[row] to its column's
 // sum in the workgroup's LDS (LDS atomics: the order of the additions inside a workgroup is not fixed), and the
 // workgroup writes its n sums to partials + blockIdx.x * n; trans_partials_sum_kernel adds the workgroups' sums in
-// order.  The scatter with global atomics (spmv_trans.hpp) takes 3.1 ms on 4 194 304 x 32 768 x 16, fp32, this 0.40: every
-// one of the scatter's 67 M atomics travels to memory.  The sums keep the element type here, so that a y of a whole LDS
+// order.  The scatter with global atomics (spmv_trans.hpp) takes 2.7 ms on 4 194 304 x 32 768 x 16, fp32, this 0.35: next
+// to every one of the scatter's 67 M atomics travels to memory.  The sums keep the element type here, so that a y of a whole LDS
 // is one slice: with sums in double precision the same matrix is three slices, 0.55 ms (csrmv_trans_slices_kernel).
 template <typename T, int W, bool CONJ>
 __global__ __launch_bounds__(kXldsThreads) void spmv_trans_ylds_kernel(int m, int n, T alpha, const T* __restrict__ val,

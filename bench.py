@@ -34,7 +34,7 @@ NO_ANALYSIS = False  # --no-analysis
 MEASURED_TRAFFIC_BYTES = {
     (3, "tiled two-phase"): (5.17e9, "profiles/spmv_tiled_C3.txt"),
     (3, "rowconst"): (34.6e9, "profiles/spmv_tiled_C3.txt"),
-    (4, "row-sum tiles"): (1.13e9, "profiles/spmv_sums_C4.txt"),
+    (4, "row-sum tiles"): (1.49e9, "profiles/spmv_sums_C4.txt"),
     (4, "merge-path"): (3.19e9, "profiles/spmv_merge_C4.txt"),
     (4, "merge-path, hot columns in LDS"): (2.85e9, "profiles/spmv_merge_hot_C4.txt"),
     (2, "ell copy"): (356.6e6, "profiles/spmv_ell_copy_C2.txt"),
@@ -362,7 +362,7 @@ def run_spmv(cfg, steps, warmup, cpu_baseline, check, transpose=False, vendor=Fa
            "dtype": {"float32": "f32", "float64": "f64", "complex64": "c64", "complex128": "c128"}[a.dtype.name],
            "parity": parity}
     # what the analysis measured when it chose the kernel (one multiply each on scratch vectors; 0 = not tried)
-    res["analysis_timings_ms"] = {k: round(float(getattr(stats, "tune_ms_" + k)), 4) for k in ("base", "tiled", "ell", "hot", "binned")}
+    res["analysis_timings_ms"] = {k: round(float(getattr(stats, "tune_ms_" + k)), 4) for k in ("base", "tiled", "ell", "hot", "binned", "sums")}
     if cx:  # a complex multiply-add is 8 real flops
         res["flops"], res["gflops"] = 8 * a.nnz, 8 * a.nnz / t["avg_ms"] / 1e6
     res["hbm_frac"] = res["gbs"] / HBM_PEAK_GBS
@@ -378,6 +378,8 @@ def run_spmv(cfg, steps, warmup, cpu_baseline, check, transpose=False, vendor=Fa
     res["workspace_bytes"] = int(stats.workspace_bytes)
     res["value_check"] = {0: "off", 1: "sampled fingerprint of csr_val before every multiply that uses a copy",
                           2: "full fingerprint"}[int(stats.value_check)]
+    if stats.value_check == 1 and stats.row_sums and stats.tiled_built + stats.ell_built == 0 and stats.xlds_slices == 0:
+        res["value_check"] = "full fingerprint (row-sum tiles in the place of a family that reads csr_val)"
     res["tune_mode"] = "model" if stats.tune_mode else "timed"
     if early_calls_ms is not None:
         res["calls_2_to_5_ms"] = [round(v, 4) for v in early_calls_ms]
