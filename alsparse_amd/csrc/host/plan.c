@@ -1421,8 +1421,10 @@ static double sums_rival_ms(const asamd_csr_plan *p) {
     kept *= p->val_size < 8 ? 0.95 : 1.1;
   }
   if (holds_values(p, algo) && algo != ASAMD_SPMV_XLDS && p->st.value_check) kept += 0.022;
-  /* (the tiled pair's estimate runs high for 16-byte values: the transpose of 2.5 M x 2.5 M x 18, complex128, 0.63 against
-   * 0.493 ms; with them 0.506) */
+  /* (the tiled pair's estimate runs high for 16-byte values.  Of 22 uniform matrices and transposes, complex128, 0.5 .. 4 M rows
+   * of 8 .. 30 entries, nine have the tiles without this factor and take 0.90 .. 1.07 of the pair's time with them: 2 M x 1 M x 16
+   * transposed 0.371 against 0.415 ms, 2.5 M x 2.5 M x 18 0.506 / 0.532, 2 M x 2 M x 24 0.528 / 0.507, 3 M x 3 M x 12 0.440 / 0.411.
+   * With it they stay with the pair; 1 M x 1 M x 40, whose family is merge-path, has the tiles: 0.645 -> 0.422.) */
   if (algo == ASAMD_SPMV_TILED && p->val_size == 16) kept *= 0.8;
   return kept;
 }
