@@ -127,7 +127,7 @@ size_t asamd_csr_plan_workspace_bytes(const asamd_csr_plan *plan);
  * asamd_csr_plan_refresh_values (or analyse again).  Row-sum tiles that stand in for a family that keeps no
  * values (merge-path, the hot columns, the row kernels) are the exception: every byte is fingerprinted for them, and a
  * single changed entry counts as it does with that family.  ALSPARSE_AMD_VALUE_CHECK=full fingerprints every
- * byte (one more pass over val per multiply), =off none (the caller then refreshes by hand).  A
+ * byte (one more pass over val per multiply), =off none, row-sum tiles included (the caller then refreshes by hand).  A
  * multiply that passes ANOTHER value array than the copies were taken from runs on the caller's arrays. */
 int asamd_csr_plan_csrmv(hipStream_t stream, asamd_csr_plan *plan, int32_t op, const void *alpha, const void *val,
                          const int32_t *row_ptr, const int32_t *col_ind, const void *x, const void *beta, void *y,

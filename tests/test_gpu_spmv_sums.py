@@ -173,6 +173,25 @@ def test_values_follow_the_caller(gpu):
         p.close()
 
 
+def test_without_a_check_a_refresh_brings_the_values(gpu, monkeypatch):
+    """ALSPARSE_AMD_VALUE_CHECK=off: the caller refreshes by hand, the tiles' values too."""
+    monkeypatch.setenv("ALSPARSE_AMD_VALUE_CHECK", "off")
+    a = _matrix(_tail(50000, 13, 20000), 200000, np.float64, 13)
+    rng = np.random.default_rng(20)
+    x, y0 = _numbers(rng, a.cols, np.float64), _numbers(rng, a.rows, np.float64)
+    p = Plan(a, 2)
+    try:
+        announce("row sums, no check")
+        assert p.stats.row_sums == 1 and p.stats.value_check == 0
+        _check(a, 1.0, x, 0.5, y0, p.multiply(1.0, x, 0.5, y0), "values of the analysis")
+        b = wl.Csr(a.rows, a.cols, a.row_ptr, a.col_ind, _numbers(rng, a.nnz, np.float64), 0, "new")
+        p.da.val.copy_from(b.values)
+        assert p.lib.asamd_csr_plan_refresh_values(None, p.plan, p.da.row_ptr.c_ptr(), p.da.col.c_ptr(), p.da.val.c_ptr()) == 0
+        _check(b, 1.0, x, 0.5, y0, p.multiply(1.0, x, 0.5, y0), "refreshed")
+    finally:
+        p.close()
+
+
 def test_single_values_poked_into_a_graph_count(gpu):
     """Merge-path and the hot-column kernel read csr_val on every multiply; the tiles that stand in for them hold a copy of
     it, 92 MB here, of which the usual check reads a quarter: one changed value anywhere has to show in the next product
