@@ -66,7 +66,7 @@ static const int kValSize[4] = {4, 8, 8, 16};
 
 static int is_complex(const asamd_csr_plan *p) { return p->dtype >= ASAMD_DTYPE_FLOAT_COMPLEX; }
 
-/* ---- environment switches (read when a plan is made; ALSPARSE_AMD_XLDS=0 also counts later) ------------------------------------------------------------ */
+/* ---- environment switches (read when a plan is made; ALSPARSE_AMD_XLDS=0 also counts later) ------------ */
 static int env_int(const char *name, int fallback) {
   const char *e = getenv(name);
   return e && *e ? atoi(e) : fallback;
@@ -447,8 +447,8 @@ static int holds_values(const asamd_csr_plan *p, int algo) {
 
 /* The transposed multiply without a copy, and its per-call scratch: sums in LDS, with the columns in slices or with all of y
  * (where it fits and the matrix is large enough for a workgroup per compute unit to pay), or the atomic scatter.  Settled
- * once: the estimates and the switches behind them cost half a microsecond, which a multiply of a few thousand entries
- * shows (a pair of products, 3 000 x 9 000 x 10: 12.4 us with them on every call, 11.6 without). */
+ * once: the estimates and the switches behind them cost 0.15 us, which a multiply of a few thousand entries shows (a pair of
+ * products, 3 000 x 9 000 x 10, in processes whose launches are quick: 9.95 us with them on every call, 9.80 without). */
 enum { TRANS_SCATTER = 0, TRANS_SLICES, TRANS_SLICES_GAPS, TRANS_YLDS };
 
 static void choose_trans_route(asamd_csr_plan *p) {
