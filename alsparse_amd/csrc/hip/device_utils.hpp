@@ -158,8 +158,10 @@ template <typename P>
 __device__ __forceinline__ P nt_load_object(const P* p) {
   typedef int V2 __attribute__((ext_vector_type(2)));
   typedef int V4 __attribute__((ext_vector_type(4)));
-  static_assert(sizeof(P) == 4 || sizeof(P) == 8 || sizeof(P) == 16 || sizeof(P) == 32, "object size");
-  if constexpr (sizeof(P) == 4) {
+  static_assert(sizeof(P) == 2 || sizeof(P) == 4 || sizeof(P) == 8 || sizeof(P) == 16 || sizeof(P) == 32, "object size");
+  if constexpr (sizeof(P) == 2) {
+    return __builtin_bit_cast(P, __builtin_nontemporal_load(reinterpret_cast<const short*>(p)));
+  } else if constexpr (sizeof(P) == 4) {
     return __builtin_bit_cast(P, __builtin_nontemporal_load(reinterpret_cast<const int*>(p)));
   } else if constexpr (sizeof(P) == 8) {
     return __builtin_bit_cast(P, __builtin_nontemporal_load(reinterpret_cast<const V2*>(p)));

@@ -267,12 +267,9 @@ static hipError_t build_sums(hipStream_t stream, asamd_sums_layout* L, const int
     if (e == hipSuccess) e = hipMemcpy(L->order, order.data(), ((size_t)spans + 1) * sizeof(int), hipMemcpyHostToDevice);
   }
   if (e == hipSuccess) e = (hipError_t)asamd_sums_refresh_values(stream, L, val, nullptr);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void*)sums_products_kernel<T, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            kLdsPerCu);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void*)sums_products_kernel<T, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            kLdsPerCu);
+  for (const void* f : {(const void*)sums_products_kernel<T, false, false>, (const void*)sums_products_kernel<T, false, true>,
+                        (const void*)sums_products_kernel<T, true, true>})
+    if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsPerCu);
   if (e == hipSuccess)
     e = hipFuncSetAttribute((const void*)tiled_reduce_kernel<T, 1, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             kLdsPerCu);
@@ -331,13 +328,21 @@ extern "C" int asamd_spmv_sums(hipStream_t s, const asamd_spmv_args* a, const as
     const T* x = (const T*)a->x;
     T* y = (T*)a->y;
     T* mid = (T*)sums;
-    // (stored past the memory-side cache where it could not hold them, as the tiled pair's products)
-    if ((int64_t)L->sums * (int64_t)sizeof(T) > ((int64_t)512 << 20))
-      sums_products_kernel<T, true><<<L->n_chunks, kProdThreads, kLdsPerCu, s>>>(
-          (const SumsChunk*)L->chunks, L->span_sum, (const T*)L->tval, L->tcol, x, mid);
-    else
-      sums_products_kernel<T, false><<<L->n_chunks, kProdThreads, kLdsPerCu, s>>>(
-          (const SumsChunk*)L->chunks, L->span_sum, (const T*)L->tval, L->tcol, x, mid);
+    const auto products = [&](auto kernel) {
+      kernel<<<L->n_chunks, kProdThreads, kLdsPerCu, s>>>((const SumsChunk*)L->chunks, L->span_sum, (const T*)L->tval, L->tcol,
+                                                          x, mid);
+    };
+    // Sums that the memory-side cache could not hold are stored past it, as the tiled pair's products.  Where it holds the
+    // sums, but not the values and columns beside them, those are loaded past it, so that the second phase finds the sums
+    // there: us, plain / past it, inputs of three matrices in turn: power law of 8 M rows fp32 331 / 307, uniform 1 M x 16
+    // fp64 (transposed, 270 MB of streams and sums) 117 / 112, 2 M x 20 fp32 144 / 141, 2 M x 20 complex128 456 / 441.  One
+    // matrix again and again is served from that cache where it fits: power law of 2 M rows (181 MB) 80 / 85, uniform 1 M x
+    // 20 fp32 (190 MB) 83 / 88.
+    const int64_t sum_bytes = (int64_t)L->sums * (int64_t)sizeof(T);
+    const int64_t stream_bytes = (int64_t)L->spans * SumsDims<T>::span * ((int64_t)sizeof(T) + 2);
+    if (sum_bytes > ((int64_t)512 << 20)) products(sums_products_kernel<T, true, true>);
+    else if (sum_bytes + stream_bytes > (int64_t)256000000) products(sums_products_kernel<T, false, true>);
+    else products(sums_products_kernel<T, false, false>);
     const unsigned grid = (unsigned)((L->row_blocks + kRedWaves - 1) / kRedWaves);
     tiled_reduce_kernel<T, 1, true><<<grid, kRedWaves * kWave, sums_red_lds<T>(L->rows_cap), s>>>(
         L->row_blocks, 0, L->rows_cap, L->row_block_start, L->run_ptr, (const TileRange*)L->runs, L->srow, mid, alpha, beta,

@@ -248,7 +248,8 @@ static __global__ __launch_bounds__(64) void sums_runs_kernel(int row_blocks, in
 // ---- phase 1 -------------------------------------------------------------------
 // Bounds: the streams, 6 bytes per fp32 entry in and 4 per sum out.  The next trip's loads are in flight while one is
 // worked on.  A span without all its entries ends in slots that no mark follows: what they form is never stored.
-template <typename T, bool NTS>
+// NTS: the sums are stored past the memory-side cache; NTL: the values and columns are loaded past it (asamd_spmv_sums).
+template <typename T, bool NTS, bool NTL>
 __global__ __launch_bounds__(kProdThreads) void sums_products_kernel(
     const SumsChunk* __restrict__ chunks, const int* __restrict__ span_sum, const T* __restrict__ t_val,
     const unsigned short* __restrict__ t_col, const T* __restrict__ x, T* __restrict__ out) {
@@ -271,8 +272,15 @@ __global__ __launch_bounds__(kProdThreads) void sums_products_kernel(
     const int64_t q = (int64_t)ch.span0 * SumsDims<T>::span + first + lane * kPer;
 #pragma unroll
     for (int i = 0; i < kPieces; ++i) {
-      v[i] = *reinterpret_cast<const Piece<T>*>(t_val + q + i * kWave * kPer);
-      c[i] = *reinterpret_cast<const ColPiece*>(t_col + q + i * kWave * kPer);
+      const auto* pv = reinterpret_cast<const Piece<T>*>(t_val + q + i * kWave * kPer);
+      const auto* pc = reinterpret_cast<const ColPiece*>(t_col + q + i * kWave * kPer);
+      if constexpr (NTL) {
+        v[i] = nt_load_object(pv);
+        c[i] = nt_load_object(pc);
+      } else {
+        v[i] = *pv;
+        c[i] = *pc;
+      }
     }
   };
   if (at < ch.slots) load(at);
