@@ -225,26 +225,43 @@ __global__ __launch_bounds__(256) void value_hash_kernel(const unsigned* __restr
   if (threadIdx.x == 0) partial[blockIdx.x] = total;
 }
 
-// Every word of a 16-byte aligned array, four per lane and load: the same sum as value_hash_kernel with runs
-// of 64 words (each word is mixed with its own position, and sums do not mind the order).
-__global__ __launch_bounds__(256) void value_hash_all_kernel(const Int4* __restrict__ quads, int64_t total_quads,
-                                                             unsigned long long* __restrict__ partial) {
+// The same sum over the same words of a 16-byte aligned array, four words per lane and load: sixteen lanes take a run's 64
+// words (ALL: the runs are those 64 words, and a position is not worked out).  Memory-bound; two loads in flight per lane
+// and full occupancy ask for enough, more of them only reach further ahead: 388 MB in 64 us with two, 67 / 70 / 73 with
+// three / four / six, 81 with eight.
+constexpr int kGuardQuads = 2;
+template <bool ALL>
+__global__ __launch_bounds__(256) void value_hash_quads_kernel(const unsigned* __restrict__ words, int64_t total_words,
+                                                               int64_t run_words, unsigned long long* __restrict__ partial) {
   const int64_t stride = (int64_t)gridDim.x * 256;
+  const int64_t lanes = ALL ? (total_words + 3) / 4 : (total_words + run_words - 1) / run_words * (kWave / 4);
+  const unsigned slot_mask = (unsigned)(run_words / kWave) - 1u;
+  const Int4* __restrict__ quads = reinterpret_cast<const Int4*>(words);
   unsigned long long mine = 0;
-  for (int64_t q0 = (int64_t)blockIdx.x * 256 + threadIdx.x; q0 < total_quads; q0 += stride * kGuardUnroll) {
-    Int4 w[kGuardUnroll];
+  for (int64_t q0 = (int64_t)blockIdx.x * 256 + threadIdx.x; q0 < lanes; q0 += stride * kGuardQuads) {
+    Int4 w[kGuardQuads];
+    int64_t idx[kGuardQuads];
 #pragma unroll
-    for (int u = 0; u < kGuardUnroll; ++u) {
+    for (int u = 0; u < kGuardQuads; ++u) {
       const int64_t q = q0 + (int64_t)u * stride;
-      w[u] = nt_load_object(quads + (q < total_quads ? q : q0));
+      int64_t pos = q * 4;
+      if constexpr (!ALL) {
+        const int64_t r = q / (kWave / 4), start = r * run_words;
+        pos = start + (int64_t)((((unsigned)r * 2654435761u) >> 7) & slot_mask) * kWave;
+        if (pos >= total_words) pos = start;  // the last, short run
+        pos += q % (kWave / 4) * 4;
+      }
+      idx[u] = q < lanes ? pos : total_words;
+      w[u] = nt_load_object(quads + (idx[u] + 4 <= total_words ? pos / 4 : 0));  // (there is a first quad)
     }
 #pragma unroll
-    for (int u = 0; u < kGuardUnroll; ++u) {
-      const int64_t q = q0 + (int64_t)u * stride;
-      if (q < total_quads) {
-        const unsigned long long i = (unsigned long long)q * 4;
+    for (int u = 0; u < kGuardQuads; ++u) {
+      const unsigned long long i = (unsigned long long)idx[u];
+      if (idx[u] + 4 <= total_words) {
         mine += mix_word((unsigned)w[u].x, i) + mix_word((unsigned)w[u].y, i + 1) + mix_word((unsigned)w[u].z, i + 2) +
                 mix_word((unsigned)w[u].w, i + 3);
+      } else {  // the array's last words
+        for (int64_t k = idx[u]; k < total_words; ++k) mine += mix_word(words[k], (unsigned long long)k);
       }
     }
   }
@@ -283,10 +300,12 @@ extern "C" int asamd_value_guard(hipStream_t stream, const void* val, size_t nby
   const int64_t total_words = (int64_t)(nbytes / 4);
   const int64_t run_words = (int64_t)((full || nbytes <= ASAMD_GUARD_FULL_BYTES ? (size_t)256 : asamd_value_guard_run(nbytes)) / 4);
   GuardWs* g = (GuardWs*)ws;
-  if (run_words == kWave && total_words % 4 == 0 && ((uintptr_t)val & 15u) == 0)
-    value_hash_all_kernel<<<kGuardBlocks, 256, 0, stream>>>((const Int4*)val, total_words / 4, g->partial);
-  else
+  if (((uintptr_t)val & 15u) == 0 && total_words >= 4) {
+    const auto hash = run_words == kWave ? value_hash_quads_kernel<true> : value_hash_quads_kernel<false>;
+    hash<<<kGuardBlocks, 256, 0, stream>>>((const unsigned*)val, total_words, run_words, g->partial);
+  } else {
     value_hash_kernel<<<kGuardBlocks, 256, 0, stream>>>((const unsigned*)val, total_words, run_words, g->partial);
+  }
   value_verdict_kernel<<<1, 256, 0, stream>>>(g, total_words, (const unsigned long long*)stored);
   return hipGetLastError();
 }

@@ -1,0 +1,58 @@
+"""The fingerprint of a value array against the same sum in numpy: every word (or every word of the sample) counts once,
+whatever the array's length and alignment -- last quads of one to three words, runs cut short, both kernels."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from alsparse_amd import capi, hiprt
+from helpers import announce
+
+pytestmark = pytest.mark.gpu
+
+GUARD_BYTES = 16384 + 64  # per-call scratch; the fingerprint lies behind 2 048 partial sums
+FULL_BYTES = 32 << 20
+
+
+def _fingerprint(words, run):
+    n = words.size
+    r = np.arange((n + run - 1) // run, dtype=np.uint64)
+    slot = ((((r * np.uint64(2654435761)) & np.uint64(0xFFFFFFFF)) >> np.uint64(7)) & np.uint64(run // 64 - 1)) * np.uint64(64)
+    pos = r * np.uint64(run) + slot
+    pos = np.where(pos >= n, r * np.uint64(run), pos)
+    idx = (pos[:, None] + np.arange(64, dtype=np.uint64)[None, :]).reshape(-1)
+    idx = idx[idx < n]
+    w = words[idx.astype(np.int64)]
+    i = idx.astype(np.uint32)  # (positions below 2^32)
+    t = i * np.uint32(0x85EBCA6B)
+    a = (w ^ t) * np.uint32(0x9E3779B1)
+    a ^= a >> np.uint32(15)
+    b = (w + ((t >> np.uint32(7)) | (t << np.uint32(25)))) * np.uint32(0x27D4EB2F)
+    b ^= b >> np.uint32(16)
+    total = int((b.astype(np.uint64) << np.uint64(32) | a.astype(np.uint64)).sum(dtype=np.uint64))
+    return total ^ (n * 0x9E3779B97F4A7C15 & (1 << 64) - 1)
+
+
+@pytest.mark.parametrize("offset", [0, 1, 2, 4], ids=lambda o: "off%d" % o)
+@pytest.mark.parametrize("words,full", [(1, 1), (2, 1), (3, 1), (4, 1), (5, 1), (63, 1), (66, 1), (255, 1), (1 << 20, 1),
+                                        (2048 * 256 * 8 + 7, 1), (FULL_BYTES // 4 + 1, 0), (FULL_BYTES // 4 + 65, 0),
+                                        (5 * (FULL_BYTES // 4) + 3, 0), (5 * (FULL_BYTES // 4) + 3, 1)])
+def test_fingerprint_is_the_sum_over_the_words(gpu, words, full, offset):
+    lib = capi.load()
+    rng = np.random.default_rng(words + offset)
+    host = rng.integers(0, 1 << 32, size=words + offset, dtype=np.uint32)
+    nbytes = words * 4
+    run = 64 if full or nbytes <= FULL_BYTES else int(lib.asamd_value_guard_run(nbytes)) // 4
+    assert (run > 64) == (not full and nbytes >= FULL_BYTES + 256), "a sample"
+    d, ws = hiprt.DeviceArray.from_numpy(host), hiprt.DeviceArray((GUARD_BYTES // 8,), np.uint64)
+    stored = hiprt.DeviceArray.from_numpy(np.array([_fingerprint(host[offset:], run)], dtype=np.uint64))
+    try:
+        announce("fingerprint", words, "full", full, "offset", offset)
+        at = ctypes.c_void_p(d.ptr + 4 * offset)
+        assert lib.asamd_value_guard(None, at, nbytes, full, stored.c_ptr(), ws.c_ptr()) == 0
+        got = ws.to_numpy()
+        assert int(got[2048]) == int(stored.to_numpy()[0])
+        assert got[2049:2050].view(np.int32)[0] == 0, "taken as changed"
+    finally:
+        for x in (d, ws, stored):
+            x.free()
