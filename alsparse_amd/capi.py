@@ -355,11 +355,11 @@ _COMMON = {
     "asamd_tiled_build": [_P, _I, _I, _I, _I, _I, _P, _P, _P, _I, _I, _P],
     "asamd_tiled_free": [_P],
     "asamd_tiled_gather_values": [_P, _P, _P, _P],
-    "asamd_spmv_tiled": [_P, POINTER(asamd_spmv_args), _P, _P, _P, _P],
+    "asamd_spmv_tiled": [_P, POINTER(asamd_spmv_args), _P, _P, _P, _P, _P],
     "asamd_sums_build": [_P, _I, _I, _I, _I, _I, _P, _P, _P, c_int64, _P],
     "asamd_sums_free": [_P],
     "asamd_sums_refresh_values": [_P, _P, _P, _P],
-    "asamd_spmv_sums": [_P, POINTER(asamd_spmv_args), _P, _P],
+    "asamd_spmv_sums": [_P, POINTER(asamd_spmv_args), _P, _P, _P],
     "asamd_hot_build": [_P, _I, _I, _I, _I, _I, _P, _P, _I, _I, _I, _P],
     "asamd_hot_free": [_P],
     "asamd_spmv_hot": [_P, POINTER(asamd_spmv_args), _P, _P, _P, _P, _P],
@@ -374,6 +374,7 @@ _COMMON = {
     "asamd_value_guard_run": [c_size_t],
     "asamd_value_guard": [_P, _P, c_size_t, _I, _P, _P],
     "asamd_value_guard_commit": [_P, _P, _P],
+    "asamd_value_guard_begin": [_P, _P, c_size_t, _I, _P, _P, _P],
     "asamd_gather_values": [_P, _I, _I, _I, _P, _P, _P, _P],
     "asamd_spmv_xlds": [_P, _P, _I],
     "asamd_spmv_xlds_fits": [_I, _I],

@@ -9,6 +9,7 @@
 
 #include "alsparse_amd_kernels.h"
 #include "launch_utils.hpp"
+#include "value_guard.hpp"
 
 using namespace asamd;
 
@@ -126,17 +127,6 @@ __device__ __forceinline__ unsigned long long mix_index(unsigned long long v, un
   return z ^ (z >> 32);
 }
 
-__device__ __forceinline__ unsigned long long block_sum_u64(unsigned long long mine) {
-  __shared__ unsigned long long s_sum[256 / kWave];
-  for (int d = kWave / 2; d > 0; d >>= 1) mine += __shfl_down(mine, d, kWave);
-  if (threadIdx.x % kWave == 0) s_sum[threadIdx.x / kWave] = mine;
-  __syncthreads();
-  unsigned long long total = 0;
-  if (threadIdx.x == 0)
-    for (int w = 0; w < 256 / kWave; ++w) total += s_sum[w];
-  return total;  // valid in thread 0
-}
-
 __global__ __launch_bounds__(256) void index_hash_kernel(int64_t n, const int* __restrict__ a, unsigned long long salt,
                                                          unsigned long long* __restrict__ hash) {
   unsigned long long mine = 0;
@@ -172,16 +162,7 @@ extern "C" int asamd_csr_structure_hash(hipStream_t stream, int32_t m, int32_t n
 // additions, so the order does not matter and equal arrays give equal words.  run_words == 64 reads
 // everything.
 // ---------------------------------------------------------------------------
-constexpr int kGuardBlocks = 2048;
 constexpr int kGuardUnroll = 8;
-static_assert(ASAMD_GUARD_WS_BYTES >= kGuardBlocks * 8 + 16, "guard scratch holds the partial sums, the word and the flag");
-
-struct GuardWs {
-  unsigned long long partial[kGuardBlocks];
-  unsigned long long fp;
-  int flag;
-};
-static_assert(offsetof(GuardWs, flag) == 8 * kGuardBlocks + 8, "ASAMD_GUARD_FLAG points at the flag");
 
 // Three 32-bit multiplications per word (they run at a quarter of the rate of an addition, and hashing a
 // whole array must stay a memory-bound pass).  For a fixed position the low half is a bijection of the word, so
@@ -269,21 +250,16 @@ __global__ __launch_bounds__(256) void value_hash_quads_kernel(const unsigned* _
   if (threadIdx.x == 0) partial[blockIdx.x] = total;
 }
 
-__global__ __launch_bounds__(256) void value_verdict_kernel(GuardWs* __restrict__ ws, int64_t total_words,
+__global__ __launch_bounds__(256) void value_verdict_kernel(GuardWs* __restrict__ ws, unsigned long long salt,
                                                             const unsigned long long* __restrict__ stored) {
-  unsigned long long mine = 0;
-  for (int i = threadIdx.x; i < kGuardBlocks; i += 256) mine += ws->partial[i];
-  unsigned long long fp = block_sum_u64(mine);
+  const unsigned long long fp = guard_fingerprint(ws, salt);
   if (threadIdx.x == 0) {
-    fp ^= (unsigned long long)total_words * 0x9E3779B97F4A7C15ull;
     ws->fp = fp;
     ws->flag = (!stored || *stored != fp) ? 1 : 0;
   }
 }
 
-__global__ void value_commit_kernel(const GuardWs* __restrict__ ws, unsigned long long* __restrict__ stored) {
-  if (ws->flag) *stored = ws->fp;
-}
+__global__ void value_commit_kernel(GuardCommit commit) { guard_commit(commit); }
 
 extern "C" size_t asamd_value_guard_run(size_t nbytes) {
   // 256 bytes of every run, 32 MiB in all at the most: the run is the smallest power of two (in 256-byte
@@ -293,8 +269,7 @@ extern "C" size_t asamd_value_guard_run(size_t nbytes) {
   return run;
 }
 
-extern "C" int asamd_value_guard(hipStream_t stream, const void* val, size_t nbytes, int32_t full,
-                                 const uint64_t* stored, void* ws) {
+static int hash_values(hipStream_t stream, const void* val, size_t nbytes, int32_t full, void* ws) {
   if (!val || !ws || ((uintptr_t)ws & 7u) || ((uintptr_t)val & 3u) || (nbytes & 3u) || nbytes == 0)
     return hipErrorInvalidValue;
   const int64_t total_words = (int64_t)(nbytes / 4);
@@ -306,8 +281,23 @@ extern "C" int asamd_value_guard(hipStream_t stream, const void* val, size_t nby
   } else {
     value_hash_kernel<<<kGuardBlocks, 256, 0, stream>>>((const unsigned*)val, total_words, run_words, g->partial);
   }
-  value_verdict_kernel<<<1, 256, 0, stream>>>(g, total_words, (const unsigned long long*)stored);
   return hipGetLastError();
+}
+
+extern "C" int asamd_value_guard(hipStream_t stream, const void* val, size_t nbytes, int32_t full,
+                                 const uint64_t* stored, void* ws) {
+  const int e = hash_values(stream, val, nbytes, full, ws);
+  if (e != hipSuccess) return e;
+  value_verdict_kernel<<<1, 256, 0, stream>>>((GuardWs*)ws, guard_salt((int64_t)(nbytes / 4)),
+                                              (const unsigned long long*)stored);
+  return hipGetLastError();
+}
+
+extern "C" int asamd_value_guard_begin(hipStream_t stream, const void* val, size_t nbytes, int32_t full, uint64_t* stored,
+                                       void* ws, asamd_value_check* check) {
+  if (!stored || !check) return hipErrorInvalidValue;
+  *check = asamd_value_check{ws, stored, (int64_t)(nbytes / 4), 0};
+  return hash_values(stream, val, nbytes, full, ws);
 }
 
 __global__ void guard_any_kernel(const GuardWs* __restrict__ a, const GuardWs* __restrict__ b, int* __restrict__ out) {
@@ -322,7 +312,7 @@ extern "C" int asamd_value_guard_any(hipStream_t stream, const void* ws_a, const
 
 extern "C" int asamd_value_guard_commit(hipStream_t stream, const void* ws, uint64_t* stored) {
   if (!ws || !stored) return hipErrorInvalidValue;
-  value_commit_kernel<<<1, 1, 0, stream>>>((const GuardWs*)ws, (unsigned long long*)stored);
+  value_commit_kernel<<<1, 1, 0, stream>>>(GuardCommit{(const GuardWs*)ws, (unsigned long long*)stored});
   return hipGetLastError();
 }
 

@@ -40,7 +40,7 @@ static std::vector<int> cut_blocks(const int* off, int groups, int max_groups, i
 }
 
 template <typename T>
-static void launch_gather_tiles(hipStream_t s, const asamd_tiled_layout* L, const void* val, const int32_t* gate) {
+static void launch_gather_tiles(hipStream_t s, const asamd_tiled_layout* L, const void* val, const GuardGate& gate) {
   // eight tiles to a wave at a time, eight workgroups abreast (one per XCD), as many as the chip holds at once
   const int64_t per_xcd = ((int64_t)(L->row_blocks + 7) / 8) * ((L->col_blocks + 7) / 8);
   int64_t grid = (per_xcd + 3) / 4 * 8;
@@ -248,7 +248,7 @@ static hipError_t build_tiled(hipStream_t stream, asamd_tiled_layout* L, const i
                                                                                 d_tile_ptr);
     if constexpr (kPayloadSort) {
       L->tile_ptr = d_tile_ptr;  // stays with the layout: the values are gathered tile by tile, now and later
-      launch_gather_tiles<T>(stream, L, val, nullptr);
+      launch_gather_tiles<T>(stream, L, val, guard_gate(nullptr));
     }
     // Entries in tiles of 65..128 entries: if they are few, phase 2 runs in its one-entry-per-lane form
     // (twice the tiles in flight) and leaves those tiles to phase 3.
@@ -434,7 +434,7 @@ extern "C" void asamd_tiled_free(asamd_tiled_layout* L) {
 // (the tiles too long for phase 2) and its ordered finish.  The layout holds zero-based local indices and
 // its own values.
 extern "C" int asamd_spmv_tiled(hipStream_t s, const asamd_spmv_args* a, const asamd_tiled_layout* L, void* products,
-                                void* long_scratch, const int32_t* skip) {
+                                void* long_scratch, const int32_t* skip, const asamd_value_check* commit) {
   if (!a || !L || !L->tval || !products || !a->alpha || !a->beta || !a->x || !a->y) return hipErrorInvalidValue;
   if (a->dtype != L->dtype || a->m != L->m || a->n != L->n || a->nnz != L->nnz) return hipErrorInvalidValue;
   if (L->n_long_finish > 0 && !long_scratch) return hipErrorInvalidValue;
@@ -459,11 +459,11 @@ extern "C" int asamd_spmv_tiled(hipStream_t s, const asamd_spmv_args* a, const a
     if (L->entries_per_lane == 1)
       tiled_reduce_kernel<T, 1, false><<<red_grid, TileDims<T>::red_threads, TileDims<T>::red_lds_bytes, s>>>(
           L->row_blocks, L->col_blocks, TileDims<T>::rows, L->row_block_start, nullptr, (const TileRange*)L->ranges,
-          L->trow, prod, alpha, beta, y, skip);
+          L->trow, prod, alpha, beta, y, skip, guard_commit_of(commit));
     else
       tiled_reduce_kernel<T, 2, false><<<red_grid, TileDims<T>::red_threads, TileDims<T>::red_lds_bytes, s>>>(
           L->row_blocks, L->col_blocks, TileDims<T>::rows, L->row_block_start, nullptr, (const TileRange*)L->ranges,
-          L->trow, prod, alpha, beta, y, skip);
+          L->trow, prod, alpha, beta, y, skip, guard_commit_of(commit));
     if (L->n_long_chunks > 0) {
       const int waves = kLongThreads / kWave, narrow = L->n_long_narrow, wide = L->n_long_chunks - narrow;
       const LongBlock* list = (const LongBlock*)L->long_list;
@@ -483,21 +483,21 @@ extern "C" int asamd_spmv_tiled(hipStream_t s, const asamd_spmv_args* a, const a
 }
 
 extern "C" int asamd_tiled_gather_values(hipStream_t s, const asamd_tiled_layout* L, const void* val,
-                                         const int32_t* gate) {
+                                         const asamd_value_check* check) {
   if (!L || !L->tval || !L->tperm || !val) return hipErrorInvalidValue;
   if (L->nnz == 0) return hipSuccess;
-  if (!L->tile_ptr) return asamd_gather_values(s, L->dtype, 0, L->nnz, L->tperm, val, L->tval, gate);
+  if (!L->tile_ptr) return asamd_gather_values(s, L->dtype, 0, L->nnz, L->tperm, val, L->tval, check);
   return by_dtype(L->dtype, [&](auto* tag) -> int {
     using T = std::remove_pointer_t<decltype(tag)>;
     if ((uintptr_t)val % alignof(T)) return hipErrorInvalidValue;
-    launch_gather_tiles<T>(s, L, val, gate);
+    launch_gather_tiles<T>(s, L, val, guard_gate(check));
     return hipGetLastError();
   });
 }
 
 // out[q] = val[perm[q]]: the values of a re-ordered copy taken afresh from the caller's array
 extern "C" int asamd_gather_values(hipStream_t s, int32_t dtype, int32_t conj, int32_t nnz, const uint32_t* perm,
-                                   const void* val, void* out, const int32_t* gate) {
+                                   const void* val, void* out, const asamd_value_check* check) {
   if (!perm || !val || !out || nnz < 0) return hipErrorInvalidValue;
   if (nnz == 0) return hipSuccess;
   return by_dtype(dtype, [&](auto* tag) -> int {
@@ -505,7 +505,10 @@ extern "C" int asamd_gather_values(hipStream_t s, int32_t dtype, int32_t conj, i
     if (((uintptr_t)val | (uintptr_t)out) % alignof(T)) return hipErrorInvalidValue;
     if (conj && kIsReal<T>) return hipErrorInvalidValue;
     int64_t grid = ((int64_t)nnz + 256 * 8 - 1) / (256 * 8);
-    if (grid > 256 * 32) grid = 256 * 32;
+    // (a check that is not settled is worked out by every workgroup: no more of them than the chip holds)
+    const int64_t most = check && !check->settled ? 256 * 8 : 256 * 32;
+    if (grid > most) grid = most;
+    const GuardGate gate = guard_gate(check);
     if constexpr (!kIsReal<T>) {
       if (conj) {
         gather_values_kernel<T, true><<<(unsigned)grid, 256, 0, s>>>(nnz, perm, (const T*)val, (T*)out, gate);

@@ -183,8 +183,8 @@ __global__ __launch_bounds__(256) void sums_spans_kernel(int spans, int col_bloc
 template <typename T>
 __global__ __launch_bounds__(256) void sums_values_kernel(int spans, const int* __restrict__ order,
                                                           const unsigned* __restrict__ t_perm, const T* __restrict__ val,
-                                                          T* __restrict__ t_val, const int* __restrict__ gate) {
-  if (gate && *gate == 0) return;
+                                                          T* __restrict__ t_val, GuardGate gate) {
+  if (!guard_open(gate)) return;
   constexpr int kSpan = SumsDims<T>::span, kU = kSpan / 256;
   static_assert(kSpan % 256 == 0, "whole workgroups");
   const int xcd = blockIdx.x % kXcds, per = (spans + kXcds - 1) / kXcds;

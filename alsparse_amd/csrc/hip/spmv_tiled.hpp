@@ -47,6 +47,7 @@
 #pragma once
 
 #include "device_utils.hpp"
+#include "value_guard.hpp"
 
 namespace asamd {
 
@@ -202,13 +203,13 @@ static __global__ __launch_bounds__(256) void tile_unpack_kernel(int nnz, const 
 }
 
 // out[q] = val[perm[q]] (CONJ: conjugated): the values of a re-ordered copy, taken afresh from the
-// caller's array.  Eight gathers in flight per lane.  gate: null, or a flag left by the value guard --
-// zero means that the values have not changed, and the kernel returns at once.
+// caller's array.  Eight gathers in flight per lane.  gate: what the value guard found -- where the values have not
+// changed, the kernel returns at once.
 template <typename T, bool CONJ>
 __global__ __launch_bounds__(256) void gather_values_kernel(int nnz, const unsigned* __restrict__ perm,
                                                             const T* __restrict__ val, T* __restrict__ out,
-                                                            const int* __restrict__ gate) {
-  if (gate && *gate == 0) return;
+                                                            GuardGate gate) {
+  if (!guard_open(gate)) return;
   constexpr int kU = 8;
   const int64_t stride = (int64_t)gridDim.x * 256;
   int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -236,8 +237,8 @@ template <typename T, bool CONJ>
 __global__ __launch_bounds__(256) void gather_values_tiles_kernel(const unsigned* __restrict__ perm,
                                                                   const T* __restrict__ val, T* __restrict__ out,
                                                                   const int* __restrict__ tile_ptr, int col_blocks,
-                                                                  int row_blocks, const int* __restrict__ gate) {
-  if (gate && *gate == 0) return;
+                                                                  int row_blocks, GuardGate gate) {
+  if (!guard_open(gate)) return;
   constexpr int kU = 8;
   const int lane = threadIdx.x % kWave;
   const int xcd = blockIdx.x % 8;
@@ -521,12 +522,14 @@ __device__ __forceinline__ void add_rows(T* acc, int r, T v, bool valid_arg) {
 // 1 takes tiles of up to kWave entries with twice as many in flight (for the same number of outstanding
 // loads: where tiles are short -- wide values make narrow column blocks -- the loads of the second half
 // would all come back empty, and the bytes in flight, which bound the speed, would halve).
+// commit: the fingerprint of the values that the copy was refreshed from in front of phase 1.
 // DISTINCT: no tile holds a row twice (row-sum tiles, spmv_sums.hpp), so nothing has to be combined first.
 template <typename T, int H, bool DISTINCT>
 __global__ __launch_bounds__(TileDims<T>::red_threads) void tiled_reduce_kernel(
     int row_blocks, int col_blocks, int rows_cap, const int* __restrict__ row_block_start,
     const int* __restrict__ run_ptr, const TileRange* __restrict__ ranges, const unsigned short* __restrict__ t_row,
-    const T* __restrict__ prod, T alpha, T beta, T* __restrict__ y, const int* __restrict__ skip) {
+    const T* __restrict__ prod, T alpha, T beta, T* __restrict__ y, const int* __restrict__ skip, GuardCommit commit) {
+  guard_commit(commit);
   if (skip && *skip) return;  // the caller's guard found that the layout no longer describes the matrix
   extern __shared__ __align__(16) unsigned char smem[];
   T* s_acc = reinterpret_cast<T*>(smem);

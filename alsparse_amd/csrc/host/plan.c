@@ -598,7 +598,9 @@ static int run_merge(hipStream_t s, const asamd_csr_plan *p, const asamd_spmv_ar
   return asamd_spmv_merge(s, a, p->merge_ipt, block_row, carry_row, carry_val, head_val);
 }
 
-static int run_algo(hipStream_t s, const asamd_csr_plan *p, int algo, const asamd_spmv_args *a, ws_cursor ws) {
+/* commit: NULL, or the check of the values that the tiled copy's multiply records (no other family takes one) */
+static int run_algo(hipStream_t s, const asamd_csr_plan *p, int algo, const asamd_spmv_args *a, ws_cursor ws,
+                    const asamd_value_check *commit) {
   const asamd_csr_stats *st = &p->st;
   const size_t vs = (size_t)p->val_size;
   switch (algo) {
@@ -609,7 +611,7 @@ static int run_algo(hipStream_t s, const asamd_csr_plan *p, int algo, const asam
       void *prod = ws_take(&ws, (size_t)st->nnz * vs);
       void *lscr = p->tiled.long_scratch_elems > 0 ? ws_take(&ws, (size_t)p->tiled.long_scratch_elems * vs) : NULL;
       if (!prod || (p->tiled.long_scratch_elems > 0 && !lscr)) return -1;
-      return asamd_spmv_tiled(s, a, &p->tiled, prod, lscr, NULL);
+      return asamd_spmv_tiled(s, a, &p->tiled, prod, lscr, NULL, commit);
     }
     case ASAMD_SPMV_ROWCONST:
       return asamd_spmv_rowconst(s, a, st->const_len);
@@ -660,13 +662,15 @@ static int run_algo(hipStream_t s, const asamd_csr_plan *p, int algo, const asam
   }
 }
 
-/* Gathers the plan's tiled / ELL / slice-by-slice copy again from val; gate: NULL, or the value guard's flag. */
+/* Gathers the plan's tiled / ELL / slice-by-slice copy again from val; check: NULL, or a settled check of the values (the
+ * tiled copy alone also takes one that is not). */
 static hipError_t refresh_main(hipStream_t s, asamd_csr_plan *p, const int32_t *rp, const int32_t *ci, const void *val,
-                               const int32_t *gate) {
+                               const asamd_value_check *check) {
   const asamd_csr_stats *st = &p->st;
+  const int32_t *gate = check ? ASAMD_GUARD_FLAG(check->ws) : NULL;
   hipError_t e = hipSuccess;
   if (st->tiled_built)
-    e = (hipError_t)asamd_tiled_gather_values(s, &p->tiled, val, gate);
+    e = (hipError_t)asamd_tiled_gather_values(s, &p->tiled, val, check);
   if (e == hipSuccess && st->ell_built)
     e = (hipError_t)asamd_csr2ell_gated(s, p->val_size, st->m, val, rp, ci, st->base, 0, st->ell_width, p->d_eval,
                                         p->d_ecol, gate);
@@ -674,12 +678,13 @@ static hipError_t refresh_main(hipStream_t s, asamd_csr_plan *p, const int32_t *
   return e;
 }
 
-/* ... and one transposed copy with everything its own analysis keeps */
-static hipError_t refresh_trans(hipStream_t s, asamd_csr_plan *p, int which, const void *val, const int32_t *gate) {
+/* ... and one transposed copy with everything its own analysis keeps; settles the check */
+static hipError_t refresh_trans(hipStream_t s, asamd_csr_plan *p, int which, const void *val, asamd_value_check *check) {
   asamd_trans_copy *t = &p->tr[which];
-  hipError_t e = (hipError_t)asamd_gather_values(s, p->dtype, which == 1, p->st.nnz, t->t.perm, val, t->t.val, gate);
-  if (e == hipSuccess) e = refresh_main(s, t->plan, t->t.row_ptr, t->t.col_ind, t->t.val, gate);
-  if (e == hipSuccess && t->plan->sums.tval) e = (hipError_t)asamd_sums_refresh_values(s, &t->plan->sums, t->t.val, gate);
+  hipError_t e = (hipError_t)asamd_gather_values(s, p->dtype, which == 1, p->st.nnz, t->t.perm, val, t->t.val, check);
+  if (check) check->settled = 1;
+  if (e == hipSuccess) e = refresh_main(s, t->plan, t->t.row_ptr, t->t.col_ind, t->t.val, check);
+  if (e == hipSuccess && t->plan->sums.tval) e = (hipError_t)asamd_sums_refresh_values(s, &t->plan->sums, t->t.val, check);
   return e;
 }
 
@@ -690,25 +695,31 @@ static int sums_check_all(const asamd_csr_plan *p) { return p->st.value_check ==
 
 /* The row-sum tiles' multiply, or -1 where they do not serve this call: none laid out, a family set from outside, other
  * values than those they hold, no room for their scratch or for the check of their values. */
-static int csrmv_sums(hipStream_t s, asamd_csr_plan *p, const asamd_spmv_args *a, ws_cursor ws, int guard) {
+static int csrmv_sums(hipStream_t s, asamd_csr_plan *p, const asamd_spmv_args *a, ws_cursor ws, int guard,
+                      const asamd_value_check *commit) {
   const asamd_csr_stats *st = &p->st;
   if (!p->sums.tval || p->pinned || a->val != p->copy_val_src) return -1;
   void *g = guard && st->value_check ? ws_take(&ws, ASAMD_GUARD_WS_BYTES) : NULL;
   void *sums = ws_take(&ws, sums_scratch(p));
   if (!sums || (guard && st->value_check && !g)) return -1;
+  asamd_value_check check;
   if (g) {
-    int e = asamd_value_guard(s, a->val, (size_t)st->nnz * (size_t)p->val_size, sums_check_all(p), p->d_fp + FP_SUMS, g);
-    if (e == hipSuccess) e = asamd_sums_refresh_values(s, &p->sums, a->val, ASAMD_GUARD_FLAG(g));
-    if (e == hipSuccess) e = asamd_value_guard_commit(s, g, p->d_fp + FP_SUMS);
+    int e = asamd_value_guard_begin(s, a->val, (size_t)st->nnz * (size_t)p->val_size, sums_check_all(p), p->d_fp + FP_SUMS, g,
+                                    &check);
+    if (e == hipSuccess) e = asamd_sums_refresh_values(s, &p->sums, a->val, &check);
     if (e != hipSuccess) return e;
+    commit = &check;
   }
-  return asamd_spmv_sums(s, a, &p->sums, sums);
+  return asamd_spmv_sums(s, a, &p->sums, sums, commit);
 }
 
-static int csrmv_inner(hipStream_t s, asamd_csr_plan *p, const asamd_spmv_args *a, ws_cursor ws, int guard) {
+/* commit: NULL, or a check whose copies have been refreshed (guard == 0): recorded by the multiply, or in front of it */
+static int csrmv_inner(hipStream_t s, asamd_csr_plan *p, const asamd_spmv_args *a, ws_cursor ws, int guard,
+                       const asamd_value_check *commit) {
   const asamd_csr_stats *st = &p->st;
-  const int summed = csrmv_sums(s, p, a, ws, guard);
+  const int summed = csrmv_sums(s, p, a, ws, guard, commit);
   if (summed != -1) return summed;
+  asamd_value_check check;
   int algo = st->algo;
   /* The tiled, ELL and slice-by-slice copies hold the values of the array they were built from.  A multiply that
    * brings another value array (same structure, new numbers) must not see the old ones: it runs the kernel that
@@ -725,15 +736,35 @@ static int csrmv_inner(hipStream_t s, asamd_csr_plan *p, const asamd_spmv_args *
       /* no room to check the copy: do not use it */
       algo = algo == ASAMD_SPMV_XLDS ? ALGO_XLDS_IN_PLACE : settle_algo(p, p->struct_algo, a->val, a->col_ind);
     } else {
-      int e = asamd_value_guard(s, a->val, (size_t)st->nnz * (size_t)p->val_size, st->value_check == 2, p->d_fp, g);
-      if (e == hipSuccess) e = (int)refresh_main(s, p, a->row_ptr, a->col_ind, a->val, ASAMD_GUARD_FLAG(g));
-      if (e == hipSuccess) e = asamd_value_guard_commit(s, g, p->d_fp);
+      const size_t bytes = (size_t)st->nnz * (size_t)p->val_size;
+      int e;
+      if (algo == ASAMD_SPMV_TILED && !st->ell_built && !p->xlds.val) {
+        /* nothing but the tiled copy: its gather finds the verdict itself, its multiply records the fingerprint */
+        e = asamd_value_guard_begin(s, a->val, bytes, st->value_check == 2, p->d_fp, g, &check);
+        commit = &check;
+        if (e == hipSuccess) e = (int)refresh_main(s, p, a->row_ptr, a->col_ind, a->val, &check);
+      } else {
+        check = (asamd_value_check){g, p->d_fp, (int64_t)(bytes / 4), 1};
+        e = asamd_value_guard(s, a->val, bytes, st->value_check == 2, p->d_fp, g);
+        if (e == hipSuccess) e = (int)refresh_main(s, p, a->row_ptr, a->col_ind, a->val, &check);
+        if (e == hipSuccess) e = asamd_value_guard_commit(s, g, p->d_fp);
+      }
       if (e != hipSuccess) return e;
     }
   }
-  int e = run_algo(s, p, algo, a, ws);
+  int e = hipSuccess;
+  if (commit && algo != ASAMD_SPMV_TILED) {
+    e = asamd_value_guard_commit(s, commit->ws, commit->stored);
+    if (e != hipSuccess) return e;
+    commit = NULL;
+  }
+  e = run_algo(s, p, algo, a, ws, commit);
   if (e == -1) {
     /* the workspace does not hold this family's scratch: a lane group per row needs none */
+    if (commit) {
+      e = asamd_value_guard_commit(s, commit->ws, commit->stored);
+      if (e != hipSuccess) return e;
+    }
     e = asamd_spmv_vector(s, a, p->auto_width);
   }
   return e;
@@ -793,7 +824,7 @@ int asamd_csr_plan_csrmv(hipStream_t s, asamd_csr_plan *p, int32_t op, const voi
   ws_cursor ws = ws_open(workspace, workspace_bytes);
   asamd_spmv_args a;
   fill_args(&a, p, alpha, val, rp, ci, x, beta, y);
-  if (op == 0) return csrmv_inner(s, p, &a, ws, 1);
+  if (op == 0) return csrmv_inner(s, p, &a, ws, 1, NULL);
 
   const int which = op - 1;
   asamd_trans_copy *t = &p->tr[which];
@@ -823,22 +854,24 @@ int asamd_csr_plan_csrmv(hipStream_t s, asamd_csr_plan *p, int32_t op, const voi
   /* the copy holds the values it was gathered from: another value array takes the scatter route below */
   if (t->plan && val == t->val_src) {
     int usable = 1;
+    asamd_value_check check;
+    const asamd_value_check *commit = NULL;
     if (st->value_check) {
       void *g = ws_take(&ws, ASAMD_GUARD_WS_BYTES);
       if (!g) {
         usable = 0; /* no room to check the copy: do not use it */
       } else {
-        int e = asamd_value_guard(s, val, (size_t)st->nnz * (size_t)p->val_size, st->value_check == 2,
-                                  p->d_fp + 1 + which, g);
-        if (e == hipSuccess) e = (int)refresh_trans(s, p, which, val, ASAMD_GUARD_FLAG(g));
-        if (e == hipSuccess) e = asamd_value_guard_commit(s, g, p->d_fp + 1 + which);
+        int e = asamd_value_guard_begin(s, val, (size_t)st->nnz * (size_t)p->val_size, st->value_check == 2,
+                                        p->d_fp + 1 + which, g, &check);
+        if (e == hipSuccess) e = (int)refresh_trans(s, p, which, val, &check);
         if (e != hipSuccess) return e;
+        commit = &check;
       }
     }
     if (usable) {
       asamd_spmv_args at;
       fill_args(&at, t->plan, alpha, t->t.val, t->t.row_ptr, t->t.col_ind, x, beta, y);
-      return csrmv_inner(s, t->plan, &at, ws, 0);
+      return csrmv_inner(s, t->plan, &at, ws, 0, commit);
     }
   }
   if (p->trans_route != TRANS_SCATTER && env_int("ALSPARSE_AMD_XLDS", 1) > 0) {
@@ -901,13 +934,14 @@ int asamd_csr_plan_csrmv_watched(hipStream_t s, asamd_csr_plan *p, const void *a
   if (e == hipSuccess) e = asamd_value_guard(s, ci, (size_t)st->nnz * 4, 1, watch + 1, g_ci);
   if (e == hipSuccess) e = asamd_value_guard_any(s, g_rp, g_ci, skip);
   if (e == hipSuccess) e = asamd_value_guard(s, val, (size_t)st->nnz * vs, 1, p->d_fp, g_val);
-  if (e == hipSuccess) e = (int)refresh_main(s, p, rp, ci, val, ASAMD_GUARD_FLAG(g_val));
+  const asamd_value_check check = {g_val, p->d_fp, (int64_t)((size_t)st->nnz * vs / 4), 1};
+  if (e == hipSuccess) e = (int)refresh_main(s, p, rp, ci, val, &check);
   if (e == hipSuccess) e = asamd_value_guard_commit(s, g_val, p->d_fp);
   asamd_spmv_args a;
   fill_args(&a, p, alpha, val, rp, ci, x, beta, y);
   /* the layout's kernels, which return at once if the structure has changed, and the stand-in on the caller's
    * arrays, which returns at once if it has not */
-  if (e == hipSuccess) e = asamd_spmv_tiled(s, &a, &p->tiled, prod, lscr, skip);
+  if (e == hipSuccess) e = asamd_spmv_tiled(s, &a, &p->tiled, prod, lscr, skip, NULL);
   if (e == hipSuccess) e = asamd_spmv_vector_if(s, &a, p->auto_width, skip);
   if (changed) *changed = skip;
   return e;
@@ -991,7 +1025,7 @@ static void time_algo(tune_ctx *t, int cand) {
   int reps = 3;
   for (int rep = 0; rep < reps && t->err == hipSuccess; ++rep) {
     t->err = hipEventRecord(t->e0, t->stream);
-    if (t->err == hipSuccess) t->err = (hipError_t)csrmv_inner(t->stream, p, &a, ws_open(t->ws, t->ws_bytes), 0);
+    if (t->err == hipSuccess) t->err = (hipError_t)csrmv_inner(t->stream, p, &a, ws_open(t->ws, t->ws_bytes), 0, NULL);
     if (t->err == hipSuccess) t->err = hipEventRecord(t->e1, t->stream);
     if (t->err == hipSuccess) t->err = hipEventSynchronize(t->e1);
     float ms = 0.f;

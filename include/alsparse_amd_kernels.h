@@ -220,6 +220,16 @@ int asamd_spmv_trans_slices(hipStream_t stream, const asamd_spmv_args *a, int32_
 /* ... for a matrix that may have long runs of empty rows */
 int asamd_spmv_trans_slices_gaps(hipStream_t stream, const asamd_spmv_args *a, int32_t conj, void *partials);
 
+#define ASAMD_GUARD_WS_BYTES (16384 + 64)
+/* A check of the values under a copy (asamd_value_guard_begin): the guard's scratch, the recorded fingerprint, the array's
+ * 4-byte words; settled: the verdict is in the scratch, otherwise only what it is worked out from. */
+typedef struct {
+  void *ws;
+  uint64_t *stored;
+  int64_t words;
+  int32_t settled;
+} asamd_value_check;
+
 /* ---- re-ordered copies of a CSR matrix ("layouts") and the kernels that multiply with them ------
  * A layout is a plain record of device pointers and counts, filled by its *_build call (which
  * allocates, launches the layout kernels on `stream` and synchronises it) and released by *_free.
@@ -254,14 +264,15 @@ int asamd_tiled_build(hipStream_t stream, int32_t dtype, int32_t m, int32_t n, i
 void asamd_tiled_free(asamd_tiled_layout *layout);
 /* layout->tval[q] = val[layout->tperm[q]] for every slot, the tiles taken row block by row block (each XCD its
  * own row blocks), so that the stretch of val a row block's tiles pick their values from is fetched from memory
- * once; gate as for asamd_gather_values */
+ * once; check as for asamd_gather_values */
 int asamd_tiled_gather_values(hipStream_t stream, const asamd_tiled_layout *layout, const void *val,
-                              const int32_t *gate);
+                              const asamd_value_check *check);
 /* y = alpha*A*x + beta*y from the layout (a->val, a->row_ptr, a->col_ind are not read).  skip: NULL, or a
  * device word; when it is non-zero the kernels that write y return at once (a guard found that the layout no
- * longer describes the caller's matrix, and asamd_spmv_vector_if on the same word computes y instead) */
+ * longer describes the caller's matrix, and asamd_spmv_vector_if on the same word computes y instead).
+ * commit: NULL, or a settled check whose fingerprint the second phase records */
 int asamd_spmv_tiled(hipStream_t stream, const asamd_spmv_args *a, const asamd_tiled_layout *layout,
-                     void *products, void *long_scratch, const int32_t *skip);
+                     void *products, void *long_scratch, const int32_t *skip, const asamd_value_check *commit);
 
 /* The tiled pair for rows that meet a column block more than once (long rows, power-law graphs): phase 1 adds up what a
  * row has in a column block and writes one value for it.  Holds the values (tval) and the CSR position of every slot
@@ -286,10 +297,12 @@ int asamd_sums_build(hipStream_t stream, int32_t dtype, int32_t m, int32_t n, in
                      const int32_t *row_ptr, const int32_t *col_ind, const void *val, int64_t most_sums,
                      asamd_sums_layout *out);
 void asamd_sums_free(asamd_sums_layout *layout);
-/* the values taken afresh from val; gate as for asamd_gather_values */
-int asamd_sums_refresh_values(hipStream_t stream, const asamd_sums_layout *layout, const void *val, const int32_t *gate);
-/* y = alpha*A*x + beta*y from the layout (a->val, a->row_ptr, a->col_ind are not read) */
-int asamd_spmv_sums(hipStream_t stream, const asamd_spmv_args *a, const asamd_sums_layout *layout, void *sums);
+/* the values taken afresh from val; check as for asamd_gather_values */
+int asamd_sums_refresh_values(hipStream_t stream, const asamd_sums_layout *layout, const void *val,
+                              const asamd_value_check *check);
+/* y = alpha*A*x + beta*y from the layout (a->val, a->row_ptr, a->col_ind are not read); commit as for asamd_spmv_tiled */
+int asamd_spmv_sums(hipStream_t stream, const asamd_spmv_args *a, const asamd_sums_layout *layout, void *sums,
+                    const asamd_value_check *commit);
 
 /* Hot-column merge-path for power-law columns: the column stream rewritten as ranks of the popular
  * columns (pcol), whose x sits in LDS (the cols_lds most popular) or in a compact front (cols_front).
@@ -380,26 +393,29 @@ int asamd_csr_locality_probe(hipStream_t stream, int32_t nnz, int32_t base, int3
  *                          full != 0, otherwise 256 bytes at a varying position of every run of
  *                          asamd_value_guard_run(nbytes) bytes, 32 MiB in all), compares with the word
  *                          at `stored` and leaves the verdict in ws: a flag and the new fingerprint;
- *   gated kernels          (asamd_gather_values, asamd_csr2ell_gated) take the flag's address and return
- *                          at once when it is 0;
+ *   gated kernels          (asamd_gather_values, asamd_csr2ell_gated) take a check, or the flag's address, and
+ *                          return at once when the values have not changed;
  *   asamd_value_guard_commit   stores the new fingerprint at `stored` if the flag is set -- AFTER the
  *                          gated kernels in stream order, so that another stream that finds the stored
  *                          word up to date also finds the copies refreshed.
  * stored == NULL in asamd_value_guard sets the flag whatever the values are (first fingerprint).
  * ws: ASAMD_GUARD_WS_BYTES of per-call device scratch, 8-byte aligned. */
-#define ASAMD_GUARD_WS_BYTES (16384 + 64)
 #define ASAMD_GUARD_FULL_BYTES ((size_t)32 << 20)
 #define ASAMD_GUARD_FLAG(ws) ((const int32_t *)((const char *)(ws) + 16384 + 8))
 size_t asamd_value_guard_run(size_t nbytes);
 int asamd_value_guard(hipStream_t stream, const void *val, size_t nbytes, int32_t full, const uint64_t *stored,
                       void *ws);
 int asamd_value_guard_commit(hipStream_t stream, const void *ws, uint64_t *stored);
+/* The same in two launches less: the fingerprint's partial sums, of which the first refreshing kernel works out the verdict
+ * itself (and leaves it in ws: `settled` for any other behind it), and which the multiply records (`commit`). */
+int asamd_value_guard_begin(hipStream_t stream, const void *val, size_t nbytes, int32_t full, uint64_t *stored, void *ws,
+                            asamd_value_check *check);
 /* *out = 1 if either of two guards' flags is set, else 0 (the guard works on any array of 4-byte words: the
  * structure arrays of a matrix that nobody promised to leave alone are watched with it too) */
 int asamd_value_guard_any(hipStream_t stream, const void *ws_a, const void *ws_b, int32_t *out);
-/* out[q] = val[perm[q]] (conj != 0: conjugated) for q < nnz; gate: NULL, or a device flag (0 = do nothing) */
+/* out[q] = val[perm[q]] (conj != 0: conjugated) for q < nnz; check: NULL, or a check (unchanged values: does nothing) */
 int asamd_gather_values(hipStream_t stream, int32_t dtype, int32_t conj, int32_t nnz, const uint32_t *perm,
-                        const void *val, void *out, const int32_t *gate);
+                        const void *val, void *out, const asamd_value_check *check);
 
 /* y = alpha*op(A)*x + beta*y without any analysis, in the traversal of the reference's plain
  * kernels: op = 0 one lane per row summing its entries in storage order
