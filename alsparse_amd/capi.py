@@ -153,7 +153,7 @@ class asamd_xlds_layout(Structure):  # include/alsparse_amd_kernels.h
 
 
 class asamd_pattern_layout(Structure):  # include/alsparse_amd_kernels.h
-    _fields_ = [("pid", c_void_p), ("dist", c_void_p), ("block_off", c_void_p), ("stride", c_int32), ("group", c_int32),
+    _fields_ = [("pid", c_void_p), ("dist", c_void_p), ("len", c_void_p), ("wave_off", c_void_p), ("stride", c_int32), ("group", c_int32),
                 ("device_bytes", ctypes.c_int64)]
 
 

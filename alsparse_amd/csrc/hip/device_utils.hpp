@@ -249,6 +249,17 @@ __device__ __forceinline__ int wave_max_scan(int v) {
   return v;
 }
 
+// inclusive running sum over the 64 lanes of a wave (DPP only)
+__device__ __forceinline__ int wave_sum_scan(int v) {
+  v += dpp_mov_rows<0x111, 0xF>(v);
+  v += dpp_mov_rows<0x112, 0xF>(v);
+  v += dpp_mov_rows<0x114, 0xF>(v);
+  v += dpp_mov_rows<0x118, 0xF>(v);
+  v += dpp_mov_rows<0x142, 0xA>(v);
+  v += dpp_mov_rows<0x143, 0xC>(v);
+  return v;
+}
+
 // value of the given lane, the same in every lane (v_readlane: no LDS crossbar)
 __device__ __forceinline__ int lane_bcast(int v, int src) { return __builtin_amdgcn_readlane(v, src); }
 __device__ __forceinline__ float lane_bcast(float v, int src) {

@@ -4,14 +4,14 @@
 //
 // The staged row blocks (spmv_rows.hpp) are bound by the bytes they stream, and a third to a half of those are column
 // numbers.  With a pattern per row the columns cost ONE byte per row instead of four per entry, and the gathers of x
-// no longer wait for a stream: a lane knows its columns from its row's pattern as soon as row_ptr is there, so they are
+// no longer wait for a stream: a lane knows its columns as soon as its row's pattern is there, so they are
 // issued beside the loads of the values, and lanes on neighbouring rows of one pattern read neighbouring elements of x.
 // The structure is promised fixed (analysed matrices only); values stay in the caller's array.
 //
 // Bound by memory.  us per multiply over four matrices in turn, before (32-bit columns, 16-bit distances or the ELL copy,
-// whichever the analysis kept) and now: 5-point Laplacian 2048^2 fp64 67.4 -> 50.4 (256 MB moved, 5.1 TB/s), fp32
-// 49.6 -> 31.9; 27-point stencil of 101 x 100 x 97 points complex64 72.5 -> 50.8, fp64 69.9 -> 50.8; of 160^3 points fp32
-// 179 -> 105; of 60 x 50 x 47 points fp32 10.7 -> 6.1.  Rows far shorter than the longest, and small matrices, stay with
+// whichever the analysis kept) and now: 5-point Laplacian 2048^2 fp64 67.4 -> 47.1 (239 MB moved, 5.1 TB/s), fp32
+// 49.6 -> 30.0; 27-point stencil of 101 x 100 x 97 points complex64 72.5 -> 48.6, fp64 69.9 -> 48.7; of 160^3 points fp32
+// 179 -> 102; of 60 x 50 x 47 points fp32 10.7 -> 6.1.  Rows far shorter than the longest, and small matrices, stay with
 // the columns (patterns_pay in plan.c).  16-byte values: the ELL copy stays
 // ahead (5-point Laplacian of 2.1 M rows 58.7 against 84.4).
 //
@@ -24,6 +24,7 @@
 namespace asamd {
 
 constexpr int kPatternSlots = 256;   // a pattern's number is one byte
+constexpr int kPatternWaves = kStreamRows / kWave;  // waves of a workgroup
 constexpr int kPatternMaxLen = 64;   // entries per row; 64 KiB of distances at most, of which a matrix touches a few lines
 
 // What the builder leaves in one allocation besides the rows' pattern numbers.
@@ -44,7 +45,7 @@ static __global__ __launch_bounds__(kStreamRows) void pattern_rows_kernel(int m,
                                                                           const int* __restrict__ col_ind,
                                                                           PatternScratch* __restrict__ tab,
                                                                           unsigned char* __restrict__ pid,
-                                                                          int* __restrict__ block_off) {
+                                                                          int* __restrict__ wave_off) {
   extern __shared__ int s_col[];
   if (__atomic_load_n(&tab->fail, __ATOMIC_RELAXED)) return;
   const int64_t row0 = (int64_t)blockIdx.x * rows_per_group;
@@ -56,9 +57,10 @@ static __global__ __launch_bounds__(kStreamRows) void pattern_rows_kernel(int m,
     if (threadIdx.x == 0) atomicOr(&tab->fail, 1);
     return;
   }
-  if (threadIdx.x == 0) {
-    block_off[blockIdx.x] = (int)lo;
-    if (row_last == m) block_off[blockIdx.x + 1] = (int)(lo + n);
+  if ((int)threadIdx.x < kPatternWaves) {
+    const int64_t r = row0 + (int64_t)threadIdx.x * (rows_per_group / kPatternWaves);
+    wave_off[(int64_t)blockIdx.x * kPatternWaves + threadIdx.x] = r < m ? row_ptr[r] - base : (int)(lo + n);
+    if (row_last == m && threadIdx.x == 0) wave_off[((int64_t)blockIdx.x + 1) * kPatternWaves] = (int)(lo + n);
   }
   for (int k = threadIdx.x; k < (int)n; k += kStreamRows) s_col[k] = col_ind[lo + k];
   __syncthreads();
@@ -138,14 +140,17 @@ static __global__ __launch_bounds__(kStreamRows) void pattern_verify_kernel(int 
 
 // y = alpha*A*x + beta*y.  256 / G rows per workgroup as in the staged row blocks: their values are one contiguous range,
 // streamed into LDS with 128-bit loads that are all in flight at once, G lanes sum a row.  U: entries per lane (rows of at
-// most U * G entries), dist: `stride` distances per pattern, block_off: where every workgroup's entries begin -- a word
-// per workgroup that its neighbours' loads have brought to the L2, so that the values need not wait for row_ptr, whose
-// lines come from memory.  NTV: the values bypass the caches.  val 16-byte aligned, row_ptr[0] == base.
+// most U * G entries), dist, lens: `stride` distances and a length per pattern, wave_off: where every wave's entries
+// begin -- words that the neighbours' loads have brought to the L2, so that the values wait for nothing from memory.
+// Where a row begins inside its wave's entries is the sum of the lengths before it, and row_ptr is not read.  us with it /
+// without, three sets of arrays in turn: 5-point Laplacian 2048^2 fp64 50.8 / 46.8, 3000 x 3001 fp64 108 / 97.4; 27-point
+// stencil 101 x 100 x 97 complex64 51.6 / 48.6, 160^3 fp32 107.9 / 102 (a length in front of its distances: 48.5 and 50.3
+// for the first and the third; workgroups that take several blocks and load the next one's values while they add one up:
+// 54 and 56).  NTV: the values bypass the caches.  val 16-byte aligned.
 template <typename T, int U, int G, bool NTV>
 __global__ __launch_bounds__(kStreamRows) void spmv_pattern_kernel(
-    int m, T alpha, const T* __restrict__ val, const int* __restrict__ row_ptr, const unsigned char* __restrict__ pid,
-    const int* __restrict__ dist, int stride, const int* __restrict__ block_off, const T* __restrict__ x, T beta,
-    T* __restrict__ y, int base) {
+    int m, T alpha, const T* __restrict__ val, const unsigned char* __restrict__ pid, const int* __restrict__ dist, int stride,
+    const int* __restrict__ lens, const int* __restrict__ wave_off, const T* __restrict__ x, T beta, T* __restrict__ y) {
   constexpr int kRows = kStreamRows / G;
   constexpr int kPer = 16 / (int)sizeof(T);       // values per 128-bit piece
   constexpr int kStaged = kStreamRows * U / kPer + 1;  // pieces of a block: one more for the values in front of its first
@@ -156,9 +161,10 @@ __global__ __launch_bounds__(kStreamRows) void spmv_pattern_kernel(
   const int lane = threadIdx.x % G;
   const int64_t row = row0 + threadIdx.x / G;
   const int64_t my_row = row < m ? row : (int64_t)m - 1;
-  const int e0 = block_off[bid], e1 = block_off[bid + 1];  // at most kStreamRows * U apart: the builder looked
+  const int* __restrict__ starts = wave_off + (int64_t)bid * kPatternWaves;
+  const int e0 = starts[0], e1 = starts[kPatternWaves];  // at most kStreamRows * U apart: the builder looked
+  const int mine0 = starts[__builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave)];
   const int pattern = pid[my_row];
-  const int first = row_ptr[my_row], last = row_ptr[my_row + 1];
   // The values through a buffer resource that ends with the block: the pieces past its end come back as zeros without a
   // request and without a condition, so that all loads are in flight before the first wait.
   const int a0 = e0 & ~(kPer - 1);
@@ -171,6 +177,7 @@ __global__ __launch_bounds__(kStreamRows) void spmv_pattern_kernel(
   // reads with it is not added below.
   const int* __restrict__ d = dist + pattern * stride;
   const T* __restrict__ xr = x + my_row;
+  const int len = row < m ? lens[pattern] : 0;
   int off[U];
   T xv[U];
 #pragma unroll
@@ -180,10 +187,10 @@ __global__ __launch_bounds__(kStreamRows) void spmv_pattern_kernel(
 #pragma unroll
   for (int s = 0; s < kPieces; ++s)
     if (threadIdx.x + s * kStreamRows < kStaged) s_words[threadIdx.x + s * kStreamRows] = v[s];
+  const int first = mine0 + wave_sum_scan(lane == 0 ? len : 0) - len;
   __syncthreads();
   if (row >= m) return;  // whole lane groups leave together
-  const T* mine = reinterpret_cast<const T*>(s_words) + (first - base - a0);
-  const int len = last - first;
+  const T* mine = reinterpret_cast<const T*>(s_words) + (first - a0);
   T mv[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) mv[u] = mine[lane + u * G < len ? lane + u * G : 0];

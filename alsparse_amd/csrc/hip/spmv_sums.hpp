@@ -339,13 +339,7 @@ __global__ __launch_bounds__(kProdThreads) void sums_products_kernel(
     if (lane == 0) in = open;
     open = lane_bcast(run, kWave - 1);
     const int mine = __builtin_popcount(marks);
-    int upto = mine;  // sums that end in this lane and below
-    upto += dpp_mov_rows<0x111, 0xF>(upto);
-    upto += dpp_mov_rows<0x112, 0xF>(upto);
-    upto += dpp_mov_rows<0x114, 0xF>(upto);
-    upto += dpp_mov_rows<0x118, 0xF>(upto);
-    upto += dpp_mov_rows<0x142, 0xA>(upto);
-    upto += dpp_mov_rows<0x143, 0xC>(upto);
+    const int upto = wave_sum_scan(mine);  // sums that end in this lane and below
     const int n = lane_bcast(upto, kWave - 1);
     // through LDS, so that they leave side by side; more than the area holds in several turns
     for (int base = 0; base < n; base += kStage) {

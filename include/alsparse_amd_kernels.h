@@ -165,7 +165,8 @@ int asamd_spmv_stream(hipStream_t stream, const asamd_spmv_args *a, int32_t grou
 typedef struct {
   unsigned char *pid;   /* m pattern numbers; NULL: no layout (owns the one allocation) */
   int32_t *dist;        /* 256 x stride distances */
-  int32_t *block_off;   /* where the entries of every workgroup's 256 / group rows begin, and the last one's end */
+  int32_t *len;         /* 256 lengths                                                  */
+  int32_t *wave_off;    /* where the entries of every 64 / group rows begin, and the last ones' end */
   int32_t stride, group;
   int64_t device_bytes;
 } asamd_pattern_layout;

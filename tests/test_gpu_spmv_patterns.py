@@ -110,6 +110,30 @@ def test_row_lengths_across_the_lane_groups(gpu, name, base, longest):
         da.free()
 
 
+@pytest.mark.parametrize("longest", [3, 9, 27])
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 31, 32, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 513])
+def test_matrices_that_end_around_a_wave(gpu, rows, longest):
+    """A row's place among its wave's entries is the sum of the lengths before it: the last wave's rows begin or end there,
+    waves without rows follow it."""
+    patterns = [np.arange(k) * 3 for k in (longest, 1, longest - 1)]
+    a = _patterned(rows + 100, rows + 300, patterns, rows, np.float64, 0)
+    rp = a.row_ptr[:rows + 1].copy()
+    rp_end = int(rp[-1])
+    b = wl.Csr(rows, a.cols, rp, a.col_ind[:rp_end].copy(), a.values[:rp_end].copy(), 0, "patterned")
+    x, y0 = wl.uniform(b.cols, b.dtype, 3), wl.uniform(b.rows, b.dtype, 4)
+    da = DeviceCsr(b)
+    layout = _build(da)
+    try:
+        assert layout.pid
+        announce("patterns: rows", rows, "longest", longest)
+        st, y = _multiply(da, layout, 1.5, x, 0.5, y0)
+        assert st == 0
+        _check(b, 1.5, x, 0.5, y0, y, "%d rows" % rows)
+    finally:
+        capi.load().asamd_patterns_free(byref(layout))
+        da.free()
+
+
 @pytest.mark.parametrize("what", ["many patterns", "an empty row", "a long row"])
 def test_matrices_without_the_layout(gpu, what):
     """More patterns than a byte can number, an empty row, rows of 65 entries: no layout, and no error."""
