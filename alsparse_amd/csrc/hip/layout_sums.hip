@@ -8,6 +8,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <functional>
+#include <utility>
 #include <vector>
 
 #include "alsparse_amd_kernels.h"
@@ -17,10 +19,36 @@
 
 using namespace asamd;
 
-// Slots of a phase-1 chunk, at most: three spans for each of its sixteen waves.  Power-law graph of 8 M rows: 48 K
-// 165 us, 64 K 167, 96 K and 128 K 162, 192 K 167 (fewer chunks fill the last round of workgroups badly, more of them
-// load x slices more often).
-constexpr int kSumsChunk = 96 * 1024;
+// Spans of a phase-1 chunk, at most.  One workgroup to a compute unit (the x slice fills its LDS), so what counts is how
+// full the last round of chunks is, and how often a slice is loaded: of the limits below the one whose rounds, each as long
+// as its longest chunk, are the shortest together.  A slice, which mostly comes from an L2, costs three quarters of its
+// bytes.  us with chunks of at most 48 spans (96 K slots), whatever the matrix, / these: uniform columns, 2 M x 2 M x 16
+// fp32 131 / 115 (256 chunks of 64 spans; 384 of up to 48), transposed 1 M x 16 fp64 106 / 100 (245 of 32; 184), 2 M x 2 M x
+// 20 fp32 135 / 129, fp64 250 / 245; power law of 8 M rows fp32 287 / 285.
+constexpr int kSumsLeastSpans = 16, kSumsMostSpans = 96, kSumsSpanStep = 4;
+constexpr int64_t kSumsSliceCost = 96 * 1024;
+
+// The limit for column blocks of spans[c] spans, span_bytes each.
+static int sums_chunk_spans(const std::vector<int>& spans, int64_t span_bytes, int64_t cus) {
+  int best = 0;
+  int64_t best_cost = 0;
+  std::vector<std::pair<int, int>> pieces(spans.size());  // a block's longest piece, and how many
+  for (int limit = kSumsLeastSpans; limit <= kSumsMostSpans; limit += kSumsSpanStep) {
+    for (size_t c = 0; c < spans.size(); ++c) {
+      const int k = (spans[c] + limit - 1) / limit;
+      pieces[c] = {k > 0 ? (spans[c] + k - 1) / k : 0, k};
+    }
+    std::sort(pieces.begin(), pieces.end(), std::greater<>());
+    int64_t cost = 0, at = 0, round = 0;  // chunks handed out, first chunk of the next round
+    for (const auto& [longest, count] : pieces)
+      for (at += count; round < at; round += cus) cost += kSumsSliceCost + longest * span_bytes;
+    if (best == 0 || cost < best_cost) {
+      best = limit;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
 
 // Tallest row block: eight waves' accumulators and dummy rows fill a compute unit's LDS
 template <typename T>
@@ -60,7 +88,6 @@ static hipError_t build_sums(hipStream_t stream, asamd_sums_layout* L, const int
   const int groups = (int)(((int64_t)m + (1 << kRowGroupLog2) - 1) >> kRowGroupLog2);
   const auto room = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
   constexpr int kSpan = SumsDims<T>::span;
-  static_assert(kSumsChunk % kSpan == 0, "a chunk is a whole number of spans");
   const int64_t spans_most = (int64_t)nnz / kSpan + cb + 1;
   const size_t cnt_n = (size_t)(spans_most > 2 * (int64_t)groups ? spans_most : 2 * (int64_t)groups) + 1;
 
@@ -225,14 +252,19 @@ static hipError_t build_sums(hipStream_t stream, asamd_sums_layout* L, const int
   // ---- 4. phase-1 work list, the values ---------------------------------------------------------------------------
   std::vector<SumsChunk> h_chunks;
   if (e == hipSuccess) {
+    std::vector<int> block_spans((size_t)cb);
+    for (int c = 0; c < cb; ++c) block_spans[(size_t)c] = colspan[(size_t)c + 1] - colspan[(size_t)c];
+    const int limit = sums_chunk_spans(block_spans, (int64_t)kSpan * ((int64_t)sizeof(T) + 2), device_cus());
     for (int c = 0; c < cb; ++c) {
-      for (int at = 0; at < colptr[(size_t)c + 1] - colptr[(size_t)c]; at += kSumsChunk) {
-        const int left = colptr[(size_t)c + 1] - colptr[(size_t)c] - at;
+      const int all = block_spans[(size_t)c], pieces = (all + limit - 1) / limit;
+      const int64_t entries = colptr[(size_t)c + 1] - colptr[(size_t)c];
+      for (int i = 0; i < pieces; ++i) {  // as even as whole spans allow
+        const int64_t first = (int64_t)all * i / pieces, end = (int64_t)all * (i + 1) / pieces * kSpan;
         SumsChunk ch;
         ch.col0 = c << kShift;
         ch.ncols = n - ch.col0 < kCols ? n - ch.col0 : kCols;
-        ch.span0 = colspan[(size_t)c] + at / kSpan;
-        ch.slots = left < kSumsChunk ? left : kSumsChunk;
+        ch.span0 = colspan[(size_t)c] + (int)first;
+        ch.slots = (int)((end < entries ? end : entries) - first * kSpan);
         h_chunks.push_back(ch);
       }
     }

@@ -92,12 +92,14 @@ SHAPES = {
     "one_block": lambda d: _matrix(_tail(70001, 1, 100), 100, d, 1),
     "block_edge": lambda d: _matrix(_tail(30000, 2, 9000), _width(d), d, 2),
     "past_the_edge": lambda d: _matrix(_tail(30000, 3, 9000), _width(d) + 1, d, 3, crowd=1),
-    # hub rows that fill whole spans (2048 entries) of one column block, beside short ones; chunks of 96 K entries
+    # hub rows that fill whole spans (2048 entries) of one column block, beside short ones
     "hubs": lambda d: _matrix([60000] * 3 + [0] * 61 + list(_tail(5000, 4, 50)), 70000, d, 4, crowd=6),
     "only_long_rows": lambda d: _matrix([5000] * 100, 50000, d, 5, crowd=1),
     # rows of exactly one and two spans, one entry more and one less
     "span_edges": lambda d: _matrix([2047, 2048, 2049, 4096, 1, 0, 1024, 1023, 1025] * 10 + [3] * 2000, 3000, d, 6, crowd=1),
     "unsorted_base_one": lambda d: _matrix(_tail(40000, 7, 4000), 2 * _width(d) + 77, d, 7, base=1, shuffled=True),
+    # column blocks of many and of few spans, cut into pieces that are not all equally long
+    "uneven_pieces": lambda d: _matrix(_tail(150001, 10, 3000), 5 * _width(d) + 11, d, 10),
     # taller than a row block: several of them, the last one short
     "many_rows": lambda d: _matrix(_tail(700001, 8, 3000), 40000, d, 8),
 }
