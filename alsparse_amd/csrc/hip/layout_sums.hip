@@ -8,47 +8,22 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <functional>
-#include <utility>
 #include <vector>
 
 #include "alsparse_amd_kernels.h"
 #include "launch_utils.hpp"
 #include "spmv_sums.hpp"
+#include "tile_chunks.hpp"
 #include "tile_sort.hpp"
 
 using namespace asamd;
 
-// Spans of a phase-1 chunk, at most.  One workgroup to a compute unit (the x slice fills its LDS), so what counts is how
-// full the last round of chunks is, and how often a slice is loaded: of the limits below the one whose rounds, each as long
-// as its longest chunk, are the shortest together.  A slice, which mostly comes from an L2, costs three quarters of its
-// bytes.  us with chunks of at most 48 spans (96 K slots), whatever the matrix, / these: uniform columns, 2 M x 2 M x 16
-// fp32 131 / 115 (256 chunks of 64 spans; 384 of up to 48), transposed 1 M x 16 fp64 106 / 100 (245 of 32; 184), 2 M x 2 M x
-// 20 fp32 135 / 129, fp64 250 / 245; power law of 8 M rows fp32 287 / 285.
+// Spans of a phase-1 chunk, between these (tile_chunks.hpp).  us with chunks of at most 48 spans (96 K slots), whatever the
+// matrix, / these: uniform columns, 2 M x 2 M x 16 fp32 131 / 115 (256 chunks of 64 spans; 384 of up to 48), transposed
+// 1 M x 16 fp64 106 / 100 (245 of 32; 184), 2 M x 2 M x 20 fp32 135 / 129, fp64 250 / 245; power law of 8 M rows fp32 287 / 285.
+// A column block's chunks on one XCD, whose L2 then has the x slice: that transposed product 99 / 96, power law of 4 M rows
+// 141 / 138, 2 M x 2 M x 20 complex128 444 / 411.
 constexpr int kSumsLeastSpans = 16, kSumsMostSpans = 96, kSumsSpanStep = 4;
-constexpr int64_t kSumsSliceCost = 96 * 1024;
-
-// The limit for column blocks of spans[c] spans, span_bytes each.
-static int sums_chunk_spans(const std::vector<int>& spans, int64_t span_bytes, int64_t cus) {
-  int best = 0;
-  int64_t best_cost = 0;
-  std::vector<std::pair<int, int>> pieces(spans.size());  // a block's longest piece, and how many
-  for (int limit = kSumsLeastSpans; limit <= kSumsMostSpans; limit += kSumsSpanStep) {
-    for (size_t c = 0; c < spans.size(); ++c) {
-      const int k = (spans[c] + limit - 1) / limit;
-      pieces[c] = {k > 0 ? (spans[c] + k - 1) / k : 0, k};
-    }
-    std::sort(pieces.begin(), pieces.end(), std::greater<>());
-    int64_t cost = 0, at = 0, round = 0;  // chunks handed out, first chunk of the next round
-    for (const auto& [longest, count] : pieces)
-      for (at += count; round < at; round += cus) cost += kSumsSliceCost + longest * span_bytes;
-    if (best == 0 || cost < best_cost) {
-      best = limit;
-      best_cost = cost;
-    }
-  }
-  return best;
-}
 
 // Tallest row block: eight waves' accumulators and dummy rows fill a compute unit's LDS
 template <typename T>
@@ -254,7 +229,8 @@ static hipError_t build_sums(hipStream_t stream, asamd_sums_layout* L, const int
   if (e == hipSuccess) {
     std::vector<int> block_spans((size_t)cb);
     for (int c = 0; c < cb; ++c) block_spans[(size_t)c] = colspan[(size_t)c + 1] - colspan[(size_t)c];
-    const int limit = sums_chunk_spans(block_spans, (int64_t)kSpan * ((int64_t)sizeof(T) + 2), device_cus());
+    const int limit = chunk_limit(block_spans, (int64_t)kSpan * ((int64_t)sizeof(T) + 2), kSumsSliceBytes, device_cus(),
+                                  kSumsLeastSpans, kSumsMostSpans, kSumsSpanStep);
     for (int c = 0; c < cb; ++c) {
       const int all = block_spans[(size_t)c], pieces = (all + limit - 1) / limit;
       const int64_t entries = colptr[(size_t)c + 1] - colptr[(size_t)c];
@@ -268,8 +244,15 @@ static hipError_t build_sums(hipStream_t stream, asamd_sums_layout* L, const int
         h_chunks.push_back(ch);
       }
     }
-    // (the short chunks last, where they even out the workgroups' ends)
-    std::stable_sort(h_chunks.begin(), h_chunks.end(), [](const SumsChunk& a, const SumsChunk& b) { return a.slots > b.slots; });
+    std::vector<int> size, block;
+    for (const SumsChunk& ch : h_chunks) {
+      size.push_back(ch.slots);
+      block.push_back(ch.col0 >> kShift);
+    }
+    const std::vector<int> order = chunk_order(size, block, kXcds);
+    std::vector<SumsChunk> ordered;
+    for (int i : order) ordered.push_back(h_chunks[(size_t)i]);
+    h_chunks.swap(ordered);
     L->n_chunks = (int)h_chunks.size();
     e = hipMalloc(&L->chunks, h_chunks.size() * sizeof(SumsChunk));
     if (e == hipSuccess) e = hipMemcpy(L->chunks, h_chunks.data(), h_chunks.size() * sizeof(SumsChunk), hipMemcpyHostToDevice);

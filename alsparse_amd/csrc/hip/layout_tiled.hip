@@ -15,6 +15,7 @@
 #include "alsparse_amd_kernels.h"
 #include "launch_utils.hpp"
 #include "spmv_tiled.hpp"
+#include "tile_chunks.hpp"
 #include "tile_sort.hpp"
 
 using namespace asamd;
@@ -338,19 +339,24 @@ static hipError_t build_tiled(hipStream_t stream, asamd_tiled_layout* L, const i
                                 (kLongThreads / kWave) * (TileDims<T>::rows + kWave) * (int)sizeof(T));
     }
   }
-  // ---- 4. phase-1 work list: every column block cut into chunks of at most kChunk entries.  48 K entries
-  // (the x slice, which neighbouring chunks find in the L2, is then loaded for every 288 KiB of fp32 streams)
-  // measured best: 16 M x 16 M with 16 entries per row 0.553 ms with 128 K -> 0.511 ms, 2 M x 2 M 83 -> 69 us;
-  // 32 K and 64 K were 3-4 % slower, equal shares for persistent workgroups no faster than 128 K.
+  // ---- 4. phase-1 work list: every column block cut into even chunks of 32 K to 96 K entries (tile_chunks.hpp).  us with
+  // chunks of 48 K and what is left, neighbours on different XCDs / these, neighbours on one XCD, whose L2 then has the x
+  // slice: uniform columns, fp32, 4.4 M x 4.4 M x 6 130 / 120, 8.7 M x 6 263 / 249, 14 M x 9 577 / 550, fp64, 5 M x 10 373 / 357;
+  // 16 M x 16 fp32 874 / 875 (even chunks with neighbours on different XCDs 895).
   if (e == hipSuccess) {
-    const int64_t kChunk = 48 * 1024;
+    constexpr int kUnit = 1024;
+    std::vector<int> units((size_t)cb);
+    for (int c = 0; c < cb; ++c) units[(size_t)c] = (h_colptr[(size_t)c + 1] - h_colptr[(size_t)c] + kUnit - 1) / kUnit;
+    const int limit = chunk_limit(units, (int64_t)kUnit * (2 * (int64_t)sizeof(T) + 2), kSliceBytes, device_cus(), 32, 96, 4);
     for (int c = 0; c < cb; ++c) {
-      for (int64_t b = h_colptr[(size_t)c]; b < h_colptr[(size_t)c + 1]; b += kChunk) {
+      const int64_t first = h_colptr[(size_t)c], len = h_colptr[(size_t)c + 1] - first;
+      const int64_t pieces = (units[(size_t)c] + limit - 1) / limit;
+      for (int64_t i = 0; i < pieces; ++i) {
         TiledChunk ch;
         ch.col0 = h_cbs[(size_t)c];
         ch.ncols = h_cbs[(size_t)c + 1] - h_cbs[(size_t)c];
-        ch.begin = (int)b;
-        ch.end = (int)(b + kChunk < h_colptr[(size_t)c + 1] ? b + kChunk : h_colptr[(size_t)c + 1]);
+        ch.begin = (int)(first + len * i / pieces);
+        ch.end = (int)(first + len * (i + 1) / pieces);
         h_chunks.push_back(ch);
       }
     }

@@ -376,7 +376,7 @@ __global__ __launch_bounds__(kProdThreads) void tiled_products_kernel(
     const unsigned short* __restrict__ t_col, const T* __restrict__ x, T* __restrict__ prod) {
   extern __shared__ __align__(16) unsigned char smem[];
   T* xs = reinterpret_cast<T*>(smem);
-  const TiledChunk ch = chunks[blockIdx.x];
+  const TiledChunk ch = chunks[xcd_contiguous_id(blockIdx.x, gridDim.x)];
   {
     // x slice -> LDS: 128-bit pieces, all of a thread's loads issued before the first LDS write
     // (a load-wait-write loop pays the memory latency once per trip: 32 trips of it were a quarter
