@@ -339,15 +339,18 @@ static hipError_t build_tiled(hipStream_t stream, asamd_tiled_layout* L, const i
                                 (kLongThreads / kWave) * (TileDims<T>::rows + kWave) * (int)sizeof(T));
     }
   }
-  // ---- 4. phase-1 work list: every column block cut into even chunks of 32 K to 96 K entries (tile_chunks.hpp).  us with
-  // chunks of 48 K and what is left, neighbours on different XCDs / these, neighbours on one XCD, whose L2 then has the x
-  // slice: uniform columns, fp32, 4.4 M x 4.4 M x 6 130 / 120, 8.7 M x 6 263 / 249, 14 M x 9 577 / 550, fp64, 5 M x 10 373 / 357;
-  // 16 M x 16 fp32 874 / 875 (even chunks with neighbours on different XCDs 895).
+  // ---- 4. phase-1 work list: every column block cut into even chunks of 32 K to 96 K entries (tile_chunks.hpp),
+  // neighbours on one XCD, whose L2 then has the x slice; where the products are stored past the caches, into chunks of 48 K
+  // and what is left, neighbours on different XCDs.  us, the second / the first: uniform columns, fp32, 4.4 M x 4.4 M x 6
+  // 130 / 120, 8.7 M x 6 263 / 249, 14 M x 9 577 / 550, fp64, 5 M x 10 373 / 357; past the caches, 16 M x 16 fp32 889 / 903,
+  // 4 M x 40 498 / 494 (a long run of rounds, whose last one matters little, and streams that are all there is).
   if (e == hipSuccess) {
     constexpr int kUnit = 1024;
+    const bool even = (int64_t)nnz_i * (int64_t)sizeof(T) <= kTiledPastCache;
     std::vector<int> units((size_t)cb);
     for (int c = 0; c < cb; ++c) units[(size_t)c] = (h_colptr[(size_t)c + 1] - h_colptr[(size_t)c] + kUnit - 1) / kUnit;
-    const int limit = chunk_limit(units, (int64_t)kUnit * (2 * (int64_t)sizeof(T) + 2), kSliceBytes, device_cus(), 32, 96, 4);
+    const int limit =
+        even ? chunk_limit(units, (int64_t)kUnit * (2 * (int64_t)sizeof(T) + 2), kSliceBytes, device_cus(), 32, 96, 4) : 48;
     for (int c = 0; c < cb; ++c) {
       const int64_t first = h_colptr[(size_t)c], len = h_colptr[(size_t)c + 1] - first;
       const int64_t pieces = (units[(size_t)c] + limit - 1) / limit;
@@ -355,8 +358,8 @@ static hipError_t build_tiled(hipStream_t stream, asamd_tiled_layout* L, const i
         TiledChunk ch;
         ch.col0 = h_cbs[(size_t)c];
         ch.ncols = h_cbs[(size_t)c + 1] - h_cbs[(size_t)c];
-        ch.begin = (int)(first + len * i / pieces);
-        ch.end = (int)(first + len * (i + 1) / pieces);
+        ch.begin = (int)(first + (even ? len * i / pieces : i * limit * kUnit));
+        ch.end = (int)(first + (even ? len * (i + 1) / pieces : std::min<int64_t>((i + 1) * limit * kUnit, len)));
         h_chunks.push_back(ch);
       }
     }
@@ -454,7 +457,7 @@ extern "C" int asamd_spmv_tiled(hipStream_t s, const asamd_spmv_args* a, const a
     T* prod = (T*)products;
     if (L->n_chunks > 0) {
       // products that the memory-side cache cannot hold anyway are stored past it
-      if ((int64_t)L->nnz * (int64_t)sizeof(T) > ((int64_t)512 << 20))
+      if ((int64_t)L->nnz * (int64_t)sizeof(T) > kTiledPastCache)
         tiled_products_kernel<T, true><<<L->n_chunks, kProdThreads, kSliceBytes, s>>>(
             (const TiledChunk*)L->chunks, (const T*)L->tval, L->tcol, x, prod);
       else

@@ -21,8 +21,9 @@ __global__ void warmup_kernel() {}
 // The array has four equal quarters of kStaticSlots 4-byte slots: block_row | carry_row | carry_val |
 // head_val.  Every slot that a call reads is written by that call first, so nothing has to be cleared
 // between calls; two calls that overlap on one device share the array and race.
-constexpr int kStaticIpt = 8;
+constexpr int kStaticIpt = 8, kStaticShortIpt = 4;
 constexpr int kStaticSlots = ASAMD_CSRMV_NOALLOC_SCRATCH_BYTES / 16;
+static_assert(ASAMD_MERGE_SHORT_ITEMS <= (int64_t)(kStaticSlots - 1) * kMergeThreads * kStaticShortIpt, "room for the shorter walks");
 static_assert((int64_t)(kStaticSlots - 1) * kMergeThreads * kStaticIpt == ASAMD_CSRMV_NOALLOC_MAX_ITEMS,
               "the documented limit is what the array holds");
 static __device__ __align__(256) unsigned char scratch[ASAMD_CSRMV_NOALLOC_SCRATCH_BYTES];
@@ -68,12 +69,14 @@ extern "C" int asamd_s_csrmv_noalloc(hipStream_t stream, int32_t m, int32_t n, i
   int* carry_row = block_row + kStaticSlots;
   float* carry_val = (float*)(carry_row + kStaticSlots);
   float* head_val = carry_val + kStaticSlots;
-  constexpr int kItems = kMergeThreads * kStaticIpt;
-  const int nb = (int)((total + kItems - 1) / kItems);
-  merge_partition_kernel<<<(nb + 1 + 255) / 256, 256, 0, stream>>>(m, nnz, row_ptr, base, nb, kItems, block_row);
-  spmv_merge_kernel<float, kStaticIpt><<<nb, kMergeThreads, 0, stream>>>(m, nnz, alpha, val, row_ptr, col_ind, x, beta,
-                                                                         y, base, block_row, carry_row, carry_val,
-                                                                         head_val);
+  // (the items per thread of the planned merge path: the same sums, bit for bit)
+  const bool few = total <= ASAMD_MERGE_SHORT_ITEMS;
+  const int items = kMergeThreads * (few ? kStaticShortIpt : kStaticIpt);
+  const int nb = (int)((total + items - 1) / items);
+  merge_partition_kernel<<<(nb + 1 + 255) / 256, 256, 0, stream>>>(m, nnz, row_ptr, base, nb, items, block_row);
+  const auto multiply = few ? spmv_merge_kernel<float, kStaticShortIpt> : spmv_merge_kernel<float, kStaticIpt>;
+  multiply<<<nb, kMergeThreads, 0, stream>>>(m, nnz, alpha, val, row_ptr, col_ind, x, beta, y, base, block_row, carry_row,
+                                             carry_val, head_val, kStreamNtValues | kStreamNtIndices, nullptr);
   if (nb > 1)
     merge_fixup_kernel<float><<<(nb + 255) / 256, 256, 0, stream>>>(nb, m, alpha, beta, carry_row, carry_val, head_val,
                                                                     y);

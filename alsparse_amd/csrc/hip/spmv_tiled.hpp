@@ -367,6 +367,7 @@ template <typename T>
 struct __attribute__((packed, aligned(alignof(T)))) LoosePiece {
   unsigned w[4];  // plain words: the piece is only moved, never computed with
 };
+constexpr int64_t kTiledPastCache = (int64_t)512 << 20;  // bytes of products that are stored so
 // NTS: the products are stored non-temporally.  Worth it when they are far more than the 256 MiB memory-side
 // cache holds (16 M x 16 M with 16 entries per row, 1 GiB of products: 0.907 -> 0.884 ms per multiply); products
 // that fit are better left where the second phase finds them (2 M x 2 M: 0.159 -> 0.164 ms with NTS).
@@ -376,7 +377,9 @@ __global__ __launch_bounds__(kProdThreads) void tiled_products_kernel(
     const unsigned short* __restrict__ t_col, const T* __restrict__ x, T* __restrict__ prod) {
   extern __shared__ __align__(16) unsigned char smem[];
   T* xs = reinterpret_cast<T*>(smem);
-  const TiledChunk ch = chunks[xcd_contiguous_id(blockIdx.x, gridDim.x)];
+  // neighbouring chunks load the same x slice: on one XCD its L2 has it (where the products are stored past the caches that
+  // was no gain: asamd_tiled_build)
+  const TiledChunk ch = chunks[NTS ? blockIdx.x : xcd_contiguous_id(blockIdx.x, gridDim.x)];
   {
     // x slice -> LDS: 128-bit pieces, all of a thread's loads issued before the first LDS write
     // (a load-wait-write loop pays the memory latency once per trip: 32 trips of it were a quarter

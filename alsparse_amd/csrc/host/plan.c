@@ -1595,7 +1595,7 @@ static hipError_t plan_create(hipStream_t stream, int32_t m, int32_t n, int32_t 
    * walks are half as long, until the matrix is so large that its streams are all there is.  us, 4 / 8 items per thread, power
    * law fp32 of 20 000 rows 8.0 / 9.8, 200 000 17.7 / 18.0, 800 000 50 / 53, 3 M (36 M items) 205 / 205, 5 M 340 / 338, 8 M
    * 580 / 572 */
-  p->merge_ipt = val_size >= 8 || total <= (int64_t)1 << 25 ? 4 : 8;
+  p->merge_ipt = val_size >= 8 || total <= ASAMD_MERGE_SHORT_ITEMS ? 4 : 8;
   const int want_ipt = env_int("ALSPARSE_AMD_MERGE_IPT", 0);
   if (want_ipt == 4 || want_ipt == 8 || (want_ipt == 16 && dtype <= ASAMD_DTYPE_DOUBLE)) p->merge_ipt = want_ipt;
   if (val_size == 16) p->merge_ipt = 4; /* the only instantiation for 16-byte values */

@@ -182,6 +182,8 @@ int asamd_spmv_patterns(hipStream_t stream, const asamd_spmv_args *a, const asam
  * that a call reads it has written before, so the scratch needs no clearing, and two multiplies that
  * run at the same time need a scratch each.  No float atomics. */
 #define ASAMD_MERGE_THREADS 256
+/* up to so many items 4-byte values take four per thread as well, not eight */
+#define ASAMD_MERGE_SHORT_ITEMS ((int64_t)1 << 25)
 int asamd_merge_partition(hipStream_t stream, int32_t m, int32_t nnz, const int32_t *row_ptr, int32_t base,
                           int32_t blocks, int32_t items_per_block, int32_t *block_row);
 /* block_row NULL: every workgroup searches row_ptr for its own two coordinates; the better form up to
