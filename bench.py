@@ -34,11 +34,11 @@ NO_ANALYSIS = False  # --no-analysis
 MEASURED_TRAFFIC_BYTES = {
     (3, "tiled two-phase"): (5.17e9, "profiles/spmv_tiled_C3.txt"),
     (3, "rowconst"): (34.6e9, "profiles/spmv_tiled_C3.txt"),
-    (4, "row-sum tiles"): (1.49e9, "profiles/spmv_sums_C4.txt"),
+    (4, "row-sum tiles"): (1.43e9, "profiles/spmv_streams_and_rounds.txt"),
     (4, "merge-path"): (3.19e9, "profiles/spmv_merge_C4.txt"),
     (4, "merge-path, hot columns in LDS"): (2.85e9, "profiles/spmv_merge_hot_C4.txt"),
     (2, "ell copy"): (356.6e6, "profiles/spmv_ell_copy_C2.txt"),
-    (2, "row-block stream, row patterns"): (256.2e6, "profiles/spmv_patterns_laplace_stencil.txt"),
+    (2, "row-block stream, row patterns"): (239.8e6, "profiles/spmv_streams_and_rounds.txt"),
     (2, "row-block stream"): (338.8e6, "profiles/spmv_stream_C2.txt"),
     (5, "spmm row-major"): (9.18e9, "profiles/spmm_rowmajor_C5.txt"),
 }
@@ -732,7 +732,7 @@ def run_ceilings(steps, warmup, short=False):
 
 def against_ceiling(cfg, r, ceilings):
     """The measured ceiling that bounds the configuration's kernel, named, and how close the kernel runs to it.
-    C2 streams its algorithmic bytes once (with row patterns: values, row offsets and a byte per row): the non-temporal
+    C2 streams its algorithmic bytes once (with row patterns: values and a byte per row): the non-temporal
     read rate.  C3's tiled pair moves its streams twice
     (products out and in again): its real traffic (counter measurement, `traffic`) against the copy rate.
     C4 and the row kernels on C3 gather single elements of x that miss the L1: entries per second against the
