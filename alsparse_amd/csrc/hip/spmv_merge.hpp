@@ -92,7 +92,10 @@ static __device__ __forceinline__ int merge_coordinate(int m, int nnz, const int
 }
 // Up to this many workgroups find their two coordinates themselves, two of a workgroup's waves one each.  A launch of
 // its own for them costs 4.4 us, three rounds of probes in the L2 about one; a workgroup's probes are 64 lines a round,
-// though, where neighbouring threads of the table's kernel share theirs, so large matrices keep the table.
+// though, where neighbouring threads of the table's kernel share theirs, so large matrices keep the table.  us, by themselves /
+// with the table, power laws, four items per thread, 4 500 / 5 100 / 5 600 workgroups: 4-byte values 31.2 / 33.2, 34.4 / 35.8,
+// 38.2 / 39.1 (6 900 and 7 800: 45.0 / 44.4, 49.9 / 48.4), 8-byte 36.9 / 38.3, 41.1 / 41.4, 45.9 / 45.7, 16-byte 58.9 / 58.5,
+// 67.3 / 65.3, 74.1 / 71.3.
 constexpr int kMergeSelfBlocks = 4096;
 
 // IPT items per thread, kMergeThreads * IPT items per workgroup.  block_row: the coordinates, or null (every workgroup

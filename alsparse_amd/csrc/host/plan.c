@@ -575,13 +575,21 @@ static int settle_algo(const asamd_csr_plan *p, int algo, const void *val, const
   return algo;
 }
 
+/* Whether the workgroups of a structure that is not promised fixed find their own coordinates: 4-byte values with four items
+ * per thread half as many again as others (spmv_merge.hpp has both sides).  With eight items, which those values took at
+ * every size, 5 M entries and rows were half the workgroups: 33.6 us by themselves; with four 35.0 behind a table, 33.2. */
+static int merge_finds_itself(const asamd_csr_plan *p) {
+  const int most = asamd_merge_self_blocks();
+  return p->st.merge_blocks <= (p->val_size == 4 && p->merge_ipt == 4 ? most / 2 * 3 : most);
+}
+
 /* merge path; perm: NULL, or where the values of the plan's entries lie in a->val */
 static int run_merge(hipStream_t s, const asamd_csr_plan *p, const asamd_spmv_args *a, ws_cursor ws, const uint32_t *perm,
                      int conj) {
   const asamd_csr_stats *st = &p->st;
   const size_t nb = (size_t)st->merge_blocks, vs = (size_t)p->val_size;
   const int32_t *block_row = p->d_block_row;
-  if (!block_row && st->merge_blocks > asamd_merge_self_blocks()) {
+  if (!block_row && !merge_finds_itself(p)) {
     /* structure not promised fixed: the coordinates are computed for this call (few workgroups: by themselves) */
     int32_t *fresh = (int32_t *)ws_take(&ws, (nb + 1) * 4);
     if (!fresh) return -1;

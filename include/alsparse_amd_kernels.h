@@ -187,7 +187,7 @@ int asamd_spmv_patterns(hipStream_t stream, const asamd_spmv_args *a, const asam
 int asamd_merge_partition(hipStream_t stream, int32_t m, int32_t nnz, const int32_t *row_ptr, int32_t base,
                           int32_t blocks, int32_t items_per_block, int32_t *block_row);
 /* block_row NULL: every workgroup searches row_ptr for its own two coordinates; the better form up to
- * asamd_merge_self_blocks() workgroups. */
+ * asamd_merge_self_blocks() workgroups (4-byte values with four items per thread: half as many again). */
 int32_t asamd_merge_self_blocks(void);
 int asamd_spmv_merge(hipStream_t stream, const asamd_spmv_args *a, int32_t ipt, const int32_t *block_row,
                      int32_t *carry_row, void *carry_val, void *head_val);

@@ -1,9 +1,11 @@
 """Merge-path without a table of coordinates: every workgroup finds its own two, 64 probes at a time.  Compared with the
 CPU oracle at one workgroup, at the edges of two and three, and with runs of empty rows and rows longer than workgroups."""
+from ctypes import byref, c_void_p, cast
+
 import numpy as np
 import pytest
 
-from alsparse_amd import workloads as wl
+from alsparse_amd import capi, hiprt, workloads as wl
 from helpers import DeviceCsr, announce, check_spmv, run_plan_csrmv
 from helpers_shapes import csr_from_lengths
 
@@ -37,3 +39,36 @@ def test_workgroups_find_their_coordinates(gpu, shape, base, dtype):
             assert np.array_equal(y, run_plan_csrmv(da, "merge", alpha, x, beta, y0, trusted=1))
     finally:
         da.free()
+
+
+@pytest.mark.parametrize("dtype,rows,alone", [(np.float32, 4096 * 64 - 64, True), (np.float32, 4096 * 64 + 64, True),
+                                              (np.float32, 6144 * 64, True), (np.float32, 6144 * 64 + 1, False),
+                                              (np.float64, 4096 * 64, True), (np.float64, 4096 * 64 + 1, False)])
+def test_how_many_workgroups_need_no_table(gpu, dtype, rows, alone):
+    """Scratch for the carries and nothing else: with it the merge path runs where its workgroups find their coordinates, the
+    same bits as behind an analysis, and where they take a table a lane group per row runs in its place."""
+    a = wl.uniform_rows(rows, 5000, 15, dtype)  # 16 items a row, 64 rows a workgroup of 1 024 items
+    x, y0 = wl.uniform(a.cols, dtype, 3), wl.uniform(a.rows, dtype, 4)
+    lib, T = capi.load(), capi.scalar_type(dtype)
+    blocks, vs = (16 * rows + 1023) // 1024, np.dtype(dtype).itemsize
+    room = -(-blocks * 4 // 256) * 256 + 2 * (-(-blocks * vs // 256) * 256)
+    da, plan = DeviceCsr(a), c_void_p()
+    ws, dx, dy = hiprt.DeviceArray((room,), np.uint8), hiprt.DeviceArray.from_numpy(x), hiprt.DeviceArray.from_numpy(y0)
+    alpha, beta = T(1.5), T(0.5)
+    try:
+        assert lib.asamd_csr_plan_create(None, a.rows, a.cols, a.nnz, da.row_ptr.c_ptr(), da.col.c_ptr(), da.val.c_ptr(), 0, vs,
+                                         0, byref(plan)) == 0
+        assert lib.asamd_csr_plan_set_algo(plan, capi.ASAMD_SPMV_MERGE) == 0
+        announce("merge without a table", rows, np.dtype(dtype).name)
+        assert lib.asamd_csr_plan_csrmv(None, plan, 0, cast(byref(alpha), c_void_p), da.val.c_ptr(), da.row_ptr.c_ptr(),
+                                        da.col.c_ptr(), dx.c_ptr(), cast(byref(beta), c_void_p), dy.c_ptr(), ws.c_ptr(), room) == 0
+        hiprt.synchronize()
+        y = dy.to_numpy()
+        check_spmv(a, 1.5, x, 0.5, y0, y, "%d rows" % rows)
+        assert np.array_equal(y, run_plan_csrmv(da, "merge" if alone else "vector", 1.5, x, 0.5, y0, trusted=1))
+        assert not np.array_equal(y, run_plan_csrmv(da, "vector" if alone else "merge", 1.5, x, 0.5, y0, trusted=1))
+    finally:
+        if plan:
+            lib.asamd_csr_plan_destroy(plan)
+        for d in (ws, dx, dy, da):
+            d.free()
