@@ -79,6 +79,7 @@ extern "C" int asamd_spmv_patterns(hipStream_t s, const asamd_spmv_args* a, cons
   const double bytes = (double)a->nnz * dtype_size(a->dtype) + 5.0 * (double)a->m +
                        ((double)a->m + (double)a->n) * dtype_size(a->dtype);
   const bool ntv = forced >= 0 ? (forced & kStreamNtValues) != 0 : bytes > 280.0e6;
+  const bool early = !ntv && bytes <= 150.0e6;  // (the kernel has both sides)
   const int g = L->group;
   const unsigned grid = (unsigned)(((int64_t)a->m * g + kStreamRows - 1) / kStreamRows);
   auto go = [&](auto* tag) -> int {
@@ -87,14 +88,15 @@ extern "C" int asamd_spmv_patterns(hipStream_t s, const asamd_spmv_args* a, cons
     constexpr int kCap = 64 / (int)sizeof(T);  // 16 KiB of values per workgroup
     if (((uintptr_t)a->val & 15u) != 0 || L->stride > kCap * g) return hipErrorInvalidValue;
     const T alpha = scalar_of<T>(a->alpha), beta = scalar_of<T>(a->beta);
-#define ASAMD_PATTERN_LAUNCH_AS(U, G, NTV)                                                                           \
-  spmv_pattern_kernel<T, U, G, NTV><<<grid, kStreamRows, 0, s>>>(a->m, alpha, (const T*)a->val, L->pid, L->dist,     \
-                                                                 L->stride, L->len, L->wave_off, (const T*)a->x,     \
-                                                                 beta, (T*)a->y)
-#define ASAMD_PATTERN_LAUNCH(U, G)                   \
-  do {                                               \
-    if (ntv) ASAMD_PATTERN_LAUNCH_AS(U, G, true);    \
-    else ASAMD_PATTERN_LAUNCH_AS(U, G, false);       \
+#define ASAMD_PATTERN_LAUNCH_AS(U, G, NTV, EARLY)                                                                    \
+  spmv_pattern_kernel<T, U, G, NTV, EARLY><<<grid, kStreamRows, 0, s>>>(a->m, alpha, (const T*)a->val, L->pid,       \
+                                                                        L->dist, L->stride, L->len, L->wave_off,     \
+                                                                        (const T*)a->x, beta, (T*)a->y)
+#define ASAMD_PATTERN_LAUNCH(U, G)                             \
+  do {                                                         \
+    if (ntv) ASAMD_PATTERN_LAUNCH_AS(U, G, true, false);       \
+    else if (early) ASAMD_PATTERN_LAUNCH_AS(U, G, false, true);\
+    else ASAMD_PATTERN_LAUNCH_AS(U, G, false, false);          \
   } while (0)
     // U: as few entries per lane as the longest row needs (each is a gather in flight, useful or not)
     const int u = (L->stride + g - 1) / g;

@@ -147,7 +147,13 @@ static __global__ __launch_bounds__(kStreamRows) void pattern_verify_kernel(int 
 // stencil 101 x 100 x 97 complex64 51.6 / 48.6, 160^3 fp32 107.9 / 102 (a length in front of its distances: 48.5 and 50.3
 // for the first and the third; workgroups that take several blocks and load the next one's values while they add one up:
 // 54 and 56).  NTV: the values bypass the caches.  val 16-byte aligned.
-template <typename T, int U, int G, bool NTV>
+// EARLY: for matrices that the caches hold, where the chain pattern - distances - x counts and not the bytes: the pattern's
+// number is asked for in front of the wait for the starts, and nothing on the way to x waits for a load of its own.  us,
+// without / with: 27-point stencil 50 x 51 x 48 fp64 8.2 / 7.7, 64 x 65 x 62 fp64 13.1 / 12.4, fp32 7.8 / 7.4, 5-point Laplacian
+// 2048^2 fp32 (138 MB) 29.9 / 27.4; beyond the caches the values' requests, which then stand behind the distances' and x',
+// are what counts: stencil 90 x 91 x 88 fp64 (163 MB) 36.3 / 36.3, 101 x 100 x 97 complex64 48.1 / 48.4, Laplacian 2600 x 2601
+// fp64 73.7 / 75.5.
+template <typename T, int U, int G, bool NTV, bool EARLY>
 __global__ __launch_bounds__(kStreamRows) void spmv_pattern_kernel(
     int m, T alpha, const T* __restrict__ val, const unsigned char* __restrict__ pid, const int* __restrict__ dist, int stride,
     const int* __restrict__ lens, const int* __restrict__ wave_off, const T* __restrict__ x, T beta, T* __restrict__ y) {
@@ -165,6 +171,10 @@ __global__ __launch_bounds__(kStreamRows) void spmv_pattern_kernel(
   const int e0 = starts[0], e1 = starts[kPatternWaves];  // at most kStreamRows * U apart: the builder looked
   const int mine0 = starts[__builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave)];
   const int pattern = pid[my_row];
+  if constexpr (EARLY) {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::"s"(mine0));  // (left alone, the compiler loads it behind the barrier, where it is needed)
+  }
   // The values through a buffer resource that ends with the block: the pieces past its end come back as zeros without a
   // request and without a condition, so that all loads are in flight before the first wait.
   const int a0 = e0 & ~(kPer - 1);
@@ -177,7 +187,13 @@ __global__ __launch_bounds__(kStreamRows) void spmv_pattern_kernel(
   // reads with it is not added below.
   const int* __restrict__ d = dist + pattern * stride;
   const T* __restrict__ xr = x + my_row;
-  const int len = row < m ? lens[pattern] : 0;
+  int len;
+  if constexpr (EARLY) {
+    const int pattern_len = lens[pattern];  // (no load under a condition: the loads behind it would wait for the branch)
+    len = row < m ? pattern_len : 0;
+  } else {
+    len = row < m ? lens[pattern] : 0;
+  }
   int off[U];
   T xv[U];
 #pragma unroll
@@ -185,8 +201,10 @@ __global__ __launch_bounds__(kStreamRows) void spmv_pattern_kernel(
 #pragma unroll
   for (int u = 0; u < U; ++u) xv[u] = xr[off[u]];
 #pragma unroll
-  for (int s = 0; s < kPieces; ++s)
+  for (int s = 0; s < kPieces; ++s) {
+    if constexpr (EARLY) asm volatile("" ::"v"(v[s].x));  // (not loaded under the condition either)
     if (threadIdx.x + s * kStreamRows < kStaged) s_words[threadIdx.x + s * kStreamRows] = v[s];
+  }
   const int first = mine0 + wave_sum_scan(lane == 0 ? len : 0) - len;
   __syncthreads();
   if (row >= m) return;  // whole lane groups leave together

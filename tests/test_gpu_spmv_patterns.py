@@ -134,6 +134,37 @@ def test_matrices_that_end_around_a_wave(gpu, rows, longest):
         da.free()
 
 
+@pytest.mark.parametrize("name,longest,mbytes", [("f32", 5, 140), ("f32", 5, 160), ("f32", 27, 270), ("f32", 27, 300), ("f64", 5, 160),
+                                                 ("f64", 27, 140), ("f64", 27, 160), ("f64", 27, 300), ("c64", 27, 200)])
+def test_forms_on_both_sides_of_their_lines(gpu, name, longest, mbytes):
+    """The form whose loads wait for as little as can be, up to 150 MB, the one whose values go first, and from 280 MB the one
+    whose values bypass the caches: a last wave with a few rows in each."""
+    dtype = DTYPES[name]
+    size = np.dtype(dtype).itemsize
+    mean = longest - 0.5  # rows of longest and longest - 1 entries
+    m = int(mbytes * 1e6 / (mean * size + 5 + 2 * size)) // 256 * 256 + 7
+    rng = np.random.default_rng(longest)
+    which = rng.integers(0, 2, size=m)
+    table = np.stack([np.arange(longest) * 3, np.arange(longest) * 3 + 1]).astype(np.int32)
+    lengths = longest - which
+    row_ptr = np.zeros(m + 1, dtype=np.int64)
+    np.cumsum(lengths, out=row_ptr[1:])
+    col = (np.arange(m, dtype=np.int32)[:, None] + table[which])[np.arange(longest)[None, :] < lengths[:, None]]
+    a = wl.Csr(m, m + 3 * longest, row_ptr.astype(np.int32), col, _vector(col.size, dtype, 9), 0, "patterned")
+    x, y0 = _vector(a.cols, dtype, 3), _vector(a.rows, dtype, 4)
+    da = DeviceCsr(a)
+    layout = _build(da)
+    try:
+        assert layout.pid
+        announce("patterns by size", name, longest, mbytes)
+        st, y = _multiply(da, layout, 1.5, x, 0.5, y0)
+        assert st == 0
+        _check(a, 1.5, x, 0.5, y0, y, "%s %d MB" % (name, mbytes))
+    finally:
+        capi.load().asamd_patterns_free(byref(layout))
+        da.free()
+
+
 @pytest.mark.parametrize("what", ["many patterns", "an empty row", "a long row"])
 def test_matrices_without_the_layout(gpu, what):
     """More patterns than a byte can number, an empty row, rows of 65 entries: no layout, and no error."""
