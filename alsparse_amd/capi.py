@@ -153,7 +153,7 @@ class asamd_xlds_layout(Structure):  # include/alsparse_amd_kernels.h
 
 
 class asamd_pattern_layout(Structure):  # include/alsparse_amd_kernels.h
-    _fields_ = [("pid", c_void_p), ("dist", c_void_p), ("len", c_void_p), ("wave_off", c_void_p), ("stride", c_int32), ("group", c_int32),
+    _fields_ = [("pid", c_void_p), ("dist", c_void_p), ("block_off", c_void_p), ("stride", c_int32), ("group", c_int32),
                 ("device_bytes", ctypes.c_int64)]
 
 
@@ -355,11 +355,15 @@ _COMMON = {
     "asamd_tiled_build": [_P, _I, _I, _I, _I, _I, _P, _P, _P, _I, _I, _P],
     "asamd_tiled_free": [_P],
     "asamd_tiled_gather_values": [_P, _P, _P, _P],
-    "asamd_spmv_tiled": [_P, POINTER(asamd_spmv_args), _P, _P, _P, _P, _P],
+    "asamd_tiled_gather_checked": [_P, _P, _P, _P],
+    "asamd_spmv_tiled": [_P, POINTER(asamd_spmv_args), _P, _P, _P, _P],
+    "asamd_spmv_tiled_commit": [_P, POINTER(asamd_spmv_args), _P, _P, _P, _P, _P],
     "asamd_sums_build": [_P, _I, _I, _I, _I, _I, _P, _P, _P, c_int64, _P],
     "asamd_sums_free": [_P],
     "asamd_sums_refresh_values": [_P, _P, _P, _P],
-    "asamd_spmv_sums": [_P, POINTER(asamd_spmv_args), _P, _P, _P],
+    "asamd_sums_refresh_checked": [_P, _P, _P, _P],
+    "asamd_spmv_sums": [_P, POINTER(asamd_spmv_args), _P, _P],
+    "asamd_spmv_sums_commit": [_P, POINTER(asamd_spmv_args), _P, _P, _P],
     "asamd_hot_build": [_P, _I, _I, _I, _I, _I, _P, _P, _I, _I, _I, _P],
     "asamd_hot_free": [_P],
     "asamd_spmv_hot": [_P, POINTER(asamd_spmv_args), _P, _P, _P, _P, _P],
@@ -376,6 +380,7 @@ _COMMON = {
     "asamd_value_guard_commit": [_P, _P, _P],
     "asamd_value_guard_begin": [_P, _P, c_size_t, _I, _P, _P, _P],
     "asamd_gather_values": [_P, _I, _I, _I, _P, _P, _P, _P],
+    "asamd_gather_checked": [_P, _I, _I, _I, _P, _P, _P, _P],
     "asamd_spmv_xlds": [_P, _P, _I],
     "asamd_spmv_xlds_fits": [_I, _I],
     "asamd_narrow_columns": [_P, _I, _I, _P, _P],

@@ -321,21 +321,30 @@ extern "C" void asamd_sums_free(asamd_sums_layout* L) {
   *L = asamd_sums_layout{};
 }
 
-extern "C" int asamd_sums_refresh_values(hipStream_t s, const asamd_sums_layout* L, const void* val,
-                                         const asamd_value_check* check) {
+static int sums_refresh(hipStream_t s, const asamd_sums_layout* L, const void* val, const GuardGate& gate) {
   if (!L || !L->tval || !L->tperm || !val) return hipErrorInvalidValue;
   return by_dtype(L->dtype, [&](auto* tag) -> int {
     using T = std::remove_pointer_t<decltype(tag)>;
     if ((uintptr_t)val % alignof(T)) return hipErrorInvalidValue;
     // few enough workgroups to return quickly where the gate is shut, and a multiple of the XCDs
     const unsigned grid = (unsigned)(L->spans >= 256 * 8 ? 256 * 8 : (L->spans + kXcds - 1) / kXcds * kXcds);
-    sums_values_kernel<T><<<grid, 256, 0, s>>>(L->spans, L->order, L->tperm, (const T*)val, (T*)L->tval, guard_gate(check));
+    sums_values_kernel<T><<<grid, 256, 0, s>>>(L->spans, L->order, L->tperm, (const T*)val, (T*)L->tval, gate);
     return hipGetLastError();
   });
 }
+extern "C" int asamd_sums_refresh_values(hipStream_t s, const asamd_sums_layout* L, const void* val, const int32_t* gate) {
+  return sums_refresh(s, L, val, guard_gate(gate));
+}
+extern "C" int asamd_sums_refresh_checked(hipStream_t s, const asamd_sums_layout* L, const void* val,
+                                          const asamd_value_check* check) {
+  return sums_refresh(s, L, val, guard_gate(check));
+}
 
-extern "C" int asamd_spmv_sums(hipStream_t s, const asamd_spmv_args* a, const asamd_sums_layout* L, void* sums,
-                               const asamd_value_check* commit) {
+extern "C" int asamd_spmv_sums(hipStream_t s, const asamd_spmv_args* a, const asamd_sums_layout* L, void* sums) {
+  return asamd_spmv_sums_commit(s, a, L, sums, nullptr);
+}
+extern "C" int asamd_spmv_sums_commit(hipStream_t s, const asamd_spmv_args* a, const asamd_sums_layout* L, void* sums,
+                                      const asamd_value_check* commit) {
   if (!a || !L || !L->tval || !sums || !a->alpha || !a->beta || !a->x || !a->y) return hipErrorInvalidValue;
   if (a->dtype != L->dtype || a->m != L->m || a->n != L->n || a->nnz != L->nnz) return hipErrorInvalidValue;
   return by_dtype(a->dtype, [&](auto* tag) -> int {

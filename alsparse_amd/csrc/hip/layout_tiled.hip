@@ -249,7 +249,7 @@ static hipError_t build_tiled(hipStream_t stream, asamd_tiled_layout* L, const i
                                                                                 d_tile_ptr);
     if constexpr (kPayloadSort) {
       L->tile_ptr = d_tile_ptr;  // stays with the layout: the values are gathered tile by tile, now and later
-      launch_gather_tiles<T>(stream, L, val, guard_gate(nullptr));
+      launch_gather_tiles<T>(stream, L, val, guard_gate((const int*)nullptr));
     }
     // Entries in tiles of 65..128 entries: if they are few, phase 2 runs in its one-entry-per-lane form
     // (twice the tiles in flight) and leaves those tiles to phase 3.
@@ -443,7 +443,11 @@ extern "C" void asamd_tiled_free(asamd_tiled_layout* L) {
 // (the tiles too long for phase 2) and its ordered finish.  The layout holds zero-based local indices and
 // its own values.
 extern "C" int asamd_spmv_tiled(hipStream_t s, const asamd_spmv_args* a, const asamd_tiled_layout* L, void* products,
-                                void* long_scratch, const int32_t* skip, const asamd_value_check* commit) {
+                                void* long_scratch, const int32_t* skip) {
+  return asamd_spmv_tiled_commit(s, a, L, products, long_scratch, skip, nullptr);
+}
+extern "C" int asamd_spmv_tiled_commit(hipStream_t s, const asamd_spmv_args* a, const asamd_tiled_layout* L, void* products,
+                                       void* long_scratch, const int32_t* skip, const asamd_value_check* commit) {
   if (!a || !L || !L->tval || !products || !a->alpha || !a->beta || !a->x || !a->y) return hipErrorInvalidValue;
   if (a->dtype != L->dtype || a->m != L->m || a->n != L->n || a->nnz != L->nnz) return hipErrorInvalidValue;
   if (L->n_long_finish > 0 && !long_scratch) return hipErrorInvalidValue;
@@ -491,22 +495,9 @@ extern "C" int asamd_spmv_tiled(hipStream_t s, const asamd_spmv_args* a, const a
   });
 }
 
-extern "C" int asamd_tiled_gather_values(hipStream_t s, const asamd_tiled_layout* L, const void* val,
-                                         const asamd_value_check* check) {
-  if (!L || !L->tval || !L->tperm || !val) return hipErrorInvalidValue;
-  if (L->nnz == 0) return hipSuccess;
-  if (!L->tile_ptr) return asamd_gather_values(s, L->dtype, 0, L->nnz, L->tperm, val, L->tval, check);
-  return by_dtype(L->dtype, [&](auto* tag) -> int {
-    using T = std::remove_pointer_t<decltype(tag)>;
-    if ((uintptr_t)val % alignof(T)) return hipErrorInvalidValue;
-    launch_gather_tiles<T>(s, L, val, guard_gate(check));
-    return hipGetLastError();
-  });
-}
-
 // out[q] = val[perm[q]]: the values of a re-ordered copy taken afresh from the caller's array
-extern "C" int asamd_gather_values(hipStream_t s, int32_t dtype, int32_t conj, int32_t nnz, const uint32_t* perm,
-                                   const void* val, void* out, const asamd_value_check* check) {
+static int gather_values(hipStream_t s, int32_t dtype, int32_t conj, int32_t nnz, const uint32_t* perm, const void* val, void* out,
+                         const GuardGate& gate) {
   if (!perm || !val || !out || nnz < 0) return hipErrorInvalidValue;
   if (nnz == 0) return hipSuccess;
   return by_dtype(dtype, [&](auto* tag) -> int {
@@ -515,9 +506,8 @@ extern "C" int asamd_gather_values(hipStream_t s, int32_t dtype, int32_t conj, i
     if (conj && kIsReal<T>) return hipErrorInvalidValue;
     int64_t grid = ((int64_t)nnz + 256 * 8 - 1) / (256 * 8);
     // (a check that is not settled is worked out by every workgroup: no more of them than the chip holds)
-    const int64_t most = check && !check->settled ? 256 * 8 : 256 * 32;
+    const int64_t most = gate.ws ? 256 * 8 : 256 * 32;
     if (grid > most) grid = most;
-    const GuardGate gate = guard_gate(check);
     if constexpr (!kIsReal<T>) {
       if (conj) {
         gather_values_kernel<T, true><<<(unsigned)grid, 256, 0, s>>>(nnz, perm, (const T*)val, (T*)out, gate);
@@ -527,4 +517,31 @@ extern "C" int asamd_gather_values(hipStream_t s, int32_t dtype, int32_t conj, i
     gather_values_kernel<T, false><<<(unsigned)grid, 256, 0, s>>>(nnz, perm, (const T*)val, (T*)out, gate);
     return hipGetLastError();
   });
+}
+extern "C" int asamd_gather_values(hipStream_t s, int32_t dtype, int32_t conj, int32_t nnz, const uint32_t* perm,
+                                   const void* val, void* out, const int32_t* gate) {
+  return gather_values(s, dtype, conj, nnz, perm, val, out, guard_gate(gate));
+}
+extern "C" int asamd_gather_checked(hipStream_t s, int32_t dtype, int32_t conj, int32_t nnz, const uint32_t* perm,
+                                    const void* val, void* out, const asamd_value_check* check) {
+  return gather_values(s, dtype, conj, nnz, perm, val, out, guard_gate(check));
+}
+
+static int tiled_gather(hipStream_t s, const asamd_tiled_layout* L, const void* val, const GuardGate& gate) {
+  if (!L || !L->tval || !L->tperm || !val) return hipErrorInvalidValue;
+  if (L->nnz == 0) return hipSuccess;
+  if (!L->tile_ptr) return gather_values(s, L->dtype, 0, L->nnz, L->tperm, val, L->tval, gate);
+  return by_dtype(L->dtype, [&](auto* tag) -> int {
+    using T = std::remove_pointer_t<decltype(tag)>;
+    if ((uintptr_t)val % alignof(T)) return hipErrorInvalidValue;
+    launch_gather_tiles<T>(s, L, val, gate);
+    return hipGetLastError();
+  });
+}
+extern "C" int asamd_tiled_gather_values(hipStream_t s, const asamd_tiled_layout* L, const void* val, const int32_t* gate) {
+  return tiled_gather(s, L, val, guard_gate(gate));
+}
+extern "C" int asamd_tiled_gather_checked(hipStream_t s, const asamd_tiled_layout* L, const void* val,
+                                          const asamd_value_check* check) {
+  return tiled_gather(s, L, val, guard_gate(check));
 }

@@ -27,19 +27,19 @@ extern "C" int asamd_patterns_build(hipStream_t s, int32_t m, int32_t nnz, int32
   const size_t lds = (size_t)rows_per_group * (size_t)max_len * sizeof(int);
   if (lds > (size_t)64 * 1024) return hipSuccess;
   const size_t pid_bytes = ((size_t)m + 255) & ~(size_t)255;
-  const size_t dist_bytes = (size_t)kPatternSlots * (size_t)max_len * sizeof(int);
+  const size_t dist_bytes = (size_t)kPatternSlots * ((size_t)max_len + 1) * sizeof(int);  // (and the lengths)
   const unsigned grid = (unsigned)(((int64_t)m + rows_per_group - 1) / rows_per_group);
-  const size_t off_bytes = ((size_t)grid * kPatternWaves + 1) * sizeof(int);
+  const size_t off_bytes = ((size_t)grid + 1 + (size_t)grid * kPatternWaves + 1) * sizeof(int);
   char* block = nullptr;
   hipError_t e = hipMalloc((void**)&block, pid_bytes + dist_bytes + sizeof(PatternScratch) + off_bytes);
   if (e != hipSuccess) return e;
   unsigned char* pid = (unsigned char*)block;
   int* dist = (int*)(block + pid_bytes);
   PatternScratch* tab = (PatternScratch*)(block + pid_bytes + dist_bytes);
-  int* wave_off = (int*)(tab + 1);
+  int* block_off = (int*)(tab + 1);
   pattern_clear_kernel<<<1, kPatternSlots, 0, s>>>(tab);
   pattern_rows_kernel<<<grid, kStreamRows, lds, s>>>(m, base, rows_per_group, max_len, row_ptr, col_ind, tab, pid,
-                                                     wave_off);
+                                                     block_off, block_off + grid + 1);
   pattern_table_kernel<<<kPatternSlots, kWave, 0, s>>>(base, max_len, row_ptr, col_ind, tab, dist);
   pattern_verify_kernel<<<grid, kStreamRows, lds, s>>>(m, base, rows_per_group, max_len, row_ptr, col_ind, pid, dist, tab);
   int fail = 1;
@@ -52,8 +52,7 @@ extern "C" int asamd_patterns_build(hipStream_t s, int32_t m, int32_t nnz, int32
   }
   out->pid = pid;
   out->dist = dist;
-  out->len = tab->len;
-  out->wave_off = wave_off;
+  out->block_off = block_off;
   out->stride = max_len;
   out->group = group;
   out->device_bytes = (int64_t)(pid_bytes + dist_bytes + sizeof(PatternScratch) + off_bytes);
@@ -67,7 +66,7 @@ extern "C" void asamd_patterns_free(asamd_pattern_layout* layout) {
 }
 
 extern "C" int asamd_spmv_patterns(hipStream_t s, const asamd_spmv_args* a, const asamd_pattern_layout* L) {
-  if (!a || !L || !L->pid || !L->dist || !L->len || !L->wave_off) return hipErrorInvalidValue;
+  if (!a || !L || !L->pid || !L->dist || !L->block_off) return hipErrorInvalidValue;
   static const int forced = getenv("ALSPARSE_AMD_STREAM_POLICY") ? atoi(getenv("ALSPARSE_AMD_STREAM_POLICY")) : -1;
   // us per multiply, the same arrays again and again / four sets in turn, values cached against not:
   //   5-point Laplacian 2048^2, fp64 (256 MB)      34 / 50 against 41 / 50     fp32 (138 MB)    22 / 32 against 28 / 28
@@ -82,16 +81,16 @@ extern "C" int asamd_spmv_patterns(hipStream_t s, const asamd_spmv_args* a, cons
   const bool early = !ntv && bytes <= 150.0e6;  // (the kernel has both sides)
   const int g = L->group;
   const unsigned grid = (unsigned)(((int64_t)a->m * g + kStreamRows - 1) / kStreamRows);
+  const int *lens = L->dist + kPatternSlots * L->stride, *wave_off = L->block_off + grid + 1;
   auto go = [&](auto* tag) -> int {
     using T = std::remove_pointer_t<decltype(tag)>;
     if (!args_ok<T>(a)) return hipErrorInvalidValue;
     constexpr int kCap = 64 / (int)sizeof(T);  // 16 KiB of values per workgroup
     if (((uintptr_t)a->val & 15u) != 0 || L->stride > kCap * g) return hipErrorInvalidValue;
     const T alpha = scalar_of<T>(a->alpha), beta = scalar_of<T>(a->beta);
-#define ASAMD_PATTERN_LAUNCH_AS(U, G, NTV, EARLY)                                                                    \
-  spmv_pattern_kernel<T, U, G, NTV, EARLY><<<grid, kStreamRows, 0, s>>>(a->m, alpha, (const T*)a->val, L->pid,       \
-                                                                        L->dist, L->stride, L->len, L->wave_off,     \
-                                                                        (const T*)a->x, beta, (T*)a->y)
+#define ASAMD_PATTERN_LAUNCH_AS(U, G, NTV, EARLY)          \
+  spmv_pattern_kernel<T, U, G, NTV, EARLY><<<grid, kStreamRows, 0, s>>>( \
+      a->m, alpha, (const T*)a->val, L->pid, L->dist, L->stride, lens, wave_off, (const T*)a->x, beta, (T*)a->y)
 #define ASAMD_PATTERN_LAUNCH(U, G)                             \
   do {                                                         \
     if (ntv) ASAMD_PATTERN_LAUNCH_AS(U, G, true, false);       \

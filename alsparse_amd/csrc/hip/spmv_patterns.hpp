@@ -45,6 +45,7 @@ static __global__ __launch_bounds__(kStreamRows) void pattern_rows_kernel(int m,
                                                                           const int* __restrict__ col_ind,
                                                                           PatternScratch* __restrict__ tab,
                                                                           unsigned char* __restrict__ pid,
+                                                                          int* __restrict__ block_off,
                                                                           int* __restrict__ wave_off) {
   extern __shared__ int s_col[];
   if (__atomic_load_n(&tab->fail, __ATOMIC_RELAXED)) return;
@@ -56,6 +57,10 @@ static __global__ __launch_bounds__(kStreamRows) void pattern_rows_kernel(int m,
   if (n < 0 || n > (int64_t)rows_per_group * max_len) {  // (not the offsets that the row statistics were taken from)
     if (threadIdx.x == 0) atomicOr(&tab->fail, 1);
     return;
+  }
+  if (threadIdx.x == 0) {
+    block_off[blockIdx.x] = (int)lo;
+    if (row_last == m) block_off[blockIdx.x + 1] = (int)(lo + n);
   }
   if ((int)threadIdx.x < kPatternWaves) {
     const int64_t r = row0 + (int64_t)threadIdx.x * (rows_per_group / kPatternWaves);
@@ -99,8 +104,8 @@ static __global__ __launch_bounds__(kStreamRows) void pattern_rows_kernel(int m,
   atomicOr(&tab->fail, 1);
 }
 
-// dist[slot * stride + s] = the s-th distance of the slot's pattern (its last one repeated up to the stride).  A
-// workgroup of one wave per slot.
+// dist[slot * stride + s] = the s-th distance of the slot's pattern (its last one repeated up to the stride), and behind
+// all of them the patterns' lengths.  A workgroup of one wave per slot.
 static __global__ __launch_bounds__(kWave) void pattern_table_kernel(int base, int stride, const int* __restrict__ row_ptr,
                                                                      const int* __restrict__ col_ind,
                                                                      const PatternScratch* __restrict__ tab,
@@ -111,6 +116,7 @@ static __global__ __launch_bounds__(kWave) void pattern_table_kernel(int base, i
   const int64_t begin = (int64_t)row_ptr[row] - base;
   for (int s = threadIdx.x; s < stride; s += kWave)
     dist[slot * stride + s] = col_ind[begin + (s < len ? s : len - 1)] - base - row;
+  if (threadIdx.x == 0) dist[kPatternSlots * stride + slot] = len;
 }
 
 // Every row against its pattern, entry by entry: the table is exact, whatever the hashes did.

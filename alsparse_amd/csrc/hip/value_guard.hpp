@@ -43,19 +43,19 @@ __device__ __forceinline__ unsigned long long guard_fingerprint(const GuardWs* w
   return block_sum_u64(mine) ^ salt;
 }
 
-// What a kernel that refreshes a copy goes by.  Not settled: the pass over the values has left partial sums, and every
-// workgroup adds them up itself (16 KB that all of them find in their L2) instead of waiting for a launch that does it
-// once; the first one leaves word and flag for the kernels behind.
+// What a kernel that refreshes a copy goes by: a flag, or a check that is not settled: the pass over the values has left
+// partial sums, and every workgroup adds them up itself (16 KB that all of them find in their L2) instead of waiting for a
+// launch that does it once; the first one leaves word and flag for the kernels behind.
 struct GuardGate {
-  GuardWs* ws;  // null: refresh
+  const int* flag;  // zero: the values have not changed
+  GuardWs* ws;      // neither this nor a flag: refresh
   const unsigned long long* stored;
   unsigned long long salt;
-  bool settled;
 };
 // whether to refresh; all 256 threads of every workgroup come here
 __device__ __forceinline__ bool guard_open(const GuardGate& g) {
+  if (g.flag) return *g.flag != 0;
   if (!g.ws) return true;
-  if (g.settled) return g.ws->flag != 0;
   __shared__ int s_changed;
   const unsigned long long fp = guard_fingerprint(g.ws, g.salt);
   if (threadIdx.x == 0) {
@@ -79,9 +79,10 @@ __device__ __forceinline__ void guard_commit(const GuardCommit& c) {
   if (c.ws && blockIdx.x == 0 && threadIdx.x == 0 && c.ws->flag) *c.stored = c.ws->fp;
 }
 
+inline GuardGate guard_gate(const int* flag) { return GuardGate{flag, nullptr, nullptr, 0}; }
 inline GuardGate guard_gate(const asamd_value_check* c) {
-  if (!c) return GuardGate{nullptr, nullptr, 0, true};
-  return GuardGate{(GuardWs*)c->ws, (const unsigned long long*)c->stored, guard_salt(c->words), c->settled != 0};
+  if (!c || c->settled) return guard_gate(c ? ASAMD_GUARD_FLAG(c->ws) : (const int*)nullptr);
+  return GuardGate{nullptr, (GuardWs*)c->ws, (const unsigned long long*)c->stored, guard_salt(c->words)};
 }
 inline GuardCommit guard_commit_of(const asamd_value_check* c) {
   return c ? GuardCommit{(const GuardWs*)c->ws, (unsigned long long*)c->stored} : GuardCommit{nullptr, nullptr};

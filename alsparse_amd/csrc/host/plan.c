@@ -619,7 +619,7 @@ static int run_algo(hipStream_t s, const asamd_csr_plan *p, int algo, const asam
       void *prod = ws_take(&ws, (size_t)st->nnz * vs);
       void *lscr = p->tiled.long_scratch_elems > 0 ? ws_take(&ws, (size_t)p->tiled.long_scratch_elems * vs) : NULL;
       if (!prod || (p->tiled.long_scratch_elems > 0 && !lscr)) return -1;
-      return asamd_spmv_tiled(s, a, &p->tiled, prod, lscr, NULL, commit);
+      return asamd_spmv_tiled_commit(s, a, &p->tiled, prod, lscr, NULL, commit);
     }
     case ASAMD_SPMV_ROWCONST:
       return asamd_spmv_rowconst(s, a, st->const_len);
@@ -678,7 +678,7 @@ static hipError_t refresh_main(hipStream_t s, asamd_csr_plan *p, const int32_t *
   const int32_t *gate = check ? ASAMD_GUARD_FLAG(check->ws) : NULL;
   hipError_t e = hipSuccess;
   if (st->tiled_built)
-    e = (hipError_t)asamd_tiled_gather_values(s, &p->tiled, val, check);
+    e = (hipError_t)asamd_tiled_gather_checked(s, &p->tiled, val, check);
   if (e == hipSuccess && st->ell_built)
     e = (hipError_t)asamd_csr2ell_gated(s, p->val_size, st->m, val, rp, ci, st->base, 0, st->ell_width, p->d_eval,
                                         p->d_ecol, gate);
@@ -689,10 +689,10 @@ static hipError_t refresh_main(hipStream_t s, asamd_csr_plan *p, const int32_t *
 /* ... and one transposed copy with everything its own analysis keeps; settles the check */
 static hipError_t refresh_trans(hipStream_t s, asamd_csr_plan *p, int which, const void *val, asamd_value_check *check) {
   asamd_trans_copy *t = &p->tr[which];
-  hipError_t e = (hipError_t)asamd_gather_values(s, p->dtype, which == 1, p->st.nnz, t->t.perm, val, t->t.val, check);
+  hipError_t e = (hipError_t)asamd_gather_checked(s, p->dtype, which == 1, p->st.nnz, t->t.perm, val, t->t.val, check);
   if (check) check->settled = 1;
   if (e == hipSuccess) e = refresh_main(s, t->plan, t->t.row_ptr, t->t.col_ind, t->t.val, check);
-  if (e == hipSuccess && t->plan->sums.tval) e = (hipError_t)asamd_sums_refresh_values(s, &t->plan->sums, t->t.val, check);
+  if (e == hipSuccess && t->plan->sums.tval) e = (hipError_t)asamd_sums_refresh_checked(s, &t->plan->sums, t->t.val, check);
   return e;
 }
 
@@ -714,11 +714,11 @@ static int csrmv_sums(hipStream_t s, asamd_csr_plan *p, const asamd_spmv_args *a
   if (g) {
     int e = asamd_value_guard_begin(s, a->val, (size_t)st->nnz * (size_t)p->val_size, sums_check_all(p), p->d_fp + FP_SUMS, g,
                                     &check);
-    if (e == hipSuccess) e = asamd_sums_refresh_values(s, &p->sums, a->val, &check);
+    if (e == hipSuccess) e = asamd_sums_refresh_checked(s, &p->sums, a->val, &check);
     if (e != hipSuccess) return e;
     commit = &check;
   }
-  return asamd_spmv_sums(s, a, &p->sums, sums, commit);
+  return asamd_spmv_sums_commit(s, a, &p->sums, sums, commit);
 }
 
 /* commit: NULL, or a check whose copies have been refreshed (guard == 0): recorded by the multiply, or in front of it */
@@ -949,7 +949,7 @@ int asamd_csr_plan_csrmv_watched(hipStream_t s, asamd_csr_plan *p, const void *a
   fill_args(&a, p, alpha, val, rp, ci, x, beta, y);
   /* the layout's kernels, which return at once if the structure has changed, and the stand-in on the caller's
    * arrays, which returns at once if it has not */
-  if (e == hipSuccess) e = asamd_spmv_tiled(s, &a, &p->tiled, prod, lscr, skip, NULL);
+  if (e == hipSuccess) e = asamd_spmv_tiled(s, &a, &p->tiled, prod, lscr, skip);
   if (e == hipSuccess) e = asamd_spmv_vector_if(s, &a, p->auto_width, skip);
   if (changed) *changed = skip;
   return e;

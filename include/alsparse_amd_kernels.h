@@ -164,9 +164,9 @@ int asamd_spmv_stream(hipStream_t stream, const asamd_spmv_args *a, int32_t grou
  * counterpart in the reference, whose kernel reads every column: dcu_gemv_vector.h:14-57.) */
 typedef struct {
   unsigned char *pid;   /* m pattern numbers; NULL: no layout (owns the one allocation) */
-  int32_t *dist;        /* 256 x stride distances */
-  int32_t *len;         /* 256 lengths                                                  */
-  int32_t *wave_off;    /* where the entries of every 64 / group rows begin, and the last ones' end */
+  int32_t *dist;        /* 256 x stride distances, then the 256 patterns' lengths */
+  int32_t *block_off;   /* where the entries of every workgroup's 256 / group rows begin, and the last one's end; then the same
+                           for the 64 / group rows of every wave of those workgroups */
   int32_t stride, group;
   int64_t device_bytes;
 } asamd_pattern_layout;
@@ -267,15 +267,20 @@ int asamd_tiled_build(hipStream_t stream, int32_t dtype, int32_t m, int32_t n, i
 void asamd_tiled_free(asamd_tiled_layout *layout);
 /* layout->tval[q] = val[layout->tperm[q]] for every slot, the tiles taken row block by row block (each XCD its
  * own row blocks), so that the stretch of val a row block's tiles pick their values from is fetched from memory
- * once; check as for asamd_gather_values */
+ * once; gate, check as for asamd_gather_values and asamd_gather_checked */
 int asamd_tiled_gather_values(hipStream_t stream, const asamd_tiled_layout *layout, const void *val,
-                              const asamd_value_check *check);
+                              const int32_t *gate);
+int asamd_tiled_gather_checked(hipStream_t stream, const asamd_tiled_layout *layout, const void *val,
+                               const asamd_value_check *check);
 /* y = alpha*A*x + beta*y from the layout (a->val, a->row_ptr, a->col_ind are not read).  skip: NULL, or a
  * device word; when it is non-zero the kernels that write y return at once (a guard found that the layout no
- * longer describes the caller's matrix, and asamd_spmv_vector_if on the same word computes y instead).
- * commit: NULL, or a settled check whose fingerprint the second phase records */
+ * longer describes the caller's matrix, and asamd_spmv_vector_if on the same word computes y instead). */
 int asamd_spmv_tiled(hipStream_t stream, const asamd_spmv_args *a, const asamd_tiled_layout *layout,
-                     void *products, void *long_scratch, const int32_t *skip, const asamd_value_check *commit);
+                     void *products, void *long_scratch, const int32_t *skip);
+/* ... commit: NULL, or the check of a refreshing kernel in front, which has left its verdict in the scratch: the second
+ * phase records the fingerprint */
+int asamd_spmv_tiled_commit(hipStream_t stream, const asamd_spmv_args *a, const asamd_tiled_layout *layout, void *products,
+                            void *long_scratch, const int32_t *skip, const asamd_value_check *commit);
 
 /* The tiled pair for rows that meet a column block more than once (long rows, power-law graphs): phase 1 adds up what a
  * row has in a column block and writes one value for it.  Holds the values (tval) and the CSR position of every slot
@@ -300,12 +305,15 @@ int asamd_sums_build(hipStream_t stream, int32_t dtype, int32_t m, int32_t n, in
                      const int32_t *row_ptr, const int32_t *col_ind, const void *val, int64_t most_sums,
                      asamd_sums_layout *out);
 void asamd_sums_free(asamd_sums_layout *layout);
-/* the values taken afresh from val; check as for asamd_gather_values */
-int asamd_sums_refresh_values(hipStream_t stream, const asamd_sums_layout *layout, const void *val,
-                              const asamd_value_check *check);
-/* y = alpha*A*x + beta*y from the layout (a->val, a->row_ptr, a->col_ind are not read); commit as for asamd_spmv_tiled */
-int asamd_spmv_sums(hipStream_t stream, const asamd_spmv_args *a, const asamd_sums_layout *layout, void *sums,
-                    const asamd_value_check *commit);
+/* the values taken afresh from val; gate, check as for asamd_gather_values and asamd_gather_checked */
+int asamd_sums_refresh_values(hipStream_t stream, const asamd_sums_layout *layout, const void *val, const int32_t *gate);
+int asamd_sums_refresh_checked(hipStream_t stream, const asamd_sums_layout *layout, const void *val,
+                               const asamd_value_check *check);
+/* y = alpha*A*x + beta*y from the layout (a->val, a->row_ptr, a->col_ind are not read) */
+int asamd_spmv_sums(hipStream_t stream, const asamd_spmv_args *a, const asamd_sums_layout *layout, void *sums);
+/* ... commit as for asamd_spmv_tiled_commit */
+int asamd_spmv_sums_commit(hipStream_t stream, const asamd_spmv_args *a, const asamd_sums_layout *layout, void *sums,
+                           const asamd_value_check *commit);
 
 /* Hot-column merge-path for power-law columns: the column stream rewritten as ranks of the popular
  * columns (pcol), whose x sits in LDS (the cols_lds most popular) or in a compact front (cols_front).
@@ -396,8 +404,8 @@ int asamd_csr_locality_probe(hipStream_t stream, int32_t nnz, int32_t base, int3
  *                          full != 0, otherwise 256 bytes at a varying position of every run of
  *                          asamd_value_guard_run(nbytes) bytes, 32 MiB in all), compares with the word
  *                          at `stored` and leaves the verdict in ws: a flag and the new fingerprint;
- *   gated kernels          (asamd_gather_values, asamd_csr2ell_gated) take a check, or the flag's address, and
- *                          return at once when the values have not changed;
+ *   gated kernels          (asamd_gather_values, asamd_csr2ell_gated) take the flag's address and return
+ *                          at once when it is 0;
  *   asamd_value_guard_commit   stores the new fingerprint at `stored` if the flag is set -- AFTER the
  *                          gated kernels in stream order, so that another stream that finds the stored
  *                          word up to date also finds the copies refreshed.
@@ -409,16 +417,20 @@ size_t asamd_value_guard_run(size_t nbytes);
 int asamd_value_guard(hipStream_t stream, const void *val, size_t nbytes, int32_t full, const uint64_t *stored,
                       void *ws);
 int asamd_value_guard_commit(hipStream_t stream, const void *ws, uint64_t *stored);
-/* The same in two launches less: the fingerprint's partial sums, of which the first refreshing kernel works out the verdict
- * itself (and leaves it in ws: `settled` for any other behind it), and which the multiply records (`commit`). */
+/* The same in two launches less: the fingerprint's partial sums, of which the first refreshing kernel (asamd_gather_checked
+ * and its like) works out the verdict itself and leaves it in ws -- the caller sets `settled` for any other behind it -- and
+ * which the multiply records (`commit`). */
 int asamd_value_guard_begin(hipStream_t stream, const void *val, size_t nbytes, int32_t full, uint64_t *stored, void *ws,
                             asamd_value_check *check);
 /* *out = 1 if either of two guards' flags is set, else 0 (the guard works on any array of 4-byte words: the
  * structure arrays of a matrix that nobody promised to leave alone are watched with it too) */
 int asamd_value_guard_any(hipStream_t stream, const void *ws_a, const void *ws_b, int32_t *out);
-/* out[q] = val[perm[q]] (conj != 0: conjugated) for q < nnz; check: NULL, or a check (unchanged values: does nothing) */
+/* out[q] = val[perm[q]] (conj != 0: conjugated) for q < nnz; gate: NULL, or a device flag (0 = do nothing) */
 int asamd_gather_values(hipStream_t stream, int32_t dtype, int32_t conj, int32_t nnz, const uint32_t *perm,
-                        const void *val, void *out, const asamd_value_check *check);
+                        const void *val, void *out, const int32_t *gate);
+/* ... check: NULL, or a check (unchanged values: does nothing) */
+int asamd_gather_checked(hipStream_t stream, int32_t dtype, int32_t conj, int32_t nnz, const uint32_t *perm,
+                         const void *val, void *out, const asamd_value_check *check);
 
 /* y = alpha*op(A)*x + beta*y without any analysis, in the traversal of the reference's plain
  * kernels: op = 0 one lane per row summing its entries in storage order

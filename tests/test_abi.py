@@ -112,6 +112,27 @@ int main(void) {
     assert nums[7] == [ctypes.sizeof(DV), DV.values.offset, DV.data_type.offset]
 
 
+def test_kernel_interfaces_that_callers_bind_stay(tmp_path):
+    """The signatures and the record of include/alsparse_amd_kernels.h that a dispatch layer outside this library was built
+    against: a device flag gates the refreshing kernels, a pattern record is five words."""
+    src = tmp_path / "bound.c"
+    src.write_text(r'''
+#include <stddef.h>
+#include "alsparse_amd_kernels.h"
+typedef const int32_t *flag;
+int (*gather)(hipStream_t, int32_t, int32_t, int32_t, const uint32_t *, const void *, void *, flag) = asamd_gather_values;
+int (*tiled_gather)(hipStream_t, const asamd_tiled_layout *, const void *, flag) = asamd_tiled_gather_values;
+int (*sums_refresh)(hipStream_t, const asamd_sums_layout *, const void *, flag) = asamd_sums_refresh_values;
+int (*tiled)(hipStream_t, const asamd_spmv_args *, const asamd_tiled_layout *, void *, void *, flag) = asamd_spmv_tiled;
+int (*sums)(hipStream_t, const asamd_spmv_args *, const asamd_sums_layout *, void *) = asamd_spmv_sums;
+_Static_assert(sizeof(asamd_pattern_layout) == 40 && offsetof(asamd_pattern_layout, block_off) == 16 &&
+               offsetof(asamd_pattern_layout, group) == 28 && offsetof(asamd_pattern_layout, device_bytes) == 32, "pattern record");
+''')
+    subprocess.check_call(["gcc", "-std=c11", "-Wall", "-Werror", "-fsyntax-only", str(src),
+                           "-I" + os.path.join(ROOT, "include"), "-I/opt/rocm/include"])
+    assert ctypes.sizeof(capi.asamd_pattern_layout) == 40
+
+
 def test_no_product_code_touches_the_oracle():
     """The shipped library and package must not import, link or call anything under oracle/."""
     bad = []

@@ -56,3 +56,22 @@ def test_fingerprint_is_the_sum_over_the_words(gpu, words, full, offset):
     finally:
         for x in (d, ws, stored):
             x.free()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.complex128], ids=["f32", "c128"])
+@pytest.mark.parametrize("flag", [None, 0, 1])
+def test_a_flag_gates_the_gather(gpu, flag, dtype):
+    """asamd_gather_values takes the address of a flag on the device, or nothing."""
+    lib = capi.load()
+    rng = np.random.default_rng(5)
+    n, code = 70001, {"float32": 0, "complex128": 3}[np.dtype(dtype).name]
+    host, perm = rng.integers(0, 1 << 20, size=n).astype(dtype), rng.permutation(n).astype(np.uint32)
+    d = [hiprt.DeviceArray.from_numpy(v) for v in (host, perm, np.full(n, 7, dtype), np.array([flag or 0], np.int32))]
+    try:
+        announce("gather behind a flag", flag, np.dtype(dtype).name)
+        assert lib.asamd_gather_values(None, code, 0, n, d[1].c_ptr(), d[0].c_ptr(), d[2].c_ptr(),
+                                       None if flag is None else d[3].c_ptr()) == 0
+        assert np.array_equal(d[2].to_numpy(), np.full(n, 7, dtype) if flag == 0 else host[perm])
+    finally:
+        for x in d:
+            x.free()
