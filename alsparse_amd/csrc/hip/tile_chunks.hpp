@@ -37,17 +37,15 @@ inline int chunk_limit(const std::vector<int>& sizes, int64_t unit_bytes, int64_
   return best;
 }
 
-// The order in which chunks are handed to workgroups: workgroup i runs on XCD i % xcds, so every XCD gets a list of its own,
-// a column block's chunks on one XCD as far as the lists stay even, the longest chunks first (the short ones even out the
-// workgroups' ends).  size[i]: chunk i; block[i]: its column block, ascending.
-inline std::vector<int> chunk_order(const std::vector<int>& size, const std::vector<int>& block, int xcds) {
-  const int n = (int)size.size();
+// A list of chunks for every XCD: a column block's chunks in one list as far as the lists stay even, the longest chunks first
+// (the short ones even out the workgroups' ends).  size[i]: chunk i; block[i]: its column block, ascending.
+inline std::vector<std::vector<int>> chunk_lists(const std::vector<int>& size, const std::vector<int>& block, int xcds) {
   int64_t all = 0;
   for (int s : size) all += s;
   std::vector<std::vector<int>> list((size_t)xcds);
   std::vector<int64_t> load((size_t)xcds, 0);
   size_t to = 0;
-  for (int i = 0; i < n; ++i) {
+  for (int i = 0; i < (int)size.size(); ++i) {
     if (i == 0 || block[(size_t)i] != block[(size_t)i - 1] || (load[to] + size[(size_t)i]) * xcds > all)
       to = (size_t)(std::min_element(load.begin(), load.end()) - load.begin());
     list[to].push_back(i);
@@ -55,9 +53,16 @@ inline std::vector<int> chunk_order(const std::vector<int>& size, const std::vec
   }
   for (auto& l : list)
     std::stable_sort(l.begin(), l.end(), [&](int a, int b) { return size[(size_t)a] > size[(size_t)b]; });
+  return list;
+}
+
+// The order in which chunks are handed to workgroups: workgroup i runs on XCD i % xcds, so the lists' chunks in turn.  Where a
+// list has ended, those behind it move up: the last, shortest chunks of the longer lists run on other XCDs than their list's.
+inline std::vector<int> chunk_order(const std::vector<int>& size, const std::vector<int>& block, int xcds) {
+  const std::vector<std::vector<int>> list = chunk_lists(size, block, xcds);
   std::vector<int> order;
-  order.reserve((size_t)n);
-  for (size_t at = 0; order.size() < (size_t)n; ++at)
+  order.reserve(size.size());
+  for (size_t at = 0; order.size() < size.size(); ++at)
     for (const auto& l : list)
       if (at < l.size()) order.push_back(l[at]);
   return order;
