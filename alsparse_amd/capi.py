@@ -152,6 +152,17 @@ class asamd_xlds_layout(Structure):  # include/alsparse_amd_kernels.h
                 ("dtype", c_int32), ("nnz", c_int32), ("base", c_int32)]
 
 
+class asamd_value_check(Structure):  # include/alsparse_amd_kernels.h
+    _fields_ = [("ws", c_void_p), ("stored", c_void_p), ("words", ctypes.c_int64), ("settled", c_int32)]
+
+
+class asamd_sums_layout(Structure):  # include/alsparse_amd_kernels.h
+    _fields_ = ([(n, c_void_p) for n in ("tval", "tperm", "tcol", "srow", "row_block_start", "run_ptr", "span_sum", "order", "runs",
+                                         "chunks")] +
+                [(n, c_int32) for n in ("dtype", "m", "n", "nnz", "col_blocks", "row_blocks", "rows_cap", "sums", "spans", "n_runs",
+                                        "n_chunks")] + [("device_bytes", ctypes.c_int64)])
+
+
 class asamd_pattern_layout(Structure):  # include/alsparse_amd_kernels.h
     _fields_ = [("pid", c_void_p), ("dist", c_void_p), ("block_off", c_void_p), ("stride", c_int32), ("group", c_int32),
                 ("device_bytes", ctypes.c_int64)]
@@ -364,6 +375,7 @@ _COMMON = {
     "asamd_sums_refresh_checked": [_P, _P, _P, _P],
     "asamd_spmv_sums": [_P, POINTER(asamd_spmv_args), _P, _P],
     "asamd_spmv_sums_commit": [_P, POINTER(asamd_spmv_args), _P, _P, _P],
+    "asamd_spmv_sums_form": [_P, POINTER(asamd_spmv_args), _P, _P, _P, _I],
     "asamd_hot_build": [_P, _I, _I, _I, _I, _I, _P, _P, _I, _I, _I, _P],
     "asamd_hot_free": [_P],
     "asamd_spmv_hot": [_P, POINTER(asamd_spmv_args), _P, _P, _P, _P, _P],

@@ -341,11 +341,16 @@ extern "C" int asamd_sums_refresh_checked(hipStream_t s, const asamd_sums_layout
 }
 
 extern "C" int asamd_spmv_sums(hipStream_t s, const asamd_spmv_args* a, const asamd_sums_layout* L, void* sums) {
-  return asamd_spmv_sums_commit(s, a, L, sums, nullptr);
+  return asamd_spmv_sums_form(s, a, L, sums, nullptr, -1);
 }
 extern "C" int asamd_spmv_sums_commit(hipStream_t s, const asamd_spmv_args* a, const asamd_sums_layout* L, void* sums,
                                       const asamd_value_check* commit) {
-  if (!a || !L || !L->tval || !sums || !a->alpha || !a->beta || !a->x || !a->y) return hipErrorInvalidValue;
+  return asamd_spmv_sums_form(s, a, L, sums, commit, -1);
+}
+extern "C" int asamd_spmv_sums_form(hipStream_t s, const asamd_spmv_args* a, const asamd_sums_layout* L, void* sums,
+                                    const asamd_value_check* commit, int32_t form) {
+  if (!a || !L || !L->tval || !sums || !a->alpha || !a->beta || !a->x || !a->y || form < -1 || form > 2)
+    return hipErrorInvalidValue;
   if (a->dtype != L->dtype || a->m != L->m || a->n != L->n || a->nnz != L->nnz) return hipErrorInvalidValue;
   return by_dtype(a->dtype, [&](auto* tag) -> int {
     using T = std::remove_pointer_t<decltype(tag)>;
@@ -366,9 +371,12 @@ extern "C" int asamd_spmv_sums_commit(hipStream_t s, const asamd_spmv_args* a, c
     // 20 fp32 (190 MB) 83 / 88.
     const int64_t sum_bytes = (int64_t)L->sums * (int64_t)sizeof(T);
     const int64_t stream_bytes = (int64_t)L->spans * SumsDims<T>::span * ((int64_t)sizeof(T) + 2);
-    if (sum_bytes > ((int64_t)512 << 20)) products(sums_products_kernel<T, true, true>);
-    else if (sum_bytes + stream_bytes > (int64_t)256000000) products(sums_products_kernel<T, false, true>);
-    else products(sums_products_kernel<T, false, false>);
+    const int by_size = sum_bytes > ((int64_t)512 << 20) ? 2 : sum_bytes + stream_bytes > (int64_t)256000000 ? 1 : 0;
+    switch (form < 0 ? by_size : form) {
+      case 0: products(sums_products_kernel<T, false, false>); break;
+      case 1: products(sums_products_kernel<T, false, true>); break;
+      default: products(sums_products_kernel<T, true, true>);
+    }
     const unsigned grid = (unsigned)((L->row_blocks + kRedWaves - 1) / kRedWaves);
     tiled_reduce_kernel<T, 1, true><<<grid, kRedWaves * kWave, sums_red_lds<T>(L->rows_cap), s>>>(
         L->row_blocks, 0, L->rows_cap, L->row_block_start, L->run_ptr, (const TileRange*)L->runs, L->srow, mid, alpha, beta,

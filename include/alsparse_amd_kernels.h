@@ -314,6 +314,10 @@ int asamd_spmv_sums(hipStream_t stream, const asamd_spmv_args *a, const asamd_su
 /* ... commit as for asamd_spmv_tiled_commit */
 int asamd_spmv_sums_commit(hipStream_t stream, const asamd_spmv_args *a, const asamd_sums_layout *layout, void *sums,
                            const asamd_value_check *commit);
+/* ... form: -1 (what the others run): by the layout's size, else 0 everything through the memory-side cache, 1 values and
+ * columns past it, 2 the sums too.  The same bits in every form. */
+int asamd_spmv_sums_form(hipStream_t stream, const asamd_spmv_args *a, const asamd_sums_layout *layout, void *sums,
+                         const asamd_value_check *commit, int32_t form);
 
 /* Hot-column merge-path for power-law columns: the column stream rewritten as ranks of the popular
  * columns (pcol), whose x sits in LDS (the cols_lds most popular) or in a compact front (cols_front).

@@ -3,7 +3,7 @@ again.  The reference has one kernel for every structure (src/kernel/dcu/level2/
 
 The tolerance is the textbook bound of a sum of L products in any order, gamma = (L + 4) u per row, against the sum of the
 absolute products in 64 bits (complex products: four roundings each, so twice that)."""
-from ctypes import byref, c_void_p
+from ctypes import addressof, byref, c_void_p, cast
 
 import numpy as np
 import pytest
@@ -121,6 +121,44 @@ def test_edges_against_64_bits(gpu, shape, dtype):
             assert np.array_equal(y, p.multiply(alpha, x, beta, y0)), "the same bits on every run"
     finally:
         p.close()
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=["f32", "f64", "c64", "c128"])
+@pytest.mark.parametrize("shape", ["past_the_edge", "hubs", "span_edges", "uneven_pieces"])
+def test_every_form_of_the_first_phase(gpu, shape, dtype):
+    """Loads and stores through the memory-side cache or past it, which the layout's size decides otherwise (256 MB of streams
+    and sums, 512 MB of sums): one sum per row and column block, the same bits in all three."""
+    a = SHAPES[shape](dtype)
+    rng = np.random.default_rng(21)
+    x, y0 = _numbers(rng, a.cols, dtype), _numbers(rng, a.rows, dtype)
+    lib, T, layout, da = capi.load(), capi.scalar_type(dtype), capi.asamd_sums_layout(), DeviceCsr(a)
+    alpha, beta = T(-1.5), T(0.5)
+    dx, dy, sums = hiprt.DeviceArray.from_numpy(x), hiprt.DeviceArray.from_numpy(y0), None
+    try:
+        assert lib.asamd_sums_build(None, capi.dtype_tag(a.dtype), a.rows, a.cols, a.nnz, a.base, da.row_ptr.c_ptr(),
+                                    da.col.c_ptr(), da.val.c_ptr(), a.nnz, byref(layout)) == 0
+        assert layout.tval and layout.nnz == a.nnz and 0 < layout.sums <= a.nnz
+        sums = hiprt.DeviceArray((layout.sums,), a.dtype)
+        args = capi.asamd_spmv_args(capi.dtype_tag(a.dtype), a.rows, a.cols, a.nnz, a.base, cast(addressof(alpha), c_void_p),
+                                    cast(addressof(beta), c_void_p), da.val.c_ptr(), da.row_ptr.c_ptr(), da.col.c_ptr(),
+                                    dx.c_ptr(), dy.c_ptr())
+        got = []
+        for form in (-1, 0, 1, 2):
+            announce("row sums, form", form, shape, np.dtype(dtype).name)
+            dy.copy_from(y0)
+            assert lib.asamd_spmv_sums_form(None, byref(args), byref(layout), sums.c_ptr(), None, form) == 0
+            hiprt.synchronize()
+            got.append(dy.to_numpy())
+        _check(a, -1.5, x, 0.5, y0, got[0], shape)
+        for y in got[1:]:
+            assert np.array_equal(y, got[0])
+        for form in (-2, 3):
+            assert lib.asamd_spmv_sums_form(None, byref(args), byref(layout), sums.c_ptr(), None, form) == 1
+    finally:
+        lib.asamd_sums_free(byref(layout))
+        for d in (dx, dy, sums, da):
+            if d:
+                d.free()
 
 
 def test_slots_without_an_entry_leave_nothing_behind(gpu):
