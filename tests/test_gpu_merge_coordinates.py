@@ -13,9 +13,11 @@ pytestmark = pytest.mark.gpu
 
 LENGTHS = {
     "one workgroup": [3] * 100,
-    "edge of two": [1] * 1024,            # rows + entries: exactly two workgroups of 1 024 items, one of 2 048
+    "edge of two": [1] * 1024,            # rows + entries: exactly two workgroups of 1 024 items, one of eight per thread
     "one item more": [1] * 1024 + [0],
     "one item less": [1] * 1023 + [0],
+    "edge of four": [1] * 2048,           # the same for 2 048 items
+    "one item past four": [1] * 2048 + [0],
     "65 rows": [0] * 64 + [5000],
     "empty runs": [0] * 3000 + [7000] + [0] * 5000 + [1, 0, 2, 4096, 0] * 3 + [0] * 2000,
     "nothing but a long row": [20000],
@@ -23,10 +25,13 @@ LENGTHS = {
 }
 
 
-@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("dtype,items", [(np.float32, None), (np.float64, None), (np.float32, 8)], ids=["f32", "f64", "f32_8"])
 @pytest.mark.parametrize("base", [0, 1])
 @pytest.mark.parametrize("shape", list(LENGTHS))
-def test_workgroups_find_their_coordinates(gpu, shape, base, dtype):
+def test_workgroups_find_their_coordinates(gpu, shape, base, dtype, items, monkeypatch):
+    """items: per thread; 4-byte values take eight, in workgroups of 2 048, where they are more than 2^25."""
+    if items:
+        monkeypatch.setenv("ALSPARSE_AMD_MERGE_IPT", str(items))
     a = csr_from_lengths(LENGTHS[shape], 30000, dtype, base=base)
     x, y0 = wl.uniform(a.cols, dtype, 3), wl.uniform(a.rows, dtype, 4)
     da = DeviceCsr(a)

@@ -61,6 +61,32 @@ def test_noalloc_matches_existing_entry_points_on_two_calls_in_a_row(gpu):
     assert all(u == 0 for u in grew[1:]), grew
 
 
+@pytest.mark.parametrize("rows,items", [(1 << 21, 4), ((1 << 21) + 1, 8)], ids=["2^25 items", "more"])
+def test_noalloc_walks_as_the_plan_does(gpu, rows, items, monkeypatch):
+    """Up to 2^25 items four per thread and eight beyond, as the planned merge path: the same bits, and not those of the
+    other walk.  Sixteen items a row but for a few that cross many workgroups."""
+    lengths = np.full(rows, 15, np.int64)
+    lengths[[5, rows // 2, rows - 3]] = [30015, 15, 15]
+    lengths[6:2006] = 0  # (as many entries as before)
+    row_ptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    nnz, cols = int(row_ptr[-1]), 5000
+    assert nnz == 15 * rows
+    rng = np.random.default_rng(rows)
+    a = wl.Csr(rows, cols, row_ptr, rng.integers(0, cols, nnz, dtype=np.int32), wl.uniform(nnz, np.float32, 5), 0, "%d items" % (16 * rows))
+    x, y0 = wl.uniform(cols, a.dtype, 3), wl.uniform(rows, a.dtype, 4)
+    da = DeviceCsr(a)
+    try:
+        announce("noalloc", a.name)
+        y, _ = _noalloc(da, 1.25, x, 0.5, y0)
+        check_spmv(a, 1.25, x, 0.5, y0, y, "noalloc/%s" % a.name)
+        assert np.array_equal(y, run_plan_csrmv(da, "merge", 1.25, x, 0.5, y0))
+        for k in (4, 8):
+            monkeypatch.setenv("ALSPARSE_AMD_MERGE_IPT", str(k))
+            assert np.array_equal(y, run_plan_csrmv(da, "merge", 1.25, x, 0.5, y0)) == (k == items), k
+    finally:
+        da.free()
+
+
 def test_noalloc_zero_entries_scales_y(gpu):
     a = csr_from_lengths([0] * 777, 50, np.float32)
     y0 = wl.uniform(a.rows, a.dtype, 4)
