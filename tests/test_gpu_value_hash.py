@@ -75,3 +75,42 @@ def test_a_flag_gates_the_gather(gpu, flag, dtype):
     finally:
         for x in d:
             x.free()
+
+
+@pytest.mark.parametrize("words", [5, 255, 70001, 2048 * 8 * 256 + 3])
+def test_the_refreshing_kernel_works_out_the_verdict(gpu, words):
+    """asamd_value_guard_begin leaves partial sums; the gather compares them with the recorded word in every workgroup, from one
+    to as many as it launches, refreshes or does not, and leaves word and flag for the kernels behind and for the record."""
+    lib = capi.load()
+    rng = np.random.default_rng(words)
+    host, perm = rng.standard_normal(words).astype(np.float32), rng.permutation(words).astype(np.uint32)
+    want = _fingerprint(host.view(np.uint32), 64)
+    d, dp = hiprt.DeviceArray.from_numpy(host), hiprt.DeviceArray.from_numpy(perm)
+    ws, out, second = hiprt.DeviceArray((GUARD_BYTES // 8,), np.uint64), hiprt.DeviceArray((words,), np.float32), hiprt.DeviceArray((words,), np.float32)
+    stored = hiprt.DeviceArray.from_numpy(np.zeros(1, np.uint64))
+    old = np.full(words, 3, np.float32)
+    try:
+        for recorded, changed in ((want ^ 1, 1), (want, 0)):
+            announce("verdict", words, changed)
+            ws.copy_from(rng.integers(0, 1 << 63, GUARD_BYTES // 8).astype(np.uint64))
+            stored.copy_from(np.array([recorded], np.uint64))
+            out.copy_from(old)
+            second.copy_from(old)
+            check = capi.asamd_value_check()
+            assert lib.asamd_value_guard_begin(None, d.c_ptr(), 4 * words, 0, stored.c_ptr(), ws.c_ptr(), ctypes.byref(check)) == 0
+            assert check.words == words and check.settled == 0
+            assert lib.asamd_gather_checked(None, 0, 0, words, dp.c_ptr(), d.c_ptr(), out.c_ptr(), ctypes.byref(check)) == 0
+            check.settled = 1
+            assert lib.asamd_gather_checked(None, 0, 0, words, dp.c_ptr(), d.c_ptr(), second.c_ptr(), ctypes.byref(check)) == 0
+            hiprt.synchronize()
+            assert int(stored.to_numpy()[0]) == recorded, "recorded before the copies are refreshed"
+            assert lib.asamd_value_guard_commit(None, ws.c_ptr(), stored.c_ptr()) == 0
+            hiprt.synchronize()
+            for got in (out, second):
+                assert np.array_equal(got.to_numpy(), host[perm] if changed else old)
+            state = ws.to_numpy()
+            assert int(state[2048]) == want and state[2049:2050].view(np.int32)[0] == changed
+            assert int(stored.to_numpy()[0]) == want
+    finally:
+        for x in (d, dp, ws, out, second, stored):
+            x.free()

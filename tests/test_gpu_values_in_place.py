@@ -322,6 +322,74 @@ def test_one_analysis_from_two_handles_at_once(gpu, shape, monkeypatch):
         da.free()
 
 
+@pytest.mark.parametrize("shape,op", [("tiled", 0), ("row_sums", 0), ("row_sums", 1)])
+def test_two_handles_find_new_values_at_once(gpu, shape, op, monkeypatch):
+    """csr_val rewritten between products that two streams make with ONE info: both find the change, or one of them finds the
+    copy refreshed by the other, and every product is that of the new values -- the same bits as one made alone."""
+    lib, hip = capi.load(), hiprt.lib()
+    monkeypatch.setenv("ALSPARSE_AMD_ROW_SUMS", "1" if shape == "row_sums" else "0")
+    a = wl.uniform_rows(1 << 21, 1 << 21, 16, np.float32)
+    da = DeviceCsr(a)
+    info = capi.alphasparse_dcu_mat_info_t()
+    assert lib.alphasparse_dcu_create_mat_info(byref(info)) == 0
+    descr = capi.make_descr(base=a.base)
+    handles, streams = [capi.Handle(), capi.Handle()], [c_void_p(), c_void_p()]
+    x = wl.uniform(a.cols, a.dtype, 10)
+    dx = hiprt.DeviceArray.from_numpy(x)
+    dys = [hiprt.DeviceArray.from_numpy(np.zeros(a.rows, a.dtype)) for _ in range(2)]
+    alpha, beta = ctypes.c_float(1.25), ctypes.c_float(0.0)
+    try:
+        announce("two handles, new values", shape, op)
+        for i in range(2):
+            hiprt.check(hip.hipStreamCreate(byref(streams[i])), "hipStreamCreate")
+            assert lib.asamd_handle_set_stream(handles[i].h, streams[i]) == 0
+        operation = capi.ALPHA_SPARSE_OPERATION_TRANSPOSE if op else capi.ALPHA_SPARSE_OPERATION_NON_TRANSPOSE
+        assert lib.alphasparse_dcu_s_csrmv_analysis(handles[0].h, operation, a.rows, a.cols, a.nnz, byref(descr), da.val.c_ptr(),
+                                                    da.row_ptr.c_ptr(), da.col.c_ptr(), info) == 0
+        if not op:
+            assert lib.asamd_analysis_stats(info).contents.row_sums == (shape == "row_sums")
+
+        def multiply(i, reps):
+            for _ in range(reps):
+                st = lib.alphasparse_dcu_s_csrmv(handles[i].h, operation, a.rows, a.cols, a.nnz, byref(alpha), byref(descr),
+                                                 da.val.c_ptr(), da.row_ptr.c_ptr(), da.col.c_ptr(), info, dx.c_ptr(),
+                                                 byref(beta), dys[i].c_ptr())
+                assert st == 0, st
+
+        for i in range(2):  # (the handles' buffers grow here)
+            multiply(i, 1)
+            hiprt.synchronize()
+        alone = None
+        for rep in range(4):
+            b = _with_values(a, _new_values(a, 40 + rep))
+            da.val.copy_from(b.values)
+            hiprt.synchronize()
+            threads = [threading.Thread(target=multiply, args=(i, 1 + 2 * i)) for i in range(2)]
+            for t in threads:
+                t.start()
+            for t in threads:
+                t.join()
+            hiprt.synchronize()
+            together = [d.to_numpy() for d in dys]
+            if op == 0 or rep == 3:  # (the oracle's transpose takes seconds)
+                _check(b, op, 1.25, x, 0.0, np.zeros(a.rows, a.dtype), together[0], "new values %d" % rep)
+            multiply(0, 1)
+            hiprt.synchronize()
+            before, alone = alone, dys[0].to_numpy()
+            assert before is None or not np.array_equal(before, alone)
+            for i in range(2):
+                assert np.array_equal(together[i], alone), "handle %d, values %d" % (i, rep)
+    finally:
+        lib.alphasparse_dcu_destroy_mat_info(info)
+        for i in range(2):
+            handles[i].close()
+            if streams[i]:
+                hip.hipStreamDestroy(streams[i])
+        for d in dys + [dx]:
+            d.free()
+        da.free()
+
+
 def test_host_pointer_mv_notices_one_changed_value_and_a_changed_structure(gpu):
     """alphasparse_d_mv reads the caller's host arrays on every call in the reference, so a single value poked
     through alphasparse_d_export_csr's pointers counts from the next call on, and so does an edited column."""
