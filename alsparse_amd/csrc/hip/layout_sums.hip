@@ -365,10 +365,14 @@ extern "C" int asamd_spmv_sums_form(hipStream_t s, const asamd_spmv_args* a, con
     };
     // Sums that the memory-side cache could not hold are stored past it, as the tiled pair's products.  Where it holds the
     // sums, but not the values and columns beside them, those are loaded past it, so that the second phase finds the sums
-    // there: us, plain / past it, inputs of three matrices in turn: power law of 8 M rows fp32 331 / 307, uniform 1 M x 16
-    // fp64 (transposed, 270 MB of streams and sums) 117 / 112, 2 M x 20 fp32 144 / 141, 2 M x 20 complex128 456 / 441.  One
-    // matrix again and again is served from that cache where it fits: power law of 2 M rows (181 MB) 80 / 85, uniform 1 M x
-    // 20 fp32 (190 MB) 83 / 88.
+    // there.  us, plain / past it, three matrices in turn and one again and again (which that cache serves where it fits):
+    //   power law fp32, 2.1 M rows (167 MB)  59.0 / 55.8  51.9 / 56.6     uniform x 16 fp64, 0.70 M (188 MB)  68.7 / 64.7  57.1 / 60.4
+    //     2.6 M (209 MB)  73.0 / 68.8  63.8 / 70.1                          0.85 M (230 MB)   83.2 / 79.4  79.3 / 74.3
+    //     3.0 M (243 MB)  83.5 / 78.2  72.6 / 77.6                          0.95 M (259 MB)   90.3 / 87.0  81.4 / 78.7
+    //     3.3 M (270 MB)  89.3 / 84.9  80.6 / 81.6                        uniform x 16 fp32, 1.6 M (242 MB)  84.6 / 80.2  75.9 / 76.3
+    //     3.8 M (312 MB)  102 / 99.0  100 / 97.6                            1.8 M (274 MB)    96.4 / 94.0  91.5 / 88.5
+    //     4.5 M (384 MB)  123 / 118  118 / 110                              4.2 M (656 MB)    230 / 215  229 / 217
+    // The line lies where one matrix again and again stops losing.
     const int64_t sum_bytes = (int64_t)L->sums * (int64_t)sizeof(T);
     const int64_t stream_bytes = (int64_t)L->spans * SumsDims<T>::span * ((int64_t)sizeof(T) + 2);
     const int by_size = sum_bytes > ((int64_t)512 << 20) ? 2 : sum_bytes + stream_bytes > (int64_t)256000000 ? 1 : 0;

@@ -342,8 +342,9 @@ static hipError_t build_tiled(hipStream_t stream, asamd_tiled_layout* L, const i
   // ---- 4. phase-1 work list: every column block cut into even chunks of 32 K to 96 K entries (tile_chunks.hpp),
   // neighbours on one XCD, whose L2 then has the x slice; where the products are stored past the caches, into chunks of 48 K
   // and what is left, neighbours on different XCDs.  us, the second / the first: uniform columns, fp32, 4.4 M x 4.4 M x 6
-  // 130 / 120, 8.7 M x 6 263 / 249, 14 M x 9 577 / 550, fp64, 5 M x 10 373 / 357; past the caches, 16 M x 16 fp32 889 / 903,
-  // 4 M x 40 498 / 494 (a long run of rounds, whose last one matters little, and streams that are all there is).
+  // 130 / 120, 8.7 M x 6 263 / 249, 14 M x 9 577 / 550, fp64, 5 M x 10 373 / 357; past the caches, 16 M x 16 fp32 889 / 903
+  // and, in another run, 874 / 875, 4 M x 40 498 / 494: no difference that two runs do not show (a long run of rounds, whose
+  // last one matters little, and streams that are all there is), so those layouts stay as they were.
   if (e == hipSuccess) {
     constexpr int kUnit = 1024;
     const bool even = (int64_t)nnz_i * (int64_t)sizeof(T) <= kTiledPastCache;

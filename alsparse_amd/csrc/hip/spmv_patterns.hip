@@ -69,12 +69,16 @@ extern "C" int asamd_spmv_patterns(hipStream_t s, const asamd_spmv_args* a, cons
   if (!a || !L || !L->pid || !L->dist || !L->block_off) return hipErrorInvalidValue;
   static const int forced = getenv("ALSPARSE_AMD_STREAM_POLICY") ? atoi(getenv("ALSPARSE_AMD_STREAM_POLICY")) : -1;
   // us per multiply, the same arrays again and again / four sets in turn, values cached against not:
-  //   5-point Laplacian 2048^2, fp64 (256 MB)      34 / 50 against 41 / 50     fp32 (138 MB)    22 / 32 against 28 / 28
-  //   27-point stencil 101 x 100 x 97, fp64 (231 MB)  33 / 51 against 47 / 47  complex64 the same
-  //   5-point Laplacian 3000 x 3001, fp64 (549 MB)    106 / 106 against 87 / 107
-  //   27-point stencil 160^3, fp32 (489 MB)           112 / 111 against 106 / 105
+  //   5-point Laplacian 2048^2, fp64 (256 MB)      34 / 47 against 40 / 44     fp32 (138 MB)    20 / 28 against 26 / 26
+  //   27-point stencil 101 x 100 x 97, fp64 (231 MB)  35 / 49 against 45 / 46
+  //   5-point Laplacian 2900 x 2901, fp32 (278 MB)    40 / 57 against 48 / 56
+  //   27-point stencil 110^3, fp64 (314 MB)           60 / 68 against 64 / 65
+  //   5-point Laplacian 2300 x 2301, fp64 (323 MB)    51 / 58 against 49 / 59
+  //   5-point Laplacian 3000 x 3001, fp64 (549 MB)    94 / 94 against 81 / 94
+  //   27-point stencil 160^3, fp32 (489 MB)           105 / 105 against 99 / 101
   // What the memory-side cache holds, or nearly, is left there for the next multiply; more than that only pushes the
-  // rest out of it.
+  // rest out of it.  (Five bytes a row, a pattern's number and four of row_ptr, which the kernel no longer reads: the lines
+  // below were drawn in these bytes.)
   const double bytes = (double)a->nnz * dtype_size(a->dtype) + 5.0 * (double)a->m +
                        ((double)a->m + (double)a->n) * dtype_size(a->dtype);
   const bool ntv = forced >= 0 ? (forced & kStreamNtValues) != 0 : bytes > 280.0e6;

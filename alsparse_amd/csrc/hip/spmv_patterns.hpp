@@ -9,9 +9,9 @@
 // The structure is promised fixed (analysed matrices only); values stay in the caller's array.
 //
 // Bound by memory.  us per multiply over four matrices in turn, before (32-bit columns, 16-bit distances or the ELL copy,
-// whichever the analysis kept) and now: 5-point Laplacian 2048^2 fp64 67.4 -> 47.1 (239 MB moved, 5.1 TB/s), fp32
-// 49.6 -> 30.0; 27-point stencil of 101 x 100 x 97 points complex64 72.5 -> 48.6, fp64 69.9 -> 48.7; of 160^3 points fp32
-// 179 -> 102; of 60 x 50 x 47 points fp32 10.7 -> 6.1.  Rows far shorter than the longest, and small matrices, stay with
+// whichever the analysis kept) and now: 5-point Laplacian 2048^2 fp64 67.4 -> 47.0 (239 MB moved, 5.1 TB/s), fp32
+// 49.6 -> 27.7; 27-point stencil of 101 x 100 x 97 points complex64 72.5 -> 48.6, fp64 69.9 -> 49.0; of 160^3 points fp32
+// 179 -> 101; of 60 x 50 x 47 points fp32 10.7 -> 6.2.  Rows far shorter than the longest, and small matrices, stay with
 // the columns (patterns_pay in plan.c).  16-byte values: the ELL copy stays
 // ahead (5-point Laplacian of 2.1 M rows 58.7 against 84.4).
 //

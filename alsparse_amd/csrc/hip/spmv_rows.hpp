@@ -81,7 +81,7 @@ __global__ __launch_bounds__(kRowsBlock) void spmv_vector_kernel(
 
 // The same with the values where they lie in another array: entry j of a row is val[perm[j]] (CONJ: its conjugate).  The
 // small transposed product: of the copy of A^T it reads the structure only, so nothing has to check that the copy's values
-// are still the caller's (the check is four launches; they are most of a small multiply).
+// are still the caller's (the check is two launches; they are most of a small multiply).
 template <typename T, int W, bool CONJ>
 __global__ __launch_bounds__(kRowsBlock) void spmv_permuted_kernel(
     int m, T alpha, const T* __restrict__ val, const unsigned* __restrict__ perm, const int* __restrict__ row_ptr,

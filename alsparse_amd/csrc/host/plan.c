@@ -795,9 +795,10 @@ static void fill_args(asamd_spmv_args *a, const asamd_csr_plan *p, const void *a
 }
 
 /* Small transposed products read the caller's values through the copy's permutation: one launch (two where a few rows of
- * A^T are long) where the check of the copy's values is four of their own, and nothing to check.  us per call, this / the
- * checked copy: 30 000 to 120 000 entries 4.6 / 18, 500 000 scattered ones 14-16 / 18-19, 1 000 000 27-30 / 19-25 (every
- * value then moves a cache line of its own), a power law of 60 000 rows 15 / 28.  With ALSPARSE_AMD_VALUE_CHECK=off the copy
+ * A^T are long) where the check of the copy's values is two of their own, and nothing to check.  us per call, this / the
+ * checked copy: 30 000 to 120 000 entries 5.4 / 14.5, 200 000 6.2 / 14.6, 300 000 8.9 / 14.7, 480 000 12 / 15.4, 500 000
+ * scattered ones 14.5-15.5 / 14.3-15.5, where the two meet (every value moves a cache line of its own: 1 000 000 27-30),
+ * a power law of 60 000 rows 14.7 / 20.  With ALSPARSE_AMD_VALUE_CHECK=off the copy
  * costs its multiply alone and is the faster one from 200 000 entries on (uniform 20 000 x 20 000 x 10 5.4 / 4.5, 40 000 x
  * 40 000 x 12 11.7 / 4.6, power law 12.6 / 9.4; level below): only another value array, which it does not hold, comes here. */
 #define PERMUTED_MOST (1 << 19)
@@ -1134,8 +1135,8 @@ static hipError_t tune_copies(hipStream_t stream, asamd_csr_plan *p, const int32
   st->tune_ms_hot = t.best[CAND_HOT];
   /* a copy has to win by a margin to be worth its memory; among the winners the fastest is kept */
   const float margin[CAND_COUNT] = {1.f, 0.9f, 0.95f, 0.95f, 0.95f};
-  /* (the timing runs launch the kernels alone: a copy that holds values is multiplied behind the value guard's four
-   * small launches later on, and is compared with them counted) */
+  /* (the timing runs launch the kernels alone: a copy that holds values is multiplied behind the value guard's two to
+   * four small launches later on, and is compared with them counted) */
   float cost[CAND_COUNT];
   for (int c = 0; c < CAND_COUNT; ++c)
     cost[c] = t.best[c] + (t.best[c] > 0.f && (c == CAND_TILED || c == CAND_ELL) && st->value_check && !p->watched ? 0.022f : 0.f);
@@ -1221,7 +1222,8 @@ static double model_ms(const asamd_csr_plan *p, int algo) {
       if (vs >= 16.0 && rate > 4.2) rate = 4.2;
       /* 16-bit distances for columns: half of the bytes they save shows (27-point stencil, 160^3 points: 0.204 ->
        * 0.181 ms with 4-byte values, 0.300 -> 0.274 with 8-byte ones) */
-      /* a pattern number per row for the columns: the values, row_ptr, the numbers, x and y are what is left */
+      /* a pattern number per row for the columns: the values, the numbers, x and y are what is left (row_ptr is counted too,
+       * as when the rate was fitted: the kernel read it then) */
       if (p->pat.pid) return hypot2((bytes - 4.0 * nnz + m) / 6.2e9, 0.5 * gather);
       if (p->d_rel16) return hypot2((bytes - 1.0 * nnz) / (rate * 1e9), gather);
       break;
@@ -1321,8 +1323,10 @@ static hipError_t model_copies(hipStream_t stream, asamd_csr_plan *p, const int3
   st->algo = p->auto_algo;
   st->tune_ms_base = (float)base;
   /* the copies in the order of their estimates; each is laid out only if it is the best one left */
-  /* a copy that holds values is multiplied behind the value guard: four small launches, 22-30 us (27-point stencil
-   * on 128 x 128 x 64 points: the ELL kernel 0.041 ms, the guarded multiply 0.057, the staged row blocks 0.046) */
+  /* a copy that holds values is multiplied behind the value guard, which the constant puts at the 22 us that its four
+   * launches took when the estimates were fitted (27-point stencil on 128 x 128 x 64 points: the ELL kernel 0.041 ms, the
+   * guarded multiply 0.057, the staged row blocks 0.046).  It takes less now: 15 us in front of the ELL copy, still four
+   * launches (5-point Laplacian 2048^2 complex128 96.8 -> 111.7), 13 to 15 in front of the tiled one, two launches less */
   const double guard_ms = st->value_check && !p->watched ? 0.022 : 0.0;
   const double est_tiled = tiled_ok ? model_ms(p, ASAMD_SPMV_TILED) + guard_ms : 0.0;
   const double est_ell = ell_ok ? model_ms(p, ASAMD_SPMV_ELL) + guard_ms : 0.0;
@@ -1425,11 +1429,13 @@ static hipError_t model_copies(hipStream_t stream, asamd_csr_plan *p, const int3
  * with power-law rows and columns (1.1 .. 8.4 M rows, P = sums per entry = 0.31 .. 0.46), power-law rows over uniform
  * columns, two and geometric row lengths, uniform rows of 3 .. 128 entries over 2 .. 64 MB of x, all types: 0.03 ms
  * (the value guard's launches, two phases' ramps) and 4.65 TB/s, 4.9 from 4 GB on; the estimate is within a tenth of 40 of 46
- * timings and within 17 % of all, the families' are within a quarter.  Before -> with them, the check included, us:
- *   power law, 8.4 M rows: fp32 527 -> 323, 2.1 M rows 124 -> 87; 1.1 M rows 62 -> 60 (not laid out)
- *   uniform rows, fp32: 1 M x 1 M x 16 93 -> 79, x 32 189 -> 137, x 64 324 -> 170, 2 M x 2 M x 16 173 -> 142;
- *     4 M x 4 M x 16 285 -> 253 (not laid out), 16 M x 16 M x 16 853 -> 910 (next to no row meets a column block twice, and
- *     the tiled pair's are wider: not laid out); fp64: 1 M x 1 M x 16 161 -> 115, 2 M x 2 M x 64 1215 -> 649
+ * timings and within 17 % of all, the families' are within a quarter.  (Timings of the kernels as they then were: cut into
+ * chunks that fill rounds and loaded past the memory-side cache, the tiles take 5 to 25 % less than the estimate, which
+ * leaves matrices near the line with their family.)  Without -> with them, the check included, inputs in turn, us:
+ *   power law, 8.4 M rows: fp32 534 -> 291, 2.1 M rows 128 -> 81; 1.1 M rows 60 (not laid out)
+ *   uniform rows, fp32: 1 M x 1 M x 16 109 -> 75, x 32 209 -> 113, x 64 325 -> 148, 2 M x 2 M x 16 166 -> 114;
+ *     4 M x 4 M x 16 278 (not laid out; the tiles alone 215), 16 M x 16 M x 16 853 -> 910 (next to no row meets a column block
+ *     twice, and the tiled pair's are wider: not laid out); fp64: 1 M x 1 M x 16 165 -> 101, 2 M x 2 M x 64 1251 -> 671
  * A matrix that they serve keeps the copy of its family, for a family set from outside and for other value arrays; the
  * copy of A^T, which has neither, does not (drop_family). */
 static double sums_bytes(const asamd_csr_plan *p, double sums) {
@@ -1445,8 +1451,8 @@ static double sums_ms(const asamd_csr_plan *p, double sums) {
   return 0.03 + bytes / (rate * 1e9);
 }
 
-/* Every byte fingerprinted (sums_check_all): 0.21 ms for 1 GiB, arrays of up to 32 MiB are read whole anyway; the copy of A^T
- * stands behind the check of A's values. */
+/* Every byte fingerprinted (sums_check_all): 0.21 ms for 1 GiB when the line was drawn (388 MB take 64 us now), arrays of up to
+ * 32 MiB are read whole anyway; the copy of A^T stands behind the check of A's values. */
 static double sums_check_ms(const asamd_csr_plan *p) {
   const asamd_csr_stats *st = &p->st;
   const double beyond = (double)st->nnz * (double)p->val_size - (double)ASAMD_GUARD_FULL_BYTES;
